@@ -1,4 +1,4 @@
-"""Builds libcpmcu_amd.so (HIP kernels + C-ABI, gfx950) and the pybind11 module ``C`` in-tree.
+"""Builds libcpmcu_amd.so (HIP kernels + C-ABI, gfx950), the pybind11 module ``C`` and the torch binding ``_torch_call`` in-tree.
 
     python -m cpm.cu_amd.build [--force]
 
@@ -35,6 +35,20 @@ HIP_FLAGS = [
 
 def pybind_module_path():
     return os.path.join(HERE, "C" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def torch_call_path():
+    return os.path.join(HERE, "_torch_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def _torch_call_command(src, out):
+    """The binding of the operators to torch tensors: the only part that is compiled against torch's headers."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include",
+            "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", src, "-o", out, f"-L{root}/lib",
+            "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{root}/lib"]
 
 
 def _stale(target, deps):
@@ -74,13 +88,17 @@ def build_all(force=False, verbose=False):
                 jobs.append([HIPCC] + HIP_FLAGS + ["-DCPMCU_TIMELINE", "-c", s, "-o", o])
         else:
             tl_objs.append(os.path.join(OBJ_DIR, src.replace(".hip", ".o")))
+    call_src, call_mod = os.path.join(CSRC, "torch_call.cpp"), torch_call_path()
+    hip_jobs = len(jobs)
+    if force or _stale(call_mod, [call_src, os.path.join(INCLUDE, "cpmcu_amd.h")]):
+        jobs.append(_torch_call_command(call_src, call_mod))
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
         for out in ex.map(_run, jobs):
             if verbose and out.strip():
                 print(out)
-    if force or jobs or _stale(LIB_PATH, objs):
+    if force or hip_jobs or _stale(LIB_PATH, objs):
         _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", LIB_PATH] + objs)
-    if force or jobs or _stale(TIMELINE_LIB_PATH, tl_objs):
+    if force or hip_jobs or _stale(TIMELINE_LIB_PATH, tl_objs):
         _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", TIMELINE_LIB_PATH] + tl_objs)
     # pybind11 module `C`: the reference's entry-point names over the C-ABI
     import pybind11

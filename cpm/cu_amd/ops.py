@@ -1,7 +1,8 @@
 """The operators of the verify/draft path on torch device tensors.
 
 torch only supplies device memory and the current stream; every function here is a thin call into
-``libcpmcu_amd.so`` through the C-ABI (``include/cpmcu_amd.h``).  Nothing falls back to torch math.
+``libcpmcu_amd.so`` through the C-ABI (``include/cpmcu_amd.h``), made by the native binding
+``_torch_call``.  Nothing falls back to torch math.
 """
 import ctypes
 import math
@@ -11,28 +12,34 @@ import torch
 from . import lib as _libmod
 from .kvcache import HEAD_DIM
 
+_native = None
+
 
 def _lib():
     return _libmod.get()
 
 
-def _ptr(t):
-    if t is None:
-        return None
-    assert t.is_cuda and t.is_contiguous(), "device-resident contiguous tensor required"
-    return ctypes.c_void_p(t.data_ptr())
+def _calls():
+    """The library's operators as native calls on tensors (csrc/torch_call.cpp), bound to the library lib.py has loaded.
+    Pointer arguments are tensors (device-resident and contiguous, or AssertionError) or None; the stream is torch's current one."""
+    global _native
+    if _native is None:
+        lib = _libmod.get()
+        try:
+            from . import _torch_call
+        except ImportError as e:
+            raise ImportError("the torch binding is not built or does not fit this torch (%s); run `python -m cpm.cu_amd.build`" % e) from e
+        _torch_call.bind(lib.raw._handle)
+        _native = _torch_call
+    return _native
 
 
 def _ptr_result(t):
-    """Like _ptr, but a pinned host tensor may stand in: the GPU writes it through the mapped address."""
-    if t is None:
-        return None
-    assert (t.is_cuda or t.is_pinned()) and t.is_contiguous(), "device-resident or pinned contiguous tensor required"
-    return ctypes.c_void_p(t.data_ptr())
-
-
-def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """A device tensor, or the address of a pinned host tensor in its place: the GPU writes it through the mapped address."""
+    if t is None or t.is_cuda:
+        return t
+    assert t.is_pinned() and t.is_contiguous(), "device-resident or pinned contiguous tensor required"
+    return t.data_ptr()
 
 
 _workspaces = {}
@@ -65,17 +72,24 @@ def release_head_workspace(ws):
     _lib().head_release_workspace(ctypes.c_void_p(ws.data_ptr()))
 
 
+_SCALE = 1.0 / math.sqrt(HEAD_DIM)
+
+
+def synchronize():
+    """Wait for torch's current stream."""
+    (_native or _calls()).synchronize()
+
+
 def mask_words(T):
     return (T + 63) // 64
 
 
 def kv_append(cache, layer, k_new, v_new, kv_len):
     """copy_to_kvcache (src/model/attn.cuh:14-21): rows go to positions [*kv_len - T, *kv_len)."""
-    T = k_new.shape[0]
+    T, Hkv = k_new.shape[0], cache.Hkv
     assert k_new.dtype == torch.float16 and v_new.dtype == torch.float16 and kv_len.dtype == torch.int32
-    assert k_new.numel() == T * cache.Hkv * HEAD_DIM and v_new.numel() == k_new.numel()
-    _lib().kv_append(_ptr(cache.k[layer]), _ptr(cache.v[layer]), _ptr(cache.block_table), _ptr(k_new), _ptr(v_new),
-                     _ptr(kv_len), T, cache.Hkv, _stream())
+    assert k_new.numel() == T * Hkv * HEAD_DIM == v_new.numel()
+    (_native or _calls()).kv_append(cache.k[layer], cache.v[layer], cache.block_table, k_new, v_new, kv_len, T, Hkv)
 
 
 def rope_table(position_ids, inv_freq):
@@ -83,7 +97,7 @@ def rope_table(position_ids, inv_freq):
     T = position_ids.numel()
     assert position_ids.dtype == torch.int32 and inv_freq.dtype == torch.float32 and inv_freq.numel() == HEAD_DIM // 2
     out = torch.empty((T, HEAD_DIM // 2, 2), dtype=torch.float32, device=position_ids.device)
-    _lib().rope_table(_ptr(position_ids), _ptr(inv_freq), T, _ptr(out), _stream())
+    _calls().rope_table(position_ids, inv_freq, T, out)
     return out
 
 
@@ -91,7 +105,7 @@ def rope_apply_(table, q, k):
     """In-place rotary embedding of q [T,Hq,128] and k [T,Hkv,128] (rotary_embedding_kernel, src/model/rotary.cuh:7-34)."""
     T, Hq, D = q.shape
     assert D == HEAD_DIM and k.shape[0] == T and k.shape[2] == D and table.shape[0] == T
-    _lib().rope_apply(_ptr(table), T, Hq, k.shape[1], _ptr(q), _ptr(k), _stream())
+    _calls().rope_apply(table, T, Hq, k.shape[1], q, k)
 
 
 def tree_attention(q, cache, layer, kv_len, max_kv_len, mask=None, scale=None, num_splits=0, out=None,
@@ -108,38 +122,30 @@ def tree_attention(q, cache, layer, kv_len, max_kv_len, mask=None, scale=None, n
     """
     T, Hq, D = q.shape
     assert D == HEAD_DIM and q.dtype == torch.float16 and kv_len.dtype == torch.int32
+    native, Hkv, max_kv_len = _native or _calls(), cache.Hkv, int(max_kv_len)
     if out is None:
         out = torch.empty_like(q)
     W = 0
     if mask is not None:
-        assert mask.dtype in (torch.uint64, torch.int64)
-        mask = mask.reshape(T, -1)
+        assert mask.dtype == torch.int64 or mask.dtype == torch.uint64
+        if mask.dim() != 2 or mask.shape[0] != T:
+            mask = mask.reshape(T, -1)
         W = mask.shape[1]
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
-    need = _lib().raw.cpmcu_tree_attention_workspace_bytes(T, Hq, cache.Hkv, int(max_kv_len))
-    ws = _workspace("attn", need, q.device)
+    ws = _workspace("attn", native.tree_attention_workspace_bytes(T, Hq, Hkv, max_kv_len), q.device)
     if k_new is not None:
         assert k_new.dtype == torch.float16 and v_new.dtype == torch.float16
-        assert k_new.numel() == T * cache.Hkv * HEAD_DIM and v_new.numel() == k_new.numel()
+        assert k_new.numel() == T * Hkv * HEAD_DIM == v_new.numel()
+    head = (q, cache.k[layer], cache.v[layer], cache.block_table, kv_len, max_kv_len, k_new, v_new)
+    tail = (mask, W, int(mask_k_range), T, Hq, Hkv, _SCALE if scale is None else scale, out, ws, ws.numel(), int(num_splits))
     if rope is not None:
         assert rope.dtype == torch.float32 and rope.numel() == T * HEAD_DIM
     if block_window_size:
-        _lib().tree_attention_window(_ptr(q), _ptr(cache.k[layer]), _ptr(cache.v[layer]), _ptr(cache.block_table), _ptr(kv_len),
-                                     int(max_kv_len), _ptr(k_new), _ptr(v_new), _ptr(rope), int(block_window_size), _ptr(mask), W,
-                                     int(mask_k_range), T, Hq, cache.Hkv, ctypes.c_float(scale), _ptr(out), _ptr(ws), ws.numel(),
-                                     int(num_splits), _stream())
-        return out
-    if rope is not None:
+        native.tree_attention_window(*head, rope, int(block_window_size), *tail)
+    elif rope is not None:
         # rotary embedding of q and of the appended K rows fused into the kernel (table from rope_table)
-        _lib().tree_attention_rope(_ptr(q), _ptr(cache.k[layer]), _ptr(cache.v[layer]), _ptr(cache.block_table), _ptr(kv_len),
-                                   int(max_kv_len), _ptr(k_new), _ptr(v_new), _ptr(rope), _ptr(mask), W, int(mask_k_range), T, Hq,
-                                   cache.Hkv, ctypes.c_float(scale), _ptr(out), _ptr(ws), ws.numel(), int(num_splits), _stream())
-        return out
-    _lib().tree_attention(_ptr(q), _ptr(cache.k[layer]), _ptr(cache.v[layer]), _ptr(cache.block_table), _ptr(kv_len),
-                          int(max_kv_len), _ptr(k_new), _ptr(v_new), _ptr(mask), W, int(mask_k_range), T, Hq, cache.Hkv,
-                          ctypes.c_float(scale), _ptr(out),
-                          _ptr(ws), ws.numel(), int(num_splits), _stream())
+        native.tree_attention_rope(*head, rope, *tail)
+    else:
+        native.tree_attention(*head, *tail)
     return out
 
 
@@ -147,7 +153,7 @@ def gather_rows(src, remap):
     """remap_copy (src/model/tree_drafter.cuh:79-86): dst[r] = src[remap[r]]."""
     assert src.dtype == torch.float16 and remap.dtype == torch.int32
     dst = torch.empty((remap.numel(), src.shape[1]), dtype=torch.float16, device=src.device)
-    _lib().gather_rows(_ptr(src), _ptr(remap), remap.numel(), src.shape[1], _ptr(dst), _stream())
+    _calls().gather_rows(src, remap, remap.numel(), src.shape[1], dst)
     return dst
 
 
@@ -171,7 +177,7 @@ def tile_head_weight(w, row_remap=None):
     H = w.shape[1]
     V = w.shape[0] if row_remap is None else row_remap.numel()
     out = torch.empty(_lib().raw.cpmcu_head_weight_tiled_bytes(V, H) // 2, dtype=torch.float16, device=w.device)
-    _lib().head_weight_tile(_ptr(w), _ptr(row_remap), V, H, _ptr(out), _stream())
+    _calls().head_weight_tile(w, row_remap, V, H, out)
     return TiledWeight(out, V, H)
 
 
@@ -188,15 +194,10 @@ def frspec_head_topk(hidden, w, token_id_remap, k):
     """
     n, H = hidden.shape
     w, layout, V = _weight(w)
-    dev = hidden.device
-    logits = torch.empty((n, V), dtype=torch.float16, device=dev)
-    stats = torch.empty((n, 2), dtype=torch.float32, device=dev)
-    val = torch.empty((n, k), dtype=torch.float16, device=dev)
-    pos = torch.empty((n, k), dtype=torch.int32, device=dev)
-    ids = torch.empty((n, k), dtype=torch.int32, device=dev)
-    ws = _workspace("head", _lib().raw.cpmcu_head_workspace_bytes(n, V), dev)
-    _lib().frspec_head_topk(_ptr(hidden), _ptr(w), layout, _ptr(token_id_remap), n, V, H, k, _ptr(logits), _ptr(stats),
-                            _ptr(val), _ptr(pos), _ptr(ids), _ptr(ws), ws.numel(), _stream())
+    native = _native or _calls()
+    logits, stats, val, pos, ids = native.empty(hidden, "h", n, V, "f", n, 2, "h", n, k, "i", n, k, "i", n, k)
+    ws = _workspace("head", native.head_workspace_bytes(n, V), hidden.device)
+    native.frspec_head_topk(hidden, w, layout, token_id_remap, n, V, H, k, logits, stats, val, pos, ids, ws, ws.numel())
     return dict(logits=logits, row_stats=stats, val=val, pos=pos, ids=ids)
 
 
@@ -218,14 +219,13 @@ def lm_head_argmax(hidden, w, head_scale=None, want_logits=False, gt=None):
     """Target head + arg-max (src/model/linear.cuh:82-101 + torch argmax of tree_drafter.py:233)."""
     n, H = hidden.shape
     w, layout, V = _weight(w)
-    dev = hidden.device
-    logits = torch.empty((n, V), dtype=torch.float16, device=dev) if want_logits else None
+    native = _native or _calls()
+    logits = native.empty(hidden, "h", n, V)[0] if want_logits else None
     if gt is None:
-        gt = torch.empty(n, dtype=torch.int32, device=dev)
-    ws = _workspace("head", _lib().raw.cpmcu_head_workspace_bytes(n, V), dev)
-    _lib().lm_head_argmax(_ptr(hidden), _ptr(w), layout, n, V, H, 0 if head_scale is None else 1,
-                          ctypes.c_float(1.0 if head_scale is None else head_scale), _ptr(logits), _ptr(gt),
-                          _ptr(ws), ws.numel(), _stream())
+        gt = torch.empty(n, dtype=torch.int32, device=hidden.device)
+    ws = _workspace("head", native.head_workspace_bytes(n, V), hidden.device)
+    native.lm_head_argmax(hidden, w, layout, n, V, H, 0 if head_scale is None else 1, 1.0 if head_scale is None else head_scale, logits, gt,
+                          ws, ws.numel())
     return (gt, logits) if want_logits else gt
 
 
@@ -240,12 +240,11 @@ def lm_head_partials(hidden, w, head_scale=None, logits=None):
     """The target head's GEMM without the launch that finishes its arg-max; see verify_tail."""
     n, H = hidden.shape
     w, layout, V = _weight(w)
-    ws = _workspace("head", _lib().raw.cpmcu_head_workspace_bytes(n, V), hidden.device)
-    num, stride = ctypes.c_int(0), ctypes.c_int(0)
-    _lib().lm_head_partials(_ptr(hidden), _ptr(w), layout, n, V, H, 0 if head_scale is None else 1,
-                            ctypes.c_float(1.0 if head_scale is None else head_scale), _ptr(logits), _ptr(ws), ws.numel(),
-                            ctypes.byref(num), ctypes.byref(stride), _stream())
-    return HeadPartials(ws, num.value, stride.value, n)
+    native = _native or _calls()
+    ws = _workspace("head", native.head_workspace_bytes(n, V), hidden.device)
+    num, stride = native.lm_head_partials(hidden, w, layout, n, V, H, 0 if head_scale is None else 1,
+                                          1.0 if head_scale is None else head_scale, logits, ws, ws.numel())
+    return HeadPartials(ws, num, stride, n)
 
 
 def verify_tail(cache, draft_ids, gt, position_ids, cache_length, attn_mask, tree_parent, hidden=None, prev_hidden=None,
@@ -257,42 +256,41 @@ def verify_tail(cache, draft_ids, gt, position_ids, cache_length, attn_mask, tre
     W = attn_mask.numel() // T
     parts = gt if isinstance(gt, HeadPartials) else None
     hidden_dim = 0 if hidden is None else hidden.shape[-1]
-    _lib().verify_tail(_ptr(cache.k_ptrs), _ptr(cache.v_ptrs), cache.num_layers, _ptr(cache.block_table), cache.Hkv, T,
-                       _ptr(draft_ids), None if parts else _ptr(gt), _ptr(parts.workspace) if parts else None,
-                       parts.num_partials if parts else 0, parts.stride if parts else 0, _ptr(position_ids), _ptr(cache_length),
-                       _ptr(attn_mask), W, _ptr(tree_parent), _ptr(hidden), hidden_dim, _ptr(prev_hidden), _ptr(gt_out), _ptr(best),
-                       _ptr(path), _ptr(accepted_ids), _ptr(next_position_ids), _ptr_result(result), _stream())
+    (_native or _calls()).verify_tail(
+        cache.k_ptrs, cache.v_ptrs, cache.num_layers, cache.block_table, cache.Hkv, T, draft_ids, None if parts else gt,
+        parts.workspace if parts else None, parts.num_partials if parts else 0, parts.stride if parts else 0, position_ids, cache_length,
+        attn_mask, W, tree_parent, hidden, hidden_dim, prev_hidden, gt_out, best, path, accepted_ids, next_position_ids, _ptr_result(result))
 
 
 def verify_tail_inplace(best, accepted_ids, pred=None, cache_length=None, kv_len=None, position_ids=None, advance_length=False,
                         next_root=False):
     """The in-place updates behind verify_tail: pred[:a] <- ids (or pred[0] <- last id), lengths and positions += a."""
     flags = (COMMIT_ADVANCE_LENGTH if advance_length else 0) | (COMMIT_NEXT_ROOT if next_root else 0)
-    _lib().verify_tail_inplace(_ptr(best), _ptr(accepted_ids), accepted_ids.numel(), _ptr(pred), _ptr(cache_length), _ptr(kv_len),
-                               _ptr(position_ids), flags, _stream())
+    _calls().verify_tail_inplace(best, accepted_ids, accepted_ids.numel(), pred, cache_length, kv_len, position_ids, flags)
 
 
 def log_softmax_(x):
     """In place (src/model/eagle.cuh:29-89); returns row_stats [n,2] (max, ln sum)."""
     n, dim = x.shape
-    stats = torch.empty((n, 2), dtype=torch.float32, device=x.device)
-    _lib().log_softmax(_ptr(x), n, dim, _ptr(stats), _stream())
+    native = _native or _calls()
+    stats, = native.empty(x, "f", n, 2)
+    native.log_softmax(x, n, dim, stats)
     return stats
 
 
 def topk(x, top):
     """TopK::prefill (src/model/topk.cuh:255-288): value descending, ties -> lower index."""
     n, dim = x.shape
-    val = torch.empty((n, top), dtype=torch.float16, device=x.device)
-    pos = torch.empty((n, top), dtype=torch.int32, device=x.device)
-    ws = _workspace("topk", _lib().raw.cpmcu_topk_workspace_bytes(n, dim, top), x.device)
-    _lib().topk(_ptr(x), n, dim, top, _ptr(val), _ptr(pos), _ptr(ws), ws.numel(), _stream())
+    native = _native or _calls()
+    val, pos = native.empty(x, "h", n, top, "i", n, top)
+    ws = _workspace("topk", native.topk_workspace_bytes(n, dim, top), x.device)
+    native.topk(x, n, dim, top, val, pos, ws, ws.numel())
     return val, pos
 
 
 def remap(pos, token_id_remap):
     out = torch.empty_like(pos)
-    _lib().remap(_ptr(pos), pos.numel(), _ptr(token_id_remap), _ptr(out), _stream())
+    _calls().remap(pos, pos.numel(), token_id_remap, out)
     return out
 
 
@@ -302,15 +300,13 @@ def tree_accept(pred, gt, position_ids, cache_length, attn_mask, tree_parent, be
     if best is None:
         best = torch.empty(2, dtype=torch.int32, device=pred.device)
     W = attn_mask.numel() // T
-    _lib().tree_accept(T, _ptr(pred), _ptr(gt), _ptr(position_ids), _ptr(cache_length), _ptr(attn_mask), W,
-                       _ptr(tree_parent), _ptr(best), _stream())
+    _calls().tree_accept(T, pred, gt, position_ids, cache_length, attn_mask, W, tree_parent, best)
     return best
 
 
 def kv_compact(cache, pred, gt, cache_length, best, max_accept):
     """fix_kv_cache (src/model/tree_drafter.cuh:48-77) on every layer of the paged cache."""
-    _lib().kv_compact(_ptr(cache.k_ptrs), _ptr(cache.v_ptrs), cache.num_layers, _ptr(cache.block_table), cache.Hkv,
-                      _ptr(pred), _ptr(gt), _ptr(cache_length), _ptr(best), int(max_accept), _stream())
+    _calls().kv_compact(cache.k_ptrs, cache.v_ptrs, cache.num_layers, cache.block_table, cache.Hkv, pred, gt, cache_length, best, int(max_accept))
 
 
 def accept_commit(cache, pred, gt, cache_length, best, max_accept, hidden=None, prev_hidden=None,
@@ -320,9 +316,8 @@ def accept_commit(cache, pred, gt, cache_length, best, max_accept, hidden=None, 
     device-side advance of cache_length, in two launches with the accept length staying on the device."""
     flags = (COMMIT_ADVANCE_LENGTH if advance_length else 0) | (COMMIT_NEXT_ROOT if next_root else 0)
     hidden_dim = 0 if hidden is None else hidden.shape[-1]
-    _lib().accept_commit(_ptr(cache.k_ptrs), _ptr(cache.v_ptrs), cache.num_layers, _ptr(cache.block_table), cache.Hkv,
-                         _ptr(pred), _ptr(gt), _ptr(cache_length), _ptr(kv_len), _ptr(best), int(max_accept), _ptr(hidden), hidden_dim,
-                         _ptr(prev_hidden), _ptr(next_position_ids), _ptr_result(result), flags, _stream())
+    _calls().accept_commit(cache.k_ptrs, cache.v_ptrs, cache.num_layers, cache.block_table, cache.Hkv, pred, gt, cache_length, kv_len, best,
+                           int(max_accept), hidden, hidden_dim, prev_hidden, next_position_ids, _ptr_result(result), flags)
 
 
 class DraftTree:
@@ -344,16 +339,15 @@ class DraftTree:
     def begin(self, topk_val, topk_pos):
         """topk_val fp16[k], topk_pos int32[k] (first row). Returns next_ids [k]."""
         assert topk_val.dtype == torch.float16 and topk_pos.dtype == torch.int32 and topk_val.numel() == self.k
-        _lib().draft_tree_begin(_ptr(self.state), self.k, self.num_iter, _ptr(topk_val), _ptr(topk_pos), _ptr(self.remap),
-                                _ptr(self.next_ids), _ptr(self.draft_mask), _stream())
+        (_native or _calls()).draft_tree_begin(self.state, self.k, self.num_iter, topk_val, topk_pos, self.remap, self.next_ids, self.draft_mask)
         return self.next_ids
 
     def extend(self, d, topk_val, topk_pos):
         """topk_val fp16[k,k] (cumulated in place), topk_pos int32[k,k] of iteration d >= 1.
         Returns (next_ids [k], parent_rows [k], draft_mask [k])."""
         assert topk_val.dtype == torch.float16 and topk_pos.dtype == torch.int32 and topk_val.numel() == self.k * self.k
-        _lib().draft_tree_extend(_ptr(self.state), self.k, self.num_iter, int(d), _ptr(topk_val), _ptr(topk_pos), _ptr(self.remap),
-                                 _ptr(self.next_ids), _ptr(self.parent_rows), _ptr(self.draft_mask), _stream())
+        (_native or _calls()).draft_tree_extend(self.state, self.k, self.num_iter, int(d), topk_val, topk_pos, self.remap, self.next_ids,
+                                                self.parent_rows, self.draft_mask)
         return self.next_ids, self.parent_rows, self.draft_mask
 
     def finish(self, tree_size, cache_length, tree_draft_ids=None):
@@ -367,8 +361,7 @@ class DraftTree:
         pos = torch.empty(T, dtype=torch.int32, device=dev)
         mask = torch.empty((T, W), dtype=torch.int64, device=dev)
         parent = torch.empty(T, dtype=torch.int32, device=dev)
-        _lib().draft_tree_finish(_ptr(self.state), self.k, self.num_iter, T, _ptr(cache_length), _ptr(self.remap),
-                                 _ptr(tree_draft_ids), _ptr(pos), _ptr(mask), _ptr(parent), _stream())
+        (_native or _calls()).draft_tree_finish(self.state, self.k, self.num_iter, T, cache_length, self.remap, tree_draft_ids, pos, mask, parent)
         return tree_draft_ids, pos, mask, parent
 
 

@@ -86,3 +86,22 @@ def test_pybind_module_has_reference_names():
         C.init_base_model(0.5, 100, 1, 512, 1024, 32, 2, 128, 1e-5, 2, 2048, 1.0, 1.0, 1.0)
     with pytest.raises(ValueError, match="head_dim"):
         C.init_base_model(0.5, 100, 1, 512, 1024, 32, 2, 64, 1e-5, 0, 2048, 1.0, 1.0, 1.0)
+
+
+@pytest.mark.parametrize("args, error", [
+    ((None,) * 6 + (1, 1), (ValueError, RuntimeError)),           # null pointers; without a device there is no stream either
+    ((None,) * 6 + (1,), TypeError),                              # one argument short
+    (("k",) + (None,) * 5 + (1, 1), TypeError),                   # neither a tensor nor an address
+    ((None,) * 6 + (1 << 40, 1), OverflowError),
+])
+def test_torch_binding_checks_its_arguments(args, error):
+    from cpm.cu_amd import ops
+    with pytest.raises(error):
+        ops._calls().kv_append(*args)
+
+
+def test_torch_binding_refuses_host_tensors():
+    import torch
+    from cpm.cu_amd import ops
+    with pytest.raises(AssertionError, match="device-resident"):
+        ops._calls().kv_append(torch.zeros(4), None, None, None, None, None, 1, 1)
