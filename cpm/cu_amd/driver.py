@@ -56,7 +56,11 @@ class VerifyStep:
         if self.commit:
             self.prev_hidden = None  # allocated at the first step, when the hidden size is known
             self.next_positions = torch.zeros(self.T, dtype=torch.int32, device=dev)
-            self.packed = torch.zeros(1 + self.T, dtype=torch.int32).pin_memory()  # (a, ids): written by the GPU
+        if self.fused:
+            # (a, ids), written by the GPU: reading them back from device memory instead (two copies with a wait each) costs
+            # 29 us behind every step
+            self.packed = torch.zeros(1 + self.T, dtype=torch.int32, pin_memory=True)
+            self._packed = self.packed.numpy()
 
     def enqueue(self, q_layers, k_new_layers, v_new_layers, hidden, draft_ids, attn_out=None, splits=0):
         """Enqueue one full verify step.  q_layers[l] [T,Hq,128]; k/v_new_layers[l] [T,Hkv,128];
@@ -77,7 +81,7 @@ class VerifyStep:
                             hidden=hidden if self.commit else None, prev_hidden=self.prev_hidden if self.commit else None,
                             gt_out=self.gt, best=self.best, path=self.path, accepted_ids=self.pred,
                             next_position_ids=self.next_positions if self.commit else None,
-                            result=self.packed if self.commit else None)
+                            result=self.packed)
             if self.commit:
                 # lengths and tree positions advance on the device: the next step of the same tree shape needs no host write
                 ops.verify_tail_inplace(self.best, self.pred, cache_length=self.cache_length, kv_len=self.kv_len,
@@ -96,12 +100,12 @@ class VerifyStep:
                           advance_length=True, kv_len=self.kv_len)
 
     def result(self):
-        """(accept length, accepted token ids) after one synchronisation.  With commit the GPU has
-        already written both into pinned host memory; otherwise they are read back from the device."""
-        torch.cuda.current_stream().synchronize()
-        if self.commit:
-            a = int(self.packed[0])
-            return a, self.packed[1:1 + a].numpy().copy()
+        """(accept length, accepted token ids) after one synchronisation.  The fused tail has already written both
+        into pinned host memory; the operator-by-operator one leaves them on the device."""
+        ops.synchronize()
+        if self.fused:
+            a = int(self._packed[0])
+            return a, self._packed[1:1 + a].copy()
         a = int(self.best[0].item())
         return a, self.pred[:a].cpu().numpy()
 
