@@ -139,6 +139,24 @@ def test_kv_append_matches_logical_write(gpu):
         assert kk.abs().sum() > 0 and vv.abs().sum() > 0
 
 
+@pytest.mark.parametrize("hkv", [1, 2, 5])
+@pytest.mark.parametrize("P,T", [(0, 1), (15, 1), (16, 16), (1, 15), (3, 17), (0, 32), (255, 33), (240, 32), (250, 60), (7, 64), (1000, 777)])
+def test_kv_append_runs_and_edges(gpu, P, T, hkv):
+    """Runs of 16 rows that start inside a 16-slot group, end short, or cross a page; what the cache held elsewhere stays."""
+    from cpm.cu_amd import ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch = gpu
+    npages = (P + T + 255) // 256 + 1
+    table = synth.rng(P + T, 4).permutation(npages).astype(np.int32)
+    a = PagedKVCache(1, hkv, npages, block_table=table, fill=7.0)
+    b = PagedKVCache(1, hkv, npages, block_table=table, fill=7.0)
+    k = to_dev(torch, synth.normal_f16((T, hkv, D), P, 10))
+    v = to_dev(torch, synth.normal_f16((T, hkv, D), P, 20))
+    ops.kv_append(a, 0, k, v, torch.tensor([P + T], dtype=torch.int32, device="cuda"))
+    b.write_logical(0, P, k, v)
+    assert torch.equal(a.k[0], b.k[0]) and torch.equal(a.v[0], b.v[0])
+
+
 @pytest.mark.parametrize("P,T,splits", [(1024, 16, 0), (4096 - 23, 60, 0), (250, 60, 1), (0, 16, 1), (700, 128, 3), (63, 64, 2)])
 def test_fused_append_equals_append_then_attend(gpu, orc, P, T, splits):
     """Handing the tree rows' K/V to the attention kernel (fused copy_to_kvcache) must give the same
