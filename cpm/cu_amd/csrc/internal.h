@@ -40,11 +40,16 @@ constexpr int kHeadModeArgmax = 1;
 #define CPMCU_HEAD_STREAM_SHAPES(X)                                                                           \
     X(1, 1, 512) X(1, 2, 256) X(1, 3, 256) X(1, 4, 256) X(2, 1, 512) X(2, 2, 256) X(2, 3, 256) X(2, 4, 128) \
     X(4, 1, 256) X(4, 2, 256) X(4, 3, 128) X(4, 4, 128) X(8, 1, 128) X(8, 2, 128)
+// The K-slice kernel <KS, NB>: H = 8 waves x KS steps of 32 columns, row groups of NB x 16 hidden rows.
+#define CPMCU_HEAD_SLICE_SHAPES(X) X(8, 1) X(8, 2) X(16, 1) X(16, 2)
 // (row-walking kernel by row blocks of hidden, the K-chunked kernel <NB, NP, KC, NBUF>, or the streaming kernel)
 enum class HeadShape { Row1, Row2, Row4, Row8, C_1_2_512_2, C_1_4_256_2, C_2_4_256_4, C_2_4_256_2, C_4_4_256_4, C_4_4_256_2, C_8_4_128_2,
                        C_2_4_512_2, C_4_4_128_4, C_8_2_128_2,
 #define CPMCU_X(nb, fp, kc) S_##nb##_##fp##_##kc,
                        CPMCU_HEAD_STREAM_SHAPES(CPMCU_X)
+#undef CPMCU_X
+#define CPMCU_X(ks, nb) T_##ks##_##nb, R_##ks##_##nb,
+                       CPMCU_HEAD_SLICE_SHAPES(CPMCU_X)
 #undef CPMCU_X
 };
 const char* head_shape_name(HeadShape s);

@@ -19,7 +19,8 @@
 //     reads one contiguous KB and consecutive k-steps are consecutive in memory; the row-major
 //     layout is read as lane = (row % 16, k-group), 4 lanes per 64 contiguous bytes of a row;
 //   * the hidden rows are the B operand, staged in LDS: resident for the whole K range with up
-//     to 16 rows on the row-major path (head_gemm_kernel), otherwise walked in K chunks that are
+//     to 16 rows on the row-major path (head_gemm_kernel), in registers where the waves split K (head_gemm_slice_kernel:
+//     vocabularies of less than one pass, row-major weights), otherwise walked in K chunks that are
 //     brought in by direct-to-LDS loads, double buffered, in the OUTER loop, with one accumulator
 //     set per row block of a sweep (head_gemm_chunked_kernel); tiled weights of at least one full pass run
 //     head_gemm_stream_kernel, which keeps the W stream in a register ring refilled fragment by fragment
@@ -58,6 +59,8 @@ struct HeadParams {
     int full_passes;
     int rem_blocks;
     int last_share;  // streaming kernel: waves that share one row block of the last pass (power of two)
+    int row_blocks;   // ceil(V / 16)
+    int part_stride;  // hidden rows per line of part_a / part_b
     int apply_scale;
     float head_scale;
     int mode;
@@ -939,6 +942,159 @@ __device__ __forceinline__ void fuse_finish_row(const HeadParams& p, const FuseP
     }
 }
 
+// K split over the waves: wave w of a workgroup multiplies columns [w * KS * 32, (w + 1) * KS * 32) of EVERY row block the
+// workgroup has, so its part of the hidden rows stays in registers (KS x NB fragments) and the loop touches neither LDS nor a barrier
+// for it, and the unit of work is one row block per workgroup instead of one per wave: a vocabulary of less than one pass over the
+// wave slots still reaches every CU.  W is requested NBUF row blocks ahead, every fragment's registers again as soon as its MFMAs
+// have read them; straight-line code per block for exact waits, as in the streaming kernel below.  The partial tiles of a
+// block (one per wave) meet in LDS in groups of eight (block, 16 hidden rows) units: wave w adds up and finishes the group's unit w.
+// More than 16 * NB hidden rows are row groups (blockIdx.y) that share the CUs: the groups' workgroups of the same blocks sit on one
+// XCD and walk them together, so W comes from HBM once.
+// us per call, x 4096 tiled, this kernel / streaming or chunked kernel: 10 rows, 8192 rows of vocabulary 13.9 / 24.1, 16384 23.8 /
+// 30.6, 20000 27.7 / 34.6, 32768 43.4 / 42.7 (where the streaming kernel takes over).  Row-major, against the row-walking kernel:
+// 8192 16.2 / 43.8, 32768 48.8 / 52, 73448 103 / 112-117 (its two loads of a 128-byte line are left to the L2: with non-temporal
+// loads 51.4 at 32768).
+template <int KS, int NB, bool TILED, typename E>
+__device__ __forceinline__ void head_gemm_slice_body(const HeadParams& p) {
+    typedef typename Elem<E>::x8 X8;
+    constexpr int NBUF = KS * (NB + 2) <= 48 ? 2 : 1;  // W buffers of one row block: what 256 registers leave beside the hidden rows
+    constexpr int kBlocks = kHeadWaves / NB;           // row blocks of a group
+    __shared__ __attribute__((aligned(1024))) f32x4 xch[2][kHeadWaves][kHeadWaves][64];  // [group parity][unit][wave][lane]
+    __shared__ float red_a[kHeadWaves][NB * 16];
+    __shared__ float red_b[kHeadWaves][NB * 16];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int l16 = lane & 15;
+    const int kgp = lane >> 4;
+    const int G = gridDim.x;
+    const int c = blockIdx.x;
+    const int row0 = blockIdx.y * (NB * 16);  // first hidden row of this row group
+    const int H = p.H;
+    const int np = (p.row_blocks - c + G - 1) / G;  // row blocks c, c + G, ... of this workgroup: at least one
+    const int k0 = wave * (KS * 32);
+
+    auto block_ptr = [&](int b) {
+        const int rb = b * G + c;
+        if constexpr (TILED) return p.w + ((size_t)rb * (H / 32) + wave * KS) * 512 + lane * 8;
+        const int row = min(rb * 16 + l16, p.V - 1);  // rows past the end are computed and discarded
+        return p.w + (size_t)row * H + k0 + kgp * 8;
+    };
+    auto load_frag = [&](const f16* base, int ks) -> X8 {
+        if constexpr (TILED) return __builtin_nontemporal_load(reinterpret_cast<const X8*>(base + ks * 512));
+        return *reinterpret_cast<const X8*>(base + ks * 32);
+    };
+    X8 wa[KS], wb[NBUF == 2 ? KS : 1], hid[KS][NB];
+    {
+        const f16* a = block_ptr(0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) wa[ks] = load_frag(a, ks);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int hrow = min(row0 + nb * 16 + l16, p.n - 1);  // rows past n: any valid data, their results are dropped
+            const f16* h = p.hidden + (size_t)hrow * H + k0 + kgp * 8;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) hid[ks][nb] = *reinterpret_cast<const X8*>(h + ks * 32);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NBUF == 2) {
+            const f16* b = block_ptr(min(1, np - 1));
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) wb[ks] = load_frag(b, ks);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // The hidden fragments are awaited here, ahead of the loop: a wait for them inside it would be one for nearly
+        // everything in flight in every later turn.
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) asm volatile("" : "+v"(hid[ks][nb]));
+        if (p.apply_scale) {  // pre-scale of the hidden rows, rounded to the element type (src/model/linear.cuh:82-101)
+            const E sc = (E)p.head_scale;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) hid[ks][nb][e] = (E)((float)hid[ks][nb][e] * (float)sc);
+        }
+    }
+    // this wave finishes blocks wave / NB, + kBlocks, ... for hidden rows row0 + my_nb * 16 ..: ascending vocabulary rows per lane
+    const int my_nb = wave % NB;
+    const float eb_none = p.mode == kHeadModeStats ? 0.f : __int_as_float(0x7fffffff);
+    float ea = -INFINITY, eb = eb_none;
+    {
+        const int first_row = (wave / NB * G + c) * 16 + kgp * 4;  // (see head_epilogue_block)
+        if (p.mode != kHeadModeStats && first_row < p.V) eb = __int_as_float(first_row);
+    }
+    auto finish_group = [&](int group) {
+        __syncthreads();
+        const int b = group * kBlocks + wave / NB;
+        if (b >= np) return;
+        const f32x4(*part)[64] = xch[group & 1][wave];
+        f32x4 acc = part[0][lane];
+#pragma unroll
+        for (int w = 1; w < kHeadWaves; ++w) {
+            const f32x4 x = part[w][lane];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[r] += x[r];
+        }
+        head_epilogue_block<E, true>(p, acc, blockIdx.y * NB + my_nb, (b * G + c) * 16 + kgp * 4, l16, ea, eb);
+    };
+    auto consume = [&](int b, auto& w, auto refill) {
+        const f16* next = refill ? block_ptr(b + NBUF) : nullptr;
+        f32x4 acc[2][NB];  // two chains per block of hidden rows
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[0][nb] = acc[1][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[ks & 1][nb] = Elem<E>::mfma_16x16x32(w[ks], hid[ks][nb], acc[ks & 1][nb]);
+            if (refill) w[ks] = load_frag(next, ks);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const int group = b / kBlocks, unit = b % kBlocks * NB;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[0][nb][r] += acc[1][nb][r];
+            xch[group & 1][unit + nb][wave][lane] = acc[0][nb];
+        }
+        // (a wave that runs ahead writes the other half: the half this group used is free again behind the next group's barrier)
+        if (b % kBlocks == kBlocks - 1) finish_group(group);
+    };
+    int b = 0;
+    if constexpr (NBUF == 2) {
+        for (; b + 3 < np; b += 2) {
+            consume(b, wa, std::true_type{});
+            consume(b + 1, wb, std::true_type{});
+        }
+        if (np - b == 3) {
+            consume(b, wa, std::true_type{});
+            consume(b + 1, wb, std::false_type{});
+            consume(b + 2, wa, std::false_type{});
+        } else {
+            consume(b, wa, std::false_type{});
+            if (np - b == 2) consume(b + 1, wb, std::false_type{});
+        }
+    } else {
+        for (; b + 1 < np; ++b) consume(b, wa, std::true_type{});
+        consume(b, wa, std::false_type{});
+    }
+    if (np % kBlocks != 0) finish_group(np / kBlocks);
+    float fa[NB], fb[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        fa[nb] = nb == my_nb ? ea : -INFINITY;
+        fb[nb] = nb == my_nb ? eb : eb_none;
+    }
+    head_finish_with<NB>(p, fa, fb, red_a, red_b, tid, wave, lane, [&](int row, float a, float bb) {
+        p.part_a[(size_t)c * p.part_stride + row0 + row] = a;
+        p.part_b[(size_t)c * p.part_stride + row0 + row] = bb;
+    });
+}
+
 // Tiled weights whose row blocks fit one sweep: FP full passes (every wave one whole row block each) and at most
 // one partly filled last pass.  The wave's W stream is a ring of 1 KB fragments held in registers and refilled
 // fragment by fragment: as soon as the MFMAs of a (row block, K step) have read their fragment, the same registers
@@ -1303,6 +1459,10 @@ template <int NB, int FP, int KC>
 __global__ __launch_bounds__(kHeadThreads) void head_gemm_stream_kernel(HeadParams p) { head_gemm_stream_body<NB, FP, KC, f16>(p); }
 template <int NB, int FP, int KC>
 __global__ __launch_bounds__(kHeadThreads) void head_gemm_stream_bf16_kernel(HeadParams p) { head_gemm_stream_body<NB, FP, KC, bf16>(p); }
+template <int KS, int NB, bool TILED>
+__global__ __launch_bounds__(kHeadThreads) void head_gemm_slice_kernel(HeadParams p) { head_gemm_slice_body<KS, NB, TILED, f16>(p); }
+template <int KS, int NB, bool TILED>
+__global__ __launch_bounds__(kHeadThreads) void head_gemm_slice_bf16_kernel(HeadParams p) { head_gemm_slice_body<KS, NB, TILED, bf16>(p); }
 // FR-Spec head + log-softmax + top-k + id map-back in one launch (one block of hidden rows).
 template <int FP, int KC>
 __global__ __launch_bounds__(kHeadThreads) void frspec_head_topk_kernel(HeadParams p, FuseParams fp) { head_gemm_stream_body<1, FP, KC, f16, true>(p, fp); }
@@ -1371,6 +1531,11 @@ const char* head_shape_name(HeadShape s) {
     case HeadShape::S_##nb##_##fp##_##kc: return "head_gemm_stream_kernel<" #nb "," #fp "," #kc ">";
             CPMCU_HEAD_STREAM_SHAPES(CPMCU_X)
 #undef CPMCU_X
+#define CPMCU_X(ks, nb)                                                                          \
+    case HeadShape::T_##ks##_##nb: return "head_gemm_slice_kernel<" #ks "," #nb ",true>";        \
+    case HeadShape::R_##ks##_##nb: return "head_gemm_slice_kernel<" #ks "," #nb ",false>";
+            CPMCU_HEAD_SLICE_SHAPES(CPMCU_X)
+#undef CPMCU_X
     }
     return "?";
 }
@@ -1413,6 +1578,34 @@ HeadShape pick_head_shape(int NB, int H, bool w_tiled, int nch, int npasses, int
     }
 }
 
+// Whether the K-slice kernel takes a call, and in which shape.  Its unit is a row block per workgroup, so it is the kernel for
+// vocabularies of less than one pass over the chip's wave slots; from one pass on the streaming kernel is level for up to 16 hidden
+// rows and ahead for more (60 rows x 32768: 46.7 us against 55.0), on exactly half a pass and more for more than 32 rows as well,
+// where it has a shape (whole passes: 16384 x 128 rows 43.9 / 46.3; 20000, where it has none, 74.1 / 56.1).  Row-major weights have
+// no streaming kernel: up to 32 rows the K slices win at every size (32 rows: 54.5 / 56.3 us at 32768, 109 / 123 at 73448, 216 / 237 at
+// 151936) but for up to 16 rows of 2048 columns from one pass on (63.9 / 61.7 at 73448); 33 to 64 rows below one pass (32768:
+// 68.9 / 69.9, 73448: 156 / 151), more below half a pass (20000 x 128 rows: 81.6 / 80.3).
+bool pick_slice_shape(int n, int H, bool w_tiled, int nrb, int cus, HeadShape* shape) {
+    const int slots = cus * kHeadWaves;
+    if (w_tiled) {
+        if (!options().head_stream_kernel || nrb >= slots) return false;
+        if (n > 32 && nrb * 2 >= slots && nrb % kHeadWaves == 0) return false;
+    } else if (n <= 32) {
+        if (n <= 16 && H < 4096 && nrb >= slots) return false;
+    } else if (nrb >= (n <= 64 ? slots : slots / 2)) {
+        return false;
+    }
+    const int snb = n <= 16 ? 1 : 2;
+#define CPMCU_X(ks, nb)                                                            \
+    if (H == ks * 32 * kHeadWaves && nb == snb) {                                  \
+        *shape = w_tiled ? HeadShape::T_##ks##_##nb : HeadShape::R_##ks##_##nb;    \
+        return true;                                                               \
+    }
+    CPMCU_HEAD_SLICE_SHAPES(CPMCU_X)
+#undef CPMCU_X
+    return false;
+}
+
 }  // namespace
 
 namespace {
@@ -1441,7 +1634,19 @@ int plan_head_gemm(const void* hidden, const void* w, int w_layout, int n, int V
     p.part_a = part_a;
     p.part_b = part_b;
     const int nrb = ceil_div(V, 16);
+    p.row_blocks = nrb;
     int G = num_cus();
+    p.part_stride = NB * 16;
+    if (pick_slice_shape(n, H, p.w_tiled, nrb, G, shape_out)) {
+        p.npasses = p.full_passes = p.rem_blocks = 0;
+        p.last_share = 1;
+        // the row groups share the CUs, in multiples of the XCD count so that the workgroups of a row block stay on one XCD
+        const int groups = ceil_div(n, NB == 1 ? 16 : 32);
+        if (groups > 1) G = G / groups / 8 * 8 > 0 ? G / groups / 8 * 8 : 1;
+        *grid_out = G < nrb ? G : nrb;
+        *p_out = p;
+        return CPMCU_OK;
+    }
     if (G * kHeadWaves > nrb) G = ceil_div(nrb, kHeadWaves);
     // The streaming kernel has accumulators for four full passes per wave (two for 65 to 128 hidden rows: three or four
     // spill), so a vocabulary of more passes than that gets a multiple of the CU count in workgroups -- they run one after
@@ -1534,6 +1739,18 @@ int launch_head_gemm(const void* hidden, const void* w, int w_layout, int n, int
         break;
             CPMCU_HEAD_STREAM_SHAPES(CPMCU_X)
 #undef CPMCU_X
+#define CPMCU_HEAD_SLICE(ks, nb, tiled)                                                                                                          \
+    do {                                                                                                                                         \
+        const dim3 grid(G, ceil_div(n, 16 * nb));                                                                                                \
+        if (is_bf16) hipLaunchKernelGGL((head_gemm_slice_bf16_kernel<ks, nb, tiled>), grid, dim3(kHeadThreads), 0, st, p);                       \
+        else hipLaunchKernelGGL((head_gemm_slice_kernel<ks, nb, tiled>), grid, dim3(kHeadThreads), 0, st, p);                                    \
+    } while (0)
+#define CPMCU_X(ks, nb)                                                     \
+    case HeadShape::T_##ks##_##nb: CPMCU_HEAD_SLICE(ks, nb, true); break;   \
+    case HeadShape::R_##ks##_##nb: CPMCU_HEAD_SLICE(ks, nb, false); break;
+            CPMCU_HEAD_SLICE_SHAPES(CPMCU_X)
+#undef CPMCU_X
+#undef CPMCU_HEAD_SLICE
     }
 #undef CPMCU_HEAD_ROW
 #undef CPMCU_HEAD_CHUNKED

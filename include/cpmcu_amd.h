@@ -84,7 +84,8 @@ const char* cpmcu_version(void);
  *                           of the head GEMM (default), 0 = plain mapping (CPMCU_HEAD_NO_SHARE set);
  *   "head_stream_kernel"    1 = tiled head weights whose row blocks make at least one full pass over the GPU's
  *                           wave slots run the streaming GEMM kernel, on a multiple of the CU count in workgroups
- *                           (up to 1024) beyond four passes (two for 65 to 128 hidden rows) (default), 0 = always
+ *                           (up to 1024) beyond four passes (two for 65 to 128 hidden rows), smaller ones of 2048 or
+ *                           4096 columns the K-slice kernel (default), 0 = always
  *                           the K-chunked kernel (CPMCU_HEAD_NO_STREAM set);
  *   "attn_merge_in_launch"  1 = the workgroups of a split tree-attention launch merge their own partials when the
  *                           launch fits the GPU's CUs and has at most 32 splits (default), 0 = always the separate
@@ -431,7 +432,8 @@ int cpmcu_frspec_head_topk(const void* hidden, const void* w, int w_layout, cons
                            int32_t* topk_ids, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The call above runs as ONE launch when the shape allows it (CPMCU_W_TILED weights, k <= 16, V a multiple of 8 with one
- * or two full passes of 16-row blocks over the GPU -- the FR-Spec vocabulary of 32768 is one) and one of the library's 8
+ * or two full passes of 16-row blocks over the GPU -- the FR-Spec vocabulary of 32768 is one -- or any smaller whole number
+ * of workgroups where the two-launch form runs the same GEMM kernel, see cpmcu_head_plan) and one of the library's 8
  * publication states per device is free for (workspace, grid size): every GEMM workgroup publishes its k..16 best
  * (value, index, token id) per hidden row as tagged 64-bit words, and the first n workgroups to finish rank one row
  * each.  Same outputs, bit for bit, as the two-launch form (cpmcu_set_option("frspec_fused", 0)); logits are complete

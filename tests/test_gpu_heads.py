@@ -643,3 +643,32 @@ def test_streaming_head_kernel_plain_last_pass(gpu, orc, set_option):
     assert_close_f16(to_np(z_s), to_np(z_p), "shared vs plain last pass", atol=8e-3, rtol=2e-3)
     assert_close_f16(to_np(z_p), orc.lm_head(hid, w), "plain last pass vs oracle")
     assert np.array_equal(to_np(gt_p), orc.argmax(to_np(z_p)))
+
+
+# (hidden rows, V, H, head scale, tiled): one row block and fewer blocks than CUs; one to three blocks per workgroup (the prologue's
+# and the tail's cases), whole and partial groups of eight (block, 16 rows) units; one to four row groups; ragged vocabularies
+_SLICE_SHAPES = [
+    (1, 9, 2048, None, True), (16, 16 * 255, 4096, None, True), (5, 16 * 256 + 1, 4096, 0.3125, True), (10, 16 * 767, 2048, None, True),
+    (16, 16 * 256 * 7 + 40, 2048, None, True), (32, 8200, 2048, None, True), (17, 5000, 4096, 2.0, True), (33, 9001, 2048, None, True),
+    (64, 20000, 2048, None, True), (100, 3001, 4096, None, True), (128, 12007, 2048, 0.5, True),
+    (1, 9, 2048, None, False), (16, 16 * 256 + 1, 4096, 0.3125, False), (3, 40001, 4096, None, False), (24, 33000, 2048, None, False),
+    (60, 7001, 4096, None, False), (128, 3000, 2048, None, False)]
+
+
+@pytest.mark.parametrize("n,V,H,scale,tiled", _SLICE_SHAPES)
+def test_k_slice_head_kernel(gpu, orc, n, V, H, scale, tiled):
+    """The kernel whose waves split K (vocabularies of less than one pass, row-major weights): logits within tolerance of the
+    oracle, arg-max exact on the kernel's own logits, with and without materialised logits."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    hid = synth.normal_f16((n, H), V + n, 1)
+    w = synth.normal_f16((V, H), V + n, 2, std=0.02)
+    d_hid, d_w = to_dev(torch, hid), to_dev(torch, w)
+    if tiled:
+        d_w = ops.tile_head_weight(d_w)
+    assert "head_gemm_slice_kernel" in ops.head_plan(n, d_w)[0]
+    gt, z = ops.lm_head_argmax(d_hid, d_w, head_scale=scale, want_logits=True)
+    gt2 = ops.lm_head_argmax(d_hid, d_w, head_scale=scale)
+    torch.cuda.synchronize()
+    assert_close_f16(to_np(z), orc.lm_head(hid, w, head_scale=scale), "K-slice kernel vs oracle")
+    assert np.array_equal(to_np(gt), orc.argmax(to_np(z))) and np.array_equal(to_np(gt), to_np(gt2))
