@@ -69,7 +69,7 @@ __host__ __device__ inline int v_slot16(int t) { return (t & ~12) | ((t & 4) << 
 
 // ---- error plumbing (thread-local message, integer status) ----
 void set_error(const char* fmt, ...);
-hipStream_t resolve_stream(void* stream);  // NULL -> the library's blocking stream
+hipStream_t resolve_stream(void* stream);  // NULL -> the library's blocking stream, CPMCU_STREAM_LEGACY -> HIP's null stream
 
 #define CPMCU_CHECK_ARG(cond, ...)                 \
     do {                                           \

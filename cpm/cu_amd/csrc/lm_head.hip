@@ -2062,12 +2062,13 @@ extern "C" int cpmcu_lm_head_argmax_static(const void* hidden, const void* w, in
     CPMCU_CHECK_ARG(head_max_grid() * 128 * 2 * sizeof(float) <= kStaticHeadScratchBytes,
                     "lm_head_argmax_static: the built-in scratch of %zu bytes is too small for %d workgroups", kStaticHeadScratchBytes,
                     head_max_grid());
-    float* part = nullptr;
-    int rc = static_head_scratch(&part, (hipStream_t)stream);
-    if (rc != CPMCU_OK) return rc;
     // NULL selects HIP's null stream here: the library's own stream is created on first use, and this entry
     // point creates nothing
-    return lm_head_argmax_on(hidden, w, w_layout, n, V, H, apply_scale, head_scale, logits, gt, part, (hipStream_t)stream);
+    hipStream_t st = stream ? resolve_stream(stream) : nullptr;
+    float* part = nullptr;
+    int rc = static_head_scratch(&part, st);
+    if (rc != CPMCU_OK) return rc;
+    return lm_head_argmax_on(hidden, w, w_layout, n, V, H, apply_scale, head_scale, logits, gt, part, st);
 }
 
 CPMCU_TIMELINE_READER(cpmcu_timeline_read_head, cpmcu::g_head_timeline)

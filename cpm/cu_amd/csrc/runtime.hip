@@ -31,6 +31,7 @@ void set_error(const char* fmt, ...) {
 }
 
 hipStream_t resolve_stream(void* stream) {
+    if (stream == CPMCU_STREAM_LEGACY) return nullptr;
     if (stream) return (hipStream_t)stream;
     if (!g_stream) {
         // a blocking stream, like the reference's calc_stream (src/utils.cu:19): work on the legacy

@@ -24,7 +24,8 @@
  *     force -- IEEE binary16 by default, bfloat16 under torch_dtype = 1 / the "dtype"
  *     option below -- row-major unless stated.
  *   - `stream` is a hipStream_t passed as void*; NULL selects the library's own
- *     blocking stream (the counterpart of calc_stream, src/utils.cu:6,19).
+ *     blocking stream (the counterpart of calc_stream, src/utils.cu:6,19), and
+ *     CPMCU_STREAM_LEGACY HIP's null stream.
  *   - operator-level calls only enqueue work; they never synchronise.
  *
  * Paged KV cache layout (this library's own; the reference keeps flat
@@ -60,6 +61,10 @@ extern "C" {
 /* flags of cpmcu_accept_commit, cpmcu_verify_tail_inplace and cpmcu_verify_step */
 #define CPMCU_COMMIT_ADVANCE_LENGTH 1
 #define CPMCU_COMMIT_NEXT_ROOT 2
+
+/* The `stream` argument that stands for HIP's null stream (the value of hipStreamLegacy): a caller whose work is there
+ * launches there, with no marker packet between its streams. */
+#define CPMCU_STREAM_LEGACY ((void*)1)
 
 #define CPMCU_PAGE_SIZE 256
 #define CPMCU_HEAD_DIM 128

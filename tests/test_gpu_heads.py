@@ -672,3 +672,20 @@ def test_k_slice_head_kernel(gpu, orc, n, V, H, scale, tiled):
     torch.cuda.synchronize()
     assert_close_f16(to_np(z), orc.lm_head(hid, w, head_scale=scale), "K-slice kernel vs oracle")
     assert np.array_equal(to_np(gt), orc.argmax(to_np(z))) and np.array_equal(to_np(gt), to_np(gt2))
+
+
+@pytest.mark.parametrize("side", [False, True])
+def test_calls_are_ordered_on_torchs_current_stream(gpu, side):
+    """Behind and ahead of torch's own work on the default (HIP's null) stream and on a stream of its own, with nothing waiting."""
+    torch = gpu
+    from cpm.cu_amd import ops
+    with torch.cuda.stream(torch.cuda.Stream() if side else torch.cuda.default_stream()):
+        x = torch.zeros((3, 5000), dtype=torch.float16, device="cuda")
+        torch.cuda._sleep(2_000_000)
+        for i in range(3):
+            x[i, 100 * i + 7] = 1.0 + i
+        val, pos = ops.topk(x, 2)
+        first, best = val[:, 0].clone(), pos[:, 0].clone()
+        val.fill_(-1.0)
+        torch.cuda.synchronize()
+    assert first.tolist() == [1.0, 2.0, 3.0] and best.tolist() == [7, 107, 207]
