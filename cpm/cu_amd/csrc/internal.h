@@ -10,6 +10,7 @@ struct Options {
     int dtype = 0;                 // element type of the 16-bit tensors handed to the operator-level entry points: 0 = fp16,
                                    // 1 = bf16 (process-wide, like the reference's model; cpmcu_init_base_model sets it)
     int attn_kv_groups = 0;        // 0 = chosen per call; 1 / 2 force that tree-attention kernel shape
+    int attn_direct = -1;          // -1 = chosen per call; 0 = never the direct shape of tree attention, 1 = always
     int head_share_last_pass = 1;  // 0 keeps the plain row-block mapping of the head GEMM
     int head_stream_kernel = 1;    // 0 keeps tiled weights on the K-chunked kernel (tests compare the two)
     int attn_merge_in_launch = 1;  // 0: the split partials of tree attention are always merged by a launch of their own

@@ -221,6 +221,9 @@ extern "C" int cpmcu_set_option(const char* name, int value) {
         // ones follow cpmcu_init_base_model's torch_dtype, which sets the same switch)
         CPMCU_CHECK_ARG(value == 0 || value == 1, "set_option: dtype=%d must be 0 (fp16) or 1 (bf16)", value);
         options().dtype = value;
+    } else if (nm == "attn_direct") {
+        CPMCU_CHECK_ARG(value >= -1 && value <= 1, "set_option: attn_direct=%d outside [-1, 1]", value);
+        options().attn_direct = value;
     } else if (nm == "attn_kv_groups") {
         CPMCU_CHECK_ARG(value >= 0 && value <= 2, "set_option: attn_kv_groups=%d outside [0, 2]", value);
         options().attn_kv_groups = value;
@@ -798,7 +801,7 @@ uint64_t step_signature(const Model& m, const StepArgs& a) {
         mix(v);
     // the options decide which kernels a capture records: a graph captured under other settings is another graph
     const Options& o = options();
-    for (int v : {o.dtype, o.attn_kv_groups, o.head_share_last_pass, o.head_stream_kernel, o.attn_merge_in_launch, o.attn_merge_wait_us, o.frspec_fused, o.frspec_wait_us, o.topk_row_kernel}) mix((uint64_t)(uint32_t)v);
+    for (int v : {o.dtype, o.attn_kv_groups, o.attn_direct, o.head_share_last_pass, o.head_stream_kernel, o.attn_merge_in_launch, o.attn_merge_wait_us, o.frspec_fused, o.frspec_wait_us, o.topk_row_kernel}) mix((uint64_t)(uint32_t)v);
     return h;
 }
 

@@ -6,6 +6,7 @@
 // three kernels: compaction reads it from device memory.
 #include "common.h"
 #include "internal.h"
+#include "kv_append.h"
 #include "topk_keys.h"
 
 namespace cpmcu {
@@ -414,64 +415,13 @@ __global__ __launch_bounds__(128) void verify_tail_inplace_kernel(const int32_t*
     }
 }
 
-// copy_to_kvcache, src/model/attn.cuh:14-21: token t of the T new rows goes to position *kv_len - T + t.
-// A launch is a chain of two round trips (rows beside length -> page ids, then the stores), so the bytes have to be whole
-// transactions: a workgroup takes kAppendRows consecutive new rows of one KV head, which it can request before it knows where
-// they go; K goes straight on as 16-byte pieces, V is transposed through LDS into 16-byte pieces of the page's dim rows (eight
-// token slots each).  Only pieces that the run covers in part are written slot by slot.  2048 rows of two heads: 7.0 us with one
-// token per workgroup and 2-byte V stores 512 bytes apart, 4.4 with runs of 32 rows (130 workgroups), 3.7 with 16 (258).
-constexpr int kAppendRows = 16;
-constexpr int kAppendStride = kHeadDim + 4;  // halves per staged V row: the lanes of a dim read rows 4 or 8 apart
-__global__ __launch_bounds__(256) void kv_append_kernel(f16* k_pool, f16* v_pool, const int32_t* block_table,
-                                                        const f16* k_new, const f16* v_new,
-                                                        const int32_t* kv_len, int T, int Hkv) {
-    __shared__ __attribute__((aligned(8))) uint16_t s_v[kAppendRows * kAppendStride];
-    const int tid = threadIdx.x;
-    const int g = blockIdx.y;
-    const int r0 = blockIdx.x * kAppendRows;
-    const int n = min(kAppendRows, T - r0);
-    const int row = tid >> 4, ch = tid & 15;  // 16 rows x 16 pieces of 16 bytes
-    const size_t o = ((size_t)(r0 + min(row, n - 1)) * Hkv + g) * kHeadDim + ch * 8;
-    const f16x8 kx = *reinterpret_cast<const f16x8*>(k_new + o);
-    const uint4 vx = *reinterpret_cast<const uint4*>(v_new + o);
-    const int p0 = kv_len[0] - T + r0;  // position of this workgroup's first row; its rows lie in at most two pages
-    const int lp = p0 / kPage;
-    const int page_lo = block_table[lp], page_hi = block_table[(p0 + n - 1) / kPage];
-    const auto page_of = [&](int pos) { return pos / kPage == lp ? page_lo : page_hi; };
-    uint2* staged = reinterpret_cast<uint2*>(s_v + row * kAppendStride + ch * 8);
-    staged[0] = make_uint2(vx.x, vx.y);
-    staged[1] = make_uint2(vx.z, vx.w);
-    if (row < n) {
-        const int pos = p0 + row;
-        *reinterpret_cast<f16x8*>(k_pool + (((size_t)page_of(pos) * Hkv + g) * kPage + pos % kPage) * kHeadDim + ch * 8) = kx;
-    }
-    __syncthreads();
-    // V^T: the one or two 16-slot groups of the run, two pieces each; the pieces of a dim on neighbouring lanes
-    const int group0 = p0 & ~15;
-    const int npieces = ((p0 + n - 1 - group0) / 16 + 1) * 2;
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-        const int x = it * 256 + tid;
-        const int d = x >> 2, piece = x & 3;
-        if (piece >= npieces) continue;
-        const int first = group0 + (piece >> 1) * 16 + (piece & 1) * 4;  // slots 0..3: tokens first .. + 3, slots 4..7: first + 8 ..
-        uint32_t v[8], in = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int r = first + (j & 3) + (j >> 2) * 8 - p0;
-            v[j] = s_v[min(max(r, 0), n - 1) * kAppendStride + d];
-            in |= r >= 0 && r < n ? 1u << j : 0u;
-        }
-        const int slot = (first & ~15) % kPage + (piece & 1) * 8;
-        uint16_t* dst = reinterpret_cast<uint16_t*>(v_pool) + (((size_t)page_of(first) * Hkv + g) * kHeadDim + d) * kPage + slot;
-        if (in == 0xFFu) {
-            *reinterpret_cast<uint4*>(dst) = make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if ((in >> j) & 1u) dst[j] = (uint16_t)v[j];
-        }
-    }
+// The rows of a prompt chunk or of a tree, appended by a launch of its own: a workgroup per run of rows and KV head.
+__global__ __launch_bounds__(kAppendThreads) void kv_append_kernel(f16* k_pool, f16* v_pool, const int32_t* block_table,
+                                                                   const f16* k_new, const f16* v_new,
+                                                                   const int32_t* kv_len, int T, int Hkv) {
+    __shared__ AppendStage stage;
+    kv_append_run<f16, false>(k_pool, v_pool, block_table, k_new, v_new, nullptr, T, Hkv, blockIdx.y, blockIdx.x * kAppendRows, threadIdx.x, stage,
+                       [&]() { return kv_len[0]; });
 }
 
 }  // namespace
@@ -604,7 +554,7 @@ extern "C" int cpmcu_kv_append(void* k_pool, void* v_pool, const int32_t* block_
                                const void* v_new, const int32_t* kv_len, int T, int Hkv, void* stream) {
     CPMCU_CHECK_ARG(k_pool && v_pool && block_table && k_new && v_new && kv_len, "kv_append: null pointer argument");
     CPMCU_CHECK_ARG(T >= 1 && Hkv >= 1, "kv_append: T=%d Hkv=%d", T, Hkv);
-    hipLaunchKernelGGL(kv_append_kernel, dim3(ceil_div(T, kAppendRows), Hkv), dim3(256), 0, resolve_stream(stream), (f16*)k_pool, (f16*)v_pool,
+    hipLaunchKernelGGL(kv_append_kernel, dim3(ceil_div(T, kAppendRows), Hkv), dim3(kAppendThreads), 0, resolve_stream(stream), (f16*)k_pool, (f16*)v_pool,
                        block_table, (const f16*)k_new, (const f16*)v_new, kv_len, T, Hkv);
     CPMCU_LAUNCH_CHECK();
     return CPMCU_OK;

@@ -38,12 +38,14 @@
 //    land on the same XCD (workgroup id modulo 8) and share its L2.
 #include "common.h"
 #include "internal.h"
+#include "kv_append.h"
 #include "timeline.h"
 
 #include <map>
 #include <mutex>
 #include <type_traits>
 #include <algorithm>
+#include <cmath>
 #include <utility>
 #include <vector>
 
@@ -302,17 +304,6 @@ __device__ inline void combine_store(const AttnParams& p, const CombineWhere<E>&
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = (E)(t.acc[e] * inv);
     *reinterpret_cast<X4*>(p.out + ((size_t)w.node * p.Hq + w.head) * kHeadDim + w.d0) = o;
-}
-
-// One rotary pair: (a, b) -> (a cos - b sin, a sin + b cos), every product and sum rounded on its own
-// (no fused multiply-add), so the result does not depend on how a compiler contracts the expression.
-template <typename E>
-__device__ inline void rotate_pair(E& a, E& b, float2 cs) {
-#pragma clang fp contract(off)
-    const float fa = (float)a, fb = (float)b;
-    const float ac = fa * cs.x, bs = fb * cs.y, as = fa * cs.y, bc = fb * cs.x;
-    a = (E)(ac - bs);
-    b = (E)(as + bc);
 }
 
 template <typename E>
@@ -1221,6 +1212,8 @@ __device__ __forceinline__ void tree_attn_combine_wide_body(const AttnParams& p)
 __global__ __launch_bounds__(64 * kCombineWideWaves) void tree_attn_combine_wide_kernel(AttnParams p) { tree_attn_combine_wide_body<f16>(p); }
 __global__ __launch_bounds__(64 * kCombineWideWaves) void tree_attn_combine_wide_bf16_kernel(AttnParams p) { tree_attn_combine_wide_body<bf16>(p); }
 
+#include "attention_direct.h"
+
 int device_cu_count() {
     static int cus[64] = {0};
     int dev = 0;
@@ -1304,6 +1297,7 @@ struct LaunchPlan {
                      // (the window starts on a block boundary at or above P - block_window_size)
     int kv_groups, num_mtiles, num_splits;
     bool merge_in_launch;  // the split workgroups merge their own partials (no combine launch)
+    bool direct;           // the direct shape: num_mtiles counts its 16-row tiles
 };
 
 // Counters of the in-launch merge.  They live in the library (zero when it is loaded, and back at zero arrivals after
@@ -1368,11 +1362,57 @@ uint32_t* merge_counters_for(const void* workspace, hipStream_t st) {
     if (it->second.use_combine) return nullptr;
     return g_merge_ctr_base[dev] + (size_t)it->second.block * kMergeUnits * kMergeUnitWords;
 }
-LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_window_size, int num_splits_override) {
+// The direct shape or one of the split shapes, and the splits of the direct one: from estimates of both, in us, fitted to a sweep
+// over 1-128 nodes x 128-120000 keys x 2, 4, 8 KV heads (replayed graphs, caches rotated through HBM).
+//   direct  3.4 for the launch up to its first block, 4 more for every further two workgroups per CU (two are resident); 1.05 per
+//           iteration, 1.2 once more than half of the CUs pull K/V, times the workgroups per CU of the fullest XCD (two that share a
+//           CU take 1.75 times as long at least); 0.4 of the time of the bytes at 5.5 TB/s; 2.3 for a merge by the last arrival and
+//           0.06 per partial it reads
+//   split   10.2, 1 per 2500 keys up to 2.2 (more splits, then longer ones), the bytes, 0.05 per node; 1.5 with the rotary embedding
+// Measured, split -> direct, one query: 10.2 -> 6.8 at 800 keys, 12.8 -> 9.2 (with rotary 14.5 -> 9.2) at 4096, 15.4 -> 11.8 at
+// 10000, 25.7 -> 23.7 (rotary) at 60000; 10 nodes: 12.4 -> 5.9 at 256, 13.7 -> 10.2 at 4096; 16 nodes 13.9 -> 11.3; 60 nodes
+// 12.4 -> 10.0 at 800.  Where the estimates change over (60 nodes at 1500, 33 at 1500, 16 at 7000, 4 at 40000) the two are within
+// 10 % of each other; beyond, the split shapes' larger tiles win (60 nodes at 4096: 15.8 / 22).
+struct DirectPlan {
+    int splits;
+    bool use;
+};
+DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope) {
+    const int units = Hkv * tiles, blocks = ceil_div(span, kBlockKeys) + 1;  // (one more for the appended rows)
+    const float stream = (float)span * Hkv * (2 * kHeadDim * sizeof(f16)) / 5.5e6f;
+    const int most = std::min(kMaxSplits, std::max(256 / units, std::max(1, std::min(4, 512 / units))));
+    DirectPlan d = {1, false};
+    float best = 1e30f;
+    for (int it = ceil_div(blocks, most); it <= blocks; it = it < 64 ? it + 1 : it * 2) {
+        const int splits = ceil_div(blocks, it);
+        const float per_cu = (float)(ceil_div(splits * Hkv, kXcds) * tiles) / 32.f;
+        const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.75f);
+        const float t = 3.4f + (units * splits > 128 ? 1.2f : 1.05f) * it * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
+                        (splits > 1 ? 2.3f + 0.06f * splits : 0.f);
+        if (t < best) best = t, d.splits = splits;
+    }
+    const float split_shape = 10.2f + std::min(2.2f, span / 2500.f) + stream + 0.05f * T + (rope ? 1.5f : 0.f);
+    d.use = options().attn_direct >= 0 ? options().attn_direct != 0 : options().attn_kv_groups == 0 && best < split_shape;
+    return d;
+}
+
+LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_window_size, int num_splits_override, bool rope, bool allow_direct = true) {
     LaunchPlan pl;
     const int window_blocks = block_window_size / 128;
     pl.span = max_kv_len;
     if (window_blocks > 0 && window_blocks * 128 + T < pl.span) pl.span = window_blocks * 128 + T;
+    const int tiles = ceil_div(group * T, kDirectRows);
+    const DirectPlan direct = choose_direct(T, Hkv, tiles, pl.span, rope);
+    // (a split count asked for is one of the split shapes', unless the direct shape is forced)
+    pl.direct = allow_direct && direct.use && (num_splits_override == 0 || options().attn_direct == 1);
+    if (pl.direct) {
+        pl.kv_groups = 0;
+        pl.num_mtiles = tiles;
+        pl.num_splits = num_splits_override > 0 ? num_splits_override : direct.splits;
+        pl.merge_in_launch = pl.num_splits > 1;
+        if (pl.num_splits == 1 || (options().attn_merge_in_launch && Hkv * tiles <= kMergeUnits)) return pl;
+        pl.direct = false;
+    }
     pl.kv_groups = choose_groups(T, group, Hkv, pl.span);
     pl.num_mtiles = ceil_div(group * T, rows_per_wg(pl.kv_groups));
     pl.num_splits = num_splits_override > 0 ? num_splits_override : choose_splits(T, group, Hkv, pl.span, pl.kv_groups);
@@ -1390,8 +1430,9 @@ extern "C" int cpmcu_tree_attention_plan(int T, int Hq, int Hkv, int max_kv_len,
                                          int num_splits_override, char* kernel_names, size_t kernel_names_bytes, int* num_splits,
                                          int* kv_groups, int* num_workgroups) {
     CPMCU_CHECK_ARG(T >= 1 && T <= kMaxTree && Hkv >= 1 && Hq >= Hkv && Hq % Hkv == 0 && max_kv_len >= T, "tree_attention_plan: bad shape");
-    const LaunchPlan pl = plan_launch(T, Hq / Hkv, Hkv, max_kv_len, block_window_size, num_splits_override);
+    const LaunchPlan pl = plan_launch(T, Hq / Hkv, Hkv, max_kv_len, block_window_size, num_splits_override, with_rope != 0);
     if (kernel_names && kernel_names_bytes > 0)
+        pl.direct ? snprintf(kernel_names, kernel_names_bytes, "tree_attn_direct_kernel") :
         snprintf(kernel_names, kernel_names_bytes, "tree_attn_split_kernel<%d,%s>%s", pl.kv_groups, with_rope ? "true" : "false",
                  pl.num_splits <= 1 || pl.merge_in_launch ? "" : pl.num_splits > kMergeMaxSplits ? "+tree_attn_combine_wide_kernel" : "+tree_attn_combine_kernel");
     if (num_splits) *num_splits = pl.num_splits;
@@ -1544,11 +1585,16 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     p.group_shift = log2_or_minus1(group);
     p.hkv_shift = log2_or_minus1(Hkv);
     p.window_blocks = block_window_size / 128;
-    const LaunchPlan plan = plan_launch(T, group, Hkv, max_kv_len, block_window_size, num_splits_override);
+    hipStream_t st = resolve_stream(stream);
+    LaunchPlan plan = plan_launch(T, group, Hkv, max_kv_len, block_window_size, num_splits_override, rope_cos_sin != nullptr);
+    p.merge_ctr = plan.merge_in_launch && workspace ? merge_counters_for(workspace, st) : nullptr;
+    // (the direct shape has no merge launch to fall back on)
+    if (plan.direct && plan.num_splits > 1 && p.merge_ctr == nullptr)
+        plan = plan_launch(T, group, Hkv, max_kv_len, block_window_size, num_splits_override, rope_cos_sin != nullptr, false);
     const int span = plan.span;
     const int G = plan.kv_groups;
     p.num_mtiles = plan.num_mtiles;
-    p.rows_pad = p.num_mtiles * rows_per_wg(G);
+    p.rows_pad = p.num_mtiles * (plan.direct ? kDirectRows : rows_per_wg(G));
     p.num_splits = plan.num_splits;
     CPMCU_CHECK_ARG(p.num_splits <= kMaxSplits, "tree_attention: max_kv_len=%d is beyond the supported context", max_kv_len);
     p.ntiles_max = ceil_div(span, kTileN);
@@ -1556,10 +1602,8 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     p.max_kv_len = max_kv_len;
     p.scale_log2 = scale * 1.4426950408889634f;
     p.out = (f16*)out;
-    hipStream_t st = resolve_stream(stream);
     p.o_part = nullptr;
     p.ml_part = nullptr;
-    p.merge_ctr = nullptr;
     p.merge_wait_ticks = 0;
     if (p.num_splits > 1) {
         const size_t o_bytes = align_up((size_t)Hkv * p.num_splits * p.rows_pad * kHeadDim * sizeof(f16), 256);
@@ -1568,12 +1612,18 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
                         "tree_attention: workspace of %zu bytes needed, %zu given", o_bytes + ml_bytes, workspace_bytes);
         p.o_part = (float*)workspace;
         p.ml_part = (float*)((char*)workspace + o_bytes);
-        if (plan.merge_in_launch) p.merge_ctr = merge_counters_for(workspace, st);
         p.merge_wait_ticks = (uint32_t)options().attn_merge_wait_us * 100u;
     }
     const int nsh = p.num_splits * Hkv;
     const dim3 grid(kXcds * ceil_div(nsh, kXcds), p.num_mtiles);
     const bool is_bf16 = options().dtype == 1;
+    if (plan.direct) {
+        const dim3 dgrid(grid.x, p.num_mtiles + (k_new != nullptr ? 1 : 0));
+        if (is_bf16) hipLaunchKernelGGL(tree_attn_direct_bf16_kernel, dgrid, dim3(kThreads), 0, st, p);
+        else hipLaunchKernelGGL(tree_attn_direct_kernel, dgrid, dim3(kThreads), 0, st, p);
+        CPMCU_LAUNCH_CHECK();
+        return CPMCU_OK;
+    }
     if (is_bf16) {
         if (p.rope != nullptr) {
             if (G == 1) hipLaunchKernelGGL((tree_attn_split_bf16_kernel<1, true>), grid, dim3(kThreads), 0, st, p);

@@ -45,6 +45,7 @@ def attention(L, torch, prefixes, T=60):
     from . import ops, synth
     from .kvcache import PagedKVCache
     Hq, Hkv, D, NL = 32, 2, 128, 8
+    L.set_option(b"attn_direct", 0)  # the stamps are the split kernel's
     mask = None  # one row, or a chain beyond 64 rows
     if 1 < T <= 64:
         mask = torch.from_numpy(synth.eagle_tree(6, 10, T, 0).mask.view(np.int64)).cuda()

@@ -85,6 +85,9 @@ const char* cpmcu_version(void);
  *                           that only move values (append, compaction, gathers, weight tiling) do not care;
  *   "attn_kv_groups"        0 = chosen per call (default), 1 / 2 = force the 256-row / the two-KV-group
  *                           shape of the tree-attention kernel (CPMCU_ATTN_KV_GROUPS=1|2);
+ *   "attn_direct"           -1 = chosen per call (default), 0 = never, 1 = always the shape of the tree-attention kernel for
+ *                           launches that are round trips rather than work (few rows, short contexts); attn_kv_groups
+ *                           other than 0 and a given split count are for the other shapes;
  *   "head_share_last_pass"  1 = the waves of a workgroup share the row blocks of a partly filled last pass
  *                           of the head GEMM (default), 0 = plain mapping (CPMCU_HEAD_NO_SHARE set);
  *   "head_stream_kernel"    1 = tiled head weights whose row blocks make at least one full pass over the GPU's
@@ -355,8 +358,8 @@ int cpmcu_tree_attention_release_workspace(const void* workspace);
 
 /* No reference counterpart: which kernels a cpmcu_tree_attention* call of this shape launches, without
  * launching -- for reports that must name the instantiation actually taken.  kernel_names receives e.g.
- * "tree_attn_split_kernel<2,false>+tree_attn_combine_kernel" (beyond 32 splits: "+tree_attn_combine_wide_kernel"); the
- * outputs may each be NULL. */
+ * "tree_attn_split_kernel<2,false>+tree_attn_combine_kernel" (beyond 32 splits: "+tree_attn_combine_wide_kernel") or
+ * "tree_attn_direct_kernel" (kv_groups 0); the outputs may each be NULL. */
 int cpmcu_tree_attention_plan(int T, int Hq, int Hkv, int max_kv_len, int with_rope, int block_window_size,
                               int num_splits_override, char* kernel_names, size_t kernel_names_bytes, int* num_splits,
                               int* kv_groups, int* num_workgroups);

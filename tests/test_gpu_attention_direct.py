@@ -1,0 +1,99 @@
+"""The direct shape of tree attention at its edges: block and row-tile remainders, splits with one block and with none, appended
+rows in more than one step, windows that start inside a page, both element types -- against the oracle, and the cache against
+what the other shapes leave behind, slots past the end included."""
+import numpy as np
+import pytest
+
+from cpm.cu_amd import synth
+from util import assert_close_f16, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+@pytest.fixture
+def option():
+    from cpm.cu_amd import lib
+    L = lib.get()
+    yield lambda name, value: L.set_option(name.encode(), int(value))
+    L.set_option(b"attn_direct", -1)
+    L.set_option(b"dtype", 0)
+
+
+@pytest.mark.parametrize("P,T,hq,hkv,splits,window,rope,fused", [
+    (0, 1, 32, 2, 1, 0, False, True), (0, 33, 32, 2, 0, 0, True, True), (1, 1, 32, 2, 2, 0, True, True), (127, 1, 32, 2, 1, 0, False, True),
+    (128, 9, 32, 2, 0, 0, True, True), (129, 16, 32, 2, 3, 0, False, True), (255, 60, 32, 2, 0, 0, False, True), (256, 31, 32, 8, 0, 0, True, True),
+    (777, 128, 32, 8, 0, 0, False, True), (300, 7, 24, 8, 2, 0, True, True), (500, 13, 28, 4, 0, 0, False, True), (90, 3, 12, 12, 0, 0, False, True),
+    (4090, 4, 32, 2, 0, 0, True, True), (4096, 1, 32, 2, 36, 0, False, True), (4700, 1, 32, 2, 37, 0, False, True), (9000, 2, 32, 4, 128, 0, True, True),
+    (20000, 1, 32, 2, 1, 0, False, True), (1500, 10, 32, 2, 0, 1024, False, True), (1537, 12, 32, 2, 3, 1024, True, True),
+    (700, 10, 32, 2, 0, 128, False, True), (640, 17, 32, 2, 0, 0, False, False), (2000, 64, 32, 2, 4, 512, False, False)])
+def test_direct_shape_against_the_oracle(gpu, orc, option, P, T, hq, hkv, splits, window, rope, fused):
+    from cpm.cu_amd import ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch = gpu
+    S, seed = P + T, 7 * P + T
+    tree = synth.random_tree(T, seed, max_children=4, max_depth=9)
+    q, k, v = (synth.normal_f16(s, seed, i) for i, s in enumerate([(T, hq, D), (S, hkv, D), (S, hkv, D)]))
+    max_len = (S + 127) // 128 * 128 + [0, 640][seed % 2]
+    npages = (max_len + 255) // 256 + 1
+    pages = synth.rng(seed, 4).permutation(npages).astype(np.int32)
+    kv_len = torch.tensor([S], dtype=torch.int32, device="cuda")
+    table, q_ref, k_ref = None, q, k
+    if rope:
+        inv_freq = (10000.0 ** (-np.arange(D // 2, dtype=np.float64) / (D // 2))).astype(np.float32)
+        table = ops.rope_table(to_dev(torch, tree.positions(P)), to_dev(torch, inv_freq))
+        q_ref, k_rot = orc.rope(q, k[P:], table=to_np(table))
+        k_ref = np.concatenate([k[:P], k_rot], 0)
+    n = P if fused else S
+    new = dict(k_new=to_dev(torch, k[P:]), v_new=to_dev(torch, v[P:])) if fused else {}
+    outs, pools = [], []
+    for direct in (0, 1):
+        option("attn_direct", direct)
+        c = PagedKVCache(1, hkv, npages, block_table=pages, fill=float("nan"))
+        if n:
+            c.write_logical(0, 0, to_dev(torch, k[:n]), to_dev(torch, v[:n]))
+        assert (ops.attention_plan(T, hq, hkv, max_len, rope, window)[0] == "tree_attn_direct_kernel") == bool(direct)
+        outs.append(ops.tree_attention(to_dev(torch, q), c, 0, kv_len, max_len, to_dev(torch, tree.mask), num_splits=splits if direct else 0,
+                                       rope=table, block_window_size=window, **new))
+        torch.cuda.synchronize()
+        pools.append([t.view(torch.int16) for t in (c.k[0], c.v[0])])
+    ref = orc.tree_attention(q_ref, k_ref, v, tree.mask, P, block_window_size=window)
+    assert_close_f16(to_np(outs[1]), ref, "direct shape")
+    assert all(torch.equal(a, b) for a, b in zip(*pools)), "the cache differs from what the split shapes leave"
+
+
+@pytest.mark.parametrize("P,T,kd", [(900, 10, 30), (130, 8, 64), (61, 4, 128)])
+def test_direct_shape_bf16_with_a_wider_mask(gpu, option, P, T, kd):
+    """bf16, a mask whose range reaches into the cached rows, replayed from a graph: the merge's arrival words are at rest behind
+    every launch."""
+    from cpm.cu_amd import ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch = gpu
+    option("dtype", 1)
+    P += kd - T
+    g = torch.Generator(device="cuda").manual_seed(P)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).to(torch.bfloat16).view(torch.float16)
+    S = P + T
+    q, k, v = rnd(T, 32, D), rnd(S, 2, D), rnd(S, 2, D)
+    mask = torch.randint(-2 ** 62, 2 ** 62, (T, (kd + 63) // 64), device="cuda", generator=g)
+    cache = PagedKVCache(1, 2, (S + 255) // 256)
+    cache.write_logical(0, 0, k[:P], v[:P])
+    kv_len = torch.tensor([S], dtype=torch.int32, device="cuda")
+    call = lambda out: ops.tree_attention(q, cache, 0, kv_len, S, mask, k_new=k[P:], v_new=v[P:], mask_k_range=kd, out=out)
+    option("attn_direct", 0)
+    ref = call(torch.empty_like(q)).view(torch.bfloat16).float()
+    option("attn_direct", 1)
+    out = call(torch.empty_like(q))
+    torch.cuda.synchronize()
+    first = out.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(3):
+            call(out)
+    for _ in range(4):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), first.view(torch.int16))
+    err = (first.view(torch.bfloat16).float() - ref).norm() / ref.norm()
+    assert err < 8e-3, float(err)
