@@ -160,13 +160,15 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(TopkParams p) 
 //      to the same fp16 value or above stays a candidate -- and only candidates are mapped;
 //   3. candidates go to LDS as exact 64-bit keys; each counts the candidates with a larger key:
 //      that count IS its output slot.
-// More than kRowCap candidates (rows dominated by one value): k rounds of a workgroup-wide maximum
-// over the register-resident values instead, each round taking the largest key below the previous winner.
+// More than kRowCap candidates (bfloat16 log-probabilities, where thousands share a value; rows dominated by one value): the exact
+// k-th largest image by bisection over workgroup-wide counts, everything above it, and as many of its equals as are missing, lowest
+// indices first.  (It was k rounds of a workgroup-wide maximum: 71 us for the 20 best of a 24483-element slice that holds fewer than
+// 20 outstanding values, 19 for one that holds more.)
 constexpr int kRowThreads = 1024;
 constexpr int kRowWaves = kRowThreads / 64;
-constexpr int kRowPieces = 4;                          // 16-byte pieces per thread
-constexpr int kRowElems = kRowPieces * 8;
-constexpr int kRowMaxDim = kRowThreads * kRowElems;    // 32768
+constexpr int kRowMaxPieces = 4;                       // 16-byte pieces per thread
+constexpr int kRowMaxDim = kRowThreads * kRowMaxPieces * 8;  // 32768
+constexpr int kRowShortDim = kRowThreads * 8;          // 8192: one piece per thread
 constexpr int kRowCap = kRowThreads;                   // candidate keys held in LDS
 constexpr int kRowBoundDrop = 4;                       // low bits of the bound that are not searched
 constexpr int kRowDenseWaves = 8;                      // waves that extract the candidates
@@ -176,11 +178,13 @@ constexpr int kRowMaxTop = 128;                        // output slots are ranks
 typedef int16_t s16x2 __attribute__((ext_vector_type(2)));
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-template <bool LOGSOFTMAX, typename E>
+template <bool LOGSOFTMAX, int kRowPieces, typename E>
 __device__ __forceinline__ void topk_row_body(const TopkParams& p) {
+    constexpr int kRowElems = kRowPieces * 8;
     __shared__ __attribute__((aligned(16))) uint64_t cand[kRowCap];
     __shared__ int rank[kRowCap];
-    __shared__ uint64_t wave_best[2][kRowWaves];
+    __shared__ __attribute__((aligned(16))) int wave_count[2][kRowWaves];
+    __shared__ int equal_count[kRowPieces * kRowWaves];
     __shared__ float row_m_lse[2];
     __shared__ uint32_t wave_kth[kRowWaves], wave_few[kRowWaves];
     __shared__ int ncand, nlanes;
@@ -207,17 +211,24 @@ __device__ __forceinline__ void topk_row_body(const TopkParams& p) {
             raw[j] = pc < npieces ? xr[pc] : make_uint4(~0u, ~0u, ~0u, ~0u);
         }
     } else {
-        // rows that do not start on 16 bytes or do not end on a whole piece: element by element
+        // rows that do not start on 16 bytes, or do not end on a whole piece: the same pieces, unaligned, and the last elements one by one
+        typedef uint32_t u32x4_unaligned __attribute__((ext_vector_type(4), aligned(2)));
         const uint16_t* xe = (const uint16_t*)xr;
 #pragma unroll
         for (int j = 0; j < kRowPieces; ++j) {
             const int e0 = (j * kRowThreads + tid) * 8;
-            uint32_t w4[4];
+            uint32_t w4[4] = {~0u, ~0u, ~0u, ~0u};
+            if (e0 + 8 <= len) {
+                const u32x4_unaligned v = *reinterpret_cast<const u32x4_unaligned*>(xe + e0);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t a = e0 + 2 * q < len ? xe[e0 + 2 * q] : 0xFFFFu;
-                const uint32_t b = e0 + 2 * q + 1 < len ? xe[e0 + 2 * q + 1] : 0xFFFFu;
-                w4[q] = a | (b << 16);
+                for (int q = 0; q < 4; ++q) w4[q] = v[q];
+            } else if (e0 < len) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t a = e0 + 2 * q < len ? xe[e0 + 2 * q] : 0xFFFFu;
+                    const uint32_t b = e0 + 2 * q + 1 < len ? xe[e0 + 2 * q + 1] : 0xFFFFu;
+                    w4[q] = a | (b << 16);
+                }
             }
             raw[j] = make_uint4(w4[0], w4[1], w4[2], w4[3]);
         }
@@ -351,6 +362,19 @@ __device__ __forceinline__ void topk_row_body(const TopkParams& p) {
         }
         return make_key(bits, idx);
     };
+    const auto mapped_id = [&](uint64_t key) { return !p.ids || sliced ? 0 : p.remap ? p.remap[key_index(key)] : key_index(key); };
+    const auto emit = [&](int slot, uint64_t key, int32_t id) {
+        if (sliced) {
+            slice_out[slot] = key;
+            return;
+        }
+        const int idx = key_index(key);
+        const size_t o = (size_t)row * p.top + slot;
+        // raw ranking: hand back the input bits (keeps -0); fused: the rounded log-prob in the key
+        p.val[o] = LOGSOFTMAX ? key_bits(key) : p.x[(size_t)row * p.dim + idx];
+        p.pos[o] = idx;
+        if (p.ids) p.ids[o] = id;
+    };
     // threads holding anything at or above the bound hand their 16 registers to LDS ...
     const bool bounded = lo != 0;
     if (bounded && lmax >= lo) {
@@ -420,8 +444,7 @@ __device__ __forceinline__ void topk_row_body(const TopkParams& p) {
         const int i = tid & ((1 << shift) - 1);
         const int part = tid >> shift, nparts = kRowThreads >> shift;
         // the mapped id of candidate tid is fetched now and used after the ranking
-        int32_t mapped = 0;
-        if (tid < C && p.ids && !sliced) mapped = p.remap ? p.remap[key_index(cand[tid])] : key_index(cand[tid]);
+        const int32_t mapped = tid < C ? mapped_id(cand[tid]) : 0;
         if (i < C) {
             // slots from C on hold key 0, so whole groups of eight can be compared
             const uint64_t my = cand[i];
@@ -438,53 +461,114 @@ __device__ __forceinline__ void topk_row_body(const TopkParams& p) {
         }
         __syncthreads();
         CPMCU_STAMP(g_topk_timeline, blockIdx.x, 5);
-        if (tid < C && rank[tid] < p.top) {
-            const uint64_t key = cand[tid];
-            if (sliced) {
-                slice_out[rank[tid]] = key;
-            } else {
-                const int idx = key_index(key);
-                const size_t o = (size_t)row * p.top + rank[tid];
-                p.val[o] = LOGSOFTMAX ? key_bits(key) : p.x[(size_t)row * p.dim + idx];
-                p.pos[o] = idx;
-                if (p.ids) p.ids[o] = mapped;
-            }
-        }
+        if (tid < C && rank[tid] < p.top) emit(rank[tid], cand[tid], mapped);
         CPMCU_STAMP(g_topk_timeline, blockIdx.x, 6);
         return;
     }
-    uint64_t prev = ~0ull;
-    for (int round = 0; round < p.top; ++round) {
-        uint64_t mine = 0;
+    // ---- the exact k-th largest image ----
+    if (LOGSOFTMAX) {  // the ranking is of the mapped values: the registers take their images (0 past the end)
 #pragma unroll
         for (int j = 0; j < kRowPieces; ++j) {
             const int e0 = (j * kRowThreads + tid) * 8;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t o = (img[j * 4 + (e >> 1)] >> ((e & 1) * 16)) & 0xFFFFu;
-                const uint64_t key = e0 + e < len ? key_from_image(o, slice_base + e0 + e) : 0ull;
-                if (key < prev && key > mine) mine = key;
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t w = img[j * 4 + q];
+                const uint32_t a = e0 + 2 * q < len ? (uint32_t)(key_from_image(w & 0xFFFFu, 0) >> 32) : 0u;
+                const uint32_t b = e0 + 2 * q + 1 < len ? (uint32_t)(key_from_image(w >> 16, 0) >> 32) : 0u;
+                img[j * 4 + q] = a | (b << 16);
             }
         }
-        const uint64_t wbest = wave_max_u64(mine);
-        uint64_t* wb = wave_best[round & 1];
-        if (lane == 0) wb[wave] = wbest;
-        __syncthreads();
-        uint64_t best = wb[0];
+    }
+    int step = 0;
+    // elements of the row whose image is c (> 0) or more
+    const auto count_from = [&](uint32_t c) {
+        const u16x2 below = __builtin_bit_cast(u16x2, (c - 1) * 0x10001u);
+        const u16x2 one2 = {1, 1};
+        u16x2 n2 = {0, 0};
 #pragma unroll
-        for (int w = 1; w < kRowWaves; ++w) best = wb[w] > best ? wb[w] : best;
-        if (tid == 0) {
-            if (sliced) slice_out[round] = best;
-            else emit_final<LOGSOFTMAX>(p, row, round, best);
+        for (int r = 0; r < kRowElems / 2; ++r)
+            n2 += __builtin_elementwise_min(__builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, img[r]), below), one2);
+        const uint32_t n = wave_reduce_b32((uint32_t)n2[0] + n2[1], [](uint32_t a, uint32_t b) { return a + b; });
+        int* const wc = wave_count[step++ & 1];  // (a wave that runs ahead writes the other buffer)
+        if (lane == 0) wc[wave] = (int)n;
+        __syncthreads();
+        int total = 0;
+#pragma unroll
+        for (int w = 0; w < kRowWaves; ++w) total += wc[w];
+        return total;
+    };
+    const auto larger = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
+    const uint32_t wmax = wave_reduce_b32(lmax, larger);
+    if (lane == 0) wave_kth[wave] = wmax;
+    __syncthreads();
+    if (tid == 0) ncand = 0;  // (everybody has read it)
+    // The largest image with k elements at or above it (0: fewer than k hold anything else), between the bound's and the maximum's.
+    uint32_t lower = bound, upper = 0;
+#pragma unroll
+    for (int w = 0; w < kRowWaves; ++w) upper = larger(upper, wave_kth[w]);
+    if (LOGSOFTMAX) {
+        lower = bound ? (uint32_t)(key_from_image(bound, 0) >> 32) : 0u;
+        upper = (uint32_t)(key_from_image(upper, 0) >> 32);
+        // (infinities and NaNs do not map in order)
+        if (lower != 0 && count_from(lower) < p.top) lower = 0;
+        if (upper != 0xFFFFu && count_from(upper + 1) != 0) upper = 0xFFFFu;
+    }
+    while (lower < upper) {
+        const uint32_t mid = (lower + upper + 1) >> 1;
+        if (count_from(mid) >= p.top) lower = mid;
+        else upper = mid - 1;
+    }
+    // -0 (0x7FFF) and +0 (0x8000) are one value
+    const uint32_t class_lo = lower == 0x8000u ? 0x7FFFu : lower, class_hi = lower == 0x7FFFu ? 0x8000u : lower;
+    const int above = class_hi == 0xFFFFu ? 0 : count_from(class_hi + 1);
+    // where this thread's members of the class come among all of them, in index order: piece by piece, then thread by thread
+    int before[kRowPieces];
+#pragma unroll
+    for (int j = 0; j < kRowPieces; ++j) {
+        int n = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t o = (img[j * 4 + (e >> 1)] >> ((e & 1) * 16)) & 0xFFFFu;
+            n += o >= class_lo && o <= class_hi ? 1 : 0;
         }
-        prev = best;
-        if (best == 0) break;
+        int total = 0;
+        before[j] = 0;
+#pragma unroll
+        for (int bit = 0; bit < 4; ++bit) {
+            const uint64_t plane = __ballot((n >> bit) & 1);
+            before[j] += __popcll(plane & ((1ull << lane) - 1ull)) << bit;
+            total += __popcll(plane) << bit;
+        }
+        if (lane == 0) equal_count[j * kRowWaves + wave] = total;
+    }
+    __syncthreads();
+    static_assert(kRowPieces * kRowWaves <= 64, "a lane per count");
+    const uint32_t counted = lane < kRowPieces * kRowWaves ? (uint32_t)equal_count[lane] : 0u;
+#pragma unroll
+    for (int j = 0; j < kRowPieces; ++j) {
+        before[j] += (int)wave_reduce_b32(lane < j * kRowWaves + wave ? counted : 0u, [](uint32_t a, uint32_t b) { return a + b; });
+        const int e0 = (j * kRowThreads + tid) * 8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t o = (img[j * 4 + (e >> 1)] >> ((e & 1) * 16)) & 0xFFFFu;
+            const uint64_t key = LOGSOFTMAX ? ((uint64_t)o << 32) | (uint32_t)(0xFFFFFFFFu - (uint32_t)(slice_base + e0 + e)) : key_from_image(o, slice_base + e0 + e);
+            if (o > class_hi) cand[atomicAdd(&ncand, 1)] = key;
+            else if (o >= class_lo && before[j]++ < p.top - above && e0 + e < len) cand[above + before[j] - 1] = key;
+        }
+    }
+    __syncthreads();
+    if (tid < min(p.top, len)) {
+        const uint64_t my = cand[tid];
+        int r = 0;
+        for (int j = 0; j < min(p.top, len); ++j) r += cand[j] > my ? 1 : 0;
+        emit(r, my, mapped_id(my));
     }
 }
 
 // The slices' k best keys of a row (at most kSliceMergeCap of them, empty slots are 0) ranked by counting: one workgroup per
 // row, the count of larger keys is the output slot.
 constexpr int kSliceMergeCap = 1024;
+constexpr int kShortSliceCand = 256, kShortSliceWorkgroups = 512;
 template <bool LOGSOFTMAX>
 __global__ __launch_bounds__(kTopkThreads) void topk_slice_merge_kernel(TopkParams p) {
     __shared__ uint64_t keys[kSliceMergeCap];
@@ -503,8 +587,11 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_merge_kernel(TopkPara
 }
 
 template <bool LOGSOFTMAX>
-__global__ __launch_bounds__(kRowThreads) void topk_row_kernel(TopkParams p) { topk_row_body<LOGSOFTMAX, f16>(p); }
-__global__ __launch_bounds__(kRowThreads) void topk_row_bf16_kernel(TopkParams p) { topk_row_body<true, bf16>(p); }
+__global__ __launch_bounds__(kRowThreads) void topk_row_kernel(TopkParams p) { topk_row_body<LOGSOFTMAX, kRowMaxPieces, f16>(p); }
+__global__ __launch_bounds__(kRowThreads) void topk_row_bf16_kernel(TopkParams p) { topk_row_body<true, kRowMaxPieces, bf16>(p); }
+template <bool LOGSOFTMAX>
+__global__ __launch_bounds__(kRowThreads) void topk_short_row_kernel(TopkParams p) { topk_row_body<LOGSOFTMAX, 1, f16>(p); }
+__global__ __launch_bounds__(kRowThreads) void topk_short_row_bf16_kernel(TopkParams p) { topk_row_body<true, 1, bf16>(p); }
 
 // log_softmax in place (src/model/eagle.cuh:29-89): one workgroup per row.  The row is walked in 16-byte pieces from its
 // first 16-byte boundary on; the first four pieces of every thread stay in registers between the three passes (maximum, sum,
@@ -631,25 +718,34 @@ int launch_topk(const void* x, int n, int dim, int top, void* val, int32_t* pos,
     p.grid = stats ? stats->grid : 0;
     p.stride = stats ? stats->stride : 0;
     p.row_stats = stats ? stats->row_stats : nullptr;
-    // rows that fit one workgroup's registers: one launch, no candidate buffer
     const bool row_kernel = options().topk_row_kernel != 0;
+    const auto launch_rows = [&](int longest, dim3 grid) {
+        if (longest <= kRowShortDim) {
+            if (stats && options().dtype == 1) hipLaunchKernelGGL(topk_short_row_bf16_kernel, grid, dim3(kRowThreads), 0, st, p);
+            else if (stats) hipLaunchKernelGGL(topk_short_row_kernel<true>, grid, dim3(kRowThreads), 0, st, p);
+            else hipLaunchKernelGGL(topk_short_row_kernel<false>, grid, dim3(kRowThreads), 0, st, p);
+        } else {
+            if (stats && options().dtype == 1) hipLaunchKernelGGL(topk_row_bf16_kernel, grid, dim3(kRowThreads), 0, st, p);
+            else if (stats) hipLaunchKernelGGL(topk_row_kernel<true>, grid, dim3(kRowThreads), 0, st, p);
+            else hipLaunchKernelGGL(topk_row_kernel<false>, grid, dim3(kRowThreads), 0, st, p);
+        }
+    };
+    // rows that fit one workgroup's registers: one launch, no candidate buffer
     if (row_kernel && dim <= kRowMaxDim && row_kernel_ranks(dim, top, stats != nullptr)) {
-        if (stats && options().dtype == 1) hipLaunchKernelGGL(topk_row_bf16_kernel, dim3(n), dim3(kRowThreads), 0, st, p);
-        else if (stats) hipLaunchKernelGGL(topk_row_kernel<true>, dim3(n), dim3(kRowThreads), 0, st, p);
-        else hipLaunchKernelGGL(topk_row_kernel<false>, dim3(n), dim3(kRowThreads), 0, st, p);
+        launch_rows(dim, dim3(n));
         CPMCU_LAUNCH_CHECK();
         return CPMCU_OK;
     }
-    // longer rows in slices of at most kRowMaxDim elements: the row kernel on every slice, and a merge of the slices' k best
-    const int nslices = ceil_div(dim, kRowMaxDim);
+    // longer rows in slices: the row kernel on every slice, and a merge of the slices' k best.  Short slices while they are all
+    // resident at once and the merge has few candidates to count: 5 rows of 73449, k = 20, 19.3 -> 11.8 us; 60 rows of 151936 (1140
+    // slices, 380 candidates) 40 -> 50 with the merge
+    const int short_slices = ceil_div(dim, kRowShortDim);
+    const int nslices = n * short_slices <= kShortSliceWorkgroups && short_slices * top <= kShortSliceCand ? short_slices : ceil_div(dim, kRowMaxDim);
     if (row_kernel && top <= kRowMaxTop && nslices * top <= kSliceMergeCap && workspace &&
         workspace_bytes >= (size_t)n * nslices * top * sizeof(uint64_t)) {
         p.slice_len = (ceil_div(dim, nslices) + 7) / 8 * 8;
         p.nchunks = nslices;
-        const dim3 grid(n, nslices);
-        if (stats && options().dtype == 1) hipLaunchKernelGGL(topk_row_bf16_kernel, grid, dim3(kRowThreads), 0, st, p);
-        else if (stats) hipLaunchKernelGGL(topk_row_kernel<true>, grid, dim3(kRowThreads), 0, st, p);
-        else hipLaunchKernelGGL(topk_row_kernel<false>, grid, dim3(kRowThreads), 0, st, p);
+        launch_rows(p.slice_len, dim3(n, nslices));
         CPMCU_LAUNCH_CHECK();
         if (stats) hipLaunchKernelGGL(topk_slice_merge_kernel<true>, dim3(n), dim3(kTopkThreads), 0, st, p);
         else hipLaunchKernelGGL(topk_slice_merge_kernel<false>, dim3(n), dim3(kTopkThreads), 0, st, p);

@@ -211,8 +211,10 @@ def frspec_head_plan(n, w, k):
     if _lib().raw.cpmcu_frspec_head_mode(ctypes.c_void_p(ws.data_ptr()), layout, n, V, H, k) == 1:
         nb, fp, kc = gemm[gemm.index("<") + 1:-1].split(",")
         return "frspec_head_topk_kernel<%s,%s>" % (fp, kc)
-    # the row kernel: on the whole row up to 32768 elements, on slices of it beyond
-    return gemm + ("+topk_row_kernel<true>" if V <= 32768 else "+topk_row_kernel<true>+topk_slice_merge_kernel<true>")
+    # the row kernel: on the whole row up to 32768 elements (in its short form up to 8192), on slices of it beyond
+    slices = (V + 8191) // 8192
+    short = V <= 8192 or (V > 32768 and n * slices <= 512 and slices * k <= 256)
+    return gemm + ("+topk_short_row_kernel<true>" if short else "+topk_row_kernel<true>") + ("" if V <= 32768 else "+topk_slice_merge_kernel<true>")
 
 
 def lm_head_argmax(hidden, w, head_scale=None, want_logits=False, gt=None):

@@ -689,3 +689,44 @@ def test_calls_are_ordered_on_torchs_current_stream(gpu, side):
         val.fill_(-1.0)
         torch.cuda.synchronize()
     assert first.tolist() == [1.0, 2.0, 3.0] and best.tolist() == [7, 107, 207]
+
+
+@pytest.mark.parametrize("n,dim,top,off", [(3, 8192, 20, 0), (2, 32761, 1, 0), (3, 73449, 20, 1), (2, 73449, 50, 0), (2, 151936, 128, 0), (4, 40000, 33, 3)])
+def test_topk_of_values_that_tie_in_thousands(gpu, orc, n, dim, top, off):
+    """Log-probabilities on a coarse grid with fewer outstanding values than k, so that the k-th best is a value thousands share:
+    the lowest indices win.  Rows on and off 16 bytes, slices included."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    g = synth.rng(dim, top)
+    x = (np.round(g.standard_normal((n, dim)) * 8) / 16 - 11).astype(np.float16)
+    x[0, g.choice(dim, top // 2, replace=False)] = (-1 - np.arange(top // 2) / 8).astype(np.float16)
+    x[1, : dim // 3] = -np.inf
+    buf = torch.zeros(n * dim + 8, dtype=torch.float16, device="cuda")
+    d = buf[off:off + n * dim].view(n, dim)
+    d.copy_(to_dev(torch, x))
+    val, pos = ops.topk(d, top)
+    torch.cuda.synchronize()
+    v_ref, p_ref = orc.topk(x, top)
+    assert np.array_equal(to_np(pos), p_ref)
+    assert np.array_equal(to_np(val).view(np.uint16), v_ref.view(np.uint16))
+
+
+@pytest.mark.parametrize("V,top", [(8192, 10), (40000, 12)])
+def test_frspec_rows_of_equal_logits(gpu, orc, V, top):
+    """Hidden rows of zeros and of one coarse value: the fused ranking of log-probabilities that are all, or nearly all, the same."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    H = 512
+    w = (synth.rng(V, 1).integers(-1, 2, size=(V, H)) / 64.0).astype(np.float16)
+    hid = np.zeros((4, H), np.float16)
+    hid[1, :3] = 1.0
+    hid[2, 7] = -2.0
+    hid[3] = synth.normal_f16((H,), V, 2)
+    remap = synth.frspec_remap(V, V, 3)
+    r = ops.frspec_head_topk(to_dev(torch, hid), ops.tile_head_weight(to_dev(torch, w)), to_dev(torch, remap), top)
+    torch.cuda.synchronize()
+    st = to_np(r["row_stats"])
+    lp = orc.log_softmax_apply(to_np(r["logits"]), st[:, 0], st[:, 1])
+    v_ref, p_ref = orc.topk(lp, top)
+    assert np.array_equal(to_np(r["pos"]), p_ref) and np.array_equal(to_np(r["ids"]), remap[p_ref])
+    assert np.array_equal(to_np(r["val"]).view(np.uint16), v_ref.view(np.uint16))
