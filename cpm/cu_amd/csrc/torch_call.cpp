@@ -113,8 +113,8 @@ struct Caller<R (*)(A...)> {
 #define CPMCU_TORCH_CALLS(X)                                                                                              \
     X(kv_append) X(rope_table) X(rope_apply) X(tree_attention) X(tree_attention_rope) X(tree_attention_window)            \
     X(tree_attention_workspace_bytes) X(gather_rows) X(head_weight_tile) X(head_workspace_bytes) X(frspec_head_topk)      \
-    X(lm_head_argmax) X(log_softmax) X(topk) X(topk_workspace_bytes) X(remap) X(tree_accept) X(kv_compact)                \
-    X(accept_commit) X(verify_tail) X(verify_tail_inplace) X(draft_tree_begin) X(draft_tree_extend) X(draft_tree_finish)
+    X(lm_head_argmax) X(log_softmax_sliced) X(log_softmax_workspace_bytes) X(topk) X(topk_workspace_bytes) X(remap)       \
+    X(tree_accept) X(kv_compact) X(accept_commit) X(verify_tail) X(verify_tail_inplace) X(draft_tree_begin) X(draft_tree_extend) X(draft_tree_finish)
 
 #define X(name)                                                                                                    \
     decltype(&cpmcu_##name) fn_##name = nullptr;                                                                   \

@@ -276,7 +276,8 @@ def log_softmax_(x):
     n, dim = x.shape
     native = _native or _calls()
     stats, = native.empty(x, "f", n, 2)
-    native.log_softmax(x, n, dim, stats)
+    ws = _workspace("softmax", native.log_softmax_workspace_bytes(n, dim), x.device)
+    native.log_softmax_sliced(x, n, dim, stats, ws, ws.numel())
     return stats
 
 

@@ -497,6 +497,9 @@ int cpmcu_lm_head_argmax_static(const void* hidden, const void* w, int w_layout,
 /* log_softmax in place -- src/model/eagle.cuh:29-89.  x [n][dim] fp16 (bf16 under the dtype option), any dim, 2-byte
  * alignment is enough; row_stats [n][2] fp32 (max, ln sum) output, may be NULL. */
 int cpmcu_log_softmax(void* x, int n, int dim, float* row_stats, void* stream);
+/* The same with a workspace (at least cpmcu_log_softmax_workspace_bytes), which lets several workgroups share a long row. */
+size_t cpmcu_log_softmax_workspace_bytes(int n, int dim);
+int cpmcu_log_softmax_sliced(void* x, int n, int dim, float* row_stats, void* workspace, size_t workspace_bytes, void* stream);
 
 /* TopK::prefill -- src/model/topk.cuh:255-288: per row the `top` largest values,
  * value descending, ties -> lower index.  top <= min(dim, 128); any dim and any 2-byte aligned x (rows of whole
