@@ -9,7 +9,7 @@
 //   * which pages a workgroup reads follows from its number alone: the page ids are requested beside the length instead of behind
 //     it, and a bound above the length costs no imbalance;
 //   * the appended rows are a block of their own, read from k_new / v_new (split 0 takes it first, while its pages are on their
-//     way), so no tile has to be patched; workgroups of their own (grid row 0) write them to the pool meanwhile;
+//     way), so no tile has to be patched; workgroups of their own (the first grid rows) write them to the pool meanwhile;
 //   * split partials are merged by the last workgroup of a unit to arrive: nobody polls or waits, so the launch may be larger than
 //     the chip, and a unit's partials are few.
 // The products are the transposed ones of the other shapes (S^T = K.Q^T, O^T = V^T.P^T), on v_mfma_f32_16x16x32: lane (c, h) =
@@ -78,7 +78,7 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int append = p.k_new != nullptr ? 1 : 0;
     const int sh = blockIdx.x;
-    const int mt = (int)blockIdx.y - append;
+    const int mt = (int)blockIdx.y - p.append_rows;
 
     int S;
     auto clamp_length = [&]() {
@@ -91,8 +91,8 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     if (mt < 0) {  // the rows on their way into the pool
         const int runs = (p.T + kAppendRows - 1) / kAppendRows;
         constexpr int kHalves = kThreads / kAppendThreads;
-        for (int x = sh * kHalves; x < runs * p.Hkv; x += gridDim.x * kHalves) {
-            const int y = x + tid / kAppendThreads;
+        const int y = (blockIdx.y * gridDim.x + sh) * kHalves + tid / kAppendThreads;
+        if (y / kHalves * kHalves < runs * p.Hkv) {
             const int gg = p.hkv_shift >= 0 ? y & (p.Hkv - 1) : y % p.Hkv;
             const int run = p.hkv_shift >= 0 ? y >> p.hkv_shift : y / p.Hkv;
             kv_append_run<E, true>(p.k_pool_w, p.v_pool_w, p.block_table, p.k_new, p.v_new, p.rope, p.T, p.Hkv, gg, run * kAppendRows,
@@ -101,7 +101,6 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
                                  clamp_length();
                                  return S;
                              });
-            __syncthreads();
         }
         return;
     }

@@ -110,6 +110,7 @@ struct AttnParams {
     int T, Hq, Hkv, group;
     int group_shift, hkv_shift;  // log2 of group / Hkv when they are powers of two (the usual case), else -1: plain division
     int num_splits, num_mtiles, rows_pad;
+    int append_rows;  // direct shape: leading grid rows whose workgroups write the appended rows to the pool, two runs each
     int ntiles_max;  // tiles the split partition spans: ceil(max_kv_len / 64), fixed by the host-side bound
                      // (with a window: the most tiles a window can hold, counted from its first tile)
     int table_pages;    // entries of block_table the caller guarantees: ceil(max_kv_len / 256)
@@ -1366,9 +1367,10 @@ uint32_t* merge_counters_for(const void* workspace, hipStream_t st) {
 // over 1-128 nodes x 128-120000 keys x 2, 4, 8 KV heads (replayed graphs, caches rotated through HBM).
 //   direct  3.4 for the launch up to its first block, 4 more for every further two workgroups per CU (two are resident); 1.05 per
 //           iteration, 1.2 once more than half of the CUs pull K/V, times the workgroups per CU of the fullest XCD (two that share a
-//           CU take 1.75 times as long at least); 0.4 of the time of the bytes at 5.5 TB/s; 2.3 for a merge by the last arrival and
+//           CU take 1.6 times as long at least); 0.6 per further 32 appended rows; 0.4 of the time of the bytes at 5.5 TB/s; 2.3 for a merge by the last arrival and
 //           0.06 per partial it reads
-//   split   10.2, 1 per 2500 keys up to 2.2 (more splits, then longer ones), the bytes, 0.05 per node; 1.5 with the rotary embedding
+//   split   10.2, 1 per 2000 keys up to 3 (more splits, then longer ones), the bytes, 0.02 per node, 3 beyond 16 units of 128 rows;
+//           1.5 with the rotary embedding
 // Measured, split -> direct, one query: 10.2 -> 6.8 at 800 keys, 12.8 -> 9.2 (with rotary 14.5 -> 9.2) at 4096, 15.4 -> 11.8 at
 // 10000, 25.7 -> 23.7 (rotary) at 60000; 10 nodes: 12.4 -> 5.9 at 256, 13.7 -> 10.2 at 4096; 16 nodes 13.9 -> 11.3; 60 nodes
 // 12.4 -> 10.0 at 800.  Where the estimates change over (60 nodes at 1500, 33 at 1500, 16 at 7000, 4 at 40000) the two are within
@@ -1379,6 +1381,7 @@ struct DirectPlan {
 };
 DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope) {
     const int units = Hkv * tiles, blocks = ceil_div(span, kBlockKeys) + 1;  // (one more for the appended rows)
+    const int new_steps = ceil_div(T, 32), split_units = Hkv * ceil_div(tiles * kDirectRows, rows_per_wg(2));
     const float stream = (float)span * Hkv * (2 * kHeadDim * sizeof(f16)) / 5.5e6f;
     const int most = std::min(kMaxSplits, std::max(256 / units, std::max(1, std::min(4, 512 / units))));
     DirectPlan d = {1, false};
@@ -1386,12 +1389,12 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope) {
     for (int it = ceil_div(blocks, most); it <= blocks; it = it < 64 ? it + 1 : it * 2) {
         const int splits = ceil_div(blocks, it);
         const float per_cu = (float)(ceil_div(splits * Hkv, kXcds) * tiles) / 32.f;
-        const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.75f);
+        const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.6f);
         const float t = 3.4f + (units * splits > 128 ? 1.2f : 1.05f) * it * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
-                        (splits > 1 ? 2.3f + 0.06f * splits : 0.f);
+                        0.6f * (new_steps - 1) + (splits > 1 ? 2.3f + 0.06f * splits : 0.f);
         if (t < best) best = t, d.splits = splits;
     }
-    const float split_shape = 10.2f + std::min(2.2f, span / 2500.f) + stream + 0.05f * T + (rope ? 1.5f : 0.f);
+    const float split_shape = 10.2f + std::min(3.f, span / 2000.f) + stream + 0.02f * T + (split_units > 16 ? 3.f : 0.f) + (rope ? 1.5f : 0.f);
     d.use = options().attn_direct >= 0 ? options().attn_direct != 0 : options().attn_kv_groups == 0 && best < split_shape;
     return d;
 }
@@ -1618,7 +1621,8 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     const dim3 grid(kXcds * ceil_div(nsh, kXcds), p.num_mtiles);
     const bool is_bf16 = options().dtype == 1;
     if (plan.direct) {
-        const dim3 dgrid(grid.x, p.num_mtiles + (k_new != nullptr ? 1 : 0));
+        p.append_rows = k_new ? ceil_div(ceil_div(T, kAppendRows) * Hkv, (int)grid.x * (kThreads / kAppendThreads)) : 0;
+        const dim3 dgrid(grid.x, p.num_mtiles + p.append_rows);
         if (is_bf16) hipLaunchKernelGGL(tree_attn_direct_bf16_kernel, dgrid, dim3(kThreads), 0, st, p);
         else hipLaunchKernelGGL(tree_attn_direct_kernel, dgrid, dim3(kThreads), 0, st, p);
         CPMCU_LAUNCH_CHECK();
