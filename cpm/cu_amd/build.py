@@ -48,7 +48,7 @@ def _torch_call_command(src, out):
     return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include",
             "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", src, "-o", out, f"-L{root}/lib",
-            "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{root}/lib"]
+            "-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{root}/lib"]
 
 
 def _stale(target, deps):

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kTopkThreads) void draft_extend_kernel(DraftState s
 constexpr int kFinishThreads = 1024;
 
 __global__ __launch_bounds__(kFinishThreads) void draft_finish_kernel(DraftState s, int k, int num_iter, int T, const int32_t* cache_length,
-                                                                      const int32_t* remap, int32_t* ids_out, int32_t* tree_pos,
+                                                                      const int32_t* remap, bool set_root, int32_t root_id, int32_t* ids_out, int32_t* tree_pos,
                                                                       uint64_t* tree_mask, int32_t* tree_parent) {
     __shared__ __attribute__((aligned(16))) uint32_t s_keys[kMaxTried];
     __shared__ int32_t s_pos[kMaxTried];     // FR-Spec index of every history entry
@@ -174,6 +174,7 @@ __global__ __launch_bounds__(kFinishThreads) void draft_finish_kernel(DraftState
         int parent = 0;
         if (tid == 0) {
             tree_pos[0] = P;
+            if (set_root) ids_out[0] = root_id;
         } else {
             int p = s_sel[tid - 1];
             tree_pos[tid] = P + (p < k ? 1 : (p - k) / kk + 2);
@@ -242,9 +243,9 @@ extern "C" int cpmcu_draft_tree_extend(void* state, int k, int num_iter, int d, 
     return CPMCU_OK;
 }
 
-extern "C" int cpmcu_draft_tree_finish(void* state, int k, int num_iter, int tree_size, const int32_t* cache_length,
-                                       const int32_t* token_id_remap, int32_t* tree_draft_ids, int32_t* tree_position_ids,
-                                       uint64_t* tree_attn_mask, int32_t* tree_parent, void* stream) {
+static int draft_tree_finish(void* state, int k, int num_iter, int tree_size, const int32_t* cache_length, const int32_t* token_id_remap,
+                             const int32_t* root_id, int32_t* tree_draft_ids, int32_t* tree_position_ids, uint64_t* tree_attn_mask,
+                             int32_t* tree_parent, void* stream) {
     CPMCU_CHECK_ARG(state && cache_length && tree_draft_ids && tree_position_ids && tree_attn_mask && tree_parent,
                     "draft_tree_finish: null pointer argument");
     if (int rc = check_shape("draft_tree_finish", k, num_iter)) return rc;
@@ -252,7 +253,20 @@ extern "C" int cpmcu_draft_tree_finish(void* state, int k, int num_iter, int tre
     CPMCU_CHECK_ARG(tree_size >= 2 && tree_size <= kMaxTree && tree_size - 1 <= total,
                     "draft_tree_finish: tree_size=%d outside [2, min(%d, history %d + 1)]", tree_size, kMaxTree, total);
     hipLaunchKernelGGL(draft_finish_kernel, dim3(1), dim3(kFinishThreads), 0, resolve_stream(stream), draft_state(state, k, num_iter), k,
-                       num_iter, tree_size, cache_length, token_id_remap, tree_draft_ids, tree_position_ids, tree_attn_mask, tree_parent);
+                       num_iter, tree_size, cache_length, token_id_remap, root_id != nullptr, root_id ? *root_id : 0, tree_draft_ids,
+                       tree_position_ids, tree_attn_mask, tree_parent);
     CPMCU_LAUNCH_CHECK();
     return CPMCU_OK;
+}
+extern "C" int cpmcu_draft_tree_finish(void* state, int k, int num_iter, int tree_size, const int32_t* cache_length,
+                                       const int32_t* token_id_remap, int32_t* tree_draft_ids, int32_t* tree_position_ids,
+                                       uint64_t* tree_attn_mask, int32_t* tree_parent, void* stream) {
+    return draft_tree_finish(state, k, num_iter, tree_size, cache_length, token_id_remap, nullptr, tree_draft_ids, tree_position_ids,
+                             tree_attn_mask, tree_parent, stream);
+}
+extern "C" int cpmcu_draft_tree_finish_root(void* state, int k, int num_iter, int tree_size, const int32_t* cache_length,
+                                            const int32_t* token_id_remap, int32_t root_id, int32_t* tree_draft_ids, int32_t* tree_position_ids,
+                                            uint64_t* tree_attn_mask, int32_t* tree_parent, void* stream) {
+    return draft_tree_finish(state, k, num_iter, tree_size, cache_length, token_id_remap, &root_id, tree_draft_ids, tree_position_ids,
+                             tree_attn_mask, tree_parent, stream);
 }

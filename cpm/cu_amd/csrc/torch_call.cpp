@@ -9,7 +9,7 @@
 // through the same module.  torch supplies memory and the stream; no torch type crosses the C-ABI.
 #include <torch/csrc/autograd/python_variable.h>
 
-#include <ATen/ops/empty.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 
 #include <dlfcn.h>
@@ -111,10 +111,10 @@ struct Caller<R (*)(A...)> {
 };
 
 #define CPMCU_TORCH_CALLS(X)                                                                                              \
-    X(kv_append) X(rope_table) X(rope_apply) X(tree_attention) X(tree_attention_rope) X(tree_attention_window)            \
-    X(tree_attention_workspace_bytes) X(gather_rows) X(head_weight_tile) X(head_workspace_bytes) X(frspec_head_topk)      \
-    X(lm_head_argmax) X(log_softmax_sliced) X(log_softmax_workspace_bytes) X(topk) X(topk_workspace_bytes) X(remap)       \
-    X(tree_accept) X(kv_compact) X(accept_commit) X(verify_tail) X(verify_tail_inplace) X(draft_tree_begin) X(draft_tree_extend) X(draft_tree_finish)
+    X(kv_append) X(rope_table) X(rope_apply) X(gather_rows) X(head_weight_tile) X(head_workspace_bytes)                   \
+    X(frspec_head_topk) X(lm_head_argmax) X(log_softmax_sliced) X(log_softmax_workspace_bytes) X(topk)                    \
+    X(topk_workspace_bytes) X(remap) X(tree_accept) X(kv_compact) X(accept_commit) X(verify_tail) X(verify_tail_inplace)  \
+    X(draft_tree_begin) X(draft_tree_extend) X(draft_tree_finish) X(draft_tree_finish_root)
 
 #define X(name)                                                                                                    \
     decltype(&cpmcu_##name) fn_##name = nullptr;                                                                   \
@@ -150,8 +150,93 @@ PyObject* call_lm_head_partials(PyObject*, PyObject* const* args, Py_ssize_t nar
     return Py_BuildValue("ii", num, stride);
 }
 
-// empty(like, dtype, rows, cols, dtype, rows, cols, ...): uninitialised [rows, cols] tensors on like's device, as a tuple.
-// dtype: 'h' 16-bit float, 'f' fp32, 'i' int32.
+// A condition on the caller's tensors; false with an AssertionError set.
+bool expect(bool ok, const char* what) {
+    if (!ok) PyErr_SetString(PyExc_AssertionError, what);
+    return ok;
+}
+const at::Tensor* tensor_or_null(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+// kv_append_rows(k_pool, v_pool, block_table, k_new, v_new, kv_len, Hkv): rows and types from the tensors.
+PyObject* call_kv_append_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 7) {
+        PyErr_Format(PyExc_TypeError, "%zd arguments given, 7 expected", nargs);
+        return nullptr;
+    }
+    void *k_pool, *v_pool;
+    const int32_t *table, *kv_len;
+    const void *k_new, *v_new;
+    int Hkv;
+    if (!(convert(args[0], &k_pool) && convert(args[1], &v_pool) && convert(args[2], &table) && convert(args[3], &k_new) &&
+          convert(args[4], &v_new) && convert(args[5], &kv_len) && convert(args[6], &Hkv)))
+        return nullptr;
+    const at::Tensor *k = tensor_or_null(args[3]), *v = tensor_or_null(args[4]), *len = tensor_or_null(args[5]);
+    if (!expect(k && v && len && k->dim() >= 1, "kv_append: tensors required") ||
+        !expect(k->scalar_type() == at::kHalf && v->scalar_type() == at::kHalf && len->scalar_type() == at::kInt, "kv_append: element types") ||
+        !expect(k->numel() == k->size(0) * Hkv * CPMCU_HEAD_DIM && v->numel() == k->numel(), "kv_append: shapes of the rows"))
+        return nullptr;
+    const int T = static_cast<int>(k->size(0));
+    void* st;
+    if (!current_stream(&st)) return nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = fn_kv_append(k_pool, v_pool, table, k_new, v_new, kv_len, T, Hkv, st);
+    Py_END_ALLOW_THREADS
+    return status(rc);
+}
+
+// tree_attention_rows(q, k_pool, v_pool, block_table, kv_len, max_kv_len, k_new, v_new, rope, block_window_size, mask, mask_k_range, Hkv,
+// scale, out, workspace, num_splits): shapes from the tensors.  None, or the bytes needed where the workspace is too small.
+decltype(&cpmcu_tree_attention_window) fn_tree_attention_window = nullptr;
+decltype(&cpmcu_tree_attention_workspace_bytes) fn_tree_attention_workspace_bytes = nullptr;
+PyObject* call_tree_attention_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 17) {
+        PyErr_Format(PyExc_TypeError, "%zd arguments given, 17 expected", nargs);
+        return nullptr;
+    }
+    const void *q, *k_new, *v_new;
+    void *k_pool, *v_pool, *out, *ws;
+    const int32_t *table, *kv_len;
+    const float* rope;
+    const uint64_t* mask;
+    int max_kv_len, window, mask_k_range, Hkv, splits;
+    float scale;
+    if (!(convert(args[0], &q) && convert(args[1], &k_pool) && convert(args[2], &v_pool) && convert(args[3], &table) && convert(args[4], &kv_len) &&
+          convert(args[5], &max_kv_len) && convert(args[6], &k_new) && convert(args[7], &v_new) && convert(args[8], &rope) &&
+          convert(args[9], &window) && convert(args[10], &mask) && convert(args[11], &mask_k_range) && convert(args[12], &Hkv) &&
+          convert(args[13], &scale) && convert(args[14], &out) && convert(args[15], &ws) && convert(args[16], &splits)))
+        return nullptr;
+    const at::Tensor *tq = tensor_or_null(args[0]), *len = tensor_or_null(args[4]), *tk = tensor_or_null(args[6]), *tv = tensor_or_null(args[7]),
+                     *tr = tensor_or_null(args[8]), *tm = tensor_or_null(args[10]), *tw = tensor_or_null(args[15]);
+    if (!expect(tq && len && tq->dim() == 3 && tq->size(2) == CPMCU_HEAD_DIM && tq->scalar_type() == at::kHalf, "tree_attention: q is [T, Hq, 128] of 16-bit floats") ||
+        !expect(len->scalar_type() == at::kInt, "tree_attention: kv_len is int32"))
+        return nullptr;
+    const int64_t T = tq->size(0), Hq = tq->size(1);
+    int W = 0;
+    if (tm) {
+        if (!expect((tm->scalar_type() == at::kLong || tm->scalar_type() == at::kUInt64) && T > 0 && tm->numel() % T == 0, "tree_attention: mask of 64-bit words, rows alike"))
+            return nullptr;
+        W = static_cast<int>(tm->numel() / T);
+    }
+    if (tk && !expect(tv && tk->scalar_type() == at::kHalf && tv->scalar_type() == at::kHalf && tk->numel() == T * Hkv * CPMCU_HEAD_DIM && tv->numel() == tk->numel(),
+                      "tree_attention: k_new and v_new are [T, Hkv, 128] of 16-bit floats"))
+        return nullptr;
+    if (tr && !expect(tr->scalar_type() == at::kFloat && tr->numel() == T * CPMCU_HEAD_DIM, "tree_attention: rope is [T, 64, 2] of floats")) return nullptr;
+    const size_t need = fn_tree_attention_workspace_bytes(static_cast<int>(T), static_cast<int>(Hq), Hkv, max_kv_len);
+    const size_t have = tw ? static_cast<size_t>(tw->nbytes()) : 0;
+    if (have < need) return PyLong_FromSize_t(need);
+    void* st;
+    if (!current_stream(&st)) return nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = fn_tree_attention_window(q, k_pool, v_pool, table, kv_len, max_kv_len, k_new, v_new, rope, window, mask, W, mask_k_range, static_cast<int>(T),
+                                  static_cast<int>(Hq), Hkv, scale, out, ws, have, splits, st);
+    Py_END_ALLOW_THREADS
+    return status(rc);
+}
+
+// empty(like, dtype, rows, cols, dtype, rows, cols, ...): uninitialised [rows, cols] tensors ([rows] where cols is 0) on like's
+// device, as a tuple.  dtype: 'h' 16-bit float, 'f' fp32, 'i' int32, 'l' int64.
 PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (nargs < 4 || (nargs - 1) % 3 != 0 || !THPVariable_Check(args[0])) {
         PyErr_SetString(PyExc_TypeError, "empty(tensor, dtype, rows, cols, ...) expected");
@@ -169,8 +254,9 @@ PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                 Py_DECREF(out);
                 return nullptr;
             }
-            const auto type = code[0] == 'h' ? at::kHalf : code[0] == 'f' ? at::kFloat : at::kInt;
-            PyObject* t = THPVariable_Wrap(at::empty({rows, cols}, at::TensorOptions().dtype(type).device(device)));
+            const auto type = code[0] == 'h' ? at::kHalf : code[0] == 'f' ? at::kFloat : code[0] == 'l' ? at::kLong : at::kInt;
+            const int64_t sizes[2] = {rows, cols};
+            PyObject* t = THPVariable_Wrap(at::detail::empty_cuda(at::IntArrayRef(sizes, cols ? 2 : 1), type, device, std::nullopt));
             if (!t) {
                 Py_DECREF(out);
                 return nullptr;
@@ -212,7 +298,9 @@ PyObject* bind(PyObject*, PyObject* handle) {
         if (!*slot) PyErr_Format(PyExc_ImportError, "the library does not export %s", name);
         return *slot != nullptr;
     };
-    bool ok = find("cpmcu_last_error", &g_last_error) && find("cpmcu_lm_head_partials", &fn_lm_head_partials);
+    bool ok = find("cpmcu_last_error", &g_last_error) && find("cpmcu_lm_head_partials", &fn_lm_head_partials) &&
+              find("cpmcu_tree_attention_window", &fn_tree_attention_window) &&
+              find("cpmcu_tree_attention_workspace_bytes", &fn_tree_attention_workspace_bytes);
 #define X(name) ok = ok && find("cpmcu_" #name, &fn_##name);
     CPMCU_TORCH_CALLS(X)
 #undef X
@@ -224,6 +312,8 @@ PyObject* bind(PyObject*, PyObject* handle) {
 PyMethodDef g_methods[] = {
     CPMCU_TORCH_CALLS(X)
     X(lm_head_partials)
+    X(kv_append_rows)
+    X(tree_attention_rows)
     {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(empty)), METH_FASTCALL, nullptr},
     {"synchronize", synchronize, METH_NOARGS, nullptr},
     {"bind", bind, METH_O, nullptr},

@@ -40,8 +40,8 @@ class VerifyStep:
         self.pos = tree_positions
         self.head_scale = head_scale
         self.P = int(prefix_len)
-        self.cache_length = torch.tensor([self.P], dtype=torch.int32, device=dev)         # P
-        self.kv_len = torch.tensor([self.P + self.T], dtype=torch.int32, device=dev)       # P + T (cpmcu/llm.py:272)
+        self.cache_length = torch.full((1,), self.P, dtype=torch.int32, device=dev)      # P
+        self.kv_len = torch.full((1,), self.P + self.T, dtype=torch.int32, device=dev)    # P + T (cpmcu/llm.py:272)
         self.max_kv_len = (self.P + self.T + 127) // 128 * 128                            # padded_length (cpmcu/llm.py:273)
         self.gt = torch.empty(self.T, dtype=torch.int32, device=dev)
         self.best = torch.zeros(2, dtype=torch.int32, device=dev)

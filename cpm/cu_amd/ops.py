@@ -86,10 +86,7 @@ def mask_words(T):
 
 def kv_append(cache, layer, k_new, v_new, kv_len):
     """copy_to_kvcache (src/model/attn.cuh:14-21): rows go to positions [*kv_len - T, *kv_len)."""
-    T, Hkv = k_new.shape[0], cache.Hkv
-    assert k_new.dtype == torch.float16 and v_new.dtype == torch.float16 and kv_len.dtype == torch.int32
-    assert k_new.numel() == T * Hkv * HEAD_DIM == v_new.numel()
-    (_native or _calls()).kv_append(cache.k[layer], cache.v[layer], cache.block_table, k_new, v_new, kv_len, T, Hkv)
+    (_native or _calls()).kv_append_rows(cache.k[layer], cache.v[layer], cache.block_table, k_new, v_new, kv_len, cache.Hkv)
 
 
 def rope_table(position_ids, inv_freq):
@@ -120,32 +117,16 @@ def tree_attention(q, cache, layer, kv_len, max_kv_len, mask=None, scale=None, n
     block_window_size (0 = none, else >= 128 tokens): the drafter layer's block sliding window
     (src/flash_attn/src/flash_blockmask.h:32): key blocks of 128 below ceil(P/128) - window/128 are skipped.
     """
-    T, Hq, D = q.shape
-    assert D == HEAD_DIM and q.dtype == torch.float16 and kv_len.dtype == torch.int32
-    native, Hkv, max_kv_len = _native or _calls(), cache.Hkv, int(max_kv_len)
+    native = _native or _calls()
     if out is None:
         out = torch.empty_like(q)
-    W = 0
-    if mask is not None:
-        assert mask.dtype == torch.int64 or mask.dtype == torch.uint64
-        if mask.dim() != 2 or mask.shape[0] != T:
-            mask = mask.reshape(T, -1)
-        W = mask.shape[1]
-    ws = _workspace("attn", native.tree_attention_workspace_bytes(T, Hq, Hkv, max_kv_len), q.device)
-    if k_new is not None:
-        assert k_new.dtype == torch.float16 and v_new.dtype == torch.float16
-        assert k_new.numel() == T * Hkv * HEAD_DIM == v_new.numel()
-    head = (q, cache.k[layer], cache.v[layer], cache.block_table, kv_len, max_kv_len, k_new, v_new)
-    tail = (mask, W, int(mask_k_range), T, Hq, Hkv, _SCALE if scale is None else scale, out, ws, ws.numel(), int(num_splits))
-    if rope is not None:
-        assert rope.dtype == torch.float32 and rope.numel() == T * HEAD_DIM
-    if block_window_size:
-        native.tree_attention_window(*head, rope, int(block_window_size), *tail)
-    elif rope is not None:
-        # rotary embedding of q and of the appended K rows fused into the kernel (table from rope_table)
-        native.tree_attention_rope(*head, rope, *tail)
-    else:
-        native.tree_attention(*head, *tail)
+    ws = _workspaces.get(("attn", q.device))
+    # (shapes and types are checked there)
+    args = (q, cache.k[layer], cache.v[layer], cache.block_table, kv_len, int(max_kv_len), k_new, v_new, rope, int(block_window_size),
+            mask, int(mask_k_range), cache.Hkv, _SCALE if scale is None else scale, out)
+    need = native.tree_attention_rows(*args, ws, int(num_splits))
+    if need is not None:
+        native.tree_attention_rows(*args, _workspace("attn", need, q.device), int(num_splits))
     return out
 
 
@@ -356,15 +337,14 @@ class DraftTree:
     def finish(self, tree_size, cache_length, tree_draft_ids=None):
         """cache_length int32[1] on the device = P.  Returns (ids [T] -- entry 0 untouched --, positions [T],
         mask [T, W] as int64 bit patterns, parent [T])."""
-        T = int(tree_size)
-        dev = self.state.device
+        native, T = _native or _calls(), int(tree_size)
         W = mask_words(T)
-        if tree_draft_ids is None:
-            tree_draft_ids = torch.full((T,), -1, dtype=torch.int32, device=dev)
-        pos = torch.empty(T, dtype=torch.int32, device=dev)
-        mask = torch.empty((T, W), dtype=torch.int64, device=dev)
-        parent = torch.empty(T, dtype=torch.int32, device=dev)
-        (_native or _calls()).draft_tree_finish(self.state, self.k, self.num_iter, T, cache_length, self.remap, tree_draft_ids, pos, mask, parent)
+        if tree_draft_ids is not None:
+            pos, mask, parent = native.empty(self.state, "i", T, 0, "l", T, W, "i", T, 0)
+            native.draft_tree_finish(self.state, self.k, self.num_iter, T, cache_length, self.remap, tree_draft_ids, pos, mask, parent)
+        else:
+            tree_draft_ids, pos, mask, parent = native.empty(self.state, "i", T, 0, "i", T, 0, "l", T, W, "i", T, 0)
+            native.draft_tree_finish_root(self.state, self.k, self.num_iter, T, cache_length, self.remap, -1, tree_draft_ids, pos, mask, parent)
         return tree_draft_ids, pos, mask, parent
 
 

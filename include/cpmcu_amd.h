@@ -607,6 +607,10 @@ int cpmcu_draft_tree_extend(void* state, int k, int num_iter, int d, void* topk_
 int cpmcu_draft_tree_finish(void* state, int k, int num_iter, int tree_size, const int32_t* cache_length,
                             const int32_t* token_id_remap, int32_t* tree_draft_ids, int32_t* tree_position_ids,
                             uint64_t* tree_attn_mask, int32_t* tree_parent, void* stream);
+/* The same with entry 0 of the ids, which finish leaves to the caller, set to root_id. */
+int cpmcu_draft_tree_finish_root(void* state, int k, int num_iter, int tree_size, const int32_t* cache_length,
+                                 const int32_t* token_id_remap, int32_t root_id, int32_t* tree_draft_ids, int32_t* tree_position_ids,
+                                 uint64_t* tree_attn_mask, int32_t* tree_parent, void* stream);
 
 #ifdef __cplusplus
 }
