@@ -714,10 +714,14 @@ __device__ __forceinline__ void log_softmax_partial_body(uint16_t* x, int dim, f
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < kSoftmaxThreads / 64; ++w) m = fmaxf(m, red[0][w]);
-    float sum = s.single >= 0 ? expf(s.single_v - m) : 0.f;
+    // A slice of nothing but -inf (a masked range, a padded vocabulary) adds nothing: its own maximum would make every term NaN.  In a
+    // row without a finite value, with +inf or with NaN the sums come out as in the form above: the apply meets -inf - -inf, this
+    // inf - inf, and NaN stays NaN.
+    const float ref = m == -INFINITY ? 0.f : m;
+    float sum = s.single >= 0 ? expf(s.single_v - ref) : 0.f;
     if (s.piece) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sum += expf(s.v[j] - m);
+        for (int j = 0; j < 8; ++j) sum += expf(s.v[j] - ref);
     }
     sum = wave_sum_f32(sum);
     if (lane == 0) red[1][wave] = sum;

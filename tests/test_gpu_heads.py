@@ -503,6 +503,47 @@ def test_log_softmax_operator(gpu, orc, n, dim, off):
     assert not to_np(buf[:off]).any() and not to_np(buf[off + n * dim:]).any()  # nothing written outside the rows
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("dim,off", [(73449, 0), (73448, 3), (16384, 0), (20001, 1)])
+def test_log_softmax_with_masked_ranges(gpu, orc, set_option, dim, off, bf16):
+    """-inf over the first, a middle and the last slice of 8192 elements (on and across slice borders), over all but one element, and
+    over a whole row; +inf and NaN in a row: a masked range takes nothing from the others, and what has no log-probabilities (no finite
+    value, +inf, NaN) is NaN throughout, as with one workgroup per row."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    set_option("dtype", int(bf16))
+    orc.set_dtype("bf16" if bf16 else "f16")
+    try:
+        S, inf, nan = 8192, float("inf"), float("nan")
+        x = (synth.rng(dim, 5 + off).standard_normal((9, dim)) * 1.3).astype(np.float32)
+        x[0, : S + 9] = -inf
+        x[1, S - 9 : 2 * S + 9] = -inf
+        x[2, dim - dim % S - 9 if dim % S else dim - S :] = -inf
+        x[3, : dim - 1] = -inf
+        x[4, 1:] = -inf
+        x[5] = -inf
+        x[6, : dim - 1] = -inf
+        x[6, 17] = nan
+        x[7, 3] = inf
+        x[8] = nan
+        t = torch.from_numpy(x).to(torch.bfloat16 if bf16 else torch.float16).view(torch.float16)
+        buf = torch.zeros(t.numel() + 8, dtype=torch.float16, device="cuda")
+        d = buf[off:off + t.numel()].view(t.shape)
+        d.copy_(t.cuda())
+        stats = to_np(ops.log_softmax_(d))
+        rows = to_np(t)[:5]
+        _, m_ref, lse_ref = orc.log_softmax(rows)
+        assert np.array_equal(stats[:5, 0], m_ref)
+        assert np.allclose(stats[:5, 1], lse_ref, atol=1e-4)
+        assert np.array_equal(to_np(d[:5]).view(np.uint16), orc.log_softmax_apply(rows, stats[:5, 0], stats[:5, 1]).view(np.uint16))
+        assert np.isnan(stats[5:, 1]).all()
+        rest = d[5:].view(torch.bfloat16 if bf16 else torch.float16)
+        assert bool(torch.isnan(rest.float()).all())
+        assert not to_np(buf[:off]).any() and not to_np(buf[off + t.numel():]).any()
+    finally:
+        orc.set_dtype("f16")
+
+
 @pytest.mark.parametrize("n,V,H", [(60, 1000 + 7, 512), (10, 4096, 1024), (24, 530, 2048), (128, 2000, 512), (1, 16, 512)])
 def test_tiled_weight_layout_gives_the_same_logits(gpu, orc, n, V, H):
     """The tiled layout holds the same numbers in another order.  The kernels chosen for the two layouts
