@@ -256,9 +256,9 @@ def log_softmax_(x):
     """In place (src/model/eagle.cuh:29-89); returns row_stats [n,2] (max, ln sum)."""
     n, dim = x.shape
     native = _native or _calls()
-    stats, = native.empty(x, "f", n, 2)
-    ws = _workspace("softmax", native.log_softmax_workspace_bytes(n, dim), x.device)
-    native.log_softmax_sliced(x, n, dim, stats, ws, ws.numel())
+    # (the slices' few bytes are the call's own, as the outputs are: calls on several streams or threads, and captured ones, share nothing)
+    stats, ws = native.empty(x, "f", n, 2, "f", native.log_softmax_workspace_bytes(n, dim) // 4, 0)
+    native.log_softmax_sliced(x, n, dim, stats, ws, ws.nbytes)
     return stats
 
 

@@ -544,6 +544,47 @@ def test_log_softmax_with_masked_ranges(gpu, orc, set_option, dim, off, bf16):
         orc.set_dtype("f16")
 
 
+def test_log_softmax_calls_share_nothing(gpu):
+    """Calls on two streams at once, and replays of a captured call between eager calls with more rows: the bits of the same call
+    made alone, every time."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rows = [torch.randn((n, 73449), device="cuda", generator=g, dtype=torch.float32).half() * s for n, s in ((3, 1.0), (5, 4.0))]
+
+    def alone(x):
+        y = x.clone()
+        st = ops.log_softmax_(y)
+        torch.cuda.synchronize()
+        return y.view(torch.int16), st.clone()
+
+    want = [alone(x) for x in rows]
+    same = lambda i, y, st: torch.equal(y.view(torch.int16), want[i][0]) and torch.equal(st, want[i][1])
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for rep in range(20):
+        work = [x.clone() for x in rows]
+        torch.cuda.synchronize()
+        stats = [None, None]
+        for i in (0, 1):
+            with torch.cuda.stream(streams[i]):
+                stats[i] = ops.log_softmax_(work[i])
+        torch.cuda.synchronize()
+        assert same(0, work[0], stats[0]) and same(1, work[1], stats[1]), rep
+    held = rows[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        st_held = ops.log_softmax_(held)
+    for rep in range(4):
+        y = rows[1].clone()
+        st = ops.log_softmax_(y)
+        later = [torch.zeros(256 * k, dtype=torch.uint8, device="cuda") for k in range(1, 9)]  # what a freed buffer would be given to
+        held.copy_(rows[0])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same(1, y, st) and same(0, held, st_held), rep
+        assert not any(bool(t.any()) for t in later)
+
+
 @pytest.mark.parametrize("n,V,H", [(60, 1000 + 7, 512), (10, 4096, 1024), (24, 530, 2048), (128, 2000, 512), (1, 16, 512)])
 def test_tiled_weight_layout_gives_the_same_logits(gpu, orc, n, V, H):
     """The tiled layout holds the same numbers in another order.  The kernels chosen for the two layouts
