@@ -11,6 +11,7 @@
 
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <dlfcn.h>
 
@@ -23,6 +24,39 @@
 namespace {
 
 const char* (*g_last_error)(void) = nullptr;
+
+template <typename Body>
+auto without_gil(Body body) {
+    struct Released {
+        PyThreadState* state = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(state); }
+    } released;
+    return body();
+}
+
+// Every entry of the module goes through one of these.  Asking a tensor for its memory or its layout throws where it has none (vmapped,
+// fake, meta or sparse tensors), as do streams without a device: that is Python's RuntimeError, and must not cross the interpreter's C frames.
+template <typename Body>
+PyObject* guarded(Body body) {
+    try {
+        return body();
+    } catch (const c10::Error& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (...) {
+        PyErr_SetString(PyExc_RuntimeError, "an exception of unknown type");
+    }
+    return nullptr;
+}
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyObject* entry(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+    return guarded([&] { return F(self, args, nargs); });
+}
+template <PyObject* (*F)(PyObject*, PyObject*)>
+PyObject* entry(PyObject* self, PyObject* arg) {
+    return guarded([&] { return F(self, arg); });
+}
 
 // One C argument from one Python object; false with a Python error set.
 template <typename T>
@@ -57,19 +91,12 @@ bool convert(PyObject* o, T* out) {
     return !PyErr_Occurred();
 }
 
-// torch's current stream; false with a Python error set where there is no device.  torch's default stream is HIP's null
-// stream, which the library has to be told apart from "its own blocking stream": every launch on a blocking stream is
-// ordered behind the null stream by a marker packet, 7-8 us between two launches (append of 9 rows in a row: 10.5 us each, 3 on
-// the null stream itself).
-bool current_stream(void** out) {
-    try {
-        *out = reinterpret_cast<void*>(c10::hip::getCurrentHIPStream().stream());
-        if (*out == nullptr) *out = CPMCU_STREAM_LEGACY;
-        return true;
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return false;
-    }
+// torch's current stream.  torch's default stream is HIP's null stream, which the library has to be told apart from "its own
+// blocking stream": every launch on a blocking stream is ordered behind the null stream by a marker packet, 7-8 us between two
+// launches (append of 9 rows in a row: 10.5 us each, 3 on the null stream itself).
+void* current_stream() {
+    void* const st = reinterpret_cast<void*>(c10::hip::getCurrentHIPStream().stream());
+    return st ? st : CPMCU_STREAM_LEGACY;
 }
 
 PyObject* status(int rc) {
@@ -99,12 +126,8 @@ struct Caller<R (*)(A...)> {
         }
         Args a;
         if (!fill(a, args, std::make_index_sequence<kGiven>{})) return nullptr;
-        if constexpr (kStream)
-            if (!current_stream(&std::get<kAll - 1>(a))) return nullptr;
-        R r;
-        Py_BEGIN_ALLOW_THREADS
-        r = std::apply(fn, a);
-        Py_END_ALLOW_THREADS
+        if constexpr (kStream) std::get<kAll - 1>(a) = current_stream();
+        const R r = without_gil([&] { return std::apply(fn, a); });
         if constexpr (std::is_same_v<R, int>) return status(r);
         else return PyLong_FromSize_t(r);
     }
@@ -140,12 +163,9 @@ PyObject* call_lm_head_partials(PyObject*, PyObject* const* args, Py_ssize_t nar
           convert(args[5], &H) && convert(args[6], &apply_scale) && convert(args[7], &scale) && convert(args[8], &logits) &&
           convert(args[9], &ws) && convert(args[10], &ws_bytes)))
         return nullptr;
-    void* st;
-    if (!current_stream(&st)) return nullptr;
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = fn_lm_head_partials(hidden, w, layout, n, V, H, apply_scale, scale, logits, ws, ws_bytes, &num, &stride, st);
-    Py_END_ALLOW_THREADS
+    void* const st = current_stream();
+    const int rc =
+        without_gil([&] { return fn_lm_head_partials(hidden, w, layout, n, V, H, apply_scale, scale, logits, ws, ws_bytes, &num, &stride, st); });
     if (rc != CPMCU_OK) return status(rc);
     return Py_BuildValue("ii", num, stride);
 }
@@ -176,13 +196,8 @@ PyObject* call_kv_append_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs
         !expect(k->numel() == k->size(0) * Hkv * CPMCU_HEAD_DIM && v->numel() == k->numel(), "kv_append: shapes of the rows"))
         return nullptr;
     const int T = static_cast<int>(k->size(0));
-    void* st;
-    if (!current_stream(&st)) return nullptr;
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = fn_kv_append(k_pool, v_pool, table, k_new, v_new, kv_len, T, Hkv, st);
-    Py_END_ALLOW_THREADS
-    return status(rc);
+    void* const st = current_stream();
+    return status(without_gil([&] { return fn_kv_append(k_pool, v_pool, table, k_new, v_new, kv_len, T, Hkv, st); }));
 }
 
 // tree_attention_rows(q, k_pool, v_pool, block_table, kv_len, max_kv_len, k_new, v_new, rope, block_window_size, mask, mask_k_range, Hkv,
@@ -225,14 +240,11 @@ PyObject* call_tree_attention_rows(PyObject*, PyObject* const* args, Py_ssize_t 
     const size_t need = fn_tree_attention_workspace_bytes(static_cast<int>(T), static_cast<int>(Hq), Hkv, max_kv_len);
     const size_t have = tw ? static_cast<size_t>(tw->nbytes()) : 0;
     if (have < need) return PyLong_FromSize_t(need);
-    void* st;
-    if (!current_stream(&st)) return nullptr;
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = fn_tree_attention_window(q, k_pool, v_pool, table, kv_len, max_kv_len, k_new, v_new, rope, window, mask, W, mask_k_range, static_cast<int>(T),
-                                  static_cast<int>(Hq), Hkv, scale, out, ws, have, splits, st);
-    Py_END_ALLOW_THREADS
-    return status(rc);
+    void* const st = current_stream();
+    return status(without_gil([&] {
+        return fn_tree_attention_window(q, k_pool, v_pool, table, kv_len, max_kv_len, k_new, v_new, rope, window, mask, W, mask_k_range,
+                                        static_cast<int>(T), static_cast<int>(Hq), Hkv, scale, out, ws, have, splits, st);
+    }));
 }
 
 // empty(like, dtype, rows, cols, dtype, rows, cols, ...): uninitialised [rows, cols] tensors ([rows] where cols is 0) on like's
@@ -243,49 +255,26 @@ PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         return nullptr;
     }
     const Py_ssize_t n = (nargs - 1) / 3;
-    PyObject* out = PyTuple_New(n);
+    THPObjectPtr out(PyTuple_New(n));
     if (!out) return nullptr;
-    try {
-        const auto device = THPVariable_Unpack(args[0]).device();
-        for (Py_ssize_t i = 0; i < n; ++i) {
-            const char* code = PyUnicode_AsUTF8(args[1 + 3 * i]);
-            const long rows = PyLong_AsLong(args[2 + 3 * i]), cols = PyLong_AsLong(args[3 + 3 * i]);
-            if (PyErr_Occurred()) {
-                Py_DECREF(out);
-                return nullptr;
-            }
-            const auto type = code[0] == 'h' ? at::kHalf : code[0] == 'f' ? at::kFloat : code[0] == 'l' ? at::kLong : at::kInt;
-            const int64_t sizes[2] = {rows, cols};
-            PyObject* t = THPVariable_Wrap(at::detail::empty_cuda(at::IntArrayRef(sizes, cols ? 2 : 1), type, device, std::nullopt));
-            if (!t) {
-                Py_DECREF(out);
-                return nullptr;
-            }
-            PyTuple_SET_ITEM(out, i, t);
-        }
-    } catch (const std::exception& e) {
-        Py_DECREF(out);
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
+    const auto device = THPVariable_Unpack(args[0]).device();
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        const char* code = PyUnicode_AsUTF8(args[1 + 3 * i]);
+        const long rows = PyLong_AsLong(args[2 + 3 * i]), cols = PyLong_AsLong(args[3 + 3 * i]);
+        if (PyErr_Occurred()) return nullptr;
+        const auto type = code[0] == 'h' ? at::kHalf : code[0] == 'f' ? at::kFloat : code[0] == 'l' ? at::kLong : at::kInt;
+        const int64_t sizes[2] = {rows, cols};
+        PyObject* t = THPVariable_Wrap(at::detail::empty_cuda(at::IntArrayRef(sizes, cols ? 2 : 1), type, device, std::nullopt));
+        if (!t) return nullptr;
+        PyTuple_SET_ITEM(out.get(), i, t);
     }
-    return out;
+    return out.release();
 }
-
-struct WithoutGil {
-    PyThreadState* state = PyEval_SaveThread();
-    ~WithoutGil() { PyEval_RestoreThread(state); }
-};
 
 // synchronize(): waits for torch's current stream.
 PyObject* synchronize(PyObject*, PyObject*) {
-    try {
-        const auto stream = c10::hip::getCurrentHIPStream();
-        WithoutGil released;
-        stream.synchronize();
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
-    }
+    const auto stream = c10::hip::getCurrentHIPStream();
+    without_gil([&] { stream.synchronize(); });
     Py_RETURN_NONE;
 }
 
@@ -308,17 +297,19 @@ PyObject* bind(PyObject*, PyObject* handle) {
     Py_RETURN_NONE;
 }
 
-#define X(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call_##name)), METH_FASTCALL, nullptr},
+#define ENTRY(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(static_cast<PyObject* (*)(PyObject*, PyObject* const*, Py_ssize_t)>(entry<fn>))), METH_FASTCALL, nullptr},
+#define X(name) ENTRY(#name, call_##name)
 PyMethodDef g_methods[] = {
     CPMCU_TORCH_CALLS(X)
     X(lm_head_partials)
     X(kv_append_rows)
     X(tree_attention_rows)
-    {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(empty)), METH_FASTCALL, nullptr},
-    {"synchronize", synchronize, METH_NOARGS, nullptr},
-    {"bind", bind, METH_O, nullptr},
+    ENTRY("empty", empty)
+    {"synchronize", entry<synchronize>, METH_NOARGS, nullptr},
+    {"bind", entry<bind>, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 #undef X
+#undef ENTRY
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_torch_call", "The library's operators on torch tensors.", -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -105,3 +105,45 @@ def test_torch_binding_refuses_host_tensors():
     from cpm.cu_amd import ops
     with pytest.raises(AssertionError, match="device-resident"):
         ops._calls().kv_append(torch.zeros(4), None, None, None, None, None, 1, 1)
+
+
+_NOT_MEMORY = """
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from cpm.cu_amd import ops
+native = ops._calls()
+with FakeTensorMode(allow_non_fake_inputs=True):
+    fake = torch.empty((4, 2, 128), dtype=torch.float16, device="cuda")
+sparse = torch.sparse_coo_tensor(torch.zeros((1, 0), dtype=torch.int64), torch.zeros(0), (4,))
+calls = [lambda t: native.kv_append(t, None, None, None, None, None, 1, 1), lambda t: native.kv_append_rows(None, None, None, t, t, t, 2),
+         lambda t: native.tree_attention_rows(t, None, None, None, t, 256, None, None, None, 0, None, 0, 2, 1.0, None, None, 0),
+         lambda t: native.lm_head_partials(t, t, 0, 1, 16, 512, 0, 1.0, None, None, 0), lambda t: native.empty(t, "h", 4, 0), lambda t: native.topk(t, 1, 4, 1, t, t, t, 0)]
+seen = []
+def vmapped(t):
+    seen.append(t)
+    for call in calls:
+        refused(call, t)
+    return t
+def refused(call, t):
+    try:
+        call(t)
+    except (RuntimeError, AssertionError):
+        return
+    raise SystemExit("accepted: %r" % t)
+for t in (fake, sparse):
+    for call in calls:
+        refused(call, t)
+with FakeTensorMode(allow_non_fake_inputs=True):
+    torch.func.vmap(vmapped)(fake)
+assert len(seen) == 1
+print("all refused")
+"""
+
+
+def test_torch_binding_raises_for_tensors_without_memory():
+    """Vmapped, fake and sparse tensors throw when they are asked for their layout or memory: a Python error, not the end of the
+    process (hence one of its own)."""
+    import subprocess
+    import sys
+    res = subprocess.run([sys.executable, "-c", _NOT_MEMORY], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert res.returncode == 0 and "all refused" in res.stdout, res.stdout
