@@ -35,11 +35,8 @@ def _calls():
 
 
 def _ptr_result(t):
-    """A device tensor, or the address of a pinned host tensor in its place: the GPU writes it through the mapped address."""
-    if t is None or t.is_cuda:
-        return t
-    assert t.is_pinned() and t.is_contiguous(), "device-resident or pinned contiguous tensor required"
-    return t.data_ptr()
+    """A device tensor, or a pinned host tensor in its place: the GPU writes it through the mapped address."""
+    return t if t is None or t.is_cuda else (_native or _calls()).pinned(t)
 
 
 _workspaces = {}

@@ -107,6 +107,25 @@ def test_torch_binding_refuses_host_tensors():
         ops._calls().kv_append(torch.zeros(4), None, None, None, None, None, 1, 1)
 
 
+@pytest.mark.parametrize("address", [4096, True, 0, 2.5, object()])
+def test_torch_binding_takes_no_bare_addresses(address):
+    """Where a pointer goes, only tensors, None and what pinned() has looked at: a number that strayed there is refused, not written to."""
+    import torch
+    from cpm.cu_amd import ops
+    native = ops._calls()
+    for pos in range(6):
+        args = [None] * 6 + [1, 1]
+        args[pos] = address
+        with pytest.raises(TypeError, match="a tensor or None required"):
+            native.kv_append(*args)
+    with pytest.raises(TypeError, match="a tensor or None required"):
+        native.tree_attention_rows(None, None, None, None, None, 256, None, None, None, 0, address, 0, 2, 1.0, None, None, 0)
+    with pytest.raises(AssertionError, match="pinned"):
+        ops._ptr_result(torch.zeros(4, dtype=torch.int32))
+    with pytest.raises(AssertionError, match="device-resident"):
+        native.empty(torch.zeros(4), "h", 4, 0)
+
+
 _NOT_MEMORY = """
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
