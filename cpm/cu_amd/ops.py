@@ -117,6 +117,8 @@ def tree_attention(q, cache, layer, kv_len, max_kv_len, mask=None, scale=None, n
     native = _native or _calls()
     if out is None:
         out = torch.empty_like(q)
+    if mask is not None and not mask.is_contiguous():
+        mask = mask.reshape(q.shape[0], -1)  # (a copy where the rows' order in memory is another one)
     ws = _workspaces.get(("attn", q.device))
     # (shapes and types are checked there)
     args = (q, cache.k[layer], cache.v[layer], cache.block_table, kv_len, int(max_kv_len), k_new, v_new, rope, int(block_window_size),

@@ -126,6 +126,22 @@ def test_torch_binding_takes_no_bare_addresses(address):
         native.empty(torch.zeros(4), "h", 4, 0)
 
 
+def test_tree_attention_takes_masks_that_reshape_makes_contiguous(monkeypatch):
+    """Mask rows that lie in another order in memory reach the binding as a contiguous copy in row order; contiguous ones as they are."""
+    import types
+    import torch
+    from cpm.cu_amd import ops
+    seen = []
+    monkeypatch.setattr(ops, "_native", types.SimpleNamespace(tree_attention_rows=lambda *args: seen.append(args[10])))
+    cache = types.SimpleNamespace(k=[None], v=[None], block_table=None, Hkv=2)
+    q = torch.zeros((6, 32, 128), dtype=torch.float16)
+    halves = torch.arange(12, dtype=torch.int64).reshape(2, 3, 2)
+    for mask in (halves.transpose(0, 1), halves.transpose(0, 1).contiguous(), None):
+        ops.tree_attention(q, cache, 0, None, 256, mask)
+    assert seen[0].is_contiguous() and seen[0].shape == (6, 2) and torch.equal(seen[0].flatten(), halves.transpose(0, 1).flatten())
+    assert seen[1].shape == (3, 2, 2) and seen[2] is None
+
+
 _NOT_MEMORY = """
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
