@@ -40,8 +40,6 @@ class VerifyStep:
         self.pos = tree_positions
         self.head_scale = head_scale
         self.P = int(prefix_len)
-        self.cache_length = torch.full((1,), self.P, dtype=torch.int32, device=dev)      # P
-        self.kv_len = torch.full((1,), self.P + self.T, dtype=torch.int32, device=dev)    # P + T (cpmcu/llm.py:272)
         self.max_kv_len = (self.P + self.T + 127) // 128 * 128                            # padded_length (cpmcu/llm.py:273)
         self.gt = torch.empty(self.T, dtype=torch.int32, device=dev)
         self.best = torch.zeros(2, dtype=torch.int32, device=dev)
@@ -61,6 +59,10 @@ class VerifyStep:
             # 29 us behind every step
             self.packed = torch.zeros(1 + self.T, dtype=torch.int32, pin_memory=True)
             self._packed = self.packed.numpy()
+        # Last, and from host memory: the host waits for these copies, and with them for the fills above, so that the step may be enqueued
+        # on another stream than the one it was built on.
+        self.cache_length = torch.tensor([self.P], dtype=torch.int32, device=dev)         # P
+        self.kv_len = torch.tensor([self.P + self.T], dtype=torch.int32, device=dev)      # P + T (cpmcu/llm.py:272)
 
     def enqueue(self, q_layers, k_new_layers, v_new_layers, hidden, draft_ids, attn_out=None, splits=0):
         """Enqueue one full verify step.  q_layers[l] [T,Hq,128]; k/v_new_layers[l] [T,Hkv,128];

@@ -101,3 +101,28 @@ def test_graph_replayed_steps_equal_host_driven_steps(gpu, orc):
         kb, vb = cache_b.read_logical(layer, 0, P)
         assert np.array_equal(to_np(ka).view(np.uint16), to_np(kb).view(np.uint16))
         assert np.array_equal(to_np(va).view(np.uint16), to_np(vb).view(np.uint16))
+
+
+@pytest.mark.parametrize("commit", [False, True])
+def test_step_is_ready_on_every_stream_when_built(gpu, commit):
+    """Built on a stream that is busy, read and written on another one without a wait: the lengths are there, and no fill of the
+    constructor is still to come."""
+    from cpm.cu_amd.driver import VerifyStep
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch = gpu
+    tree = synth.random_tree(T, 1, max_children=3, max_depth=6)
+    args = [torch.from_numpy(x).cuda() for x in (tree.mask.view(np.int64), tree.parent, tree.positions(P0))]
+    cache = PagedKVCache(1, HKV, 5)
+    used, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(used):
+        torch.cuda._sleep(20_000_000)
+        step = VerifyStep(cache, None, *args, P0, commit=commit)
+    with torch.cuda.stream(other):
+        lengths = torch.cat([step.cache_length, step.kv_len]).cpu()
+        for t in [step.best, step.path] + ([step.next_positions] if commit else []):
+            t.fill_(7)
+    torch.cuda.synchronize()
+    assert lengths.tolist() == [P0, P0 + T]
+    assert bool((step.best == 7).all()) and bool((step.path == 7).all())
+    assert not commit or bool((step.next_positions == 7).all())
