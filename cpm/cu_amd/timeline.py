@@ -1,6 +1,7 @@
 """Where the time of a launch goes, from wall-clock stamps taken inside the kernels.
 
-    python -m cpm.cu_amd.timeline attention [P ...] [--rows T]   tree attention, T-node tree (default 60), prefix lengths P (default 4096)
+    python -m cpm.cu_amd.timeline attention [P ...] [--rows T]   tree attention in its split shapes, T-node tree (default 60), prefix lengths P
+                                                        (default 4096); the direct shape of short launches has no stamps
     python -m cpm.cu_amd.timeline head [n ...]          target head 73448 x 4096, n hidden rows (default 60 16)
     python -m cpm.cu_amd.timeline frspec                FR-Spec head 32768 x 4096, 10 rows: two launches and one launch
 
@@ -42,10 +43,18 @@ def _spread(name, x):
 
 
 def attention(L, torch, prefixes, T=60):
+    """The split shapes, also where the library would take the direct one, which has no stamps."""
+    L.set_option(b"attn_direct", 0)
+    try:
+        _attention(torch, L, prefixes, T)
+    finally:
+        L.set_option(b"attn_direct", -1)
+
+
+def _attention(torch, L, prefixes, T):
     from . import ops, synth
     from .kvcache import PagedKVCache
     Hq, Hkv, D, NL = 32, 2, 128, 8
-    L.set_option(b"attn_direct", 0)  # the stamps are the split kernel's
     mask = None  # one row, or a chain beyond 64 rows
     if 1 < T <= 64:
         mask = torch.from_numpy(synth.eagle_tree(6, 10, T, 0).mask.view(np.int64)).cuda()

@@ -142,6 +142,18 @@ def test_tree_attention_takes_masks_that_reshape_makes_contiguous(monkeypatch):
     assert seen[1].shape == (3, 2, 2) and seen[2] is None
 
 
+@pytest.mark.parametrize("prefixes, error", [([], None), ([None], TypeError)])
+def test_attention_timeline_gives_the_choice_of_shape_back(prefixes, error):
+    import contextlib
+    import types
+    import torch
+    from cpm.cu_amd import timeline
+    told = []
+    with pytest.raises(error) if error else contextlib.nullcontext():
+        timeline.attention(types.SimpleNamespace(set_option=lambda *a: told.append(a)), torch, prefixes, 1)
+    assert told == [(b"attn_direct", 0), (b"attn_direct", -1)]
+
+
 _NOT_MEMORY = """
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
