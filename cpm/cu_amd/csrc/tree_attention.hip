@@ -1364,17 +1364,20 @@ uint32_t* merge_counters_for(const void* workspace, hipStream_t st) {
     return g_merge_ctr_base[dev] + (size_t)it->second.block * kMergeUnits * kMergeUnitWords;
 }
 // The direct shape or one of the split shapes, and the splits of the direct one: from estimates of both, in us, fitted to a sweep
-// over 1-128 nodes x 128-120000 keys x 2, 4, 8 KV heads (replayed graphs, caches rotated through HBM).
+// over 1-128 nodes x 128-120000 keys x 2, 4, 8 KV heads (replayed graphs, caches rotated).
 //   direct  3.4 for the launch up to its first block, 4 more for every further two workgroups per CU (two are resident); 1.05 per
 //           iteration, 1.2 once more than half of the CUs pull K/V, times the workgroups per CU of the fullest XCD (two that share a
-//           CU take 1.6 times as long at least); 0.6 per further 32 appended rows; 0.4 of the time of the bytes at 5.5 TB/s; 2.3 for a merge by the last arrival and
-//           0.06 per partial it reads
+//           CU take 1.6 times as long at least); 0.6 per further 32 appended rows; 0.4 of the time of the bytes at 5.5 TB/s; 2.3
+//           for a merge by the last arrival and 0.06 per partial it reads
 //   split   10.2, 1 per 2000 keys up to 3 (more splits, then longer ones), the bytes, 0.02 per node, 3 beyond 16 units of 128 rows;
 //           1.5 with the rotary embedding
-// Measured, split -> direct, one query: 10.2 -> 6.8 at 800 keys, 12.8 -> 9.2 (with rotary 14.5 -> 9.2) at 4096, 15.4 -> 11.8 at
-// 10000, 25.7 -> 23.7 (rotary) at 60000; 10 nodes: 12.4 -> 5.9 at 256, 13.7 -> 10.2 at 4096; 16 nodes 13.9 -> 11.3; 60 nodes
-// 12.4 -> 10.0 at 800.  Where the estimates change over (60 nodes at 1500, 33 at 1500, 16 at 7000, 4 at 40000) the two are within
-// 10 % of each other; beyond, the split shapes' larger tiles win (60 nodes at 4096: 15.8 / 22).
+// Measured, split / direct, us per layer, 2 KV heads (`python -m cpm.cu_amd.sweep attention --direct --graph`): one query 10.4 / 6.3 at
+// 1024 keys, 12.6 / 8.9 (with rotary 14.0 / 8.9) at 4096, 18.8 / 16.4 at 32768, 24.3 / 24.2 at 65536, 37.3 / 37.0 at 131072: direct at every
+// length.  The estimates change over at about 30000 keys with 4 nodes (19.1 / 18.2 at 32768), 12000 with 8 (15.3 / 12.4 at 8192, 16.3 /
+// 16.7 at 16384), 7000 with 16 (16.0 / 16.0 at 8192), 3000 with 24 (13.5 / 10.6 at 2048, 14.5 / 14.7 at 4096) and 900 with 33 and 60
+// (11.9 / 9.4 and 12.2 / 9.9 at 512, 13.5 / 13.4 and 13.2 / 13.9 at 1536), and leave 128 nodes to the split shapes (15.6 / 26.0 at
+// 512), whose larger tiles win beyond (60 nodes at 4096: 16.0 / 21.8).  The shape taken is within 9 % of the other one in
+// every cell of the sweep but 33 nodes at 1024 (13.0 / 11.0) and 8 nodes at 65536 on 8 KV heads (62.8 / 56.6).  The estimates cost up to 0.5 us of host time a call.
 struct DirectPlan {
     int splits;
     bool use;
@@ -1383,14 +1386,15 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope) {
     const int units = Hkv * tiles, blocks = ceil_div(span, kBlockKeys) + 1;  // (one more for the appended rows)
     const int new_steps = ceil_div(T, 32), split_units = Hkv * ceil_div(tiles * kDirectRows, rows_per_wg(2));
     const float stream = (float)span * Hkv * (2 * kHeadDim * sizeof(f16)) / 5.5e6f;
-    const int most = std::min(kMaxSplits, std::max(256 / units, std::max(1, std::min(4, 512 / units))));
+    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const int most = std::min(kMaxSplits, std::max(cus / units, std::max(1, std::min(4, 2 * cus / units))));
     DirectPlan d = {1, false};
     float best = 1e30f;
     for (int it = ceil_div(blocks, most); it <= blocks; it = it < 64 ? it + 1 : it * 2) {
         const int splits = ceil_div(blocks, it);
-        const float per_cu = (float)(ceil_div(splits * Hkv, kXcds) * tiles) / 32.f;
+        const float per_cu = (float)(ceil_div(splits * Hkv, kXcds) * tiles * kXcds) / (float)cus;
         const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.6f);
-        const float t = 3.4f + (units * splits > 128 ? 1.2f : 1.05f) * it * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
+        const float t = 3.4f + (units * splits * 2 > cus ? 1.2f : 1.05f) * it * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
                         0.6f * (new_steps - 1) + (splits > 1 ? 2.3f + 0.06f * splits : 0.f);
         if (t < best) best = t, d.splits = splits;
     }

@@ -1,9 +1,12 @@
 """Timings of the operators over ranges of shapes, with the kernels the library picks for each: looks for cliffs in the launch plans.
 
-    python -m cpm.cu_amd.sweep attention [--groups] [--heads Hq,Hkv] [--graph]
+    python -m cpm.cu_amd.sweep attention [--groups] [--direct] [--heads Hq,Hkv] [--graph] [--rope]
                                                       tree attention, prefix 256..131072 x tree rows 1..128 (us per layer);
                                                       --groups: the automatic choice beside both kernel shapes forced;
+                                                      --direct: prefix 128..262144, the split shapes beside the direct one,
+                                                      the library's choice marked;
                                                       --heads: query / KV head counts other than 32,2;
+                                                      --rope: with the rotary embedding fused;
                                                       --graph: timed inside replayed graphs (short contexts are
                                                       launch-bound when enqueued from Python)
     python -m cpm.cu_amd.sweep head                   target head (arg-max), rows 1..128 x vocabulary 8K..256K x hidden 2048/4096/8192
@@ -47,14 +50,20 @@ def _time_graph(torch, fn, reps, inner):
     return _time(torch, g.replay, reps) / inner
 
 
-def attention(torch, with_groups, Hq=32, Hkv=2, graph=False):
+def attention(torch, with_groups, Hq=32, Hkv=2, graph=False, with_direct=False, with_rope=False):
     from . import lib, ops, synth
     from .kvcache import PagedKVCache
     D = 128
     L = lib.get()
     prefixes = [256, 1024, 2048, 4096, 8192, 16384, 32768, 65536, 131072]
     rows = [1, 8, 16, 24, 32, 40, 48, 60, 64, 96, 128]
-    print("tree attention, %d query / %d KV heads: us per layer (kernel shape <G>, KV splits, +c: merge launch)" % (Hq, Hkv))
+    if with_direct:
+        prefixes = [128, 512, 1024, 1536] + prefixes[2:] + [262144]
+        rows = [1, 2, 4, 8, 10, 16, 24, 33, 60, 128]
+    inv_freq = (10000.0 ** (-torch.arange(0, D, 2, dtype=torch.float64) / D)).float().cuda()
+    print("tree attention, %d query / %d KV heads%s: us per layer (%s)" %
+          (Hq, Hkv, ", rotary embedding" if with_rope else "",
+           "split shape / direct shape with its splits, * the library's choice" if with_direct else "kernel shape <G>, KV splits, +c: merge launch; <0>: the direct shape"))
     print("%8s" % "P \\ T" + "".join("%22d" % t for t in rows))
     for P in prefixes:
         line = "%8d" % P
@@ -63,7 +72,7 @@ def attention(torch, with_groups, Hq=32, Hkv=2, graph=False):
             if 1 < T <= 64:
                 mask = torch.from_numpy(synth.eagle_tree(6, 10, T, 0).mask.view(np.int64)).cuda()
             S = P + T
-            nl = 6 if P <= 32768 else 3
+            nl = 16 if P <= 4096 else 6 if P <= 32768 else 3
             cache = PagedKVCache(nl, Hkv, (S + 255) // 256 + 1)
             for l in range(nl):
                 cache.k[l].normal_()
@@ -74,21 +83,29 @@ def attention(torch, with_groups, Hq=32, Hkv=2, graph=False):
             kv_len = torch.tensor([S], dtype=torch.int32, device="cuda")
             out = torch.empty_like(q)
             pad = (S + 127) // 128 * 128
+            table = ops.rope_table(torch.arange(P, S, dtype=torch.int32, device="cuda"), inv_freq) if with_rope else None
 
             def run():
                 for l in range(nl):
-                    ops.tree_attention(q, cache, l, kv_len, pad, mask, out=out, k_new=kn, v_new=vn)
+                    ops.tree_attention(q, cache, l, kv_len, pad, mask, out=out, k_new=kn, v_new=vn, rope=table)
             cell = []
-            for G in ((0, 1, 2) if with_groups else (0,)):
-                L.set_option(b"attn_kv_groups", G)
+            chosen = ops.attention_plan(T, Hq, Hkv, pad, with_rope)[0]
+            for G in ((0, 1, 2) if with_groups else (0, -1) if with_direct else (0,)):
+                L.set_option(b"attn_kv_groups", max(G, 0))
+                if with_direct:
+                    L.set_option(b"attn_direct", 1 if G < 0 else 0)
                 for _ in range(3):
                     run()
                 torch.cuda.synchronize()
                 us = (_time_graph(torch, run, 12, 1) if graph else _time(torch, run, 12 if P <= 32768 else 6)) / nl
-                kernels, splits, groups, _ = ops.attention_plan(T, Hq, Hkv, pad)
-                cell.append("%.1f <%d> s%d%s" % (us, groups, splits, "+c" if "combine" in kernels else ""))
+                kernels, splits, groups, _ = ops.attention_plan(T, Hq, Hkv, pad, with_rope)
+                if with_direct:
+                    cell.append("%.1f%s%s" % (us, "*" if kernels == chosen else "", " s%d" % splits if G < 0 else ""))
+                else:
+                    cell.append("%.1f <%d> s%d%s" % (us, groups, splits, "+c" if "combine" in kernels else ""))
             L.set_option(b"attn_kv_groups", 0)
-            line += "%22s" % cell[0] if not with_groups else "  [" + " | ".join(cell) + "]"
+            L.set_option(b"attn_direct", -1)
+            line += "%22s" % " / ".join(cell) if with_direct else "%22s" % cell[0] if not with_groups else "  [" + " | ".join(cell) + "]"
             del cache
         print(line, flush=True)
 
@@ -217,7 +234,7 @@ def main(argv):
     torch.cuda.set_device(0)
     if argv[0] == "attention":
         heads = argv[argv.index("--heads") + 1].split(",") if "--heads" in argv else (32, 2)
-        attention(torch, "--groups" in argv[1:], int(heads[0]), int(heads[1]), "--graph" in argv[1:])
+        attention(torch, "--groups" in argv[1:], int(heads[0]), int(heads[1]), "--graph" in argv[1:], "--direct" in argv[1:], "--rope" in argv[1:])
     elif argv[0] == "head":
         head(torch)
     elif argv[0] == "topk":
