@@ -19,6 +19,7 @@ namespace cpmcu {
 namespace {
 thread_local std::string g_error;
 hipStream_t g_stream = nullptr;
+bool capture_open();
 }  // namespace
 
 void set_error(const char* fmt, ...) {
@@ -31,8 +32,9 @@ void set_error(const char* fmt, ...) {
 }
 
 hipStream_t resolve_stream(void* stream) {
-    if (stream == CPMCU_STREAM_LEGACY) return nullptr;
-    if (stream) return (hipStream_t)stream;
+    // (work on the null stream would end a capture of the library's blocking stream: between cpmcu_capture_begin and _end it is recorded)
+    if (stream == CPMCU_STREAM_LEGACY && !capture_open()) return nullptr;
+    if (stream && stream != CPMCU_STREAM_LEGACY) return (hipStream_t)stream;
     if (!g_stream) {
         // a blocking stream, like the reference's calc_stream (src/utils.cu:19): work on the legacy
         // default stream is implicitly ordered with it
@@ -121,6 +123,7 @@ struct Model {
 };
 
 Model* g_model = nullptr;
+bool capture_open() { return g_model != nullptr && g_model->capturing; }
 constexpr int kMaxStepGraphs = 16;  // captured verify steps kept at a time (least recently used goes first)
 
 int require_model(bool need_storage) {

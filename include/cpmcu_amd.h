@@ -63,7 +63,8 @@ extern "C" {
 #define CPMCU_COMMIT_NEXT_ROOT 2
 
 /* The `stream` argument that stands for HIP's null stream (the value of hipStreamLegacy): a caller whose work is there
- * launches there, with no marker packet between its streams. */
+ * launches there, with no marker packet between its streams.  Between cpmcu_capture_begin and cpmcu_capture_end it is the
+ * library's own stream, as NULL is: the call is recorded with the others. */
 #define CPMCU_STREAM_LEGACY ((void*)1)
 
 #define CPMCU_PAGE_SIZE 256

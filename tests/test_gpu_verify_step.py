@@ -345,6 +345,55 @@ def test_step_graph_cache_is_bounded(gpu, orc):
         m.close()
 
 
+def test_operator_calls_are_recorded_in_a_caller_made_graph(gpu):
+    """Operator calls on torch's default stream between capture_begin and capture_end: recorded in order with the model-level calls
+    around them, not run; every replay gives what the eager calls give."""
+    from cpm.cu_amd import ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    from cpm.cu_amd.model import PathModel
+    torch = gpu
+    V, H, T, P = 3000, 512, 12, 300
+    m = PathModel(V, 1, H, HQ, HKV, memory_limit=0.005, tree_size=T, num_iter=4, topk=3)
+    try:
+        m.load_head(synth.normal_f16((V, H), 8, 2, std=0.02))
+        hiddens = [to_dev(torch, synth.normal_f16((T, H), 8, 100 + i)) for i in range(4)]
+        hidden, gt, ids = torch.empty_like(hiddens[0]), torch.zeros(T, dtype=torch.int32, device="cuda"), torch.zeros(T, dtype=torch.int32, device="cuda")
+        kn, vn = (to_dev(torch, synth.normal_f16((T, HKV, D), 8, i)) for i in (4, 5))
+        kv_len = torch.tensor([P + T], dtype=torch.int32, device="cuda")
+        cache = PagedKVCache(1, HKV, 3)
+
+        def calls():
+            ops.kv_append(cache, 0, kn, vn, kv_len)
+            m.L.decode_lm_head(T, hidden.data_ptr(), 0, gt.data_ptr())
+            ops._calls().remap(gt, T, table, ids)
+        table = torch.arange(V, 0, -1, dtype=torch.int32, device="cuda")
+        hidden.copy_(hiddens[0])
+        calls()
+        m.synchronize()
+        torch.cuda.synchronize()
+        k_ref, v_ref = cache.k[0].clone(), cache.v[0].clone()
+        cache.k[0].zero_(), cache.v[0].zero_(), ids.zero_()
+        torch.cuda.synchronize()
+        graph = m.capture(calls)
+        torch.cuda.synchronize()
+        assert not bool(ids.any()) and not bool(cache.k[0].any()), "the calls ran instead of being recorded"
+        for h in hiddens:
+            hidden.copy_(h)
+            cache.k[0].zero_(), cache.v[0].zero_(), ids.zero_()
+            torch.cuda.synchronize()
+            m.replay(graph)
+            m.synchronize()
+            got = ids.clone()
+            assert torch.equal(cache.k[0], k_ref) and torch.equal(cache.v[0], v_ref)
+            calls()
+            m.synchronize()
+            torch.cuda.synchronize()
+            assert torch.equal(got, ids) and bool(ids.any())
+        m.L.graph_destroy(graph)
+    finally:
+        m.close()
+
+
 @pytest.mark.parametrize("frspec", [True, False])
 def test_model_level_draft_rounds(gpu, orc, frspec):
     """cpmcu_draft_round / cpmcu_draft_finish (the drafter's state owned by the library, driven through the pybind module)
