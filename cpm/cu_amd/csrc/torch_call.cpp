@@ -9,7 +9,9 @@
 // through the same module.  torch supplies memory and the stream; no torch type crosses the C-ABI.
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/utils/object_ptr.h>
 
@@ -281,8 +283,9 @@ PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return out.release();
 }
 
-// pinned(tensor): a contiguous pinned host tensor's memory, in the place of a device tensor; the GPU writes it through the mapped
-// address.
+// pinned(tensor): a contiguous pinned host tensor's memory, in the place of a device tensor, for a call on the current stream: the GPU writes
+// it through the mapped address.  The allocator is told of the stream, so that a tensor dropped before the work is done is not
+// given to somebody else ahead of it (device memory is reused in stream order by itself).
 PyObject* pinned(PyObject*, PyObject* o) {
     if (!THPVariable_Check(o)) {
         PyErr_SetString(PyExc_TypeError, "pinned(tensor) expected");
@@ -290,6 +293,7 @@ PyObject* pinned(PyObject*, PyObject* o) {
     }
     const at::Tensor& t = THPVariable_Unpack(o);
     if (!expect(t.is_contiguous() && t.is_pinned(), "device-resident or pinned contiguous tensor required")) return nullptr;
+    at::getHostAllocator(at::kCUDA)->record_event(t.data_ptr(), t.storage().data_ptr().get_context(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
     return PyCapsule_New(t.data_ptr(), kPinned, nullptr);
 }
 

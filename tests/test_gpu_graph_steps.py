@@ -126,3 +126,23 @@ def test_step_is_ready_on_every_stream_when_built(gpu, commit):
     assert lengths.tolist() == [P0, P0 + T]
     assert bool((step.best == 7).all()) and bool((step.path == 7).all())
     assert not commit or bool((step.next_positions == 7).all())
+
+
+def test_pinned_result_outlives_the_work_that_writes_it(gpu):
+    """The pinned memory a call is to write is not handed out again while the call's stream is busy, dropped or not; afterwards it is."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    n = 12345
+    pinned = lambda: torch.empty(n, dtype=torch.int32, pin_memory=True)
+    used = torch.cuda.Stream()
+    result = pinned()
+    address = result.data_ptr()
+    with torch.cuda.stream(used):
+        torch.cuda._sleep(20_000_000)
+        ops._ptr_result(result)
+    del result
+    others = [pinned() for _ in range(4)]
+    assert not used.query(), "the stream was to be busy until here"
+    assert address not in [t.data_ptr() for t in others]
+    torch.cuda.synchronize()
+    assert address in [t.data_ptr() for t in [pinned() for _ in range(4)]]
