@@ -39,17 +39,24 @@ def _ptr_result(t):
     return t if t is None or t.is_cuda else (_native or _calls()).pinned(t)
 
 
+# One scratch buffer per operator family and device, handed to every call: calls that use it have to follow one another (one stream, or
+# streams that wait for each other).  A call that needs more gets a buffer of at least twice the size, and the old one is
+# kept, because captured launches go on writing to the addresses they were recorded with; all those kept are less than the one in use.
 _workspaces = {}
+_outgrown = []
 
 
 def _workspace(kind, nbytes, device):
     key = (kind, device)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        if ws is not None and kind == "attn":
-            release_attention_workspace(ws)
-        if ws is not None and kind == "head":
-            release_head_workspace(ws)
+        if ws is not None:
+            if kind == "attn":
+                release_attention_workspace(ws)
+            if kind == "head":
+                release_head_workspace(ws)
+            _outgrown.append(ws)
+            nbytes = max(nbytes, 2 * ws.numel())
         ws = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
     return ws

@@ -154,6 +154,25 @@ def test_attention_timeline_gives_the_choice_of_shape_back(prefixes, error):
     assert told == [(b"attn_direct", 0), (b"attn_direct", -1)]
 
 
+def test_outgrown_workspaces_stay(monkeypatch):
+    """Captured launches hold the addresses of the workspace they were recorded with: a larger one does not give it away, and what
+    is kept stays below what is in use."""
+    import torch
+    from cpm.cu_amd import ops
+    monkeypatch.setattr(ops, "_workspaces", {})
+    monkeypatch.setattr(ops, "_outgrown", [])
+    monkeypatch.setattr(ops, "release_attention_workspace", lambda ws: None)
+    cpu = torch.device("cpu")
+    for kind in ("topk", "attn"):
+        seen = []
+        for nbytes in (10, 300, 301, 40000, 39999, 70000, 10 ** 6):
+            ws = ops._workspace(kind, nbytes, cpu)
+            assert ws.numel() >= nbytes
+            seen += [ws.data_ptr()] if ws.data_ptr() not in seen else []
+        kept = [t for t in ops._outgrown if t.data_ptr() in seen]
+        assert [t.data_ptr() for t in kept] == seen[:-1] and sum(t.numel() for t in kept) < ws.numel()
+
+
 _NOT_MEMORY = """
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode

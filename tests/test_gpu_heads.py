@@ -793,6 +793,30 @@ def test_topk_of_values_that_tie_in_thousands(gpu, orc, n, dim, top, off):
     assert np.array_equal(to_np(val).view(np.uint16), v_ref.view(np.uint16))
 
 
+def test_captured_topk_outlives_its_workspace(gpu):
+    """A captured call replayed after a larger eager call has taken another workspace: its candidates still go to memory of its own."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(11)
+    x, wide = (torch.randn(s, device="cuda", generator=g).half() for s in ((2, 73449), (9, 151936)))
+    ops._workspaces.pop(("topk", x.device), None)
+    val, pos = ops.topk(x, 7)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        val_g, pos_g = ops.topk(x, 7)
+    wide_ref = ops.topk(wide, 100)
+    later = [torch.zeros(256 * k, dtype=torch.uint8, device="cuda") for k in range(1, 40)]
+    for rep in range(4):
+        x.copy_(torch.randn(x.shape, device="cuda", generator=g))
+        graph.replay()
+        again = ops.topk(wide, 100)
+        val, pos = ops.topk(x, 7)
+        torch.cuda.synchronize()
+        assert torch.equal(val, val_g) and torch.equal(pos, pos_g), rep
+        assert torch.equal(again[0], wide_ref[0]) and torch.equal(again[1], wide_ref[1]), rep
+    assert not any(bool(t.any()) for t in later)
+
+
 @pytest.mark.parametrize("V,top", [(8192, 10), (40000, 12)])
 def test_frspec_rows_of_equal_logits(gpu, orc, V, top):
     """Hidden rows of zeros and of one coarse value: the fused ranking of log-probabilities that are all, or nearly all, the same."""
