@@ -9,11 +9,13 @@
                                                       --rope: with the rotary embedding fused;
                                                       --graph: timed inside replayed graphs (short contexts are
                                                       launch-bound when enqueued from Python)
-    python -m cpm.cu_amd.sweep head                   target head (arg-max), rows 1..128 x vocabulary 8K..256K x hidden 2048/4096/8192
+    python -m cpm.cu_amd.sweep head [--row-major]     target head (arg-max), rows 1..128 x vocabulary 8K..256K x hidden 2048/4096/8192, tiled weights
+                                                      or the matrix as a checkpoint holds it
     python -m cpm.cu_amd.sweep frspec                 FR-Spec head + log-softmax + top-k + id map-back, vocabulary 8K..73448 x rows x k
     python -m cpm.cu_amd.sweep topk                   top-k of fp16 rows, row length 64..152K x rows 1..60 x k 1..128
+    python -m cpm.cu_amd.sweep softmax                log-softmax of fp16 rows: one workgroup per row beside the operator's own choice (slices)
     python -m cpm.cu_amd.sweep window                 the drafter layer's attention (k queries, block window of 1024 tokens): the
-                                                      library's plan beside both kernel shapes and forced split counts
+                                                      library's plan beside both split shapes and forced split counts
 
 Eager launches on cuda:0, random fp16 data, event-timed; attention rotates over several layers' K/V pools and the heads over
 copies of the weight matrix, so that no pass is served from the last-level cache.  Fractions are of 8 TB/s (heads) and TFLOP/s
@@ -110,20 +112,20 @@ def attention(torch, with_groups, Hq=32, Hkv=2, graph=False, with_direct=False, 
         print(line, flush=True)
 
 
-def head(torch):
+def head(torch, row_major=False):
     from . import ops
     rows = [1, 16, 17, 32, 33, 60, 64, 100, 128]
     for H in (2048, 4096, 8192):
-        print("target head, hidden size %d: fraction of 8 TB/s (kernel)" % H)
+        print("target head, hidden size %d, %s weights: fraction of 8 TB/s (kernel)" % (H, "row-major" if row_major else "tiled"))
         print("%8s" % "V \\ n" + "".join("%20d" % n for n in rows))
         for V in (8192, 16384, 32768, 50000, 73448, 100000, 131072, 151936, 200000, 262144):
             w = (torch.randn(V, H, device="cuda") * 0.02).half()
-            copies = [ops.tile_head_weight(w) for _ in range(2 if V * H * 2 < 1.5e9 else 1)]
+            copies = [w.clone() if row_major else ops.tile_head_weight(w) for _ in range(2 if V * H * 2 < 1.5e9 else 1)]
             del w
             line = "%8d" % V
             for n in rows:
                 hid = torch.randn(n, H, device="cuda").half()
-                name = ops.head_plan(n, copies[0])[0].replace("head_gemm_", "").replace("stream_kernel", "S").replace("chunked_kernel", "C")
+                name = ops.head_plan(n, copies[0])[0].replace("head_gemm_", "").replace("stream_kernel", "S").replace("chunked_kernel", "C").replace("slice_kernel", "K").replace("kernel", "R")
 
                 def run():
                     for c in copies:
@@ -188,6 +190,31 @@ def topk(torch):
             print(line, flush=True)
 
 
+def softmax(torch):
+    import ctypes
+    from . import lib, ops
+    L = lib.get()
+    print("log-softmax of fp16 rows: us per call in a replayed graph, one workgroup per row / the operator's choice")
+    rows = (1, 5, 16, 60, 128, 256)
+    print("%8s" % "dim \\ n" + "".join("%16d" % n for n in rows))
+    for dim in (4096, 8192, 8200, 16384, 32768, 50000, 73448, 73449, 151936):
+        line = "%8d" % dim
+        for n in rows:
+            xs = [torch.randn(n, dim, device="cuda").half() for _ in range(4)]
+            st = torch.empty((n, 2), dtype=torch.float32, device="cuda")
+            p = lambda t: ctypes.c_void_p(t.data_ptr())
+
+            def whole():
+                for x in xs:
+                    L.log_softmax(p(x), n, dim, p(st), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+            def own():
+                for x in xs:
+                    ops.log_softmax_(x)
+            line += "%16s" % " / ".join("%.1f" % (_time_graph(torch, fn, 12, 2) / len(xs)) for fn in (whole, own))
+        print(line, flush=True)
+
+
 def window(torch):
     from . import lib, ops
     from .kvcache import PagedKVCache
@@ -225,7 +252,7 @@ def window(torch):
 
 
 def main(argv):
-    if not argv or argv[0] not in ("attention", "head", "frspec", "topk", "window"):
+    if not argv or argv[0] not in ("attention", "head", "frspec", "topk", "softmax", "window"):
         print(__doc__)
         return 2
     import torch
@@ -236,9 +263,11 @@ def main(argv):
         heads = argv[argv.index("--heads") + 1].split(",") if "--heads" in argv else (32, 2)
         attention(torch, "--groups" in argv[1:], int(heads[0]), int(heads[1]), "--graph" in argv[1:], "--direct" in argv[1:], "--rope" in argv[1:])
     elif argv[0] == "head":
-        head(torch)
+        head(torch, "--row-major" in argv[1:])
     elif argv[0] == "topk":
         topk(torch)
+    elif argv[0] == "softmax":
+        softmax(torch)
     elif argv[0] == "window":
         window(torch)
     else:
