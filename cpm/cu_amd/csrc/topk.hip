@@ -672,7 +672,8 @@ __device__ __forceinline__ void log_softmax_body(uint16_t* x, int dim, float* ro
 }
 
 // The same for long rows, in slices of 8192 elements with a workgroup each: partial (max, sum), then the map.  One workgroup per row
-// is bound by the exponentials of its CU: 14.9 us for five rows of 73449, 9.5 in two launches; 60 rows of 151936 29 and 16.
+// is bound by the exponentials of its CU: 14.7 us for five rows of 73449 in a replayed graph, 6.8 in two launches; 60 rows of 151936 32
+// and 17.
 constexpr int kSoftmaxThreads = 1024;
 constexpr int kSoftmaxSlice = kSoftmaxThreads * 8;
 template <typename E>
@@ -911,10 +912,14 @@ extern "C" int cpmcu_log_softmax_sliced(void* x, int n, int dim, float* row_stat
     CPMCU_CHECK_ARG(((uintptr_t)x & 1) == 0, "log_softmax_sliced: x is not aligned to its elements");
     const size_t need = cpmcu_log_softmax_workspace_bytes(n, dim);
     CPMCU_CHECK_ARG(workspace && workspace_bytes >= need, "log_softmax_sliced: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
-    // a row of one slice has nothing to share; where the rows fill the GPU, each is read once by a workgroup of its own
-    if (dim <= kSoftmaxSlice || n > 65535 || (n >= 256 && dim <= 32768)) return cpmcu_log_softmax(x, n, dim, row_stats, stream);
+    // Slices take 6 to 7 us while each has a CU of its own and then grow with their number, a workgroup per row takes 4.5 us and one for
+    // every 7000 elements, whatever the number of rows up to 256.  us, whole rows / slices: 16384 elements x 1 row 5.5 / 6.1, x 128 rows
+    // 6.3 / 7.4; 24576 x 16 6.6 / 6.7; 28000 x 1 6.8 / 5.9, x 64 7.6 / 7.3, x 80 (320 slices) 7.7 / 8.8; 50000 x 80 12.0 / 11.5, x 128 13.7 /
+    // 14.7, x 256 16.5 / 22.2; 73448 x 5 14.7 / 6.8, x 128 18.8 / 17.6, x 160 19.4 / 20.1; 151936 x 60 32.2 / 17.8, x 256 54.3 / 53.9.
+    const int slices = ceil_div(dim, kSoftmaxSlice);
+    if (dim <= 3 * kSoftmaxSlice || n > 65535 || ((long long)n * slices > 256 && (long long)n * 560 > dim)) return cpmcu_log_softmax(x, n, dim, row_stats, stream);
     hipStream_t st = resolve_stream(stream);
-    const dim3 grid(ceil_div(dim, kSoftmaxSlice), n);
+    const dim3 grid(slices, n);
     if (options().dtype == 1) {
         hipLaunchKernelGGL(log_softmax_partial_bf16_kernel, grid, dim3(kSoftmaxThreads), 0, st, (uint16_t*)x, dim, (float2*)workspace);
         hipLaunchKernelGGL(log_softmax_apply_bf16_kernel, grid, dim3(kSoftmaxThreads), 0, st, (uint16_t*)x, dim, (const float2*)workspace, row_stats);

@@ -504,7 +504,7 @@ def test_log_softmax_operator(gpu, orc, n, dim, off):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("dim,off", [(73449, 0), (73448, 3), (16384, 0), (20001, 1)])
+@pytest.mark.parametrize("dim,off", [(73449, 0), (73448, 3), (32768, 0), (28001, 1), (16384, 0)])
 def test_log_softmax_with_masked_ranges(gpu, orc, set_option, dim, off, bf16):
     """-inf over the first, a middle and the last slice of 8192 elements (on and across slice borders), over all but one element, and
     over a whole row; +inf and NaN in a row: a masked range takes nothing from the others, and what has no log-probabilities (no finite
@@ -542,6 +542,25 @@ def test_log_softmax_with_masked_ranges(gpu, orc, set_option, dim, off, bf16):
         assert not to_np(buf[:off]).any() and not to_np(buf[off + t.numel():]).any()
     finally:
         orc.set_dtype("f16")
+
+
+@pytest.mark.parametrize("n,dim", [(2, 24576), (2, 24577), (64, 32768), (65, 32768), (89, 50000), (90, 50000), (1, 8 * 8192 + 1)])
+def test_log_softmax_on_either_side_of_the_choice(gpu, orc, n, dim):
+    """The last shapes that one workgroup per row takes and the first in slices (and the other way round where the slices get too many):
+    statistics and rounded values as staged from the oracle's, and the two forms' statistics beside each other.  The sums differ in
+    their order only: 1e-6 of a sum of at most 2^17 positive terms, 1e-5 of its logarithm."""
+    import ctypes
+    from cpm.cu_amd import lib, ops
+    torch = gpu
+    x = (synth.rng(dim, n).standard_normal((n, dim)) * 1.3).astype(np.float16)
+    d, whole = to_dev(torch, x), to_dev(torch, x)
+    stats = ops.log_softmax_(d)
+    st = torch.empty_like(stats)
+    lib.get().log_softmax(ctypes.c_void_p(whole.data_ptr()), n, dim, ctypes.c_void_p(st.data_ptr()), None)
+    torch.cuda.synchronize()
+    assert torch.equal(st[:, 0], stats[:, 0]) and torch.allclose(st[:, 1], stats[:, 1], rtol=0, atol=1e-5)
+    staged = orc.log_softmax_apply(x, to_np(stats)[:, 0], to_np(stats)[:, 1])
+    assert np.array_equal(to_np(d).view(np.uint16), staged.view(np.uint16))
 
 
 def test_log_softmax_calls_share_nothing(gpu):
