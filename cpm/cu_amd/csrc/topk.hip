@@ -786,8 +786,8 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const f16x8* src, cons
 
 }  // namespace
 
-// Whether the row kernel finds a bound for the k-th largest of a row of `dim` elements (else it would fall to its k rounds):
-// up to 64 any wave's lanes do; beyond, the waves that are full of elements share k, at most 64 lanes' worth each.
+// Whether the row kernel finds a bound for the k-th largest of a row of `dim` elements (else every row would take its search for
+// the exact k-th): up to 64 any wave's lanes do; beyond, the waves that are full of elements share k, at most 64 lanes' worth each.
 static bool row_kernel_ranks(int dim, int top, bool fused_stats) {
     if (top <= 64 || dim <= kRowCap) return top <= kRowMaxTop;
     const int sharing = std::min(kRowWaves, dim / 8 / 64) - (fused_stats ? 1 : 0);

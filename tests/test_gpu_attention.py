@@ -1,6 +1,6 @@
 """GPU parity of the tree-verify attention and KV append kernels against the CPU oracle.
 
-Every call goes through the C-ABI (cpm.cu_amd.ops -> ctypes -> libcpmcu_amd.so).  Tolerance of the
+Every call goes through the C-ABI (cpm.cu_amd.ops -> _torch_call -> libcpmcu_amd.so).  Tolerance of the
 path for fp16 outputs: max-abs 2e-2 and max-rel 1e-2 (see tests/util.py).
 """
 import numpy as np
