@@ -76,17 +76,43 @@ def main(argv):
         mode = ["in_cache", "append", "append_rope"][int(g.integers(3))]
         splits = [0, 0, 0, 1, 2, 3, 5, 7, 16, 17, 24, 32, 33, 64, 100, 128][int(g.integers(16))]
         slack = [0, 0, 1, 63, 64, 200, 1000][int(g.integers(7))]
-        lib.get().set_option(b"attn_kv_groups", int(g.integers(3)))  # 0 = the library's choice
+        shape = int(g.integers(4))  # 0 = the library's choice, 1 / 2 a split shape, 3 the direct shape
+        lib.get().set_option(b"attn_kv_groups", shape % 3)
+        lib.get().set_option(b"attn_direct", 1 if shape == 3 else -1)
         try:
             t_attention.test_randomised_shape_sweep(torch, orc, P, T, mode, splits, slack, seed)
         finally:
             lib.get().set_option(b"attn_kv_groups", 0)
+            lib.get().set_option(b"attn_direct", -1)
 
     def head_counts(seed):
         g = synth.rng(seed, 102)
         HKV = int([1, 1, 2, 3, 4, 8, 16, 32][g.integers(8)])
         HQ = HKV * int([1, 1, 2, 3, 4, 5, 8, 16][g.integers(8)])
-        t_attention._heads_case(torch, orc, HQ, HKV, int(g.integers(0, 4000)), int(g.integers(1, 129)), ["in_cache", "append", "append_rope"][int(g.integers(3))], seed)
+        lib.get().set_option(b"attn_direct", -1 if seed % 2 else 1)
+        try:
+            t_attention._heads_case(torch, orc, HQ, HKV, int(g.integers(0, 4000)), int(g.integers(1, 129)), ["in_cache", "append", "append_rope"][int(g.integers(3))], seed)
+        finally:
+            lib.get().set_option(b"attn_direct", -1)
+
+    def log_softmax(seed):
+        g = synth.rng(seed, 103)
+        n, dim, off = int(g.integers(1, 70)), int(np.exp(g.uniform(0, np.log(160000)))), int(g.integers(8))
+        x = (g.standard_normal((n, dim)) * float([1.3, 0.1, 20.0][g.integers(3)])).astype(np.float16)
+        for i in range(n):  # masked ranges, whole slices among them; one element at least is left
+            if g.random() < 0.5:
+                a, b = sorted(g.integers(0, dim + 1, size=2))
+                keep, value = int(g.integers(dim)), x[i].copy()
+                x[i, a:b] = -np.inf
+                x[i, keep] = value[keep]
+        buf = torch.zeros(n * dim + 8, dtype=torch.float16, device="cuda")
+        d = buf[off:off + n * dim].view(n, dim)
+        d.copy_(to_dev(torch, x))
+        stats = to_np(ops.log_softmax_(d))
+        _, m_ref, lse_ref = orc.log_softmax(x)
+        assert np.array_equal(stats[:, 0], m_ref) and np.allclose(stats[:, 1], lse_ref, atol=1e-4), "statistics"
+        assert np.array_equal(to_np(d).view(np.uint16), orc.log_softmax_apply(x, stats[:, 0], stats[:, 1]).view(np.uint16)), "rounded values"
+        assert not to_np(buf[:off]).any() and not to_np(buf[off + n * dim:]).any(), "outside the rows"
 
     def target_head(seed):
         g = synth.rng(seed, 92)
@@ -244,7 +270,7 @@ def main(argv):
         t_fused._assert_same(one, two, "V=%d n=%d k=%d std=%g" % (V, n, k, std))
         lib.get().synchronize()  # a wait that ran out would be an error here
 
-    stages = [("attention", "tree attention", attention), ("heads", "tree attention with other query / KV head counts", head_counts), ("head", "target head", target_head), ("frspec", "FR-Spec head", frspec_head),
+    stages = [("attention", "tree attention", attention), ("heads", "tree attention with other query / KV head counts", head_counts), ("head", "target head", target_head), ("frspec", "FR-Spec head", frspec_head), ("softmax", "log-softmax with masked ranges", log_softmax),
               ("topk", "top-k", topk), ("tail", "accept / compaction / tail", tail), ("draft", "draft tree", draft_tree),
               ("steps", "verify steps, eager and as graph replays", verify_steps), ("loop", "speculative loop against greedy decoding", speculative_loop),
               ("window", "drafter-layer attention: mask range, block window; window under a tree with rotary embedding", windows),
