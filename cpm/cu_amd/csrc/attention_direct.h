@@ -10,8 +10,8 @@
 //     it, and a bound above the length costs no imbalance;
 //   * the appended rows are a block of their own, read from k_new / v_new (split 0 takes it first, while its pages are on their
 //     way), so no tile has to be patched; workgroups of their own (the first grid rows) write them to the pool meanwhile;
-//   * split partials are merged by the last workgroup of a unit to arrive: nobody polls or waits, so the launch may be larger than
-//     the chip, and a unit's partials are few.
+//   * the partials of few splits are merged by the last workgroup of a unit to arrive: nobody polls or waits, so the launch may be larger
+//     than the chip.  Those of many splits are merged in shares: one query at 60001 keys 23.0 -> 19.0 us per layer, at 4096 9.0 -> 7.9.
 // The products are the transposed ones of the other shapes (S^T = K.Q^T, O^T = V^T.P^T), on v_mfma_f32_16x16x32: lane (c, h) =
 // (lane & 15, lane >> 4) of a score block holds query row c and four keys.  Which key sits in which row of the K operand is free;
 // it is chosen so that the eight probabilities of a lane of the B operand belong to eight neighbouring slots of a V^T row.
@@ -22,6 +22,8 @@
 
 constexpr int kDirectRows = 16;        // packed query rows per workgroup
 constexpr int kBlockKeys = kPage / 2;  // keys per iteration
+constexpr int kDirectItems = kDirectRows * 4;  // pieces of a unit's output that are merged by themselves: 32 dims of a row
+constexpr int kDirectLastMerges = 15;         // up to here the last arrival merges all splits
 static_assert(kThreads == kDirectRows * 32, "the merge: 32 threads per row");
 // The keys of a group of 32 make two operand blocks.  Row m of the K operand of block b of a group is its key direct_key_of_row(m) + 8 b;
 // probability j of lane (., h) of the group's B operand belongs to key 16 (h / 2) + 4 (h % 2) + j % 4 + 8 (j / 4), whose slots in
@@ -52,6 +54,23 @@ __device__ inline float half_wave(float x) {
     return with(__uint_as_float(a[0]), __uint_as_float(a[1]));
 }
 
+// the same over all 64 lanes
+template <bool MAX>
+__device__ inline float full_wave(float x) {
+    x = half_wave<MAX>(x);
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return MAX ? fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])) : __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+// x over the 16 lanes of the same number modulo 4
+__device__ inline float over_splits(float x) {
+    x += __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(x), 0x124, 0xf, 0xf, true));  // rotated by 4 in 16
+    x += __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(x), 0x128, 0xf, 0xf, true));  // by 8
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 template <typename E>
 __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     typedef typename Elem<E>::x8 X8;
@@ -65,12 +84,14 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
             char v[kWaves][kWaveBytes];
         } block;
         AppendStage append[kThreads / kAppendThreads];
-        float weight[kMaxSplits][kDirectRows];  // of the merge
+        float weight[kMaxSplits][kDirectRows];  // of the merge by the last arrival
+        f32x4 sums[kWaves][8];                  // of the merge in shares: 32 dims
     } s;
     __shared__ __attribute__((aligned(1024))) char s_q[kDirectRows * kHeadDim * 2];
     __shared__ X8 s_p[kGroups][64];                   // the probabilities of an iteration
     __shared__ f32x4 s_max[kDirectRows][kWaves / 4];  // each wave's row maxima
-    __shared__ int s_last;
+    __shared__ Arrival s_arrival;
+    __shared__ uint32_t s_abandoned[kDirectItems / 32];
     asm volatile("" ::"s"(p.q), "s"(p.k_pool), "s"(p.v_pool), "s"(p.block_table), "s"(p.kv_len), "s"(p.k_new), "s"(p.v_new), "s"(p.rope),
                  "s"(p.mask), "s"(p.mask_words), "s"(p.mask_k_range), "s"(p.T), "s"(p.Hq), "s"(p.Hkv), "s"(p.group), "s"(p.group_shift),
                  "s"(p.hkv_shift), "s"(p.num_splits), "s"(p.num_mtiles), "s"(p.table_pages), "s"(p.window_blocks), "s"(p.max_kv_len));
@@ -421,22 +442,81 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0) {
-        // the word of the other shapes: arrivals below, a generation above; the last arrival moves it on
-        uint32_t* const ctr = p.merge_ctr + kMergeUnitWords * unit;
-        const uint32_t before = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int last = (before & 0xffffu) + 1u == (uint32_t)p.num_splits ? 1 : 0;
-        if (last) __hip_atomic_fetch_add(ctr, 0x10000u - (uint32_t)p.num_splits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = last;
-    }
+    uint32_t* const ctr = p.merge_ctr + kMergeUnitWords * unit;
+    if (tid == 0) s_arrival = arrive_at_unit(p, ctr, split < p.merge_shares ? split : -1);
     __syncthreads();
-    if (!s_last) return;
+    const auto o_rsrc = __builtin_amdgcn_make_buffer_rsrc(o_part, 0, p.num_splits * kPartBytes, 0x00027000);
+    constexpr int kSc1 = 16;  // past the (per-XCD) L2
+    if (p.merge_shares > 0) {
+        // The merge in shares.  An item is 32 dims of a row, 64 bytes of each partial: a wave reads 16 splits' worth at once, and as many
+        // waves as the splits need work on an item, so that a share is one round trip.  (The last arrival alone has all 4 KB of every
+        // split to read: 0.04 us per split, 23.0 us for one query at 60001 keys on 64 splits.)
+        const int item_waves = p.num_splits <= 16 ? 1 : p.num_splits <= 32 ? 2 : p.num_splits <= 64 ? 4 : 8;
+        const int at_once = kWaves / item_waves;
+        const int items = min(kDirectRows, last_row + 1 - mt * kDirectRows) * 4;
+        auto merge_share = [&](int share) {
+            for (int i0 = share * at_once; i0 < items; i0 += p.merge_shares * at_once) {
+                const int slot = wave / item_waves, part = wave % item_waves;
+                const int item = min(i0 + slot, items - 1), row = item >> 2;
+                const int split0 = part * 16;
+                const X8 x = bits_as<X8>(__builtin_amdgcn_raw_buffer_load_b128(
+                    o_rsrc, (split0 + (lane >> 2)) * kPartBytes + item * 64 + (lane & 3) * 16, 0, kSc1));  // (zeros past the last split)
+                // the weights of all splits in every wave: lane i has those of splits i and i + 64
+                float m[2] = {-INFINITY, -INFINITY}, w[2] = {0.f, 0.f};
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const int sp = lane + 64 * k;
+                    if (64 * k < p.num_splits && sp < p.num_splits) {
+                        const uint64_t ml = load_dev64(ml_part + (sp * kDirectRows + row) * 8);
+                        m[k] = __uint_as_float((uint32_t)ml);
+                        w[k] = __uint_as_float((uint32_t)(ml >> 32));
+                    }
+                }
+                float top = full_wave<true>(fmaxf(m[0], m[1]));
+                top = top == -INFINITY ? 0.f : top;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) w[k] *= __builtin_amdgcn_exp2f(m[k] - top);
+                const float sum = full_wave<false>(w[0] + w[1]);
+                const float inv = (sum == 0.f || sum != sum) ? 1.f : 1.f / sum;
+                const float weight = __shfl(part < 4 ? w[0] : w[1], (split0 + (lane >> 2)) & 63) * inv;
+                f32x4 lo, hi;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    lo[e] = over_splits(weight * (float)x[e]);
+                    hi[e] = over_splits(weight * (float)x[e + 4]);
+                }
+                __syncthreads();  // (the area: the blocks, the items before)
+                if (lane < 4) {
+                    s.sums[wave][lane * 2] = lo;
+                    s.sums[wave][lane * 2 + 1] = hi;
+                }
+                __syncthreads();
+                const int t_slot = tid >> 3, quad = tid & 7;
+                if (t_slot < at_once && i0 + t_slot < items) {
+                    f32x4 o = s.sums[t_slot * item_waves][quad];
+                    for (int v = 1; v < item_waves; ++v) o += s.sums[t_slot * item_waves + v][quad];
+                    X4 y;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) y[e] = (E)o[e];
+                    const int R = mt * kDirectRows + ((i0 + t_slot) >> 2);
+                    *reinterpret_cast<X4*>(p.out + ((size_t)node_of(R) * p.Hq + head_of(R)) * kHeadDim + ((i0 + t_slot) & 3) * 32 + quad * 4) = y;
+                }
+            }
+        };
+        if (s_arrival.go) merge_share(split);
+        if (s_arrival.last) {
+            if (tid < kDirectItems / 32) s_abandoned[tid] = collect_abandoned(ctr, tid);
+            __syncthreads();
+            for (int v = 0; v < kDirectItems / 32; ++v)
+                for (uint32_t left = s_abandoned[v]; left != 0; left &= left - 1) merge_share(v * 32 + __builtin_ctz(left));
+        }
+        return;
+    }
+    if (!s_arrival.last) return;
 
     // The merge: a thread has four dims of a row; the weights of a row's splits are worked out once, by 32 threads.
     // Everything is requested before any of it is used, in groups of four splits that a launch of few skips.  Loads past the last
     // split return zeros, and meet a weight of zero.
-    const auto o_rsrc = __builtin_amdgcn_make_buffer_rsrc(o_part, 0, p.num_splits * kPartBytes, 0x00027000);
-    constexpr int kSc1 = 16;  // past the (per-XCD) L2
     constexpr int kInFlight = 36;
     static_assert(kMaxSplits % 4 == 0, "weights are filled up to a multiple of four");
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};

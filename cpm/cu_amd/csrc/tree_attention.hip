@@ -130,6 +130,7 @@ struct AttnParams {
     // unit, arrivals in its low 16 bits, a generation count above them.  Between launches arrivals is 0; the last
     // workgroup of a unit to arrive turns the full count into the next generation.
     uint32_t* merge_ctr;
+    int merge_shares;            // direct shape: workgroups of a unit that merge a share each (0: the last arrival merges everything)
     uint32_t merge_wait_ticks;  // longest wait for the other workgroups of a unit, in ticks of the 100 MHz wall clock
 };
 
@@ -148,6 +149,59 @@ template <typename To, typename From>
 __device__ inline To bits_as(const From& v) {
     static_assert(sizeof(To) == sizeof(From), "bits_as: size mismatch");
     return __builtin_bit_cast(To, v);
+}
+
+// A workgroup whose partials are in memory arrives at its unit (the workgroups of one KV head and M-tile, one per split) and, if
+// it has a share of the merge (share >= 0), waits until all have.  One thread.
+// The last to arrive never waits; the others wait for it, with a limit -- workgroups that wait for each other
+// must all be resident, which the host checks against the CU count but cannot promise when another launch
+// holds CUs (two such launches on one GPU could wait for each other's unstarted workgroups).  A workgroup
+// whose wait runs out marks its share as abandoned and leaves, which frees its CU; the last to arrive merges
+// the abandoned shares after its own, so the output is complete either way.
+struct Arrival {
+    int go;    // the partials of all splits are there, and this workgroup merges its share
+    int last;  // nobody arrives behind this one: it also merges what was abandoned
+};
+__device__ inline Arrival arrive_at_unit(const AttnParams& p, uint32_t* unit_ctr, int share) {
+    Arrival a = {share >= 0 ? 1 : 0, 0};
+    // One bit per share; zero between launches (a mark that was made just behind the last arrival's collection is taken back
+    // by its maker).
+    uint32_t* const mark = unit_ctr + 1 + (max(share, 0) >> 5);
+    const uint32_t bit = 1u << (share & 31);
+    // The word as this workgroup's arrival found it: the generation of this launch above, the arrivals before it below.
+    const uint32_t before = __hip_atomic_fetch_add(unit_ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t full = (before & 0xffff0000u) + (uint32_t)p.num_splits;
+    // either the full count or, once the last one has moved it on, the next generation
+    auto complete = [&](uint32_t now) { return now == full || (now & 0xffff0000u) != (before & 0xffff0000u); };
+    if (before + 1u == full) {
+        // last to arrive: full count -> next generation, no arrivals (nobody needs the result of this one)
+        __hip_atomic_fetch_add(unit_ctr, 0x10000u - (uint32_t)p.num_splits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        a.last = 1;
+    } else if (share >= 0) {
+        const unsigned long long t_begin = wall_clock64();
+        while (!complete(__hip_atomic_load(unit_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+            if (wall_clock64() - t_begin >= p.merge_wait_ticks) {
+                // The mark is in memory before this workgroup looks once more: if the others have all arrived by
+                // then, the last of them may have read the marks already, and this workgroup merges its share
+                // itself (twice the same values at worst); if not, the last one will find the mark.
+                // (acquire-release on the mark, acquire on the look that follows: the two stay in this order)
+                (void)__hip_atomic_fetch_or(mark, bit, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+                a.go = complete(__hip_atomic_load(unit_ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)) ? 1 : 0;
+                // everyone is there after all: this workgroup merges its share itself and takes its mark back, so that
+                // no mark outlives the launch (if the last arrival has collected it already, the share is merged twice
+                // with the same values)
+                if (a.go) (void)__hip_atomic_fetch_and(mark, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(&g_attn_report.abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(4);
+        }
+    }
+    return a;
+}
+// The last arrival: shares 32 w .. 32 w + 31 that were abandoned.
+__device__ inline uint32_t collect_abandoned(uint32_t* unit_ctr, int w) {
+    return __hip_atomic_exchange(unit_ctr + 1 + w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Merge of the split partials of one 32-row block and one quad of output dims (one wave; lane = accumulator lane):
@@ -1072,55 +1126,16 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         // Every workgroup of the unit (same KV head and M-tile, one per split) announces its partials once they
         // have reached memory; when all have, each merges its share of the unit's 32-row x 4-dim-quad blocks
         // (share s: the blocks b with b % splits == s).
-        // The last to arrive never waits; the others wait for it, with a limit -- workgroups that wait for each other
-        // must all be resident, which the host checks against the CU count but cannot promise when another launch
-        // holds CUs (two such launches on one GPU could wait for each other's unstarted workgroups).  A workgroup
-        // whose wait runs out marks its share as abandoned and leaves, which frees its CU; the last to arrive merges
-        // the abandoned shares after its own, so the output is complete either way.
         __shared__ int s_merge_go, s_merge_last;
         __shared__ uint32_t s_merge_abandoned;
         CPMCU_CLOCK(tl_stored);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         CPMCU_CLOCK(tl_acked);
-        uint32_t* const unit_abandoned = unit_ctr + 1;  // one bit per share; zero between launches (a mark that was made just
-                                                        // behind the last arrival's collection is taken back by its maker)
         if (tid == 0) {
-            int go = 1, last = 0;
-            // The word as this workgroup's arrival found it: the generation of this launch above, the arrivals before it below.
-            const uint32_t before = __hip_atomic_fetch_add(unit_ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint32_t full = (before & 0xffff0000u) + (uint32_t)p.num_splits;
-            auto all_arrived = [&]() {  // either the full count or, once the last one has moved it on, the next generation
-                const uint32_t now = __hip_atomic_load(unit_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                return now == full || (now & 0xffff0000u) != (before & 0xffff0000u);
-            };
-            if (before + 1u == full) {
-                // last to arrive: full count -> next generation, no arrivals (nobody needs the result of this one)
-                __hip_atomic_fetch_add(unit_ctr, 0x10000u - (uint32_t)p.num_splits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                last = 1;
-            } else {
-                const unsigned long long t_begin = wall_clock64();
-                while (!all_arrived()) {
-                    if (wall_clock64() - t_begin >= p.merge_wait_ticks) {
-                        // The mark is in memory before this workgroup looks once more: if the others have all arrived by
-                        // then, the last of them may have read the marks already, and this workgroup merges its share
-                        // itself (twice the same values at worst); if not, the last one will find the mark.
-                        // (acquire-release on the mark, acquire on the look that follows: the two stay in this order)
-                        (void)__hip_atomic_fetch_or(unit_abandoned, 1u << split, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-                        const uint32_t now = __hip_atomic_load(unit_ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-                        go = (now == full || (now & 0xffff0000u) != (before & 0xffff0000u)) ? 1 : 0;
-                        // everyone is there after all: this workgroup merges its share itself and takes its mark back, so that
-                        // no mark outlives the launch (if the last arrival has collected it already, the share is merged twice
-                        // with the same values)
-                        if (go) (void)__hip_atomic_fetch_and(unit_abandoned, ~(1u << split), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        __hip_atomic_fetch_add(&g_attn_report.abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(4);
-                }
-            }
-            s_merge_go = go;
-            s_merge_last = last;
+            const Arrival a = arrive_at_unit(p, unit_ctr, split);
+            s_merge_go = a.go;
+            s_merge_last = a.last;
         }
         __syncthreads();
         CPMCU_CLOCK(tl_go);
@@ -1128,7 +1143,7 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         const bool last = s_merge_last != 0;
         // the last one collects the abandoned shares while it merges its own
         uint32_t abandoned = 0;
-        if (last && tid == 0) abandoned = __hip_atomic_exchange(unit_abandoned, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (last && tid == 0) abandoned = collect_abandoned(unit_ctr, 0);
         const int nblocks = kRowWaves * 16;
         auto merge_share = [&](int share) {
             for (int b = share + p.num_splits * wave; b < nblocks; b += p.num_splits * kWaves)
@@ -1363,21 +1378,29 @@ uint32_t* merge_counters_for(const void* workspace, hipStream_t st) {
     if (it->second.use_combine) return nullptr;
     return g_merge_ctr_base[dev] + (size_t)it->second.block * kMergeUnits * kMergeUnitWords;
 }
+// The direct shape's merge.  Up to kDirectLastMerges splits the last arrival reads one round trip's worth of partials and nobody waits;
+// from there on sharing is the faster form (one query, last arrival / shares, us per layer: 7.07 / 7.86 on 8 splits, 7.25 / 7.47 on 12, 7.63 /
+// 7.45 on 16, 8.30 / 7.56 on 24, 9.06 / 7.90 on 33, 22.99 / 20.41 on 64, 25.42 / 19.01 on 128), if there is a CU for each
+// workgroup: those with a share wait for all others, so all have to be resident (two to a CU are not, always).
+int direct_merge_shares(int num_splits, int workgroups, int cus) {
+    return num_splits > kDirectLastMerges && workgroups <= cus ? std::min(num_splits, kDirectItems) : 0;
+}
+
 // The direct shape or one of the split shapes, and the splits of the direct one: from estimates of both, in us, fitted to a sweep
 // over 1-128 nodes x 128-120000 keys x 2, 4, 8 KV heads (replayed graphs, caches rotated).
 //   direct  3.4 for the launch up to its first block, 4 more for every further two workgroups per CU (two are resident); 1.05 per
 //           iteration, 1.2 once more than half of the CUs pull K/V, times the workgroups per CU of the fullest XCD (two that share a
 //           CU take 1.6 times as long at least); 0.6 per further 32 appended rows; 0.4 of the time of the bytes at 5.5 TB/s; 2.3
-//           for a merge by the last arrival and 0.06 per partial it reads
+//           for a merge and per partial 0.06 by the last arrival, 0.025 in shares
 //   split   10.2, 1 per 2000 keys up to 3 (more splits, then longer ones), the bytes, 0.02 per node, 3 beyond 16 units of 128 rows;
 //           1.5 with the rotary embedding
 // Measured, split / direct, us per layer, 2 KV heads (`python -m cpm.cu_amd.sweep attention --direct --graph`): one query 10.4 / 6.3 at
-// 1024 keys, 12.6 / 8.9 (with rotary 14.0 / 8.9) at 4096, 18.8 / 16.4 at 32768, 24.3 / 24.2 at 65536, 37.3 / 37.0 at 131072: direct at every
-// length.  The estimates change over at about 30000 keys with 4 nodes (19.1 / 18.2 at 32768), 12000 with 8 (15.3 / 12.4 at 8192, 16.3 /
-// 16.7 at 16384), 7000 with 16 (16.0 / 16.0 at 8192), 3000 with 24 (13.5 / 10.6 at 2048, 14.5 / 14.7 at 4096) and 900 with 33 and 60
-// (11.9 / 9.4 and 12.2 / 9.9 at 512, 13.5 / 13.4 and 13.2 / 13.9 at 1536), and leave 128 nodes to the split shapes (15.6 / 26.0 at
-// 512), whose larger tiles win beyond (60 nodes at 4096: 16.0 / 21.8).  The shape taken is within 9 % of the other one in
-// every cell of the sweep but 33 nodes at 1024 (13.0 / 11.0) and 8 nodes at 65536 on 8 KV heads (62.8 / 56.6).  The estimates cost up to 0.5 us of host time a call.
+// 1024 keys, 12.7 / 7.6 at 4096, 18.8 / 13.6 at 32768, 24.1 / 19.5 at 65536, 37.6 / 31.3 at 131072: direct at every
+// length.  The estimates change over at about 30000 keys with 4 nodes (16.1 / 12.8 at 16384, 19.0 / 17.8 at 32768), 12000 with 8 (15.3 / 12.3 at
+// 8192, 16.4 / 16.5 at 16384), 7000 with 16 (16.0 / 16.7 at 8192), 3000 with 24 (13.4 / 10.5 at 2048, 14.5 / 14.5 at 4096) and 900 with 33 and 60
+// (11.9 / 9.4 and 12.2 / 9.9 at 512, 13.5 / 13.1 and 13.2 / 13.6 at 1536), and leave 128 nodes to the split shapes (15.6 / 26.0 at
+// 512), whose larger tiles win beyond (60 nodes at 4096: 16.0 / 21.5).  The shape taken is within 9 % of the other one in
+// every cell of the sweep but 33 nodes at 1024 (12.9 / 11.2) and 8 nodes at 65536 on 8 KV heads (62.8 / 56.6).  The estimates cost up to 0.5 us of host time a call.
 struct DirectPlan {
     int splits;
     bool use;
@@ -1392,10 +1415,12 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope) {
     float best = 1e30f;
     for (int it = ceil_div(blocks, most); it <= blocks; it = it < 64 ? it + 1 : it * 2) {
         const int splits = ceil_div(blocks, it);
-        const float per_cu = (float)(ceil_div(splits * Hkv, kXcds) * tiles * kXcds) / (float)cus;
+        const int workgroups = kXcds * ceil_div(splits * Hkv, kXcds) * tiles;
+        const float per_cu = (float)workgroups / (float)cus;
         const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.6f);
+        const float merge = splits == 1 ? 0.f : 2.3f + (direct_merge_shares(splits, workgroups, cus) > 0 ? 0.025f : 0.06f) * splits;
         const float t = 3.4f + (units * splits * 2 > cus ? 1.2f : 1.05f) * it * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
-                        0.6f * (new_steps - 1) + (splits > 1 ? 2.3f + 0.06f * splits : 0.f);
+                        0.6f * (new_steps - 1) + merge;
         if (t < best) best = t, d.splits = splits;
     }
     const float split_shape = 10.2f + std::min(3.f, span / 2000.f) + stream + 0.02f * T + (split_units > 16 ? 3.f : 0.f) + (rope ? 1.5f : 0.f);
@@ -1612,6 +1637,7 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     p.o_part = nullptr;
     p.ml_part = nullptr;
     p.merge_wait_ticks = 0;
+    p.merge_shares = 0;
     if (p.num_splits > 1) {
         const size_t o_bytes = align_up((size_t)Hkv * p.num_splits * p.rows_pad * kHeadDim * sizeof(f16), 256);
         const size_t ml_bytes = (size_t)Hkv * p.num_splits * p.rows_pad * 2 * sizeof(float);
@@ -1625,6 +1651,7 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     const dim3 grid(kXcds * ceil_div(nsh, kXcds), p.num_mtiles);
     const bool is_bf16 = options().dtype == 1;
     if (plan.direct) {
+        p.merge_shares = direct_merge_shares(p.num_splits, (int)(grid.x * grid.y), device_cu_count());
         p.append_rows = k_new ? ceil_div(ceil_div(T, kAppendRows) * Hkv, (int)grid.x * (kThreads / kAppendThreads)) : 0;
         const dim3 dgrid(grid.x, p.num_mtiles + p.append_rows);
         if (is_bf16) hipLaunchKernelGGL(tree_attn_direct_bf16_kernel, dgrid, dim3(kThreads), 0, st, p);

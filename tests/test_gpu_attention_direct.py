@@ -97,3 +97,45 @@ def test_direct_shape_bf16_with_a_wider_mask(gpu, option, P, T, kd):
         assert torch.equal(out.view(torch.int16), first.view(torch.int16))
     err = (first.view(torch.bfloat16).float() - ref).norm() / ref.norm()
     assert err < 8e-3, float(err)
+
+
+@pytest.mark.parametrize("P,T,hq,hkv,splits,rope", [
+    (1900, 1, 32, 2, 15, False), (2040, 1, 32, 2, 16, True), (2100, 1, 32, 8, 17, False), (4090, 2, 32, 8, 32, True), (4200, 2, 28, 4, 33, False),
+    (4500, 1, 32, 1, 40, False), (8190, 1, 32, 2, 64, False), (8300, 5, 4, 1, 65, True), (8400, 3, 16, 2, 64, False), (16500, 1, 32, 2, 128, False),
+    (700, 1, 32, 2, 128, False), (8000, 2, 32, 2, 128, False)])
+def test_merge_in_shares_against_the_oracle(gpu, orc, option, P, T, hq, hkv, splits, rope):
+    """Around the split counts where the merge changes its form (one to eight waves an item, two row tiles, splits without a share,
+    rows that fill a tile in part, more workgroups than CUs) and with splits that have no keys."""
+    test_direct_shape_against_the_oracle(gpu, orc, option, P, T, hq, hkv, splits, 0, rope, True)
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("hkv,splits", [(2, 20), (2, 100), (8, 32)])
+def test_shares_left_behind_are_merged_by_the_last_arrival(gpu, option, hkv, splits, dtype):
+    """A wait limit of zero: every workgroup but a unit's last gives its share up (unless all have arrived); the output is the
+    same to the bit, and the launch behind it is whole again."""
+    from cpm.cu_amd import lib, ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch, L = gpu, lib.get()
+    option("dtype", dtype)
+    option("attn_direct", 1)
+    option("attn_merge_in_launch", 1)
+    S = 12901
+    g = torch.Generator(device="cuda").manual_seed(S + splits)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).to(torch.bfloat16 if dtype else torch.float16).view(torch.float16)
+    cache = PagedKVCache(1, hkv, (S + 255) // 256)
+    cache.write_logical(0, 0, rnd(S, hkv, D), rnd(S, hkv, D))
+    q, kv_len = rnd(1, 32, D), torch.tensor([S], dtype=torch.int32, device="cuda")
+    ref = ops.tree_attention(q, cache, 0, kv_len, S, num_splits=splits)
+    torch.cuda.synchronize()
+    try:
+        for wait_us in (0, 0, 2000, 0):
+            option("attn_merge_wait_us", wait_us)
+            out = torch.full_like(q, float("nan"))
+            ops.tree_attention(q, cache, 0, kv_len, S, num_splits=splits, out=out)
+            torch.cuda.synchronize()
+            assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), wait_us
+    finally:
+        option("attn_merge_wait_us", 2000)
+        L.synchronize()
+        option("attn_merge_in_launch", 1)  # (the waits that ran out had sent the workspaces back to the merge launch)
