@@ -653,6 +653,14 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
             load_to_lds16_v(p.v_new + ((size_t)r * p.Hkv + g) * kHeadDim + (lane & 15) * 8, vstage + inst * 1024);
         }
     }
+    // The rows beyond the staging area (trees of more than kVStageRows nodes, whose new rows reach into three tiles at most) go to the
+    // ring stage of the tile behind this workgroup's last, as soon as every wave has left the tile that was there: when
+    // the first tile with new rows is mended, or the one behind it.  (Read from v_new element by element where a tile is
+    // mended, they kept the last split 11 us behind the others with 128 nodes.)
+    enum { kNoLate, kLateWanted, kLateOnTheWay, kLateHere };
+    int late = p.k_new != nullptr && p.T > kVStageRows && (t0 + n) * kTileN > P + kVStageRows ? kLateWanted : kNoLate;
+    char* const late_rows = ring + (n % kStages) * kStageBytes;
+    static_assert(kMaxTree <= 2 * kVStageRows, "the new rows: staged and late");
     // The first tiles are requested into the stages the Q rows do not occupy ...
     constexpr int kPrologueTiles = (kDepth + 1) * G;  // = kStages
     constexpr int kEarlyTiles = kStages - kQStages;
@@ -758,6 +766,15 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         const int iter_end = (t0 + it * G) * kTileN + G * kTileN;
         const bool iter_needs_fix = iter_end > S || (p.k_new != nullptr && iter_end > P);
         if (iter_needs_fix) {
+            if (late == kLateWanted && it * G > n - kStages) {  // (trees of more than kVStageRows nodes)
+#pragma unroll
+                for (int qq = 0; qq < kVStageRows / (4 * kWaves); ++qq) {
+                    const int inst = wave_u + kWaves * qq;
+                    const int r = min(kVStageRows + inst * 4 + (lane >> 4), p.T - 1);
+                    load_to_lds16_v(p.v_new + ((size_t)r * p.Hkv + g) * kHeadDim + (lane & 15) * 8, late_rows + inst * 1024);
+                }
+                late = kLateOnTheWay;
+            }
             for (int e = 0; e < G; ++e) {
                 const int ie = it * G + e;
                 const int ce = (t0 + ie) * kTileN;
@@ -811,10 +828,14 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
                     // V^T, one 16-byte piece (8 token slots of one dim) per thread, read-modify-write:
                     // slots of appended tokens take the value from the staged row-major copy (the
                     // transposition), slots at or beyond S become zero, the others keep the pool's value.
-                    // Trees of more than kVStageRows nodes read the rows beyond the staging area from
-                    // v_new; the choice is uniform, so the usual case issues no global load here.
-                    auto patch_v = [&](auto all_staged_c) {
-                        constexpr bool kAllStaged = decltype(all_staged_c)::value;
+                    // (Late rows: an instance of its own, so that trees without any keep their shorter one.)
+                    auto patch_v = [&](auto late_c) {
+                        constexpr bool kLateRows = decltype(late_c)::value;
+                        if (kLateRows && late == kLateOnTheWay && append && ce + kTileN > P + kVStageRows) {
+                            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                            __syncthreads();
+                            late = kLateHere;
+                        }
                         // A wave works on one group of 8 token slots at a time, so which of them are appended rows, which lie
                         // beyond the end and which staged row each takes its value from are scalar quantities: the per-slot
                         // index arithmetic and the case distinctions stay off the vector pipe.
@@ -831,50 +852,37 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
                             uint16_t nv[8];
 #pragma unroll
                             for (int j = 0; j < 8; ++j) {
-                                const int r = min(max(ce + v_slot16(sg * 8 + j) - P, 0), kAllStaged ? p.T - 1 : kVStageRows - 1);
-                                nv[j] = reinterpret_cast<const uint16_t*>(vstage)[r * kHeadDim + d];
+                                const int r = min(max(ce + v_slot16(sg * 8 + j) - P, 0), p.T - 1);
+                                if (kLateRows) nv[j] = reinterpret_cast<const uint16_t*>(r < kVStageRows ? vstage : late_rows)[(r % kVStageRows) * kHeadDim + d];
+                                else nv[j] = reinterpret_cast<const uint16_t*>(vstage)[r * kHeadDim + d];
                             }
-                            if constexpr (kAllStaged) {
-                                // The eight slots of a group are two runs of four consecutive token positions (v_slot16
-                                // swaps bits 2 and 3 of the slot number), so which of them take the staged value
-                                // ([P, S)), keep the pool's (below P, or below S when nothing is appended) or become
-                                // zero (from S on) are two bit ranges per run: a handful of scalar instructions and one
-                                // and-or per 64 bits, where a comparison chain per slot cost more than the tile's MFMAs.
-                                uint64_t w2[2] = {__builtin_bit_cast(uint4, cur).x | ((uint64_t)__builtin_bit_cast(uint4, cur).y << 32),
-                                                  __builtin_bit_cast(uint4, cur).z | ((uint64_t)__builtin_bit_cast(uint4, cur).w << 32)};
+                            // The eight slots of a group are two runs of four consecutive token positions (v_slot16
+                            // swaps bits 2 and 3 of the slot number), so which of them take the staged value
+                            // ([P, S)), keep the pool's (below P, or below S when nothing is appended) or become
+                            // zero (from S on) are two bit ranges per run: a handful of scalar instructions and one
+                            // and-or per 64 bits, where a comparison chain per slot cost more than the tile's MFMAs.
+                            uint64_t w2[2] = {__builtin_bit_cast(uint4, cur).x | ((uint64_t)__builtin_bit_cast(uint4, cur).y << 32),
+                                              __builtin_bit_cast(uint4, cur).z | ((uint64_t)__builtin_bit_cast(uint4, cur).w << 32)};
 #pragma unroll
-                                for (int h = 0; h < 2; ++h) {
-                                    const int c0 = ce + v_slot16(sg * 8 + 4 * h);
-                                    const int end = min(max(S - c0, 0), 4);
-                                    const int beg = append ? min(max(P - c0, 0), end) : end;
-                                    const uint64_t below_end = end >= 4 ? ~0ull : (1ull << (16 * end)) - 1ull;
-                                    const uint64_t below_beg = beg >= 4 ? ~0ull : (1ull << (16 * beg)) - 1ull;
-                                    const uint64_t staged = (uint64_t)nv[4 * h] | ((uint64_t)nv[4 * h + 1] << 16) | ((uint64_t)nv[4 * h + 2] << 32) |
-                                                            ((uint64_t)nv[4 * h + 3] << 48);
-                                    w2[h] = (staged & below_end & ~below_beg) | (w2[h] & below_beg);
-                                    has_new = has_new || end > beg;
-                                }
-                                cur = __builtin_bit_cast(f16x8, make_uint4((uint32_t)w2[0], (uint32_t)(w2[0] >> 32), (uint32_t)w2[1], (uint32_t)(w2[1] >> 32)));
-                            } else {
-#pragma unroll
-                                for (int j = 0; j < 8; ++j) {
-                                    const int c = ce + v_slot16(sg * 8 + j);
-                                    if (append && c >= P && c < S) {
-                                        if (c - P < kVStageRows) cur[j] = __builtin_bit_cast(f16, nv[j]);
-                                        else cur[j] = p.v_new[((size_t)(c - P) * p.Hkv + g) * kHeadDim + d];
-                                        has_new = true;
-                                    } else if (c >= S) {
-                                        cur[j] = (f16)0.f;
-                                    }
-                                }
+                            for (int h = 0; h < 2; ++h) {
+                                const int c0 = ce + v_slot16(sg * 8 + 4 * h);
+                                const int end = min(max(S - c0, 0), 4);
+                                const int beg = append ? min(max(P - c0, 0), end) : end;
+                                const uint64_t below_end = end >= 4 ? ~0ull : (1ull << (16 * end)) - 1ull;
+                                const uint64_t below_beg = beg >= 4 ? ~0ull : (1ull << (16 * beg)) - 1ull;
+                                const uint64_t staged = (uint64_t)nv[4 * h] | ((uint64_t)nv[4 * h + 1] << 16) | ((uint64_t)nv[4 * h + 2] << 32) |
+                                                        ((uint64_t)nv[4 * h + 3] << 48);
+                                w2[h] = (staged & below_end & ~below_beg) | (w2[h] & below_beg);
+                                has_new = has_new || end > beg;
                             }
+                            cur = __builtin_bit_cast(f16x8, make_uint4((uint32_t)w2[0], (uint32_t)(w2[0] >> 32), (uint32_t)w2[1], (uint32_t)(w2[1] >> 32)));
                             *pp = cur;
                             if (has_new && mt == 0)  // the same 8 slots are 16 contiguous bytes of the pool's page row
                                 *reinterpret_cast<f16x8*>(p.v_pool_w + (((size_t)pg * p.Hkv + g) * kHeadDim + d) * kPage + ce % kPage + sg * 8) = cur;
                         }
                     };
-                    if (p.T <= kVStageRows) patch_v(std::true_type{});
-                    else patch_v(std::false_type{});
+                    if (p.T <= kVStageRows) patch_v(std::false_type{});
+                    else patch_v(std::true_type{});
                 }
             }
             CPMCU_CLOCK(tl_fix0);
