@@ -414,49 +414,62 @@ __device__ inline void scalar_load3(const int32_t* pa, const int32_t* pb, const 
                  : "=&s"(a), "=&s"(b), "=&s"(c) : "s"(pa), "s"(pb), "s"(pc) : "memory");
 }
 
-// Per-thread byte offsets of its pieces inside a K tile and a V^T tile of a page (second piece of each:
-// + 32 keys = 8192 bytes for K, + 64 dims = 64 * 512 bytes for V^T; the swizzle terms do not change).
-__device__ inline uint32_t k_piece_off(int wave, int lane) {
-    const int key = wave * 4 + (lane >> 4);
-    const int piece = (lane & 15) ^ (key & 15);
-    return (uint32_t)(key * kHeadDim + piece * 8) * 2u;
+// A wave requests 2 KB of a K tile (8 rows) and as much of a V^T tile (16 dims), 1 KB in lane order by each request; the swizzle is
+// applied on the global side.  The two requests fill consecutive KB of LDS, so that one LDS address (m0) and one base serve both: the
+// immediate offset of the second is added to both addresses, and the lane's own offset makes up the difference.  (44 -> 14 scalar
+// instructions a tile; with registers freed in the paths of few tiles, 60 nodes at 32K 45.2 -> 44.8 us a layer, 128 at 4K 24.8 -> 22.5.)
+constexpr int kRequests = 16 / kWaves;  // of a wave, for K and for V^T
+static_assert(kRequests == 2, "TileOffsets");
+struct TileOffsets {
+    uint32_t k0, v0;  // of the first requests
+    __device__ inline TileOffsets(int wave, int lane) {
+        const int key = wave * (4 * kRequests) + (lane >> 4);
+        k0 = (uint32_t)(key * kHeadDim + ((lane & 15) ^ (key & 15)) * 8) * 2u;
+        const int d = wave * (8 * kRequests) + (lane >> 3);
+        v0 = (uint32_t)(d * kPage + ((lane & 7) ^ ((d >> 1) & 7)) * 8) * 2u;
+    }
+    // of request h, less 1 KB times h: four keys or eight dims on, where the swizzle is another one by bit 2 of the piece
+    __device__ inline uint32_t k(int h) const { return k0 ^ (64u * h); }
+    __device__ inline uint32_t v(int h) const { return (v0 ^ (64u * h)) + (8u * kPage * 2u - 1024u) * h; }
+};
+template <int H>
+__device__ inline void load_to_lds16_nth(const void* base, uint32_t byte_off) {
+    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(byte_off), "s"(base), "i"(1024 * H) : "memory");
 }
-__device__ inline uint32_t v_piece_off(int wave, int lane) {
-    const int d = wave * 8 + (lane >> 3);
-    const int piece = (lane & 7) ^ ((d >> 1) & 7);
-    return (uint32_t)(d * kPage + piece * 8) * 2u;
-}
+__device__ inline void set_lds_address(uint32_t addr) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(addr) : "memory", "m0"); }
 
-// Issues this thread's four 16-byte direct-to-LDS loads of one tile (2 for K, 2 for V^T).  Each
-// wave-level instruction fills 1 KB of LDS in lane order; the swizzle is applied on the global side.
-// Everything but the two per-thread offsets is wave-uniform, so the address arithmetic is scalar.
-__device__ inline void issue_tile(const AttnParams& p, int g, int tile, int page, char* stage, int wave, uint32_t koff, uint32_t voff) {
+// Issues this thread's direct-to-LDS loads of one tile.  `lds`: where the wave's part of the K tile goes.
+// Everything but the per-thread offsets is wave-uniform, so the address arithmetic is scalar.
+__device__ inline void issue_tile(const AttnParams& p, int g, int tile, int page, uint32_t lds, const TileOffsets& off) {
     const int slot0 = (tile * kTileN) % kPage;
     const char* kbase = reinterpret_cast<const char*>(p.k_pool + (((size_t)page * p.Hkv + g) * kPage + slot0) * kHeadDim);
     const char* vbase = reinterpret_cast<const char*>(p.v_pool + ((size_t)page * p.Hkv + g) * kHeadDim * kPage + slot0);
-    load_to_lds16(kbase, koff, stage + wave * 1024);
-    load_to_lds16(vbase, voff, stage + kKTileBytes + wave * 1024);
-    load_to_lds16(kbase + 32 * kHeadDim * 2, koff, stage + (wave + kWaves) * 1024);
-    load_to_lds16(vbase + 64 * kPage * 2, voff, stage + kKTileBytes + (wave + kWaves) * 1024);
+    set_lds_address(lds);
+    load_to_lds16_nth<0>(kbase, off.k(0));
+    load_to_lds16_nth<1>(kbase, off.k(1));
+    set_lds_address(lds + kKTileBytes);
+    load_to_lds16_nth<0>(vbase, off.v(0));
+    load_to_lds16_nth<1>(vbase, off.v(1));
 }
 
 // The same for a tile that reaches the rows being appended: keys at positions [P, S) take their K
 // pieces straight from k_new (same 16-byte pieces, so the fused append costs K nothing); V^T comes
 // from the pool as usual and is patched in LDS afterwards.
-__device__ inline void issue_tile_append(const AttnParams& p, int g, int tile, int page, char* stage, int wave, int lane, uint32_t koff,
-                                         uint32_t voff, int P, int S) {
+__device__ inline void issue_tile_append(const AttnParams& p, int g, int tile, int page, char* stage, int wave, int lane, const TileOffsets& off, int P,
+                                         int S) {
     const int slot0 = (tile * kTileN) % kPage;
     const char* kbase = reinterpret_cast<const char*>(p.k_pool + (((size_t)page * p.Hkv + g) * kPage + slot0) * kHeadDim);
     const char* vbase = reinterpret_cast<const char*>(p.v_pool + ((size_t)page * p.Hkv + g) * kHeadDim * kPage + slot0);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int key = h * 32 + wave * 4 + (lane >> 4);
+    for (int h = 0; h < kRequests; ++h) {
+        const int part = wave * kRequests + h;
+        const int key = part * 4 + (lane >> 4);
         const int c = tile * kTileN + key;
         const int piece = (lane & 15) ^ (key & 15);
-        const char* src = kbase + h * (32 * kHeadDim * 2) + koff;
+        const char* src = kbase + off.k(h) + 1024 * h;
         if (c >= P && c < S) src = reinterpret_cast<const char*>(p.k_new + ((size_t)(c - P) * p.Hkv + g) * kHeadDim + piece * 8);
-        load_to_lds16_v(src, stage + (wave + kWaves * h) * 1024);
-        load_to_lds16(vbase + h * (64 * kPage * 2), voff, stage + kKTileBytes + (wave + kWaves * h) * 1024);
+        load_to_lds16_v(src, stage + part * 1024);
+        load_to_lds16(vbase, off.v(h) + 1024 * h, stage + kKTileBytes + part * 1024);
     }
 }
 
@@ -504,6 +517,12 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     const int g = p.hkv_shift >= 0 ? sh & (p.Hkv - 1) : sh % p.Hkv;
     const int split = p.hkv_shift >= 0 ? sh >> p.hkv_shift : sh / p.Hkv;
 
+    // The value as it is known here: keeps what is worked out from it in paths that few tiles take from being worked out ahead of
+    // the loop, where it would hold registers that the loop needs.
+    auto here = [](int v) {
+        asm volatile("" : "+v"(v));
+        return v;
+    };
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
@@ -611,16 +630,19 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     const int n = max(t1 - t0, 0);
     const int niter = (n + G - 1) / G;  // one iteration consumes G tiles, one per KV group
 
-    const uint32_t koff = k_piece_off(wave, lane), voff = v_piece_off(wave, lane);
+    TileOffsets off(wave, lane);
+    const uint32_t ring_lds = (uint32_t)(uintptr_t)(lds_ptr_t)ring + wave_u * (kKTileBytes / kWaves);
     auto issue_tile_i = [&](int i) {  // the i-th tile of this workgroup's range, into its ring stage
         const int tile = t0 + i;
         const int page = page_of_tile(tile);
+        off.k0 = here(off.k0);  // (the other requests' offsets are worked out from these each time: two registers less)
+        off.v0 = here(off.v0);
         if (p.k_new != nullptr && (tile + 1) * kTileN > P) {
             // (the page is kept for the patch of the landed tile: a table load there would sit in front of its LDS reads)
             if (tid == 0) s_append_page[min(max(tile - P / kTileN, 0), 2)] = page;
-            issue_tile_append(p, g, tile, page, ring + (i % kStages) * kStageBytes, wave_u, lane, koff, voff, P, S);
+            issue_tile_append(p, g, tile, page, ring + (i % kStages) * kStageBytes, wave_u, here(lane), off, P, S);
         } else
-            issue_tile(p, g, tile, page, ring + (i % kStages) * kStageBytes, wave_u, koff, voff);
+            issue_tile(p, g, tile, page, ring_lds + (i % kStages) * kStageBytes, off);
     };
     auto issue_iter = [&](int it) {
 #pragma unroll
@@ -766,7 +788,9 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         const int iter_end = (t0 + it * G) * kTileN + G * kTileN;
         const bool iter_needs_fix = iter_end > S || (p.k_new != nullptr && iter_end > P);
         if (iter_needs_fix) {
+            const int tid = G == 1 ? here(threadIdx.x) : (int)threadIdx.x;
             if (late == kLateWanted && it * G > n - kStages) {  // (trees of more than kVStageRows nodes)
+                const int lane = here(threadIdx.x) & 63;
 #pragma unroll
                 for (int qq = 0; qq < kVStageRows / (4 * kWaves); ++qq) {
                     const int inst = wave_u + kWaves * qq;
@@ -840,10 +864,11 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
                         // beyond the end and which staged row each takes its value from are scalar quantities: the per-slot
                         // index arithmetic and the case distinctions stay off the vector pipe.
                         static_assert(kThreads % kHeadDim == 0 && (kHeadDim * 8) % kThreads == 0, "whole waves per slot group");
-                        const int d = tid & (kHeadDim - 1);
+                        const int thread = kLateRows ? here(tid) : tid;
+                        const int d = thread & (kHeadDim - 1);
 #pragma unroll
                         for (int pass = 0; pass < (kHeadDim * 8) / kThreads; ++pass) {
-                            const int sg = __builtin_amdgcn_readfirstlane(tid / kHeadDim + pass * (kThreads / kHeadDim));
+                            const int sg = __builtin_amdgcn_readfirstlane(thread / kHeadDim + pass * (kThreads / kHeadDim));
                             f16x8* pp = reinterpret_cast<f16x8*>(st + v_lds_off(d, sg));
                             f16x8 cur = *pp;
                             bool has_new = false;
