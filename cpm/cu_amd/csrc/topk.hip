@@ -49,8 +49,9 @@ __device__ inline void emit_final(const TopkParams& p, int row, int round, uint6
     if (key == 0) return;
     const int idx = key_index(key);
     const size_t o = (size_t)row * p.top + round;
-    // raw ranking: hand back the input bits (keeps -0); fused: the rounded log-prob in the key
-    p.val[o] = LOGSOFTMAX ? key_bits(key) : p.x[(size_t)row * p.dim + idx];
+    // raw ranking: hand back the input bits, which are the key's but for -0; fused: the rounded log-prob in the key
+    const uint16_t bits = key_bits(key);
+    p.val[o] = LOGSOFTMAX || bits != 0 ? bits : p.x[(size_t)row * p.dim + idx];
     p.pos[o] = idx;
     if (p.ids) p.ids[o] = p.remap ? p.remap[idx] : idx;
 }
@@ -170,7 +171,10 @@ constexpr int kRowMaxPieces = 4;                       // 16-byte pieces per thr
 constexpr int kRowMaxDim = kRowThreads * kRowMaxPieces * 8;  // 32768
 constexpr int kRowShortDim = kRowThreads * 8;          // 8192: one piece per thread
 constexpr int kRowCap = kRowThreads;                   // candidate keys held in LDS
-constexpr int kRowBoundDrop = 4;                       // low bits of the bound that are not searched
+constexpr int kRowBoundDrop = 4;                       // low bits of the bound that fp16 rows do not search:
+// 16 ulps of an fp16 value are 1/64 of it.  Of a bfloat16 value they are 1/8 -- with log-probabilities around -12 more than a nat, which let
+// thousands of candidates in; those rows search to the bit, in instances of their own (a switch among the arguments cost
+// fp16 rows 0.3 us a launch; the 50 best of 151936: 24.1 -> 12.9 us, of 64 such rows 35 -> 18).
 constexpr int kRowDenseWaves = 8;                      // waves that extract the candidates
 constexpr int kRowLaneCap = 512;                       // threads with candidates whose registers LDS can take
 constexpr int kRowMaxTop = 128;                        // output slots are ranks below k <= kRowCap; beyond 64 see row_kernel_ranks()
@@ -271,7 +275,7 @@ __device__ __forceinline__ void topk_row_body(const TopkParams& p) {
     asm volatile("" ::"v"(lmax));
 #endif
     CPMCU_STAMP(g_topk_timeline, blockIdx.x, 1);
-    // k-th largest of this wave's lane maxima, rounded down to a multiple of 2^kRowBoundDrop (0 when
+    // k-th largest of this wave's lane maxima, rounded down to a multiple of 2^kRowBoundDrop where that is fine enough (0 when
     // fewer than k lanes hold anything): a slightly lower bound is as valid and costs fewer steps
     // (with fused statistics wave 0 reduces those meanwhile and contributes no bound: any subset of
     // the waves gives a valid one)
@@ -282,20 +286,28 @@ __device__ __forceinline__ void topk_row_body(const TopkParams& p) {
     // (bfloat16 rows tie so often that the shared bound pays at every k: 6.0 against 6.4 us for the top 10 of 32768; fp16: 5.9 either way)
     const bool spread = (p.top > 16 || !std::is_same<E, f16>::value) && full_waves - first_wave >= 2;
     if (!(LOGSOFTMAX && wave == 0)) {
-        for (int bit = 15; bit >= kRowBoundDrop; --bit) {
-            const uint32_t c = kth | (1u << bit);
-            if (__popcll(__ballot(lmax >= c)) >= p.top) kth = c;
-        }
+        const auto search = [&](int lanes) {
+            uint32_t at = 0;
+            const auto step = [&](int bit) {
+                const uint32_t c = at | (1u << bit);
+                if (__popcll(__ballot(lmax >= c)) >= lanes) at = c;
+            };
+#pragma unroll
+            for (int bit = 15; bit >= kRowBoundDrop; --bit) step(bit);
+            if (!std::is_same<E, f16>::value) {
+#pragma unroll
+                for (int bit = kRowBoundDrop - 1; bit >= 0; --bit) step(bit);
+            }
+            return at;
+        };
+        kth = search(p.top);
         if (spread && wave < full_waves) {
             const int few = (p.top + full_waves - first_wave - 1) / (full_waves - first_wave);
             uint32_t kf = 0;
             if (few == 1) {
                 kf = wave_reduce_b32(lmax, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
             } else {
-                for (int bit = 15; bit >= kRowBoundDrop; --bit) {
-                    const uint32_t c = kf | (1u << bit);
-                    if (__popcll(__ballot(lmax >= c)) >= few) kf = c;
-                }
+                kf = search(few);
             }
             if (lane == 0) wave_few[wave] = kf;
         }
@@ -566,32 +578,46 @@ __device__ __forceinline__ void topk_row_body(const TopkParams& p) {
 }
 
 // The slices' k best keys of a row (at most kSliceMergeCap of them, empty slots are 0) ranked by counting: one workgroup per
-// row, the count of larger keys is the output slot.
+// row, the count of larger keys is the output slot.  Four lanes share the counting for a candidate, and a value is read from the row
+// again only where the key has lost its sign (with one lane for each and all values read: the 20 best of five fp16 rows of 73449 10.2 us against 8.9, the
+// 50 best of 151936 11.6 against 10.5).
 constexpr int kSliceMergeCap = 1024;
 constexpr int kShortSliceCand = 256, kShortSliceWorkgroups = 512;
+constexpr int kMergeThreads = 1024, kMergeLanes = 4;
 template <bool LOGSOFTMAX>
-__global__ __launch_bounds__(kTopkThreads) void topk_slice_merge_kernel(TopkParams p) {
+__global__ __launch_bounds__(kMergeThreads) void topk_slice_merge_kernel(TopkParams p) {
     __shared__ uint64_t keys[kSliceMergeCap];
-    const int row = blockIdx.x;
+    const int row = blockIdx.x, tid = threadIdx.x;
     const int ncand = p.nchunks * p.top;
     const uint64_t* in = p.cand + (size_t)row * ncand;
-    for (int i = threadIdx.x; i < ncand; i += kTopkThreads) keys[i] = in[i];
+    const int padded = (ncand + 8 * kMergeLanes - 1) / (8 * kMergeLanes) * (8 * kMergeLanes);
+    if (tid < padded) keys[tid] = tid < ncand ? in[tid] : 0;
     __syncthreads();
-    for (int i = threadIdx.x; i < ncand; i += kTopkThreads) {
+    const int part = tid % kMergeLanes;
+    for (int i = tid / kMergeLanes; i < ncand; i += kMergeThreads / kMergeLanes) {
         const uint64_t my = keys[i];
-        if (my == 0) continue;
-        int r = 0;
-        for (int j = 0; j < ncand; ++j) r += keys[j] > my ? 1 : 0;
-        if (r < p.top) emit_final<LOGSOFTMAX>(p, row, r, my);
+        uint32_t r = 0;
+        for (int j = part; j < padded; j += 8 * kMergeLanes) {
+            uint64_t o[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) o[u] = keys[j + u * kMergeLanes];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) r += o[u] > my ? 1u : 0u;
+        }
+        r += dpp_mov<kDppXor1>(r);
+        r += dpp_mov<kDppXor2>(r);
+        if (my != 0 && part == 0 && (int)r < p.top) emit_final<LOGSOFTMAX>(p, row, (int)r, my);
     }
 }
 
 template <bool LOGSOFTMAX>
 __global__ __launch_bounds__(kRowThreads) void topk_row_kernel(TopkParams p) { topk_row_body<LOGSOFTMAX, kRowMaxPieces, f16>(p); }
-__global__ __launch_bounds__(kRowThreads) void topk_row_bf16_kernel(TopkParams p) { topk_row_body<true, kRowMaxPieces, bf16>(p); }
+template <bool LOGSOFTMAX>
+__global__ __launch_bounds__(kRowThreads) void topk_row_bf16_kernel(TopkParams p) { topk_row_body<LOGSOFTMAX, kRowMaxPieces, bf16>(p); }
 template <bool LOGSOFTMAX>
 __global__ __launch_bounds__(kRowThreads) void topk_short_row_kernel(TopkParams p) { topk_row_body<LOGSOFTMAX, 1, f16>(p); }
-__global__ __launch_bounds__(kRowThreads) void topk_short_row_bf16_kernel(TopkParams p) { topk_row_body<true, 1, bf16>(p); }
+template <bool LOGSOFTMAX>
+__global__ __launch_bounds__(kRowThreads) void topk_short_row_bf16_kernel(TopkParams p) { topk_row_body<LOGSOFTMAX, 1, bf16>(p); }
 
 // log_softmax in place (src/model/eagle.cuh:29-89): one workgroup per row.  The row is walked in 16-byte pieces from its
 // first 16-byte boundary on; the first four pieces of every thread stay in registers between the three passes (maximum, sum,
@@ -818,11 +844,13 @@ int launch_topk(const void* x, int n, int dim, int top, void* val, int32_t* pos,
     const bool row_kernel = options().topk_row_kernel != 0;
     const auto launch_rows = [&](int longest, dim3 grid) {
         if (longest <= kRowShortDim) {
-            if (stats && options().dtype == 1) hipLaunchKernelGGL(topk_short_row_bf16_kernel, grid, dim3(kRowThreads), 0, st, p);
+            if (stats && options().dtype == 1) hipLaunchKernelGGL(topk_short_row_bf16_kernel<true>, grid, dim3(kRowThreads), 0, st, p);
+            else if (options().dtype == 1) hipLaunchKernelGGL(topk_short_row_bf16_kernel<false>, grid, dim3(kRowThreads), 0, st, p);
             else if (stats) hipLaunchKernelGGL(topk_short_row_kernel<true>, grid, dim3(kRowThreads), 0, st, p);
             else hipLaunchKernelGGL(topk_short_row_kernel<false>, grid, dim3(kRowThreads), 0, st, p);
         } else {
-            if (stats && options().dtype == 1) hipLaunchKernelGGL(topk_row_bf16_kernel, grid, dim3(kRowThreads), 0, st, p);
+            if (stats && options().dtype == 1) hipLaunchKernelGGL(topk_row_bf16_kernel<true>, grid, dim3(kRowThreads), 0, st, p);
+            else if (options().dtype == 1) hipLaunchKernelGGL(topk_row_bf16_kernel<false>, grid, dim3(kRowThreads), 0, st, p);
             else if (stats) hipLaunchKernelGGL(topk_row_kernel<true>, grid, dim3(kRowThreads), 0, st, p);
             else hipLaunchKernelGGL(topk_row_kernel<false>, grid, dim3(kRowThreads), 0, st, p);
         }
@@ -844,8 +872,8 @@ int launch_topk(const void* x, int n, int dim, int top, void* val, int32_t* pos,
         p.nchunks = nslices;
         launch_rows(p.slice_len, dim3(n, nslices));
         CPMCU_LAUNCH_CHECK();
-        if (stats) hipLaunchKernelGGL(topk_slice_merge_kernel<true>, dim3(n), dim3(kTopkThreads), 0, st, p);
-        else hipLaunchKernelGGL(topk_slice_merge_kernel<false>, dim3(n), dim3(kTopkThreads), 0, st, p);
+        if (stats) hipLaunchKernelGGL(topk_slice_merge_kernel<true>, dim3(n), dim3(kMergeThreads), 0, st, p);
+        else hipLaunchKernelGGL(topk_slice_merge_kernel<false>, dim3(n), dim3(kMergeThreads), 0, st, p);
         CPMCU_LAUNCH_CHECK();
         return CPMCU_OK;
     }

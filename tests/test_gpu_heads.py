@@ -370,6 +370,39 @@ def test_topk_of_rows_that_start_off_16_bytes(gpu, orc, n, dim, top, off):
     assert np.array_equal(to_np(val).view(np.uint16), v_ref.view(np.uint16))
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("n,dim,top,kind", [(2, 32776, 1, "narrow"), (3, 151936, 50, "narrow"), (3, 151936, 50, "close"), (2, 131072, 128, "close"),
+                                            (1, 262144, 128, "narrow"), (70, 65544, 17, "close"), (2, 151936, 33, "zeros"), (3, 98304, 64, "neg_inf"),
+                                            (4, 8200, 64, "close"), (4, 32768, 128, "zeros")])
+def test_topk_of_slices_and_of_close_values(gpu, orc, set_option, n, dim, top, kind, bf16):
+    """What bounds a row (to the last bit where the format is bfloat16) and what ranks the slices of a long one (four lanes a candidate):
+    one candidate to as many as the merge takes, values a few codes apart, both zeros, rows nearly all -inf.  Positions and bits exactly."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    set_option("dtype", int(bf16))
+    orc.set_dtype("bf16" if bf16 else "f16")
+    try:
+        g = synth.rng(dim + top, 17)
+        if kind == "narrow":      # one binade: every value of bfloat16 there is held by hundreds of elements
+            x = (1 + g.random((n, dim))).astype(np.float32)
+        elif kind == "zeros":     # the top is the zeros, of both signs
+            x = -np.abs(g.standard_normal((n, dim))).astype(np.float32)
+            at = g.random((n, dim)) < 0.01
+            x[at] = np.where(g.random(at.sum()) < 0.5, np.float32(0.0), np.float32(-0.0))
+        else:
+            x = g.standard_normal((n, dim)).astype(np.float32)
+        if kind == "neg_inf":
+            x[:, g.random(dim) < 0.9995] = -np.inf
+        t = torch.from_numpy(x).to(torch.bfloat16 if bf16 else torch.float16).view(torch.float16)
+        val, pos = ops.topk(t.cuda(), top)
+        torch.cuda.synchronize()
+        v_ref, p_ref = orc.topk(t.numpy(), top)
+        assert np.array_equal(to_np(pos), p_ref)
+        assert np.array_equal(to_np(val).view(np.uint16), v_ref.view(np.uint16))
+    finally:
+        orc.set_dtype("f16")
+
+
 @pytest.mark.parametrize("n,dim,top,kind", [(3, 510, 59, "normal"), (10, 32768, 10, "normal"), (2, 32768, 64, "ties"), (4, 5000, 32, "ties"),
                                             (2, 73448, 25, "normal"), (3, 20000, 100, "normal"), (2, 32001, 63, "ties"), (5, 64, 64, "normal"),
                                             (2, 16384, 40, "neg_inf")])
