@@ -27,21 +27,17 @@ constexpr int kMaxTried = kTopkThreads * kPerThread;  // history entries one wor
 __device__ inline uint32_t key32(uint16_t bits, int idx) { return (ord16(bits) << 16) | (uint32_t)(0xFFFF - idx); }
 static_assert(kMaxTried <= 0x10000, "the index must fit the low half of a 32-bit key");
 
-// Places of the `top` largest of s_keys[0, n): emit(place, index) is called by the thread that owns the
-// entry.  s_keys must be padded with zeros to a multiple of 4 and be visible (barrier) on entry.
-template <typename Emit>
-__device__ inline void rank_select(const uint32_t* s_keys, int n, int top, Emit emit) {
+// How many of s_keys[0, n) are larger: the place of a key among them.  s_keys must be padded with zeros to a multiple of 4 and be
+// visible (barrier) on entry.
+__device__ inline int keys_above(const uint32_t* s_keys, int n, uint32_t mine) {
     const int n4 = (n + 3) & ~3;
-    for (int x = threadIdx.x; x < n; x += blockDim.x) {
-        const uint32_t mine = s_keys[x];
-        int above = 0;
+    int above = 0;
 #pragma unroll 8
-        for (int j = 0; j < n4; j += 4) {  // every lane reads the same 16 bytes: an LDS broadcast
-            const uint4 o = *reinterpret_cast<const uint4*>(s_keys + j);
-            above += (o.x > mine) + (o.y > mine) + (o.z > mine) + (o.w > mine);
-        }
-        if (above < top) emit(above, x);
+    for (int j = 0; j < n4; j += 4) {  // every lane reads the same 16 bytes: an LDS broadcast
+        const uint4 o = *reinterpret_cast<const uint4*>(s_keys + j);
+        above += (o.x > mine) + (o.y > mine) + (o.z > mine) + (o.w > mine);
     }
+    return above;
 }
 
 struct DraftState {
@@ -87,44 +83,58 @@ __global__ void draft_begin_kernel(DraftState s, int k, const uint16_t* val, con
     next_ids[i] = remap ? remap[pos[i]] : pos[i];
 }
 
+// A chain of round trips (arguments, candidates, vocabulary ids) around a short count, so an entry stays with its thread: what a chosen one
+// needs -- its id is looked up for every candidate, under the count -- is in registers when its place is known.  (A draft of 6 rounds of 10 in a
+// replayed graph 364.9 -> 361.4 us, one of 4 rounds of 4 call by call 105.7 -> 103.4, against looking the chosen ones' ids up behind the count.)
+// kEntries: entries of a thread, at most.  The loads have no branches around them (an entry past the end repeats the last one): behind a
+// branch the compiler would wait for the ids in front of the count.
+template <int kEntries>
 __global__ __launch_bounds__(kTopkThreads) void draft_extend_kernel(DraftState s, int k, int d, uint16_t* val, const int32_t* pos,
                                                                     const int32_t* remap, int32_t* next_ids, int32_t* parent_rows,
                                                                     uint64_t* mask_out, int is_bf16) {
-    __shared__ __attribute__((aligned(16))) uint32_t s_keys[kMaxK * kMaxK];
-    __shared__ int32_t s_sel[kMaxK];
-    __shared__ uint16_t s_val[kMaxK * kMaxK];
-    __shared__ uint64_t s_oldmask[kMaxK];
+    __shared__ __attribute__((aligned(16))) uint32_t s_keys[kEntries * kTopkThreads];
     const int tid = threadIdx.x;
     const int kk = k * k;
     const int base = k + (d - 1) * kk;
-    if (tid < k) s_oldmask[tid] = s.mask[tid];
-    for (int x = tid; x < ((kk + 3) & ~3); x += kTopkThreads) {
-        uint32_t key = 0;
+    uint32_t key[kEntries];
+    int32_t id[kEntries];
+    int parent[kEntries];
+    uint64_t mask[kEntries];
+    uint16_t cum[kEntries];
+#pragma unroll
+    for (int e = 0; e < kEntries; ++e) {
+        const int x = tid + e * kTopkThreads, at = min(x, kk - 1);
+        parent[e] = (unsigned)at / (unsigned)k;
+        const uint16_t v = val[at], c = s.cum[parent[e]];
+        const int32_t p = pos[at];
+        mask[e] = s.mask[parent[e]];
+        id[e] = *(remap ? remap + p : pos + at);
+        // the running log-prob of the parent is added in the element type: 16 bits += 16 bits, rounded to 16 bits
+        const uint16_t sum_f16 = Elem<f16>::to_bits(Elem<f16>::from_bits(v) + Elem<f16>::from_bits(c));
+        const uint16_t sum_bf16 = Elem<bf16>::to_bits(Elem<bf16>::from_bits(v) + Elem<bf16>::from_bits(c));
+        cum[e] = is_bf16 ? sum_bf16 : sum_f16;
+        key[e] = x < kk ? key32(cum[e], x) : 0;
+        s_keys[x] = key[e];
         if (x < kk) {
-            // the running log-prob of the parent is added in the element type: 16 bits += 16 bits, rounded to 16 bits
-            const uint16_t bits = is_bf16 ? Elem<bf16>::to_bits(Elem<bf16>::from_bits(val[x]) + Elem<bf16>::from_bits(s.cum[x / k]))
-                                          : Elem<f16>::to_bits(Elem<f16>::from_bits(val[x]) + Elem<f16>::from_bits(s.cum[x / k]));
-            val[x] = bits;
-            s.tried_val[base + x] = bits;
-            s.tried_pos[base + x] = pos[x];
-            s_val[x] = bits;
-            key = key32(bits, x);
+            val[x] = cum[e];
+            s.tried_val[base + x] = cum[e];
+            s.tried_pos[base + x] = p;
         }
-        s_keys[x] = key;
     }
     __syncthreads();
-    rank_select(s_keys, kk, k, [&](int place, int x) { s_sel[place] = x; });
-    __syncthreads();
-    if (tid < k) {
-        const int p2 = s_sel[tid];
-        s.tried_parent[(d - 1) * k + tid] = p2 + base;
-        const uint64_t m = s_oldmask[p2 / k] | (1ull << (k * d + tid));
-        s.mask[tid] = m;
-        if (mask_out) mask_out[tid] = m;
-        if (parent_rows) parent_rows[tid] = p2 / k;
-        const int32_t fr = pos[p2];
-        next_ids[tid] = remap ? remap[fr] : fr;
-        s.cum[tid] = s_val[p2];
+#pragma unroll
+    for (int e = 0; e < kEntries; ++e) {
+        const int x = tid + e * kTopkThreads;
+        if (x >= kk) break;
+        const int place = keys_above(s_keys, kk, key[e]);
+        if (place >= k) continue;
+        const uint64_t m = mask[e] | (1ull << (k * d + place));
+        s.tried_parent[(d - 1) * k + place] = x + base;
+        s.mask[place] = m;
+        if (mask_out) mask_out[place] = m;
+        if (parent_rows) parent_rows[place] = parent[e];
+        next_ids[place] = id[e];
+        s.cum[place] = cum[e];
     }
 }
 
@@ -157,13 +167,14 @@ __global__ __launch_bounds__(kFinishThreads) void draft_finish_kernel(DraftState
     if (tid < k * (num_iter - 1)) s_hpar[tid] = s.tried_parent[tid];
     const int P = cache_length[0];
     __syncthreads();
-    rank_select(s_keys, total, T - 1, [&](int place, int x) { s_sel[place] = x; });
-    __syncthreads();
-    if (tid >= 1 && tid < T) {
-        const int p = s_sel[tid - 1];
-        s_reverse[p] = tid;
-        const int32_t fr = s_pos[p];
-        ids_out[tid] = remap ? remap[fr] : fr;
+    for (int x = tid; x < total; x += kFinishThreads) {
+        const int place = keys_above(s_keys, total, s_keys[x]);
+        if (place < T - 1) {
+            s_sel[place] = x;
+            s_reverse[x] = place + 1;
+            const int32_t fr = s_pos[x];
+            ids_out[place + 1] = remap ? remap[fr] : fr;
+        }
     }
     __syncthreads();
     // build_dynamic_tree (src/model/eagle.cuh:188-214), every node on its own thread: its parent is the
@@ -237,7 +248,8 @@ extern "C" int cpmcu_draft_tree_extend(void* state, int k, int num_iter, int d, 
     CPMCU_CHECK_ARG(state && topk_val && topk_pos && next_ids, "draft_tree_extend: null pointer argument");
     if (int rc = check_shape("draft_tree_extend", k, num_iter)) return rc;
     CPMCU_CHECK_ARG(d >= 1 && d < num_iter, "draft_tree_extend: iteration d=%d outside [1, %d)", d, num_iter);
-    hipLaunchKernelGGL(draft_extend_kernel, dim3(1), dim3(kTopkThreads), 0, resolve_stream(stream), draft_state(state, k, num_iter), k, d,
+    const auto kernel = k * k <= kTopkThreads ? draft_extend_kernel<1> : draft_extend_kernel<kMaxK * kMaxK / kTopkThreads>;
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kTopkThreads), 0, resolve_stream(stream), draft_state(state, k, num_iter), k, d,
                        (uint16_t*)topk_val, topk_pos, token_id_remap, next_ids, parent_rows, draft_mask, options().dtype == 1 ? 1 : 0);
     CPMCU_LAUNCH_CHECK();
     return CPMCU_OK;

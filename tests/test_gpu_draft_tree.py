@@ -48,6 +48,25 @@ def test_draft_tree_equals_oracle(gpu, orc, k, num_iter, T, seed, with_remap, dy
     assert np.array_equal(g_mask, o_mask)
 
 
+@pytest.mark.parametrize("k,num_iter,T,with_remap", [(15, 4, 64, True), (16, 4, 64, True), (16, 2, 30, False), (17, 3, 60, True), (24, 2, 128, False)])
+def test_rounds_of_one_and_of_several_candidates_a_thread(gpu, orc, k, num_iter, T, with_remap):
+    """Up to 256 candidates a thread of the extend kernel holds one, beyond up to four: both sides of that line, with ties and with
+    zeros of either sign (whose bits the running log-probs keep)."""
+    torch = gpu
+    remap = synth.frspec_remap(2000, 500, k) if with_remap else None
+    vals, poss = make_rows(k, num_iter, 500, k, dyadic=True)
+    for d in range(num_iter):
+        vals[d][:, 0] = np.float16(-0.0 if d % 2 == 0 else 0.0)
+    (o_ids, o_pos, o_mask, o_parent), o_trace = run_oracle(orc, k, num_iter, T, 99, vals, poss, remap)
+    (g_ids, g_pos, g_mask, g_parent), g_trace, _ = run_gpu(torch, k, num_iter, T, 99, vals, poss, remap)
+    assert np.array_equal(g_trace[0], o_trace[0])
+    for d in range(1, num_iter):
+        for a, b in zip(g_trace[d], o_trace[d]):
+            assert np.array_equal(a, b), "iteration %d" % d
+    assert np.array_equal(g_ids[1:], o_ids[1:]) and np.array_equal(g_pos, o_pos)
+    assert np.array_equal(g_parent, o_parent) and np.array_equal(g_mask, o_mask)
+
+
 def test_heavy_ties(gpu, orc):
     """All log-probs equal: every choice is made by the index rule alone."""
     torch = gpu
