@@ -949,12 +949,12 @@ __device__ __forceinline__ void fuse_finish_row(const HeadParams& p, const FuseP
 // have read them; straight-line code per block for exact waits, as in the streaming kernel below.  The partial tiles of a
 // block (one per wave) meet in LDS in groups of eight (block, 16 hidden rows) units: wave w adds up and finishes the group's unit w.
 // More than 16 * NB hidden rows are row groups (blockIdx.y) that share the CUs: the groups' workgroups of the same blocks sit on one
-// XCD and walk them together, so W comes from HBM once.
+// XCD and walk them together, so W comes from HBM once -- SHARED: W is then requested without the non-temporal hint, which would
+// take a line out of the L2 before a group that is a little behind has read it.
 // us per call, x 4096 tiled, this kernel / streaming or chunked kernel: 10 rows, 8192 rows of vocabulary 13.9 / 24.1, 16384 23.8 /
-// 30.6, 20000 27.7 / 34.6, 32768 43.4 / 42.7 (where the streaming kernel takes over).  Row-major, against the row-walking kernel:
-// 8192 16.2 / 43.8, 32768 48.8 / 52, 73448 103 / 112-117 (its two loads of a 128-byte line are left to the L2: with non-temporal
-// loads 51.4 at 32768).
-template <int KS, int NB, bool TILED, typename E>
+// 30.6, 20000 27.7 / 34.6, 32768 43.4 / 42.7 (where the streaming kernel takes over).  Row-major (below), one row: 8192 15.8, 32768 45.9,
+// 73449 96.3.
+template <int KS, int NB, bool TILED, bool SHARED, typename E>
 __device__ __forceinline__ void head_gemm_slice_body(const HeadParams& p) {
     typedef typename Elem<E>::x8 X8;
     constexpr int NBUF = KS * (NB + 2) <= 48 ? 2 : 1;  // W buffers of one row block: what 256 registers leave beside the hidden rows
@@ -974,19 +974,46 @@ __device__ __forceinline__ void head_gemm_slice_body(const HeadParams& p) {
     const int np = (p.row_blocks - c + G - 1) / G;  // row blocks c, c + G, ... of this workgroup: at least one
     const int k0 = wave * (KS * 32);
 
-    auto block_ptr = [&](int b) {
+    // Row-major weights: the lanes of an MFMA operand take 64 bytes of each of 16 rows, half a line, and two such requests for every line
+    // cost a tenth of the stream.  So a pair of K steps is requested by lines, the even rows' with the first and the odd rows' with the
+    // second -- eight lanes, those of rows 2 i and 2 i + 1, take a row's 128 bytes -- and the two lanes of a pair of rows exchange what is
+    // the other one's in front of the MFMAs.  Call by halves of lines / by lines, us, x 4096: one row 8192 17.8 / 15.8, 32768 51.2 / 45.9, 73449
+    // 107 / 96; 32 rows 25.1 / 23.3, 59.6 / 53.5, 126 / 113.
+    struct Block {
+        const f16 *first, *second;  // TILED: first only
+    };
+    auto block_ptr = [&](int b) -> Block {
         const int rb = b * G + c;
-        if constexpr (TILED) return p.w + ((size_t)rb * (H / 32) + wave * KS) * 512 + lane * 8;
-        const int row = min(rb * 16 + l16, p.V - 1);  // rows past the end are computed and discarded
-        return p.w + (size_t)row * H + k0 + kgp * 8;
+        if constexpr (TILED) return {p.w + ((size_t)rb * (H / 32) + wave * KS) * 512 + lane * 8, nullptr};
+        const int row = rb * 16 + (l16 & ~1), last = p.V - 1;  // rows past the end are computed and discarded
+        const f16* at = p.w + k0 + ((l16 & 1) * 4 + kgp) * 8;
+        return {at + (size_t)min(row, last) * H, at + (size_t)min(row + 1, last) * H};
     };
-    auto load_frag = [&](const f16* base, int ks) -> X8 {
-        if constexpr (TILED) return __builtin_nontemporal_load(reinterpret_cast<const X8*>(base + ks * 512));
-        return *reinterpret_cast<const X8*>(base + ks * 32);
+    auto load_frag = [&](const Block& base, int ks) -> X8 {
+        const X8* at = reinterpret_cast<const X8*>(TILED ? base.first + ks * 512 : (ks & 1 ? base.second : base.first) + (ks >> 1) * 64);
+        if constexpr (SHARED) return *at;
+        return __builtin_nontemporal_load(at);
     };
+    // What was requested for a pair of K steps, as the operands of the two: of an even row's lane its own first register quad and its
+    // neighbour's, of an odd row's its neighbour's second and its own.
+    auto exchange = [&](const X8& first, const X8& second, X8& even, X8& odd) {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        const u32x4 f = __builtin_bit_cast(u32x4, first), g = __builtin_bit_cast(u32x4, second);
+        u32x4 a, o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t fi = f[i], gi = g[i];
+            const uint32_t of_odd = dpp_mov<kDppXor1>(fi), of_even = dpp_mov<kDppXor1>(gi);  // (with all lanes: a lane that is off has nothing)
+            a[i] = (l16 & 1) ? of_even : fi;
+            o[i] = (l16 & 1) ? gi : of_odd;
+        }
+        even = __builtin_bit_cast(X8, a);
+        odd = __builtin_bit_cast(X8, o);
+    };
+    static_assert(TILED || KS % 2 == 0, "K steps go in pairs");
     X8 wa[KS], wb[NBUF == 2 ? KS : 1], hid[KS][NB];
     {
-        const f16* a = block_ptr(0);
+        const Block a = block_ptr(0);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) wa[ks] = load_frag(a, ks);
         __builtin_amdgcn_sched_barrier(0);
@@ -999,7 +1026,7 @@ __device__ __forceinline__ void head_gemm_slice_body(const HeadParams& p) {
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (NBUF == 2) {
-            const f16* b = block_ptr(min(1, np - 1));
+            const Block b = block_ptr(min(1, np - 1));
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) wb[ks] = load_frag(b, ks);
             __builtin_amdgcn_sched_barrier(0);
@@ -1043,14 +1070,18 @@ __device__ __forceinline__ void head_gemm_slice_body(const HeadParams& p) {
         head_epilogue_block<E, true>(p, acc, blockIdx.y * NB + my_nb, (b * G + c) * 16 + kgp * 4, l16, ea, eb);
     };
     auto consume = [&](int b, auto& w, auto refill) {
-        const f16* next = refill ? block_ptr(b + NBUF) : nullptr;
+        const Block next = refill ? block_ptr(b + NBUF) : Block{};
         f32x4 acc[2][NB];  // two chains per block of hidden rows
+        X8 pair[2];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[0][nb] = acc[1][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
+            if constexpr (!TILED) {
+                if (ks % 2 == 0) exchange(w[ks], w[ks + 1], pair[0], pair[1]);
+            }
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc[ks & 1][nb] = Elem<E>::mfma_16x16x32(w[ks], hid[ks][nb], acc[ks & 1][nb]);
+            for (int nb = 0; nb < NB; ++nb) acc[ks & 1][nb] = Elem<E>::mfma_16x16x32(TILED ? w[ks] : pair[ks & 1], hid[ks][nb], acc[ks & 1][nb]);
             if (refill) w[ks] = load_frag(next, ks);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -1459,10 +1490,10 @@ template <int NB, int FP, int KC>
 __global__ __launch_bounds__(kHeadThreads) void head_gemm_stream_kernel(HeadParams p) { head_gemm_stream_body<NB, FP, KC, f16>(p); }
 template <int NB, int FP, int KC>
 __global__ __launch_bounds__(kHeadThreads) void head_gemm_stream_bf16_kernel(HeadParams p) { head_gemm_stream_body<NB, FP, KC, bf16>(p); }
-template <int KS, int NB, bool TILED>
-__global__ __launch_bounds__(kHeadThreads) void head_gemm_slice_kernel(HeadParams p) { head_gemm_slice_body<KS, NB, TILED, f16>(p); }
-template <int KS, int NB, bool TILED>
-__global__ __launch_bounds__(kHeadThreads) void head_gemm_slice_bf16_kernel(HeadParams p) { head_gemm_slice_body<KS, NB, TILED, bf16>(p); }
+template <int KS, int NB, bool TILED, bool SHARED>
+__global__ __launch_bounds__(kHeadThreads) void head_gemm_slice_kernel(HeadParams p) { head_gemm_slice_body<KS, NB, TILED, SHARED, f16>(p); }
+template <int KS, int NB, bool TILED, bool SHARED>
+__global__ __launch_bounds__(kHeadThreads) void head_gemm_slice_bf16_kernel(HeadParams p) { head_gemm_slice_body<KS, NB, TILED, SHARED, bf16>(p); }
 // FR-Spec head + log-softmax + top-k + id map-back in one launch (one block of hidden rows).
 template <int FP, int KC>
 __global__ __launch_bounds__(kHeadThreads) void frspec_head_topk_kernel(HeadParams p, FuseParams fp) { head_gemm_stream_body<1, FP, KC, f16, true>(p, fp); }
@@ -1582,17 +1613,16 @@ HeadShape pick_head_shape(int NB, int H, bool w_tiled, int nch, int npasses, int
 // vocabularies of less than one pass over the chip's wave slots; from one pass on the streaming kernel is level for up to 16 hidden
 // rows and ahead for more (60 rows x 32768: 46.7 us against 55.0), on exactly half a pass and more for more than 32 rows as well,
 // where it has a shape (whole passes: 16384 x 128 rows 43.9 / 46.3; 20000, where it has none, 74.1 / 56.1).  Row-major weights have
-// no streaming kernel: up to 32 rows the K slices win at every size (32 rows: 54.5 / 56.3 us at 32768, 109 / 123 at 73448, 216 / 237 at
-// 151936) but for up to 16 rows of 2048 columns from one pass on (63.9 / 61.7 at 73448); 33 to 64 rows below one pass (32768:
-// 68.9 / 69.9, 73448: 156 / 151), more below half a pass (20000 x 128 rows: 81.6 / 80.3).
+// no streaming kernel: the K slices win at every size up to 96 rows (the row-walking kernel / K slices, x 4096: 64 rows 75.9 / 63.8 at
+// 32768, 177 / 147 at 73449, 308 / 287 at 151936; 96 rows 92.3 / 86.3 at 32768; x 2048: one row 66.4 / 58.9 and 64 rows 91.9 / 82.3 at 73449),
+// and with more unless the row-walking kernel's passes over the wave slots are full: 128 rows 241 / 219 at 73449 (0.75 of three passes),
+// 92.0 / 97.5 at 32768 (one whole pass), 406 / 409 at 151936 (0.93 of five).
 bool pick_slice_shape(int n, int H, bool w_tiled, int nrb, int cus, HeadShape* shape) {
     const int slots = cus * kHeadWaves;
     if (w_tiled) {
         if (!options().head_stream_kernel || nrb >= slots) return false;
         if (n > 32 && nrb * 2 >= slots && nrb % kHeadWaves == 0) return false;
-    } else if (n <= 32) {
-        if (n <= 16 && H < 4096 && nrb >= slots) return false;
-    } else if (nrb >= (n <= 64 ? slots : slots / 2)) {
+    } else if (n > 96 && nrb * 13 > ceil_div(nrb, slots) * slots * 12) {
         return false;
     }
     const int snb = n <= 16 ? 1 : 2;
@@ -1739,11 +1769,15 @@ int launch_head_gemm(const void* hidden, const void* w, int w_layout, int n, int
         break;
             CPMCU_HEAD_STREAM_SHAPES(CPMCU_X)
 #undef CPMCU_X
+// Tiled weights are shared through the L2 with either kind of request where the row groups are alike; a last group of one block of rows runs
+// ahead of the others (x 4096 tiled, non-temporal / plain: 33 rows 55.0 / 37.7 at 20000, 26.6 / 21.3 at 8192; 64 rows 42.7 / 42.6 and 24.5 / 25.4).
 #define CPMCU_HEAD_SLICE(ks, nb, tiled)                                                                                                          \
     do {                                                                                                                                         \
         const dim3 grid(G, ceil_div(n, 16 * nb));                                                                                                \
-        if (is_bf16) hipLaunchKernelGGL((head_gemm_slice_bf16_kernel<ks, nb, tiled>), grid, dim3(kHeadThreads), 0, st, p);                       \
-        else hipLaunchKernelGGL((head_gemm_slice_kernel<ks, nb, tiled>), grid, dim3(kHeadThreads), 0, st, p);                                    \
+        const bool shared = grid.y > 1 && (!(tiled) || (n - 1) % 32 < 16);                                                                      \
+        const auto kernel = is_bf16 ? (shared ? head_gemm_slice_bf16_kernel<ks, nb, tiled, (nb > 1)> : head_gemm_slice_bf16_kernel<ks, nb, tiled, false>) \
+                                    : (shared ? head_gemm_slice_kernel<ks, nb, tiled, (nb > 1)> : head_gemm_slice_kernel<ks, nb, tiled, false>);           \
+        hipLaunchKernelGGL(kernel, grid, dim3(kHeadThreads), 0, st, p);                                                                          \
     } while (0)
 #define CPMCU_X(ks, nb)                                                     \
     case HeadShape::T_##ks##_##nb: CPMCU_HEAD_SLICE(ks, nb, true); break;   \

@@ -316,6 +316,15 @@ def test_row_major_head_with_many_k_chunks(gpu, orc, n, H):
     _frspec_check(gpu, orc, n=n, V=2600, Vs=2048 + 24, H=H, k=10, seed=50 + n)
 
 
+@pytest.mark.parametrize("n,V,H,tiled", [(1, 17, 2048, False), (5, 4099, 4096, False), (16, 8177, 2048, False), (17, 4111, 4096, False), (33, 6001, 2048, False),
+                                         (48, 4096, 4096, False), (64, 3999, 2048, False), (96, 5001, 4096, False), (97, 2047, 2048, False), (128, 32768, 2048, False),
+                                         (128, 30241, 2048, False), (128, 30240, 2048, False), (33, 8200, 4096, True), (48, 5000, 2048, True), (49, 5000, 2048, True)])
+def test_head_by_k_slices_over_row_groups_and_ragged_ends(gpu, orc, n, V, H, tiled):
+    """Row-major weights requested by lines, a pair of rows by eight lanes: vocabularies that end inside a pair and inside a block of 16,
+    one row group and several (whose last one is half full or not), and both sides of the line to the row-walking kernel at 128 rows."""
+    _argmax_check(gpu, orc, n, V=V, H=H, seed=n + V % 89, tiled=tiled)
+
+
 def test_target_head_c2_full_size(gpu, orc):
     """Config 2 head: 60 tree rows against the 73448x4096 head."""
     _argmax_check(gpu, orc, 60, V=73448, H=4096, seed=0)
