@@ -335,9 +335,9 @@ size_t cpmcu_tree_attention_workspace_bytes(int T, int Hq, int Hkv, int max_kv_l
  *           when that is 0.  Calls that may overlap on one GPU must use different
  *           workspaces: the split partials live there, and the library keys the
  *           arrival counters of the in-launch merge by this pointer (a launch with at
- *           most 32 splits and at most one workgroup per CU merges its own partials;
- *           its workgroups wait for each other, which needs them all resident -- see
- *           "attn_merge_in_launch" above).
+ *           most 32 splits, of the direct shape with 16 to 128, and at most one workgroup
+ *           per CU merges its own partials; its workgroups wait for each other, which
+ *           needs them all resident -- see "attn_merge_in_launch" above).
  *   num_splits_override: 0 = choose from max_kv_len; >0 forces the KV split count.
  * max_kv_len is limited to 2^30. */
 int cpmcu_tree_attention(const void* q, void* k_pool, void* v_pool, const int32_t* block_table,
