@@ -697,11 +697,10 @@ __device__ __forceinline__ void log_softmax_body(uint16_t* x, int dim, float* ro
     }
 }
 
-// The same for long rows, in slices of 4096 elements with a workgroup each: partial (max, sum), then the map.  One workgroup per row
-// is bound by the exponentials of its CU: 14.8 us for five rows of 73448 in a replayed graph, 6.1 in two launches; 64 rows of 151936 32.2
-// and 16.5.  (Both launches are a round trip and two exchanges between waves, which sixteen waves do later than eight: 6.9 and 17.9 with
-// slices of 8192; four waves 5.8 and 17.8.)
-constexpr int kSoftmaxThreads = 512;
+// The same for long rows, in slices of 8192 elements with a workgroup each: partial (max, sum), then the map.  One workgroup per row
+// is bound by the exponentials of its CU: 14.7 us for five rows of 73449 in a replayed graph, 6.8 in two launches; 60 rows of 151936 32
+// and 17.
+constexpr int kSoftmaxThreads = 1024;
 constexpr int kSoftmaxSlice = kSoftmaxThreads * 8;
 template <typename E>
 struct SoftmaxSlice {
@@ -765,14 +764,11 @@ template <typename E>
 __device__ __forceinline__ void log_softmax_apply_body(uint16_t* x, int dim, const float2* part, float* row_stats) {
     const int row = blockIdx.y, nslices = gridDim.x, lane = threadIdx.x & 63;
     const SoftmaxSlice<E> s(x, dim, row, blockIdx.x);
-    const float2* pr = part + (size_t)row * nslices;
-    const float2 first = lane < nslices ? pr[lane] : make_float2(-INFINITY, 0.f);
-    float m = first.x;
-    for (int i = lane + 64; i < nslices; i += 64) m = fmaxf(m, pr[i].x);
+    float m = -INFINITY, sum = 0.f;
+    for (int i = lane; i < nslices; i += 64) m = fmaxf(m, part[(size_t)row * nslices + i].x);
     m = wave_max_f32(m);
-    float sum = lane < nslices ? first.y * expf(first.x - m) : 0.f;
-    for (int i = lane + 64; i < nslices; i += 64) {
-        const float2 t = pr[i];
+    for (int i = lane; i < nslices; i += 64) {
+        const float2 t = part[(size_t)row * nslices + i];
         sum += t.y * expf(t.x - m);
     }
     const float lse = logf(wave_sum_f32(sum));
@@ -944,13 +940,12 @@ extern "C" int cpmcu_log_softmax_sliced(void* x, int n, int dim, float* row_stat
     CPMCU_CHECK_ARG(((uintptr_t)x & 1) == 0, "log_softmax_sliced: x is not aligned to its elements");
     const size_t need = cpmcu_log_softmax_workspace_bytes(n, dim);
     CPMCU_CHECK_ARG(workspace && workspace_bytes >= need, "log_softmax_sliced: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
-    // Slices take 5.5 to 6 us while each has a CU of its own and then grow with their number, a workgroup per row takes 4.5 us and one for
-    // every 7000 elements, whatever the number of rows up to 256.  us, whole rows / slices: 12000 elements x 5 rows 5.4 / 5.8; 16400 x 1 5.6 /
-    // 5.2, x 16 6.2 / 6.0, x 64 (320 slices) 6.3 / 6.8; 24576 x 5 6.5 / 5.6, x 64 7.0 / 6.9, x 128 7.5 / 8.2; 32768 x 80 8.2 / 8.3, x 128 9.2 / 9.5;
-    // 50000 x 64 11.4 / 9.3, x 128 13.6 / 13.0; 73448 x 5 14.8 / 6.2, x 128 18.9 / 15.7, x 256 24.1 / 26.6; 151936 x 64 32.3 / 16.8, x 256
-    // 54.6 / 50.5.
+    // Slices take 6 to 7 us while each has a CU of its own and then grow with their number, a workgroup per row takes 4.5 us and one for
+    // every 7000 elements, whatever the number of rows up to 256.  us, whole rows / slices: 16384 elements x 1 row 5.5 / 6.1, x 128 rows
+    // 6.3 / 7.4; 24576 x 16 6.6 / 6.7; 28000 x 1 6.8 / 5.9, x 64 7.6 / 7.3, x 80 (320 slices) 7.7 / 8.8; 50000 x 80 12.0 / 11.5, x 128 13.7 /
+    // 14.7, x 256 16.5 / 22.2; 73448 x 5 14.7 / 6.8, x 128 18.8 / 17.6, x 160 19.4 / 20.1; 151936 x 60 32.2 / 17.8, x 256 54.3 / 53.9.
     const int slices = ceil_div(dim, kSoftmaxSlice);
-    if (dim <= 4 * kSoftmaxSlice || n > 65535 || ((long long)n * slices > 256 && (long long)n * 400 > dim)) return cpmcu_log_softmax(x, n, dim, row_stats, stream);
+    if (dim <= 3 * kSoftmaxSlice || n > 65535 || ((long long)n * slices > 256 && (long long)n * 560 > dim)) return cpmcu_log_softmax(x, n, dim, row_stats, stream);
     hipStream_t st = resolve_stream(stream);
     const dim3 grid(slices, n);
     if (options().dtype == 1) {

@@ -605,22 +605,6 @@ def test_log_softmax_on_either_side_of_the_choice(gpu, orc, n, dim):
     assert np.array_equal(to_np(d).view(np.uint16), staged.view(np.uint16))
 
 
-@pytest.mark.parametrize("n,dim", [(2, 16384), (2, 16385), (64, 16400), (65, 20481), (64, 28001), (2, 64 * 4096), (2, 64 * 4096 + 1), (2, 65 * 4096 + 9)])
-def test_log_softmax_in_slices_of_4096(gpu, orc, n, dim):
-    """Both sides of the choice, and as many slices as a wave has lanes and one and two more -- with a row that is finite in its
-    last slice only."""
-    from cpm.cu_amd import ops
-    torch = gpu
-    test_log_softmax_on_either_side_of_the_choice(gpu, orc, n, dim)
-    x = (synth.rng(dim, n).standard_normal((n, dim)) * 1.3).astype(np.float16)
-    x[0, : (dim - 1) // 4096 * 4096] = -np.inf
-    d = to_dev(torch, x)
-    stats = to_np(ops.log_softmax_(d))
-    _, m_ref, lse_ref = orc.log_softmax(x)
-    assert np.array_equal(stats[:, 0], m_ref) and np.allclose(stats[:, 1], lse_ref, rtol=0, atol=1e-4)
-    assert np.array_equal(to_np(d).view(np.uint16), orc.log_softmax_apply(x, stats[:, 0], stats[:, 1]).view(np.uint16))
-
-
 def test_log_softmax_calls_share_nothing(gpu):
     """Calls on two streams at once, and replays of a captured call between eager calls with more rows: the bits of the same call
     made alone, every time."""
