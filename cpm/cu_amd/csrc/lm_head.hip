@@ -17,7 +17,7 @@
 //   * W goes HBM -> registers directly as the A operand of v_mfma_f32_16x16x32_f16.  In the tiled
 //     layout (cpmcu_head_weight_tile: [V/16][H/32][64 lanes][8 halves]) every wave instruction
 //     reads one contiguous KB and consecutive k-steps are consecutive in memory; the row-major
-//     layout is read as lane = (row % 16, k-group), 4 lanes per 64 contiguous bytes of a row;
+//     layout is read as lane = (row % 16, k-group), 4 lanes per 64 contiguous bytes of a row (by whole lines in head_gemm_slice_kernel);
 //   * the hidden rows are the B operand, staged in LDS: resident for the whole K range with up
 //     to 16 rows on the row-major path (head_gemm_kernel), in registers where the waves split K (head_gemm_slice_kernel:
 //     vocabularies of less than one pass, row-major weights), otherwise walked in K chunks that are
