@@ -40,6 +40,10 @@ __device__ inline int keys_above(const uint32_t* s_keys, int n, uint32_t mine) {
     return above;
 }
 
+// Vocabulary id of a candidate.  A position of -1 stands for no candidate (a row that a one-launch FR-Spec head left unfinished, a list that
+// was padded): it reads the table's first entry rather than what lies in front of the table.  Without a table the position itself.
+__device__ inline const int32_t* id_address(const int32_t* remap, const int32_t* pos) { return remap ? remap + max(*pos, 0) : pos; }
+
 struct DraftState {
     uint16_t* tried_val;    // [total] fp16 bits
     int32_t* tried_pos;     // [total]
@@ -80,7 +84,7 @@ __global__ void draft_begin_kernel(DraftState s, int k, const uint16_t* val, con
     s.cum[i] = val[i];
     s.mask[i] = 1ull << i;
     if (mask_out) mask_out[i] = 1ull << i;
-    next_ids[i] = remap ? remap[pos[i]] : pos[i];
+    next_ids[i] = *id_address(remap, pos + i);
 }
 
 // A chain of round trips (arguments, candidates, vocabulary ids) around a short count, so an entry stays with its thread: what a chosen one
@@ -108,7 +112,7 @@ __global__ __launch_bounds__(kTopkThreads) void draft_extend_kernel(DraftState s
         const uint16_t v = val[at], c = s.cum[parent[e]];
         const int32_t p = pos[at];
         mask[e] = s.mask[parent[e]];
-        id[e] = *(remap ? remap + p : pos + at);
+        id[e] = *id_address(remap, pos + at);
         // the running log-prob of the parent is added in the element type: 16 bits += 16 bits, rounded to 16 bits
         const uint16_t sum_f16 = Elem<f16>::to_bits(Elem<f16>::from_bits(v) + Elem<f16>::from_bits(c));
         const uint16_t sum_bf16 = Elem<bf16>::to_bits(Elem<bf16>::from_bits(v) + Elem<bf16>::from_bits(c));
@@ -173,7 +177,7 @@ __global__ __launch_bounds__(kFinishThreads) void draft_finish_kernel(DraftState
             s_sel[place] = x;
             s_reverse[x] = place + 1;
             const int32_t fr = s_pos[x];
-            ids_out[place + 1] = remap ? remap[fr] : fr;
+            ids_out[place + 1] = remap ? remap[max(fr, 0)] : fr;
         }
     }
     __syncthreads();

@@ -594,6 +594,8 @@ int cpmcu_verify_tail_inplace(const int32_t* best, const int32_t* accepted_ids, 
  *          [k], parent_rows int32[k] (row of the previous hidden states each new node continues:
  *          remap_hidden's index, may be NULL), draft_mask [k] for the next draft-layer attention.
  *          Every position is looked up in token_id_remap, not only the chosen ones.
+ *          (Throughout, a position of -1 -- no candidate: a row that a one-launch head left unfinished, a padded list --
+ *          is looked up as position 0; the rest have to be valid ones.)
  *   finish (:385-393): selects the tree_size - 1 best candidates of the history and writes
  *          tree_draft_ids[1..tree_size) (entry 0, the root token, is the caller's),
  *          tree_position_ids [tree_size] (P + depth; P read from the device scalar

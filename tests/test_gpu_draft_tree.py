@@ -67,6 +67,35 @@ def test_rounds_of_one_and_of_several_candidates_a_thread(gpu, orc, k, num_iter,
     assert np.array_equal(g_parent, o_parent) and np.array_equal(g_mask, o_mask)
 
 
+@pytest.mark.parametrize("bits", [0xFC00, 0xFFFF])  # -inf of a padded list, and what an unfinished row of a one-launch head holds
+@pytest.mark.parametrize("k,num_iter,T,rows_lost,cols_lost", [(4, 4, 30, 1, 2), (10, 3, 60, 9, 3), (17, 3, 128, 5, 0), (6, 2, 40, 6, 6)])
+def test_positions_of_minus_one_stay_inside_the_table(gpu, orc, k, num_iter, T, rows_lost, cols_lost, bits):
+    """Candidates that are none (position -1, the lowest value): they read the table's first entry and not the one in front of it,
+    ranked among the chosen or not.  The last rows of every round lost, and the last columns of the first."""
+    from cpm.cu_amd import ops
+    torch = gpu
+    vals, poss = make_rows(k, num_iter, 500, k, dyadic=True)
+    table = synth.frspec_remap(2000, 500, k)
+    lost = [np.zeros(p.shape, bool) for p in poss]
+    lost[0][:, k - cols_lost:] = True
+    for d in range(1, num_iter):
+        lost[d][k - rows_lost:] = True
+    o_vals = [np.where(m, np.float16(-np.inf), v) for m, v in zip(lost, vals)]
+    (o_ids, o_pos, o_mask, o_parent), o_trace = run_oracle(orc, k, num_iter, T, 99, o_vals, [np.where(m, 0, p) for m, p in zip(lost, poss)], table)
+    g_vals = [np.where(m, np.uint16(bits), v.view(np.uint16)).view(np.float16) for m, v in zip(lost, vals)]
+    g_poss = [np.where(m, -1, p).astype(np.int32) for m, p in zip(lost, poss)]
+    around = to_dev(torch, np.concatenate([[-777], table]).astype(np.int32))
+    t = ops.DraftTree(k, num_iter, around[1:])
+    assert np.array_equal(to_np(t.begin(to_dev(torch, g_vals[0][0]), to_dev(torch, g_poss[0][0]))), o_trace[0])
+    for d in range(1, num_iter):
+        ids, rows, mask = t.extend(d, to_dev(torch, g_vals[d]), to_dev(torch, g_poss[d]))
+        for a, b in zip((to_np(ids), to_np(rows), to_np(mask).view(np.uint64)), o_trace[d]):
+            assert np.array_equal(a, b), "iteration %d" % d
+    ids, pos, mask, parent = (to_np(x) for x in t.finish(T, torch.tensor([99], dtype=torch.int32, device="cuda")))
+    assert np.array_equal(ids[1:], o_ids[1:]) and np.array_equal(pos, o_pos)
+    assert np.array_equal(parent, o_parent) and np.array_equal(mask.view(np.uint64), o_mask)
+
+
 def test_heavy_ties(gpu, orc):
     """All log-probs equal: every choice is made by the index rule alone."""
     torch = gpu
