@@ -242,7 +242,7 @@ extern "C" int cpmcu_set_option(const char* name, int value) {
     } else if (nm == "attn_merge_in_launch") {
         CPMCU_CHECK_ARG(value == 0 || value == 1, "set_option: attn_merge_in_launch=%d must be 0 or 1", value);
         options().attn_merge_in_launch = value;
-        if (value) attention_merge_reenable();  // also for workspaces that went back to the combine launch after an abandoned wait
+        if (value) attention_merge_reenable();  // also for workspaces whose launches have not waited since an abandoned wait
     } else if (nm == "frspec_fused") {
         CPMCU_CHECK_ARG(value == 0 || value == 1, "set_option: frspec_fused=%d must be 0 or 1", value);
         options().frspec_fused = value;

@@ -1373,7 +1373,7 @@ bool can_merge_in_launch(int Hkv, int num_mtiles, int num_splits) {
 
 struct MergeState {
     int block = -1;
-    bool use_combine = false;  // a wait was abandoned on this device: the workspace's launches are merged by the combine launch
+    bool no_waits = false;  // a wait was abandoned on this device: nobody waits in the workspace's launches any more
 };
 std::mutex g_merge_mu;
 std::map<std::pair<int, const void*>, MergeState> g_merge_states;
@@ -1381,10 +1381,15 @@ std::vector<int> g_merge_free_blocks[64];
 bool g_merge_blocks_listed[64] = {false};
 uint32_t* g_merge_ctr_base[64] = {nullptr};
 
-// The counter block of a workspace on the current device; null: the launch has to be merged by the combine launch.
-uint32_t* merge_counters_for(const void* workspace, hipStream_t st) {
+// The counter block of a workspace on the current device.  words null: the launch has to be merged by the combine launch.  may_wait
+// false: so does one whose workgroups would wait for each other; the direct shape's last arrival, which waits for nobody, still merges.
+struct MergeCounters {
+    uint32_t* words = nullptr;
+    bool may_wait = false;
+};
+MergeCounters merge_counters_for(const void* workspace, hipStream_t st) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return {};
     std::lock_guard<std::mutex> lock(g_merge_mu);
     auto it = g_merge_states.find({dev, workspace});
     if (it == g_merge_states.end()) {
@@ -1393,12 +1398,12 @@ uint32_t* merge_counters_for(const void* workspace, hipStream_t st) {
             hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
             if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
                 (void)hipGetLastError();
-                return nullptr;
+                return {};
             }
             void* ptr = nullptr;
             if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_merge_ctr)) != hipSuccess) {
                 (void)hipGetLastError();
-                return nullptr;
+                return {};
             }
             g_merge_ctr_base[dev] = (uint32_t*)ptr;
         }
@@ -1406,14 +1411,13 @@ uint32_t* merge_counters_for(const void* workspace, hipStream_t st) {
             for (int b = kMergeBlocks - 1; b >= 0; --b) g_merge_free_blocks[dev].push_back(b);
             g_merge_blocks_listed[dev] = true;
         }
-        if (g_merge_free_blocks[dev].empty()) return nullptr;
+        if (g_merge_free_blocks[dev].empty()) return {};
         MergeState ns;
         ns.block = g_merge_free_blocks[dev].back();
         g_merge_free_blocks[dev].pop_back();
         it = g_merge_states.emplace(std::make_pair(dev, workspace), ns).first;
     }
-    if (it->second.use_combine) return nullptr;
-    return g_merge_ctr_base[dev] + (size_t)it->second.block * kMergeUnits * kMergeUnitWords;
+    return {g_merge_ctr_base[dev] + (size_t)it->second.block * kMergeUnits * kMergeUnitWords, !it->second.no_waits};
 }
 // The direct shape's merge.  Up to kDirectLastMerges splits the last arrival reads one round trip's worth of partials and nobody waits;
 // from there on sharing is the faster form (one query, last arrival / shares, us per layer: 7.07 / 7.86 on 8 splits, 7.25 / 7.47 on 12, 7.63 /
@@ -1442,7 +1446,7 @@ struct DirectPlan {
     int splits;
     bool use;
 };
-DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope) {
+DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope, bool may_wait) {
     const int units = Hkv * tiles, blocks = ceil_div(span, kBlockKeys) + 1;  // (one more for the appended rows)
     const int new_steps = ceil_div(T, 32), split_units = Hkv * ceil_div(tiles * kDirectRows, rows_per_wg(2));
     const float stream = (float)span * Hkv * (2 * kHeadDim * sizeof(f16)) / 5.5e6f;
@@ -1455,7 +1459,7 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope) {
         const int workgroups = kXcds * ceil_div(splits * Hkv, kXcds) * tiles;
         const float per_cu = (float)workgroups / (float)cus;
         const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.6f);
-        const float merge = splits == 1 ? 0.f : 2.3f + (direct_merge_shares(splits, workgroups, cus) > 0 ? 0.025f : 0.06f) * splits;
+        const float merge = splits == 1 ? 0.f : 2.3f + (may_wait && direct_merge_shares(splits, workgroups, cus) > 0 ? 0.025f : 0.06f) * splits;
         const float t = 3.4f + (units * splits * 2 > cus ? 1.2f : 1.05f) * it * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
                         0.6f * (new_steps - 1) + merge;
         if (t < best) best = t, d.splits = splits;
@@ -1465,15 +1469,18 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope) {
     return d;
 }
 
-LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_window_size, int num_splits_override, bool rope, bool allow_direct = true) {
+// What a launch finds of merge counters: the direct shape with its shares, with the last arrival's merge, or not at all beyond one split.
+enum class DirectMerge { kMayWait, kNoWaits, kNone };
+LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_window_size, int num_splits_override, bool rope,
+                       DirectMerge merge = DirectMerge::kMayWait) {
     LaunchPlan pl;
     const int window_blocks = block_window_size / 128;
     pl.span = max_kv_len;
     if (window_blocks > 0 && window_blocks * 128 + T < pl.span) pl.span = window_blocks * 128 + T;
     const int tiles = ceil_div(group * T, kDirectRows);
-    const DirectPlan direct = choose_direct(T, Hkv, tiles, pl.span, rope);
+    const DirectPlan direct = choose_direct(T, Hkv, tiles, pl.span, rope, merge == DirectMerge::kMayWait);
     // (a split count asked for is one of the split shapes', unless the direct shape is forced)
-    pl.direct = allow_direct && direct.use && (num_splits_override == 0 || options().attn_direct == 1);
+    pl.direct = merge != DirectMerge::kNone && direct.use && (num_splits_override == 0 || options().attn_direct == 1);
     if (pl.direct) {
         pl.kv_groups = 0;
         pl.num_mtiles = tiles;
@@ -1527,7 +1534,8 @@ void attention_release_workspace(const void* workspace) {
 // The report words of the current device, read without a round trip of their own: `attention_report_enqueue` puts a copy
 // into pinned host memory in stream order (call it ahead of a synchronisation of that stream, outside any capture),
 // `attention_report_take` looks at that copy afterwards and clears the device words only when something is there.
-// After any abandoned wait every workspace of the device goes back to the combine launch.
+// After any abandoned wait nobody waits in the launches of the device's workspaces: the split shapes go back to the combine launch, the
+// direct one to the merge by the last arrival.
 namespace {
 AttnReport* g_report_host[64] = {nullptr};
 }
@@ -1556,34 +1564,35 @@ int attention_report_take(int* bad_length, unsigned int* abandoned) {
         if (r.abandoned != 0) {
             std::lock_guard<std::mutex> lock(g_merge_mu);
             for (auto& kv : g_merge_states)
-                if (kv.first.first == dev) kv.second.use_combine = true;
+                if (kv.first.first == dev) kv.second.no_waits = true;
         }
     }
     *bad_length = r.bad_length;
     *abandoned = r.abandoned;
     return CPMCU_OK;
 }
-// Lets the workspaces of the current device merge inside the launch again (cpmcu_set_option attn_merge_in_launch = 1).
+// Lets the launches on the workspaces of the current device wait again (cpmcu_set_option attn_merge_in_launch = 1).
 void attention_merge_reenable() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return;
     std::lock_guard<std::mutex> lock(g_merge_mu);
     for (auto& kv : g_merge_states)
-        if (kv.first.first == dev) kv.second.use_combine = false;
+        if (kv.first.first == dev) kv.second.no_waits = false;
 }
 }  // namespace cpmcu
 
 // 1: a launch on this workspace (outside a stream capture, of a shape that allows it) merges its split partials itself;
-// 0: it is merged by the combine launch (no counter block left for the workspace, or the device has seen an abandoned wait).
+// 0: it is merged by the combine launch (no counter block left for the workspace, or the device has seen an abandoned wait -- then
+// launches of the direct shape are merged by their last arrivals).
 extern "C" int cpmcu_tree_attention_merge_mode(const void* workspace) {
     int dev = 0;
     if (workspace == nullptr || hipGetDevice(&dev) != hipSuccess) return 0;
     {
         std::lock_guard<std::mutex> lock(g_merge_mu);
         auto it = g_merge_states.find({dev, workspace});
-        if (it != g_merge_states.end()) return it->second.use_combine || !options().attn_merge_in_launch ? 0 : 1;
+        if (it != g_merge_states.end()) return it->second.no_waits || !options().attn_merge_in_launch ? 0 : 1;
     }
-    return merge_counters_for(workspace, nullptr) != nullptr && options().attn_merge_in_launch ? 1 : 0;
+    return merge_counters_for(workspace, nullptr).may_wait && options().attn_merge_in_launch ? 1 : 0;
 }
 
 extern "C" int cpmcu_tree_attention_release_workspace(const void* workspace) {
@@ -1656,10 +1665,12 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     p.window_blocks = block_window_size / 128;
     hipStream_t st = resolve_stream(stream);
     LaunchPlan plan = plan_launch(T, group, Hkv, max_kv_len, block_window_size, num_splits_override, rope_cos_sin != nullptr);
-    p.merge_ctr = plan.merge_in_launch && workspace ? merge_counters_for(workspace, st) : nullptr;
-    // (the direct shape has no merge launch to fall back on)
-    if (plan.direct && plan.num_splits > 1 && p.merge_ctr == nullptr)
-        plan = plan_launch(T, group, Hkv, max_kv_len, block_window_size, num_splits_override, rope_cos_sin != nullptr, false);
+    const MergeCounters counters = plan.merge_in_launch && workspace ? merge_counters_for(workspace, st) : MergeCounters{};
+    // (the direct shape has no merge launch to fall back on, but a merge that waits for nobody)
+    if (plan.direct && plan.num_splits > 1 && !counters.may_wait)
+        plan = plan_launch(T, group, Hkv, max_kv_len, block_window_size, num_splits_override, rope_cos_sin != nullptr,
+                           counters.words != nullptr ? DirectMerge::kNoWaits : DirectMerge::kNone);
+    p.merge_ctr = plan.direct || counters.may_wait ? counters.words : nullptr;
     const int span = plan.span;
     const int G = plan.kv_groups;
     p.num_mtiles = plan.num_mtiles;
@@ -1688,7 +1699,7 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     const dim3 grid(kXcds * ceil_div(nsh, kXcds), p.num_mtiles);
     const bool is_bf16 = options().dtype == 1;
     if (plan.direct) {
-        p.merge_shares = direct_merge_shares(p.num_splits, (int)(grid.x * grid.y), device_cu_count());
+        p.merge_shares = counters.may_wait ? direct_merge_shares(p.num_splits, (int)(grid.x * grid.y), device_cu_count()) : 0;
         p.append_rows = k_new ? ceil_div(ceil_div(T, kAppendRows) * Hkv, (int)grid.x * (kThreads / kAppendThreads)) : 0;
         const dim3 dgrid(grid.x, p.num_mtiles + p.append_rows);
         if (is_bf16) hipLaunchKernelGGL(tree_attn_direct_bf16_kernel, dgrid, dim3(kThreads), 0, st, p);

@@ -285,8 +285,9 @@ int cpmcu_synchronize(void);
  * so far (cpmcu_synchronize, cpmcu_verify_and_fix; also printed by cpmcu_print_perf_summary).  A split workgroup that
  * has waited attn_merge_wait_us for the other workgroups of its unit leaves its share of the merge to the last of them
  * and ends: the output is complete, only late.  It happens when the launch's workgroups are not all resident at once,
- * i.e. when another launch holds CUs.  After the first such wait is seen, the device's workspaces go back to the
- * separate merge launch; cpmcu_set_option("attn_merge_in_launch", 1) lets them merge inside the launch again. */
+ * i.e. when another launch holds CUs.  After the first such wait is seen, nobody waits in launches on the device's
+ * workspaces: split ones go back to the separate merge launch, those of the direct shape to the merge by the workgroup
+ * that arrives last.  cpmcu_set_option("attn_merge_in_launch", 1) lets them wait again. */
 long cpmcu_attention_abandoned_waits(void);
 /* Free everything the global model owns (the reference never frees). */
 int cpmcu_shutdown(void);
@@ -350,7 +351,8 @@ int cpmcu_tree_attention(const void* q, void* k_pool, void* v_pool, const int32_
  * to the separate merge launch (0).  The library keeps a block of arrival counters per workspace pointer it has met on a
  * device (32 per device, kept until the library's own workspace is freed at cpmcu_shutdown; further workspaces get
  * none), and takes every workspace of a device off the in-launch merge once a merge wait has been abandoned there
- * (see cpmcu_attention_abandoned_waits).  Asking assigns a block to a workspace that has none yet. */
+ * (see cpmcu_attention_abandoned_waits; launches of the direct shape, whose last arrival can merge without a wait,
+ * stay single ones).  Asking assigns a block to a workspace that has none yet. */
 int cpmcu_tree_attention_merge_mode(const void* workspace);
 /* No reference counterpart: tells the library that an attention workspace is about to be freed, so that its block of
  * arrival counters can go to another workspace.  None of its launches may be in flight, and no captured graph that holds

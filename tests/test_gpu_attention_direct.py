@@ -139,3 +139,69 @@ def test_shares_left_behind_are_merged_by_the_last_arrival(gpu, option, hkv, spl
         option("attn_merge_wait_us", 2000)
         L.synchronize()
         option("attn_merge_in_launch", 1)  # (the waits that ran out had sent the workspaces back to the merge launch)
+
+
+@pytest.mark.parametrize("hkv,T,splits", [(2, 1, 2), (2, 4, 15), (2, 1, 16), (8, 2, 32), (2, 1, 37), (1, 1, 128), (2, 3, 0)])
+def test_direct_launches_after_an_abandoned_wait(gpu, option, hkv, T, splits):
+    """After a merge wait that ran out on the device a launch of the direct shape stays one: nobody waits in it, and the last arrival
+    merges.  Its partials, in the workspace, are those of the launch that waits, bit for bit."""
+    import ctypes
+    from cpm.cu_amd import lib, ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch, L = gpu, lib.get()
+    option("attn_direct", 1)
+    S = 16500
+    g = torch.Generator(device="cuda").manual_seed(S + splits)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).half()
+    cache = PagedKVCache(1, hkv, (S + 255) // 256)
+    k, v = rnd(S, hkv, D), rnd(S, hkv, D)
+    cache.write_logical(0, 0, k, v)
+    q, kv_len = rnd(T, 32, D), torch.tensor([S], dtype=torch.int32, device="cuda")
+    hidden = torch.arange(S, device="cuda")[None] > S - T + torch.arange(T, device="cuda")[:, None]
+    exact = torch.empty((T, 32, D), dtype=torch.float64, device="cuda")
+    for h in range(32):
+        x = (q[:, h].double() @ k[:, h * hkv // 32].double().t().contiguous()) * D ** -0.5
+        exact[:, h] = torch.softmax(x.masked_fill(hidden, -float("inf")), 1) @ v[:, h * hkv // 32].double()
+    key = ("attn", q.device)
+    ws = torch.empty(L.raw.cpmcu_tree_attention_workspace_bytes(T, 32, hkv, S), dtype=torch.uint8, device="cuda")
+    saved, ops._workspaces[key] = ops._workspaces.get(key), ws
+
+    def call():
+        ws.zero_()
+        out = torch.full_like(q, float("nan"))
+        ops.tree_attention(q, cache, 0, kv_len, S, num_splits=splits, out=out)
+        torch.cuda.synchronize()
+        used = splits or ops.attention_plan(T, 32, hkv, S)[1]
+        return out, ws[:hkv * -(-32 // hkv * T // 16) * used * 16 * D * 2].clone()
+    try:
+        if not L.raw.cpmcu_tree_attention_merge_mode(ctypes.c_void_p(ws.data_ptr())):
+            option("attn_merge_in_launch", 1)
+        if not L.raw.cpmcu_tree_attention_merge_mode(ctypes.c_void_p(ws.data_ptr())):
+            pytest.skip("this process has used up the library's counter blocks")
+        ref, ref_parts = call()
+        # a wait that runs out: with a limit of zero a launch of 64 splits leaves shares behind
+        option("attn_merge_wait_us", 0)
+        for _ in range(4):
+            ops.tree_attention(q[:1], cache, 0, kv_len, S, num_splits=64 // hkv * 2)
+        before = L.raw.cpmcu_attention_abandoned_waits()
+        L.synchronize()
+        seen = L.raw.cpmcu_attention_abandoned_waits()
+        assert seen > before and L.raw.cpmcu_tree_attention_merge_mode(ctypes.c_void_p(ws.data_ptr())) == 0
+        for _ in range(2):
+            out, parts = call()
+            if splits:  # (else the number of splits is chosen anew)
+                assert torch.equal(parts, ref_parts)
+                # two orders of the same fp32 sums, rounded to fp16 once: a unit in the last place apart, at most
+                assert float((out.float() - ref.float()).abs().max()) <= 2.0 ** -10 * float(ref.float().abs().max())
+            # three roundings to fp16 (probabilities, partials, output) of 2.1e-4 of the norm each, added up in full
+            assert float((out.double() - exact).norm() / exact.norm()) < 6.3e-4
+        L.synchronize()
+        assert L.raw.cpmcu_attention_abandoned_waits() == seen, "somebody waited"
+    finally:
+        option("attn_merge_wait_us", 2000)
+        L.synchronize()
+        option("attn_merge_in_launch", 1)
+        ops.release_attention_workspace(ws)
+        ops._workspaces.pop(key)
+        if saved is not None:
+            ops._workspaces[key] = saved
