@@ -432,11 +432,11 @@ struct TileOffsets {
     __device__ inline uint32_t k(int h) const { return k0 ^ (64u * h); }
     __device__ inline uint32_t v(int h) const { return (v0 ^ (64u * h)) + (8u * kPage * 2u - 1024u) * h; }
 };
-template <int H>
-__device__ inline void load_to_lds16_nth(const void* base, uint32_t byte_off) {
-    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(byte_off), "s"(base), "i"(1024 * H) : "memory");
+// (one statement: nothing else can come between m0 and the two requests that read it)
+__device__ inline void load_to_lds16_pair(const void* base, uint32_t off_0, uint32_t off_1, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024"
+                 : : "v"(off_0), "v"(off_1), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
-__device__ inline void set_lds_address(uint32_t addr) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(addr) : "memory", "m0"); }
 
 // Issues this thread's direct-to-LDS loads of one tile.  `lds`: where the wave's part of the K tile goes.
 // Everything but the per-thread offsets is wave-uniform, so the address arithmetic is scalar.
@@ -444,12 +444,8 @@ __device__ inline void issue_tile(const AttnParams& p, int g, int tile, int page
     const int slot0 = (tile * kTileN) % kPage;
     const char* kbase = reinterpret_cast<const char*>(p.k_pool + (((size_t)page * p.Hkv + g) * kPage + slot0) * kHeadDim);
     const char* vbase = reinterpret_cast<const char*>(p.v_pool + ((size_t)page * p.Hkv + g) * kHeadDim * kPage + slot0);
-    set_lds_address(lds);
-    load_to_lds16_nth<0>(kbase, off.k(0));
-    load_to_lds16_nth<1>(kbase, off.k(1));
-    set_lds_address(lds + kKTileBytes);
-    load_to_lds16_nth<0>(vbase, off.v(0));
-    load_to_lds16_nth<1>(vbase, off.v(1));
+    load_to_lds16_pair(kbase, off.k(0), off.k(1), lds);
+    load_to_lds16_pair(vbase, off.v(0), off.v(1), lds + kKTileBytes);
 }
 
 // The same for a tile that reaches the rows being appended: keys at positions [P, S) take their K

@@ -213,3 +213,19 @@ def test_torch_binding_raises_for_tensors_without_memory():
     import sys
     res = subprocess.run([sys.executable, "-c", _NOT_MEMORY], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
     assert res.returncode == 0 and "all refused" in res.stdout, res.stdout
+
+
+def test_requests_into_lds_set_their_own_lds_address():
+    """A load into LDS takes its LDS address from m0, which the compiler may use between two statements: every inline assembly
+    statement with such a load sets m0 itself, in front of the load, and says that it does."""
+    csrc = os.path.join(ROOT, "cpm", "cu_amd", "csrc")
+    found = 0
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".hip", ".h")):
+            continue
+        for statement in re.findall(r"\basm\b[^;]*?;", open(os.path.join(csrc, name)).read(), flags=re.S):
+            if re.search(r"load_lds|\blds\b", statement):
+                found += 1
+                assert 0 <= statement.find("s_mov_b32 m0") < re.search(r"load_lds|\blds\b", statement).start(), (name, statement)
+                assert '"m0"' in statement, (name, statement)
+    assert found >= 5
