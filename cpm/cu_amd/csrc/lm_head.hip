@@ -1613,17 +1613,23 @@ HeadShape pick_head_shape(int NB, int H, bool w_tiled, int nch, int npasses, int
 // vocabularies of less than one pass over the chip's wave slots; from one pass on the streaming kernel is level for up to 16 hidden
 // rows and ahead for more (60 rows x 32768: 46.7 us against 55.0), on exactly half a pass and more for more than 32 rows as well,
 // where it has a shape (whole passes: 16384 x 128 rows 43.9 / 46.3; 20000, where it has none, 74.1 / 56.1).  Row-major weights have
-// no streaming kernel: the K slices win at every size up to 96 rows (the row-walking kernel / K slices, x 4096: 64 rows 75.9 / 63.8 at
-// 32768, 177 / 147 at 73449, 308 / 287 at 151936; 96 rows 92.3 / 86.3 at 32768; x 2048: one row 66.4 / 58.9 and 64 rows 91.9 / 82.3 at 73449),
-// and with more unless the row-walking kernel's passes over the wave slots are full: 128 rows 241 / 219 at 73449 (0.75 of three passes),
-// 92.0 / 97.5 at 32768 (one whole pass), 406 / 409 at 151936 (0.93 of five).
+// no streaming kernel.  Up to 96 rows the K slices win at every size (the row-walking or chunked kernel / K slices: one row 1.17 at whole passes to
+// 2.8 at 8192 rows of 4096 columns, 1.08 to 2.1 of 2048; 65 and 96 rows 1.05 / 1.03 at 98304 x 4096, 1.32 / 1.29 at 65600), but for 65 to
+// 96 rows of 4096 columns on exactly two or four passes (0.985 / 0.96 at 65536, 1.01 / 0.98 at 131072).  With more rows they read W for four groups, and
+// the chunked kernel, whose time goes by whole passes of the wave slots, wins where those are nearly full: `full`, in fortieths.  97 and
+// 128 rows x 4096, one pass: 1.10 / 1.08 at 30000 (0.92), 1.03 / 0.98 at 31000, 1.04 to 0.95 at 32768 with the weights' place in memory; several: 1.13 / 1.10
+// at 65600 (0.67 of three), 1.04 / 1.01 at 73448 (0.75), 1.02 / 0.99 at 51200 (0.78 of two), 1.00 / 0.98 at 78656 (0.80 of three), 0.97 / 0.94 at 53744 (0.82 of
+// two), 0.89 / 0.87 at 60000 (0.92), 0.84 / 0.82 at 65536; x 2048: 1.07 / 1.04 at 32768, 1.10 / 1.11 at 53744, 1.01 / 1.00 at 107488 (0.82 of four), 1.05 / 1.04 at
+// 57344 (0.875 of two), 1.00 / 0.98 at 85000 (0.86 of three), 0.98 / 0.97 at 140000 (0.85 of five), 0.93 / 0.93 at 120000 and 151936 (0.92 and 0.93).
 bool pick_slice_shape(int n, int H, bool w_tiled, int nrb, int cus, HeadShape* shape) {
     const int slots = cus * kHeadWaves;
     if (w_tiled) {
         if (!options().head_stream_kernel || nrb >= slots) return false;
         if (n > 32 && nrb * 2 >= slots && nrb % kHeadWaves == 0) return false;
-    } else if (n > 96 && nrb * 13 > ceil_div(nrb, slots) * slots * 12) {
-        return false;
+    } else if (n > 96) {
+        const int passes = ceil_div(nrb, slots);
+        const int full = passes == 1 ? (H >= 4096 ? 37 : 40) : H >= 4096 ? 32 : 35;
+        if (nrb * 40 > passes * slots * full) return false;
     }
     const int snb = n <= 16 ? 1 : 2;
 #define CPMCU_X(ks, nb)                                                            \

@@ -229,3 +229,17 @@ def test_requests_into_lds_set_their_own_lds_address():
                 assert 0 <= statement.find("s_mov_b32 m0") < re.search(r"load_lds|\blds\b", statement).start(), (name, statement)
                 assert '"m0"' in statement, (name, statement)
     assert found >= 5
+
+
+@pytest.mark.parametrize("n,V,H,sliced", [
+    (96, 65536, 4096, True), (97, 30304, 4096, True), (97, 30320, 4096, False), (128, 32768, 2048, True), (128, 32784, 4096, True), (97, 52416, 4096, True), (97, 52432, 4096, False), (128, 60000, 4096, False),
+    (128, 65536, 2048, False), (128, 65552, 4096, True), (100, 57344, 2048, True), (100, 57360, 2048, False), (128, 120000, 4096, False),
+    (128, 104848, 4096, True), (128, 104864, 4096, False), (100, 151936, 4096, False)])
+def test_row_major_heads_of_many_rows_take_the_faster_kernel(n, V, H, sliced):
+    """More than 96 rows: the K slices unless the chunked kernel's passes over the wave slots are nearly full, 37 fortieths of one, 32 of several
+    (2048 columns: always with one, 35 of several).
+    (The plan counts 256 CUs where there is no device.)"""
+    from cpm.cu_amd import lib
+    name, wg = ctypes.create_string_buffer(96), ctypes.c_int(0)
+    lib.get().head_plan(n, V, H, 0, name, 96, ctypes.byref(wg))
+    assert ("slice_kernel" in name.value.decode()) == sliced, name.value

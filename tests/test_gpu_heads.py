@@ -795,7 +795,7 @@ _SLICE_SHAPES = [
     (16, 16 * 256 * 7 + 40, 2048, None, True), (32, 8200, 2048, None, True), (17, 5000, 4096, 2.0, True), (33, 9001, 2048, None, True),
     (64, 20000, 2048, None, True), (100, 3001, 4096, None, True), (128, 12007, 2048, 0.5, True),
     (1, 9, 2048, None, False), (16, 16 * 256 + 1, 4096, 0.3125, False), (3, 40001, 4096, None, False), (24, 33000, 2048, None, False),
-    (60, 7001, 4096, None, False), (128, 3000, 2048, None, False)]
+    (60, 7001, 4096, None, False), (128, 3000, 2048, None, False), (97, 32768, 2048, None, False)]
 
 
 @pytest.mark.parametrize("n,V,H,scale,tiled", _SLICE_SHAPES)
