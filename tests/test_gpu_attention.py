@@ -454,6 +454,17 @@ def test_randomised_shape_sweep(gpu, orc, P, T, mode, splits, slack, seed):
         assert np.array_equal(to_np(vc).view(np.uint16), v.view(np.uint16))
 
 
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("P,T,splits", [
+    (0, 65, 1), (0, 128, 1), (1, 128, 1), (63, 128, 1), (64, 65, 1), (64, 128, 1), (65, 127, 1), (127, 66, 1), (129, 128, 1), (191, 128, 1), (192, 100, 1),
+    (255, 128, 1), (257, 127, 1), (319, 128, 1), (400, 128, 1),  # one split of two to nine tiles: every stage of the ring is the free one
+    (0, 128, 2), (63, 128, 3), (190, 128, 2), (300, 127, 4), (520, 128, 3), (700, 65, 13), (700, 128, 13), (961, 128, 8), (1000, 128, 17), (1337, 97, 6)])
+def test_appended_rows_beyond_the_staged_ones(gpu, orc, P, T, splits, rope):
+    """Trees of more than 64 nodes: the rows behind the first 64 pass through the ring stage that the last tile leaves free.  Splits of few
+    tiles and of many, new rows in the tiles of one split, of two and of three, at the edges of tiles and pages."""
+    test_randomised_shape_sweep(gpu, orc, P, T, "append_rope" if rope else "append", splits, [0, 65, 300][P % 3], 3000 + P + T)
+
+
 def _heads_case(torch, orc, HQ_, HKV_, P, T, mode, seed):
     """One attention call with HQ_ query heads on HKV_ KV heads (any ratio) against the oracle; appended rows bit for bit."""
     from cpm.cu_amd import ops
