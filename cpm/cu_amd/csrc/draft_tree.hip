@@ -88,8 +88,9 @@ __global__ void draft_begin_kernel(DraftState s, int k, const uint16_t* val, con
 }
 
 // A chain of round trips (arguments, candidates, vocabulary ids) around a short count, so an entry stays with its thread: what a chosen one
-// needs -- its id is looked up for every candidate, under the count -- is in registers when its place is known.  (A draft of 6 rounds of 10 in a
-// replayed graph 364.9 -> 361.4 us, one of 4 rounds of 4 call by call 105.7 -> 103.4, against looking the chosen ones' ids up behind the count.)
+// needs -- its id is looked up for every candidate, under the count -- is in registers when its place is known.  (Against looking the chosen ones' ids up behind the
+// count, replayed graphs, three runs of either build in turn within 0.2 us: the launch 3.06 -> 2.69 us with 10 x 10 candidates, 2.41 -> 2.00 with 4 x 4,
+// 38.4 -> 37.9 with 32 x 32; a draft of 6 rounds of 10 361.3 -> 358.4, one of 4 rounds of 4 104.5 -> 102.6.  A first pass on new inputs shows no gain.)
 // kEntries: entries of a thread, at most.  The loads have no branches around them (an entry past the end repeats the last one): behind a
 // branch the compiler would wait for the ids in front of the count.
 template <int kEntries>

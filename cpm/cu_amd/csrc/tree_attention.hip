@@ -417,7 +417,9 @@ __device__ inline void scalar_load3(const int32_t* pa, const int32_t* pb, const 
 // A wave requests 2 KB of a K tile (8 rows) and as much of a V^T tile (16 dims), 1 KB in lane order by each request; the swizzle is
 // applied on the global side.  The two requests fill consecutive KB of LDS, so that one LDS address (m0) and one base serve both: the
 // immediate offset of the second is added to both addresses, and the lane's own offset makes up the difference.  (44 -> 14 scalar
-// instructions a tile; with registers freed in the paths of few tiles, 60 nodes at 32K 45.2 -> 44.8 us a layer, 128 at 4K 24.8 -> 22.5.)
+// instructions a tile.  With registers freed in the paths of few tiles, us a layer in replayed graphs, both builds in turn, three times on each of three
+// boards: 60 nodes at 4K 16.0 -> 15.8, at 8K 20.0 -> 19.7, at 32K 44.1 -> 43.8, there with the rotary embedding 46.2 -> 45.1; 24 nodes at 32K 26.9 -> 26.4;
+// 128 nodes level; 8 KV heads 33 nodes at 10007 21.6 -> 21.7, 16 at 20000 28.0 -> 28.3.)
 constexpr int kRequests = 16 / kWaves;  // of a wave, for K and for V^T
 static_assert(kRequests == 2, "TileOffsets");
 struct TileOffsets {
@@ -633,7 +635,9 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         const int page = page_of_tile(tile);
         if constexpr (G == 1 || ROPE) {
             // (the other requests' offsets are worked out from these each time: two registers less.  Two groups have them to spare without the
-            // rotary embedding: 33 nodes at 10007 keys on 8 KV heads in bfloat16, a step of 32 layers, 805 -> 798 us)
+            // rotary embedding: us a layer in replayed graphs, both builds in turn, three times on each of three boards: 33 nodes at
+            // 10007 keys on 8 KV heads in bfloat16 21.72 -> 21.57, every run; in fp16 level; 24 at 32K on 2 26.3 -> 26.05; 16 at 20000 on 8 28.3 -> 28.45;
+            // 60 nodes level)
             off.k0 = here(off.k0);
             off.v0 = here(off.v0);
         }
@@ -678,7 +682,8 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     // The rows beyond the staging area (trees of more than kVStageRows nodes, whose new rows reach into three tiles at most) go to the
     // ring stage of the tile behind this workgroup's last, as soon as every wave has left the tile that was there: when
     // the first tile with new rows is mended, or the one behind it.  (Read from v_new element by element where a tile is
-    // mended, they kept the last split 11 us behind the others with 128 nodes.)
+    // mended, they kept the last split 11 us behind the others with 128 nodes: 24.8 -> 22.1 us a layer at 4K, 82.2 -> 77.9 at 32K.
+    // A kernel of its own for these trees is no faster, theirs or the others': 22.3 at 4K, 60 nodes level.)
     enum { kNoLate, kLateWanted, kLateOnTheWay, kLateHere };
     int late = p.k_new != nullptr && p.T > kVStageRows && (t0 + n) * kTileN > P + kVStageRows ? kLateWanted : kNoLate;
     char* const late_rows = ring + (n % kStages) * kStageBytes;
