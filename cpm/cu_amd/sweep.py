@@ -114,7 +114,7 @@ def attention(torch, with_groups, Hq=32, Hkv=2, graph=False, with_direct=False, 
 
 def head(torch, row_major=False):
     from . import ops
-    rows = [1, 16, 17, 32, 33, 60, 64, 100, 128]
+    rows = [1, 16, 17, 32, 33, 60, 64] + [96] * row_major + [100, 128]
     for H in (2048, 4096, 8192):
         print("target head, hidden size %d, %s weights: fraction of 8 TB/s (kernel)" % (H, "row-major" if row_major else "tiled"))
         print("%8s" % "V \\ n" + "".join("%20d" % n for n in rows))
