@@ -68,8 +68,8 @@ constexpr int kVTileBytes = kHeadDim * kTileN * 2;  // 16 KB, row = one dim (128
 constexpr int kStageBytes = kKTileBytes + kVTileBytes;
 constexpr int kVStageRows = 64;  // appended V rows staged in LDS ahead of their transposition
 constexpr int kMaxSplits = 128;
-constexpr int kMergeMaxSplits = 32;  // most splits of a launch that merges its own partials: arrivals on one counter
-                                     // serialise, about 0.15 us each
+constexpr int kMergeMaxSplits = 32;  // most splits of a launch of the split shapes that merges its own partials: arrivals on one
+                                     // counter serialise, about 0.15 us each (the direct shape: direct_merge_shares)
 constexpr int kXcds = 8;
 constexpr float kLazyLog2 = 8.f;  // slack of the lazily updated softmax reference, in log2 units
 

@@ -97,8 +97,10 @@ const char* cpmcu_version(void);
  *                           4096 columns the K-slice kernel (default), 0 = always
  *                           the K-chunked kernel (CPMCU_HEAD_NO_STREAM set);
  *   "attn_merge_in_launch"  1 = the workgroups of a split tree-attention launch merge their own partials when the
- *                           launch fits the GPU's CUs and has at most 32 splits (default), 0 = always the separate
- *                           merge launch (CPMCU_ATTN_SEPARATE_MERGE set);
+ *                           launch fits the GPU's CUs and has at most 32 splits, those of the direct shape always (in
+ *                           shares from 16 splits on if the launch fits, else by the last to arrive) (default), 0 = always
+ *                           the separate merge launch, and the direct shape for launches of one split only
+ *                           (CPMCU_ATTN_SEPARATE_MERGE set);
  *   "attn_merge_wait_us"    longest time a workgroup of such a launch waits for the others of its merge before it
  *                           leaves its share to the last one to arrive (default 2000; 0 = never wait);
  *   "topk_row_kernel"       1 = top-k by the one-launch row kernel (rows of more than 32768 elements in slices and a
