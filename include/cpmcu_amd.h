@@ -102,7 +102,8 @@ const char* cpmcu_version(void);
  *                           the separate merge launch, and the direct shape for launches of one split only
  *                           (CPMCU_ATTN_SEPARATE_MERGE set);
  *   "attn_merge_wait_us"    longest time a workgroup of such a launch waits for the others of its merge before it
- *                           leaves its share to the last one to arrive (default 2000; 0 = never wait);
+ *                           leaves its share to the last one to arrive (default 2000; 0 = never wait: split launches leave
+ *                           their shares at once, those of the direct shape are merged whole by the last to arrive);
  *   "topk_row_kernel"       1 = top-k by the one-launch row kernel (rows of more than 32768 elements in slices and a
  *                           merge of the slices' k best) (default), 0 = k rounds of a maximum search per chunk of 2048
  *                           elements and a merge launch, for chunks x k up to 2048: the same results, bit for bit,

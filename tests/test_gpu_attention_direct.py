@@ -112,8 +112,9 @@ def test_merge_in_shares_against_the_oracle(gpu, orc, option, P, T, hq, hkv, spl
 @pytest.mark.parametrize("dtype", [0, 1])
 @pytest.mark.parametrize("hkv,splits", [(2, 20), (2, 100), (8, 32)])
 def test_shares_left_behind_are_merged_by_the_last_arrival(gpu, option, hkv, splits, dtype):
-    """A wait limit of zero: every workgroup but a unit's last gives its share up (unless all have arrived); the output is the
-    same to the bit, and the launch behind it is whole again."""
+    """A wait limit of 1 us, which the arrivals of 20 workgroups and more on one word do not keep: those that it runs out for give their
+    share up; the output is the same to the bit, and the launch behind it is whole again.  That the launches are direct ones with a CU for every workgroup, and that
+    shares were given up, is asserted: without either the outputs would be the same."""
     from cpm.cu_amd import lib, ops
     from cpm.cu_amd.kvcache import PagedKVCache
     torch, L = gpu, lib.get()
@@ -126,10 +127,16 @@ def test_shares_left_behind_are_merged_by_the_last_arrival(gpu, option, hkv, spl
     cache = PagedKVCache(1, hkv, (S + 255) // 256)
     cache.write_logical(0, 0, rnd(S, hkv, D), rnd(S, hkv, D))
     q, kv_len = rnd(1, 32, D), torch.tensor([S], dtype=torch.int32, device="cuda")
+    kernel, used, _, workgroups = ops.attention_plan(1, 32, hkv, S, num_splits=splits)
+    assert (kernel, used) == ("tree_attn_direct_kernel", splits)
+    assert workgroups <= torch.cuda.get_device_properties(0).multi_processor_count
+    L.synchronize()
+    option("attn_merge_in_launch", 1)
     ref = ops.tree_attention(q, cache, 0, kv_len, S, num_splits=splits)
-    torch.cuda.synchronize()
+    L.synchronize()
+    before = L.raw.cpmcu_attention_abandoned_waits()
     try:
-        for wait_us in (0, 0, 2000, 0):
+        for wait_us in (1, 1, 2000, 1, 1, 1, 1):
             option("attn_merge_wait_us", wait_us)
             out = torch.full_like(q, float("nan"))
             ops.tree_attention(q, cache, 0, kv_len, S, num_splits=splits, out=out)
@@ -138,13 +145,16 @@ def test_shares_left_behind_are_merged_by_the_last_arrival(gpu, option, hkv, spl
     finally:
         option("attn_merge_wait_us", 2000)
         L.synchronize()
-        option("attn_merge_in_launch", 1)  # (the waits that ran out had sent the workspaces back to the merge launch)
+        option("attn_merge_in_launch", 1)  # (nobody had waited in these workspaces' launches from the synchronisation on)
+    assert L.raw.cpmcu_attention_abandoned_waits() > before, "no share was left behind"
 
 
+@pytest.mark.parametrize("zero_limit", [False, True])
 @pytest.mark.parametrize("hkv,T,splits", [(2, 1, 2), (2, 4, 15), (2, 1, 16), (8, 2, 32), (2, 1, 37), (1, 1, 128), (2, 3, 0)])
-def test_direct_launches_after_an_abandoned_wait(gpu, option, hkv, T, splits):
+def test_direct_launches_after_an_abandoned_wait(gpu, option, hkv, T, splits, zero_limit):
     """After a merge wait that ran out on the device a launch of the direct shape stays one: nobody waits in it, and the last arrival
-    merges.  Its partials, in the workspace, are those of the launch that waits, bit for bit."""
+    merges.  Its partials, in the workspace, are those of the launch that waits, bit for bit.  A wait limit of zero does the same from the
+    first launch on: nothing is left behind for the last arrival to merge share by share."""
     import ctypes
     from cpm.cu_amd import lib, ops
     from cpm.cu_amd.kvcache import PagedKVCache
@@ -179,14 +189,20 @@ def test_direct_launches_after_an_abandoned_wait(gpu, option, hkv, T, splits):
         if not L.raw.cpmcu_tree_attention_merge_mode(ctypes.c_void_p(ws.data_ptr())):
             pytest.skip("this process has used up the library's counter blocks")
         ref, ref_parts = call()
-        # a wait that runs out: with a limit of zero a launch of 64 splits leaves shares behind
-        option("attn_merge_wait_us", 0)
-        for _ in range(4):
-            ops.tree_attention(q[:1], cache, 0, kv_len, S, num_splits=64 // hkv * 2)
-        before = L.raw.cpmcu_attention_abandoned_waits()
         L.synchronize()
         seen = L.raw.cpmcu_attention_abandoned_waits()
-        assert seen > before and L.raw.cpmcu_tree_attention_merge_mode(ctypes.c_void_p(ws.data_ptr())) == 0
+        option("attn_merge_wait_us", 0)
+        if not zero_limit:
+            # a wait that runs out: with a limit of zero the split shapes leave shares behind
+            option("attn_direct", 0)
+            for _ in range(4):
+                ops.tree_attention(q[:1], cache, 0, kv_len, S, num_splits=32)
+            before = seen
+            L.synchronize()
+            seen = L.raw.cpmcu_attention_abandoned_waits()
+            assert seen > before and L.raw.cpmcu_tree_attention_merge_mode(ctypes.c_void_p(ws.data_ptr())) == 0
+            option("attn_direct", 1)
+            option("attn_merge_wait_us", 2000)
         for _ in range(2):
             out, parts = call()
             if splits:  # (else the number of splits is chosen anew)
