@@ -1001,8 +1001,8 @@ extern "C" int cpmcu_print_perf_summary(void) {
 
 // Extension: merge waits of tree-attention launches that ran out since the library was loaded, as seen by the
 // synchronising calls so far (cpmcu_synchronize, cpmcu_verify_and_fix).  Each is a workgroup that stopped waiting for the
-// others of its unit and left its share of the merge to the last of them: the output was complete, but late, and the
-// device's workspaces have gone back to the separate merge launch (cpmcu_set_option("attn_merge_in_launch", 1) undoes that).
+// others of its unit and left its share of the merge to the last of them: the output was complete, but late, and nobody
+// waits in later launches on the device's workspaces (cpmcu_set_option("attn_merge_in_launch", 1) undoes that).
 extern "C" long cpmcu_attention_abandoned_waits(void) { return g_abandoned_waits; }
 
 // Rows of one-launch FR-Spec heads seen by the library's synchronisations so far: finished from the published candidates,

@@ -290,7 +290,8 @@ int cpmcu_synchronize(void);
  * and ends: the output is complete, only late.  It happens when the launch's workgroups are not all resident at once,
  * i.e. when another launch holds CUs.  After the first such wait is seen, nobody waits in launches on the device's
  * workspaces: split ones go back to the separate merge launch, those of the direct shape to the merge by the workgroup
- * that arrives last.  cpmcu_set_option("attn_merge_in_launch", 1) lets them wait again. */
+ * that arrives last.  Launches that a graph holds already keep the form in which they were recorded.
+ * cpmcu_set_option("attn_merge_in_launch", 1) lets later ones wait again. */
 long cpmcu_attention_abandoned_waits(void);
 /* Free everything the global model owns (the reference never frees). */
 int cpmcu_shutdown(void);
