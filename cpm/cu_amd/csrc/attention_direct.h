@@ -11,7 +11,8 @@
 //   * the appended rows are a block of their own, read from k_new / v_new (split 0 takes it first, while its pages are on their
 //     way), so no tile has to be patched; workgroups of their own (the first grid rows) write them to the pool meanwhile;
 //   * the partials of few splits are merged by the last workgroup of a unit to arrive: nobody polls or waits, so the launch may be larger
-//     than the chip.  Those of many splits are merged in shares: one query at 60001 keys 23.0 -> 19.0 us per layer, at 4096 9.0 -> 7.9.
+//     than the chip.  Those of many splits are merged in shares, by words that say themselves whether they are there: a kernel of its own
+//     (tree_attn_direct_shares_kernel), since code that a launch jumps over is fetched all the same, 0.1-0.2 us.
 // The products are the transposed ones of the other shapes (S^T = K.Q^T, O^T = V^T.P^T), on v_mfma_f32_16x16x32: lane (c, h) =
 // (lane & 15, lane >> 4) of a score block holds query row c and four keys.  Which key sits in which row of the K operand is free;
 // it is chosen so that the eight probabilities of a lane of the B operand belong to eight neighbouring slots of a V^T row.
@@ -23,7 +24,25 @@
 constexpr int kDirectRows = 16;        // packed query rows per workgroup
 constexpr int kBlockKeys = kPage / 2;  // keys per iteration
 constexpr int kDirectItems = kDirectRows * 4;  // pieces of a unit's output that are merged by themselves: 32 dims of a row
-constexpr int kDirectLastMerges = 15;         // up to here the last arrival merges all splits
+constexpr int kDirectLastMerges = 15;          // up to here the last arrival merges all splits
+// A partial that is merged in shares changes hands through memory of the library: every 8-byte word carries two outputs (or half of a
+// row's statistics) and the generation of its slot, so that a reader that sees the generation has the payload, and nothing is acknowledged
+// or counted in front of the reads (acknowledgement, arrival, poll and read were four round trips, store and poll are two).  A slot's
+// generation is read when a launch begins and advanced by the last arrival of its unit, so no older word passes for a fresh one (but for one
+// of exactly 2^32 launches ago).  us per layer in replayed graphs, partials counted in / words: one query with the rotary embedding on 2 KV
+// heads 7.4 / 7.1 at 4096 keys, 11.4 / 10.4 at 16384, 19.5 / 17.9 at 60001, 30.0 / 28.6 at 131072; on 8 heads 10.0 / 9.6 at 4096, 21.0 / 19.6 at
+// 20000; two queries 9.0 / 8.6 at 9000; four 8.5 / 8.5 at 4096, on 4 heads 11.2 / 11.45 at 8192.  A plain copy of the partials beside the words: 0.1-0.4 more.
+constexpr int kDirectSlots = 256;                           // workgroups of such a launch
+constexpr int kSlotQuads = kDirectRows * 32 + kDirectRows;  // of 16 bytes: four dims of a row, then a row's maximum and sum
+constexpr int kSlotBytes = kSlotQuads * 16;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+struct DirectSlots {
+    uint32_t generation[kDirectSlots];
+    u32x4 words[kDirectSlots][kSlotQuads];
+    // the partials of such a launch where nobody is to wait: the last arrival reads them once it has counted all
+    f16 o[kDirectSlots][kDirectRows][kHeadDim];
+    float2 ml[kDirectSlots][kDirectRows];
+};
 static_assert(kThreads == kDirectRows * 32, "the merge: 32 threads per row");
 // The keys of a group of 32 make two operand blocks.  Row m of the K operand of block b of a group is its key direct_key_of_row(m) + 8 b;
 // probability j of lane (., h) of the group's B operand belongs to key 16 (h / 2) + 4 (h % 2) + j % 4 + 8 (j / 4), whose slots in
@@ -31,47 +50,46 @@ static_assert(kThreads == kDirectRows * 32, "the merge: 32 threads per row");
 __device__ inline int direct_key_of_row(int m) { return 16 * (m >> 3) + 4 * ((m >> 2) & 1) + (m & 3); }
 // Swizzled 16-byte pieces of a 256-byte row: the 16 lanes of an operand read touch 16 different columns.
 __device__ inline int direct_off(int row, int piece) { return row * 256 + ((piece ^ (row & 15)) << 4); }
-// x over the four lanes of a column (lanes c, c + 16, c + 32, c + 48)
-__device__ inline float column_max(float x) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+// Exchanges between lanes that take no LDS: max (or sum) with the lane 16 or 32 away, the value of the lane 8 or so away.
+template <bool MAX>
+__device__ inline float max_or_sum(float a, float b) {
+    return MAX ? fmaxf(a, b) : a + b;
 }
-
-// max (or sum) over the 32 lanes of a half wave
+template <int CTRL>
+__device__ inline float dpp(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+__device__ inline float lanes_8(float x) { return dpp<0x128>(x); }  // rotated by 8 in 16
+template <bool MAX>
+__device__ inline float with_lanes_16(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return max_or_sum<MAX>(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+template <bool MAX>
+__device__ inline float with_lanes_32(float x) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return max_or_sum<MAX>(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+// x over the four lanes of a column (lanes c, c + 16, c + 32, c + 48)
+__device__ inline float column_max(float x) { return with_lanes_32<true>(with_lanes_16<true>(x)); }
+// over the 32 lanes of a half wave
 template <bool MAX>
 __device__ inline float half_wave(float x) {
-    auto with = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
-    auto dpp = [](float v, auto ctrl) {
-        return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), decltype(ctrl)::value, 0xf, 0xf, true));
-    };
-    x = with(x, dpp(x, std::integral_constant<int, 0xB1>{}));   // lane ^ 1
-    x = with(x, dpp(x, std::integral_constant<int, 0x4E>{}));   // lane ^ 2
-    x = with(x, dpp(x, std::integral_constant<int, 0x141>{}));  // mirrored in 8
-    x = with(x, dpp(x, std::integral_constant<int, 0x140>{}));  // mirrored in 16
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return with(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    x = max_or_sum<MAX>(x, dpp<0xB1>(x));   // lane ^ 1
+    x = max_or_sum<MAX>(x, dpp<0x4E>(x));   // lane ^ 2
+    x = max_or_sum<MAX>(x, dpp<0x141>(x));  // mirrored in 8
+    x = max_or_sum<MAX>(x, dpp<0x140>(x));  // mirrored in 16
+    return with_lanes_16<MAX>(x);
 }
-
-// the same over all 64 lanes
+// over the 16 lanes of the same number modulo 4
 template <bool MAX>
-__device__ inline float full_wave(float x) {
-    x = half_wave<MAX>(x);
-    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return MAX ? fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])) : __uint_as_float(a[0]) + __uint_as_float(a[1]);
-}
-// x over the 16 lanes of the same number modulo 4
 __device__ inline float over_splits(float x) {
-    x += __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(x), 0x124, 0xf, 0xf, true));  // rotated by 4 in 16
-    x += __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(x), 0x128, 0xf, 0xf, true));  // by 8
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    x = max_or_sum<MAX>(x, dpp<0x124>(x));  // rotated by 4 in 16
+    x = max_or_sum<MAX>(x, lanes_8(x));
+    return with_lanes_32<MAX>(with_lanes_16<MAX>(x));
 }
 
-template <typename E>
+template <bool SHARES, typename E>
 __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     typedef typename Elem<E>::x8 X8;
     typedef typename Elem<E>::x4 X4;
@@ -85,16 +103,15 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         } block;
         AppendStage append[kThreads / kAppendThreads];
         float weight[kMaxSplits][kDirectRows];  // of the merge by the last arrival
-        f32x4 sums[kWaves][8];                  // of the merge in shares: 32 dims
     } s;
     __shared__ __attribute__((aligned(1024))) char s_q[kDirectRows * kHeadDim * 2];
     __shared__ X8 s_p[kGroups][64];                   // the probabilities of an iteration
     __shared__ f32x4 s_max[kDirectRows][kWaves / 4];  // each wave's row maxima
     __shared__ Arrival s_arrival;
-    __shared__ uint32_t s_abandoned[kDirectItems / 32];
+    __shared__ int s_late[2];  // the merge in shares: a wave's wait for partials ran out
     asm volatile("" ::"s"(p.q), "s"(p.k_pool), "s"(p.v_pool), "s"(p.block_table), "s"(p.kv_len), "s"(p.k_new), "s"(p.v_new), "s"(p.rope),
-                 "s"(p.mask), "s"(p.mask_words), "s"(p.mask_k_range), "s"(p.T), "s"(p.Hq), "s"(p.Hkv), "s"(p.group), "s"(p.group_shift),
-                 "s"(p.hkv_shift), "s"(p.num_splits), "s"(p.num_mtiles), "s"(p.table_pages), "s"(p.window_blocks), "s"(p.max_kv_len));
+                 "s"(p.mask), "s"(p.mask_words), "s"(p.mask_k_range), "s"(p.T), "s"(p.Hq), "s"(p.Hkv), "s"(p.group), "s"(p.group_inv),
+                 "s"(p.hkv_inv), "s"(p.num_splits), "s"(p.num_mtiles), "s"(p.table_pages), "s"(p.window_blocks), "s"(p.max_kv_len));
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int append = p.k_new != nullptr ? 1 : 0;
@@ -114,8 +131,8 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         constexpr int kHalves = kThreads / kAppendThreads;
         const int y = (blockIdx.y * gridDim.x + sh) * kHalves + tid / kAppendThreads;
         if (y / kHalves * kHalves < runs * p.Hkv) {
-            const int gg = p.hkv_shift >= 0 ? y & (p.Hkv - 1) : y % p.Hkv;
-            const int run = p.hkv_shift >= 0 ? y >> p.hkv_shift : y / p.Hkv;
+            const Quotient y_of = divide(y, p.Hkv, p.hkv_inv);
+            const int gg = y_of.r, run = y_of.q;
             kv_append_run<E, true>(p.k_pool_w, p.v_pool_w, p.block_table, p.k_new, p.v_new, p.rope, p.T, p.Hkv, gg, run * kAppendRows,
                              tid % kAppendThreads, s.append[tid / kAppendThreads], [&]() {
                                  S = scalar_load(p.kv_len);
@@ -126,10 +143,18 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         return;
     }
     if (sh >= p.num_splits * p.Hkv) return;
-    const int g = p.hkv_shift >= 0 ? sh & (p.Hkv - 1) : sh % p.Hkv;
-    const int split = p.hkv_shift >= 0 ? sh >> p.hkv_shift : sh / p.Hkv;
+    const Quotient sh_of = divide(sh, p.Hkv, p.hkv_inv);
+    const int g = sh_of.r, split = sh_of.q;
     const int unit = g * p.num_mtiles + mt;
     const int c = lane & 15, h = lane >> 4;
+    // lane i: the generation that the words of splits i and i + 64 carry in this launch
+    uint32_t fresh[2] = {0, 0};
+    if constexpr (SHARES) {
+        const uint32_t* gen = p.slots->generation + unit * p.num_splits;
+        fresh[0] = __hip_atomic_load(gen + min(lane, p.num_splits - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        if (tid < 2) s_late[tid] = 0;
+        if (p.num_splits > 64) fresh[1] = __hip_atomic_load(gen + min(lane + 64, p.num_splits - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    }
 
     // This workgroup's blocks: base + block_of(i), i = 0, 1, ...  The appended rows come in front of the stream, as its block 0.
     const bool has_new = append && split == 0;
@@ -149,8 +174,12 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     int pages = 0;
     if (may_iterate) pages = pages_from(0);
 
-    auto node_of = [&](int R) { return p.group_shift >= 0 ? R >> p.group_shift : R / p.group; };
-    auto head_of = [&](int R) { return g * p.group + (p.group_shift >= 0 ? R & (p.group - 1) : R % p.group); };
+    auto node_of = [&](int R) { return divide(R, p.group, p.group_inv).q; };
+    // where row R of q and out begins
+    auto row_at = [&](int R) {
+        const Quotient row = divide(R, p.group, p.group_inv);
+        return ((size_t)row.q * p.Hq + g * p.group + row.r) * kHeadDim;
+    };
     const int last_row = p.group * p.T - 1;
     const int my_node = node_of(min(mt * kDirectRows + c, last_row));
     // What this lane's row sees of the tree: needed where keys of the mask's range are met.
@@ -195,7 +224,7 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     if (tid < kQThreads) {
         const int R = min(mt * kDirectRows + t_row, last_row);
         const int node = node_of(R);
-        fetch_row(rq, rq_cs, p.q + ((size_t)node * p.Hq + head_of(R)) * kHeadDim, node);
+        fetch_row(rq, rq_cs, p.q + row_at(R), node);
     }
     // 32 appended rows at a time, by the upper half of the threads: K row t is row m of block b, in the K area of wave b ...
     constexpr int kNewRows = 32;
@@ -237,6 +266,7 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     // counts its outstanding requests by hand, four for its keys and four for its dims of a block: everything the compiler
     // has requested so far (page ids, mask words, rows) is waited for first.
     asm volatile("" : "+v"(mw0), "+v"(mw1), "+v"(pages));
+    if constexpr (SHARES) asm volatile("" : "+v"(fresh[0]), "+v"(fresh[1]));
     if (tid < kQThreads) arrived(rq, rq_cs);
     if (has_new && wave >= kWaves / 2) arrived(rk, rk_cs);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -374,7 +404,6 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         __syncthreads();
         if (late_keys && has(0)) load_k(0);
     }
-
     // A block's keys are requested ahead of its dims (but for late ones), each as soon as its area has been read.
     constexpr auto kAll = std::integral_constant<int, kGroups>{};
     for (int i = 0; has(i); ++i) {
@@ -415,103 +444,175 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (more) load_v(i + 1);
     }
-
-    const bool whole = p.num_splits == 1;
-    // Results leave normalised: the output rows themselves, or partials
-    //   o_part [unit][split][16 rows][128],  ml_part [unit][split][16 rows] x (max * scale_log2, sum)
-    // written through to memory.
-    char* const o_part = reinterpret_cast<char*>(p.o_part) + (size_t)unit * p.num_splits * kPartBytes;
-    char* const ml_part = reinterpret_cast<char*>(p.ml_part) + (size_t)unit * p.num_splits * (kDirectRows * 8);
+    const bool whole = !SHARES && p.num_splits == 1;
+    constexpr int kSc1 = 16;  // past the (per-XCD) L2
+    const float L = l[0];
+    X4 result;
     {
-        const float L = l[0];
         const float inv = (L == 0.f || L != L) ? (whole ? 1.f : 0.f) : 1.f / L;
-        X4 x;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = (E)(o[e] * inv);
-        const int R = mt * kDirectRows + c, dim = wave * 16 + h * 4;
-        if (whole) {
-            if (R <= last_row) *reinterpret_cast<X4*>(p.out + ((size_t)my_node * p.Hq + head_of(R)) * kHeadDim + dim) = x;
-        } else {
-            store_dev64(o_part + split * kPartBytes + (c * kHeadDim + dim) * 2, bits_as<uint64_t>(x));
-            if (wave == 0 && h == 0)
-                store_dev64(ml_part + (split * kDirectRows + c) * 8, (uint64_t)__float_as_uint(M) | ((uint64_t)__float_as_uint(L) << 32));
-        }
+        for (int e = 0; e < 4; ++e) result[e] = (E)(o[e] * inv);
     }
+    const int my_dim = wave * 16 + h * 4;
     if (whole) {
+        const int R = mt * kDirectRows + c;
+        if (R <= last_row) *reinterpret_cast<X4*>(p.out + row_at(R) + my_dim) = result;
         return;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
     uint32_t* const ctr = p.merge_ctr + kMergeUnitWords * unit;
-    if (tid == 0) s_arrival = arrive_at_unit(p, ctr, split < p.merge_shares ? split : -1);
-    __syncthreads();
-    const auto o_rsrc = __builtin_amdgcn_make_buffer_rsrc(o_part, 0, p.num_splits * kPartBytes, 0x00027000);
-    constexpr int kSc1 = 16;  // past the (per-XCD) L2
-    if (p.merge_shares > 0) {
-        // The merge in shares.  An item is 32 dims of a row, 64 bytes of each partial: a wave reads 16 splits' worth at once, and as many
-        // waves as the splits need work on an item, so that a share is one round trip.  (The last arrival alone has all 4 KB of every
-        // split to read: 0.04 us per split, 23.0 us for one query at 60001 keys on 64 splits.)
-        const int item_waves = p.num_splits <= 16 ? 1 : p.num_splits <= 32 ? 2 : p.num_splits <= 64 ? 4 : 8;
-        const int at_once = kWaves / item_waves;
+    if constexpr (SHARES) {
+        __shared__ f32x4 s_sums[2][kWaves][8];   // 32 dims
+        __shared__ float2 s_sums_ml[2][kWaves];  // their (maximum, sum of the weights)
+        __shared__ uint32_t s_abandoned[kDirectItems / 32];
+        // The merge in shares, by words that say themselves whether they are there (DirectSlots).  An item is 32 dims of a row, 128 bytes of
+        // each slot: a wave reads 16 splits' worth at once, and as many waves as the splits need work on an item, so that a share is
+        // one round trip.
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(p.slots->words[unit * p.num_splits], 0, p.num_splits * kSlotBytes, 0x00027000);
+        {
+            const uint32_t mine = (uint32_t)__builtin_amdgcn_readlane((int)(split < 64 ? fresh[0] : fresh[1]), split & 63);
+            const uint64_t bits = bits_as<uint64_t>(result);
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4{(uint32_t)bits, mine, (uint32_t)(bits >> 32), mine}, rsrc,
+                                                   split * kSlotBytes + (c * 32 + (my_dim >> 2)) * 16, 0, kSc1);
+            if (wave == 0 && h == 0)
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(M), mine, __float_as_uint(L), mine}, rsrc,
+                                                       split * kSlotBytes + (kDirectRows * 32 + c) * 16, 0, kSc1);
+        }
+        const int item_shift = (p.num_splits > 16) + (p.num_splits > 32) + (p.num_splits > 64);
+        const int item_waves = 1 << item_shift, at_once = kWaves >> item_shift;
         const int items = min(kDirectRows, last_row + 1 - mt * kDirectRows) * 4;
-        auto merge_share = [&](int share) {
+        const int slot = wave >> item_shift, part = wave & (item_waves - 1);
+        const int my_split = part * 16 + (lane >> 2);  // whose words this lane reads
+        const uint32_t my_fresh = (uint32_t)__shfl((int)(part < 4 ? fresh[0] : fresh[1]), my_split & 63);
+        int parity = 0;
+        // False (in every wave): the wait for the words ran out.
+        auto merge_share = [&](int share, uint32_t limit) {
+            const unsigned long long t_begin = wall_clock64();
             for (int i0 = share * at_once; i0 < items; i0 += p.merge_shares * at_once) {
-                const int slot = wave / item_waves, part = wave % item_waves;
                 const int item = min(i0 + slot, items - 1), row = item >> 2;
-                const int split0 = part * 16;
-                const X8 x = bits_as<X8>(__builtin_amdgcn_raw_buffer_load_b128(
-                    o_rsrc, (split0 + (lane >> 2)) * kPartBytes + item * 64 + (lane & 3) * 16, 0, kSc1));  // (zeros past the last split)
-                // the weights of all splits in every wave: lane i has those of splits i and i + 64
-                float m[2] = {-INFINITY, -INFINITY}, w[2] = {0.f, 0.f};
-#pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const int sp = lane + 64 * k;
-                    if (64 * k < p.num_splits && sp < p.num_splits) {
-                        const uint64_t ml = load_dev64(ml_part + (sp * kDirectRows + row) * 8);
-                        m[k] = __uint_as_float((uint32_t)ml);
-                        w[k] = __uint_as_float((uint32_t)(ml >> 32));
+                const int at = my_split * kSlotBytes + item * 128 + (lane & 3) * 32, ml_at = my_split * kSlotBytes + (kDirectRows * 32 + row) * 16;
+                u32x4 xa = {0, 0, 0, 0}, xb = xa, ml = xa;
+                bool there = my_split >= p.num_splits;
+                for (;;) {
+                    if (!there) {  // (the lanes that still wait)
+                        xa = __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, kSc1);
+                        xb = __builtin_amdgcn_raw_buffer_load_b128(rsrc, at + 16, 0, kSc1);
+                        ml = __builtin_amdgcn_raw_buffer_load_b128(rsrc, ml_at, 0, kSc1);
+                        there = ((xa[1] ^ my_fresh) | (xa[3] ^ my_fresh) | (xb[1] ^ my_fresh) | (xb[3] ^ my_fresh) | (ml[1] ^ my_fresh) | (ml[3] ^ my_fresh)) == 0;
                     }
+                    if (__all(there) || wall_clock64() - t_begin >= limit) break;
+                    asm volatile("" ::: "memory");  // (loads anew)
                 }
-                float top = full_wave<true>(fmaxf(m[0], m[1]));
-                top = top == -INFINITY ? 0.f : top;
-#pragma unroll
-                for (int k = 0; k < 2; ++k) w[k] *= __builtin_amdgcn_exp2f(m[k] - top);
-                const float sum = full_wave<false>(w[0] + w[1]);
-                const float inv = (sum == 0.f || sum != sum) ? 1.f : 1.f / sum;
-                const float weight = __shfl(part < 4 ? w[0] : w[1], (split0 + (lane >> 2)) & 63) * inv;
+                if (!__all(there)) s_late[parity] = 1;
+                // sums over the wave's splits, relative to their own maximum
+                const float m = my_split < p.num_splits ? __uint_as_float(ml[0]) : -INFINITY;
+                const float top = over_splits<true>(m);
+                const float weight = __uint_as_float(ml[2]) * __builtin_amdgcn_exp2f(m - (top == -INFINITY ? 0.f : top));
+                const X8 x = bits_as<X8>(u32x4{xa[0], xa[2], xb[0], xb[2]});
                 f32x4 lo, hi;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    lo[e] = over_splits(weight * (float)x[e]);
-                    hi[e] = over_splits(weight * (float)x[e + 4]);
+                    lo[e] = over_splits<false>(weight * (float)x[e]);
+                    hi[e] = over_splits<false>(weight * (float)x[e + 4]);
                 }
-                __syncthreads();  // (the area: the blocks, the items before)
+                const float sum = over_splits<false>(weight);
                 if (lane < 4) {
-                    s.sums[wave][lane * 2] = lo;
-                    s.sums[wave][lane * 2 + 1] = hi;
+                    s_sums[parity][wave][lane * 2] = lo;
+                    s_sums[parity][wave][lane * 2 + 1] = hi;
+                    if (lane == 0) s_sums_ml[parity][wave] = make_float2(top, sum);
                 }
                 __syncthreads();
-                const int t_slot = tid >> 3, quad = tid & 7;
-                if (t_slot < at_once && i0 + t_slot < items) {
-                    f32x4 o = s.sums[t_slot * item_waves][quad];
-                    for (int v = 1; v < item_waves; ++v) o += s.sums[t_slot * item_waves + v][quad];
+                if (s_late[parity]) return false;
+                if (wave == 0) {
+                    // lane (v, quad): four dims of what wave v has summed up; the waves of an item lie 8, 16 and 32 lanes apart
+                    const int v = lane >> 3, quad = lane & 7;
+                    const float2 v_ml = s_sums_ml[parity][v];
+                    f32x4 acc = s_sums[parity][v][quad];
+                    float all = v_ml.x;
+                    if (item_waves >= 2) all = fmaxf(all, lanes_8(all));
+                    if (item_waves >= 4) all = with_lanes_16<true>(all);
+                    if (item_waves >= 8) all = with_lanes_32<true>(all);
+                    const float scale = __builtin_amdgcn_exp2f(v_ml.x - (all == -INFINITY ? 0.f : all));
+                    float den = v_ml.y * scale;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[e] *= scale;
+                    if (item_waves >= 2) {
+                        den += lanes_8(den);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[e] += lanes_8(acc[e]);
+                    }
+                    if (item_waves >= 4) {
+                        den = with_lanes_16<false>(den);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[e] = with_lanes_16<false>(acc[e]);
+                    }
+                    if (item_waves >= 8) {
+                        den = with_lanes_32<false>(den);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[e] = with_lanes_32<false>(acc[e]);
+                    }
+                    const float inv = (den == 0.f || den != den) ? 1.f : 1.f / den;
                     X4 y;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = (E)o[e];
-                    const int R = mt * kDirectRows + ((i0 + t_slot) >> 2);
-                    *reinterpret_cast<X4*>(p.out + ((size_t)node_of(R) * p.Hq + head_of(R)) * kHeadDim + ((i0 + t_slot) & 3) * 32 + quad * 4) = y;
+                    for (int e = 0; e < 4; ++e) y[e] = (E)(acc[e] * inv);
+                    const int t_item = i0 + (v >> item_shift);
+                    if (t_item < items && (v & (item_waves - 1)) == 0)
+                        *reinterpret_cast<X4*>(p.out + row_at(mt * kDirectRows + (t_item >> 2)) + (t_item & 3) * 32 + quad * 4) = y;
                 }
+                parity ^= 1;  // (the other one was read ahead of the barrier)
             }
+            return true;
         };
-        if (s_arrival.go) merge_share(split);
-        if (s_arrival.last) {
+        // Everyone has arrived: the words are on their way, and are waited for (the limit has the launch end whatever happens).
+        auto merge_what_comes = [&](int share) {
+            if (!merge_share(share, 100000000u) && tid == 0) __hip_atomic_fetch_add(&g_attn_report.lost, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        // The arrival stands for nothing but this workgroup's having looked at the generations and sent its words off.
+        // (its answer is looked at behind the merge: in front of it would be a round trip)
+        __shared__ uint32_t s_before;
+        uint32_t before = 0;
+        if (tid == 0) before = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool merged = split >= p.merge_shares || merge_share(split, p.merge_wait_ticks);
+        if (tid == 0) s_before = before;
+        __syncthreads();
+        const UnitWord word(ctr, p.num_splits, s_before);
+        if (word.last()) {
+            // (every workgroup of the unit has read the generations)
+            if (wave == 0) {
+                uint32_t* gen = p.slots->generation + unit * p.num_splits;
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    if (lane + 64 * k < p.num_splits) __hip_atomic_store(gen + lane + 64 * k, fresh[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (tid == 0) word.next_generation();
+        }
+        if (!merged) {
+            if (tid == 0) {
+                s_arrival.go = word.last() || word.abandon(split);
+                s_late[0] = s_late[1] = 0;
+            }
+            __syncthreads();
+            if (s_arrival.go) merge_what_comes(split);
+        }
+        if (word.last()) {
             if (tid < kDirectItems / 32) s_abandoned[tid] = collect_abandoned(ctr, tid);
             __syncthreads();
             for (int v = 0; v < kDirectItems / 32; ++v)
-                for (uint32_t left = s_abandoned[v]; left != 0; left &= left - 1) merge_share(v * 32 + __builtin_ctz(left));
+                for (uint32_t left = s_abandoned[v]; left != 0; left &= left - 1) merge_what_comes(v * 32 + __builtin_ctz(left));
         }
         return;
     }
+    // Merged by the last arrival.  Partials, written through to memory:
+    //   o_part [unit][split][16 rows][128],  ml_part [unit][split][16 rows] x (max * scale_log2, sum)
+    char* const o_part = reinterpret_cast<char*>(p.o_part) + (size_t)unit * p.num_splits * kPartBytes;
+    char* const ml_part = reinterpret_cast<char*>(p.ml_part) + (size_t)unit * p.num_splits * (kDirectRows * 8);
+    store_dev64(o_part + split * kPartBytes + (c * kHeadDim + my_dim) * 2, bits_as<uint64_t>(result));
+    if (wave == 0 && h == 0)
+        store_dev64(ml_part + (split * kDirectRows + c) * 8, (uint64_t)__float_as_uint(M) | ((uint64_t)__float_as_uint(L) << 32));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) s_arrival = arrive_at_unit(p, ctr, -1);
+    __syncthreads();
+    const auto o_rsrc = __builtin_amdgcn_make_buffer_rsrc(o_part, 0, p.num_splits * kPartBytes, 0x00027000);
     if (!s_arrival.last) return;
 
     // The merge: a thread has four dims of a row; the weights of a row's splits are worked out once, by 32 threads.
@@ -572,9 +673,11 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     X4 x;
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = (E)acc[e];
-    if (R <= last_row) *reinterpret_cast<X4*>(p.out + ((size_t)node_of(R) * p.Hq + head_of(R)) * kHeadDim + (tid & 31) * 4) = x;
+    if (R <= last_row) *reinterpret_cast<X4*>(p.out + row_at(R) + (tid & 31) * 4) = x;
 }
 
 // (two workgroups per CU)
-__global__ __launch_bounds__(kThreads, 4) void tree_attn_direct_kernel(AttnParams p) { tree_attn_direct_body<f16>(p); }
-__global__ __launch_bounds__(kThreads, 4) void tree_attn_direct_bf16_kernel(AttnParams p) { tree_attn_direct_body<bf16>(p); }
+__global__ __launch_bounds__(kThreads, 4) void tree_attn_direct_kernel(AttnParams p) { tree_attn_direct_body<false, f16>(p); }
+__global__ __launch_bounds__(kThreads, 4) void tree_attn_direct_bf16_kernel(AttnParams p) { tree_attn_direct_body<false, bf16>(p); }
+__global__ __launch_bounds__(kThreads, 4) void tree_attn_direct_shares_kernel(AttnParams p) { tree_attn_direct_body<true, f16>(p); }
+__global__ __launch_bounds__(kThreads, 4) void tree_attn_direct_shares_bf16_kernel(AttnParams p) { tree_attn_direct_body<true, bf16>(p); }

@@ -26,7 +26,7 @@ Options& options();
 // attention_report_enqueue copies both words to pinned host memory in stream order (ahead of a synchronisation, never
 // under a capture); attention_report_take reads that copy afterwards and clears what it found.
 int attention_report_enqueue(hipStream_t st);
-int attention_report_take(int* bad_length, unsigned int* abandoned);
+int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int* lost);
 void attention_merge_reenable();
 // Assigns the counters of the in-launch merge to a workspace on the current device (otherwise done by the first
 // launch that uses it outside a stream capture); they stay with it until it is released.

@@ -177,8 +177,8 @@ int synchronize_and_check(hipStream_t st) {
     if (rc) return rc;
     CPMCU_HIP(hipStreamSynchronize(st));
     int bad = 0;
-    unsigned int abandoned = 0;
-    rc = attention_report_take(&bad, &abandoned);
+    unsigned int abandoned = 0, lost = 0;
+    rc = attention_report_take(&bad, &abandoned, &lost);
     if (rc) return rc;
     g_abandoned_waits += abandoned;
     unsigned int fr_timeouts = 0, fr_slow = 0, fr_fused = 0;
@@ -190,6 +190,10 @@ int synchronize_and_check(hipStream_t st) {
     if (fr_timeouts != 0) {
         set_error("%u row(s) of a one-launch FR-Spec head were not finished: the workgroups of the launch were not all resident within "
                   "the wait (frspec_wait_us); those rows hold index -1, and the head runs as two launches from now on", fr_timeouts);
+        return CPMCU_ERR_RUNTIME;
+    }
+    if (lost != 0) {
+        set_error("%u partial result(s) of a tree-attention launch did not reach the workgroup that merges them; its output is not valid", lost);
         return CPMCU_ERR_RUNTIME;
     }
     if (bad != 0) {

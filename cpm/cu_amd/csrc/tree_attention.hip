@@ -83,6 +83,7 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 struct AttnReport {
     int bad_length;
     unsigned int abandoned;
+    unsigned int lost;  // words of a partial that never came (direct shape; a second after the last arrival): nothing makes this happen
 };
 __device__ AttnReport g_attn_report;
 
@@ -92,6 +93,23 @@ __device__ AttnReport g_attn_report;
 // 11 M-tile; 12 / 13 second / third iteration entered, 14 / 15 last patch of landed tiles (appended rows, end of the
 // stream) begun / done.
 CPMCU_TIMELINE_STORAGE(g_attn_timeline)
+
+// Quotient and remainder without a branch: a division, and a branch around it for powers of two, are 200 bytes of instructions each on the
+// way to the first request, in a launch that finds its instructions in no cache.
+struct Quotient {
+    int q, r;
+};
+__host__ __device__ inline uint32_t inverse_of(int d) { return 0xffffffffu / (uint32_t)d; }
+// x / d and x % d for 0 <= x < 2^31 - 1: (x + 1) / d less than one too small, so its floor is the quotient or one less
+__device__ inline Quotient divide(int x, int d, uint32_t inv) {
+    Quotient a;
+    a.q = (int)__umulhi((uint32_t)x + 1u, inv);
+    a.r = x - a.q * d;
+    const bool more = a.r >= d;
+    a.q += more ? 1 : 0;
+    a.r -= more ? d : 0;
+    return a;
+}
 
 struct AttnParams {
     const f16* q;
@@ -108,7 +126,7 @@ struct AttnParams {
     int mask_words;
     int mask_k_range;  // trailing key columns the mask bits refer to (>= T; = T for the verify tree)
     int T, Hq, Hkv, group;
-    int group_shift, hkv_shift;  // log2 of group / Hkv when they are powers of two (the usual case), else -1: plain division
+    uint32_t group_inv, hkv_inv;  // inverse_of(group), inverse_of(Hkv)
     int num_splits, num_mtiles, rows_pad;
     int append_rows;  // direct shape: leading grid rows whose workgroups write the appended rows to the pool, two runs each
     int ntiles_max;  // tiles the split partition spans: ceil(max_kv_len / 64), fixed by the host-side bound
@@ -130,6 +148,7 @@ struct AttnParams {
     // unit, arrivals in its low 16 bits, a generation count above them.  Between launches arrivals is 0; the last
     // workgroup of a unit to arrive turns the full count into the next generation.
     uint32_t* merge_ctr;
+    struct DirectSlots* slots;   // direct shape, merged in shares: where the partials change hands
     int merge_shares;            // direct shape: workgroups of a unit that merge a share each (0: the last arrival merges everything)
     uint32_t merge_wait_ticks;  // longest wait for the other workgroups of a unit, in ticks of the 100 MHz wall clock
 };
@@ -162,36 +181,51 @@ struct Arrival {
     int go;    // the partials of all splits are there, and this workgroup merges its share
     int last;  // nobody arrives behind this one: it also merges what was abandoned
 };
+// A unit's word as an arrival found it: the generation of this launch above, the arrivals before it below.
+struct UnitWord {
+    uint32_t* ctr;
+    uint32_t before, full;
+    __device__ inline UnitWord(uint32_t* c, int num_splits)
+        : ctr(c), before(__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)), full((before & 0xffff0000u) + (uint32_t)num_splits) {}
+    __device__ inline UnitWord(uint32_t* c, int num_splits, uint32_t b) : ctr(c), before(b), full((b & 0xffff0000u) + (uint32_t)num_splits) {}
+    __device__ inline bool last() const { return before + 1u == full; }
+    // last to arrive: full count -> next generation, no arrivals (nobody needs the result of this one)
+    __device__ inline void next_generation() const {
+        __hip_atomic_fetch_add(ctr, 0x10000u - (full & 0xffffu), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // either the full count or, once the last one has moved it on, the next generation
+    __device__ inline bool complete(uint32_t now) const { return now == full || (now & 0xffff0000u) != (before & 0xffff0000u); }
+    // Marks a share as abandoned.  True: everyone has arrived after all, and the workgroup merges its share itself.
+    __device__ inline bool abandon(int share) const {
+        // One bit per share; zero between launches (a mark that was made just behind the last arrival's collection is taken back
+        // by its maker).
+        uint32_t* const mark = ctr + 1 + (share >> 5);
+        const uint32_t bit = 1u << (share & 31);
+        // The mark is in memory before this workgroup looks once more: if the others have all arrived by
+        // then, the last of them may have read the marks already, and this workgroup merges its share
+        // itself (twice the same values at worst); if not, the last one will find the mark.
+        // (acquire-release on the mark, acquire on the look that follows: the two stay in this order)
+        (void)__hip_atomic_fetch_or(mark, bit, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        const bool go = complete(__hip_atomic_load(ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT));
+        // everyone is there after all: this workgroup merges its share itself and takes its mark back, so that
+        // no mark outlives the launch (if the last arrival has collected it already, the share is merged twice
+        // with the same values)
+        if (go) (void)__hip_atomic_fetch_and(mark, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(&g_attn_report.abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return go;
+    }
+};
 __device__ inline Arrival arrive_at_unit(const AttnParams& p, uint32_t* unit_ctr, int share) {
     Arrival a = {share >= 0 ? 1 : 0, 0};
-    // One bit per share; zero between launches (a mark that was made just behind the last arrival's collection is taken back
-    // by its maker).
-    uint32_t* const mark = unit_ctr + 1 + (max(share, 0) >> 5);
-    const uint32_t bit = 1u << (share & 31);
-    // The word as this workgroup's arrival found it: the generation of this launch above, the arrivals before it below.
-    const uint32_t before = __hip_atomic_fetch_add(unit_ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t full = (before & 0xffff0000u) + (uint32_t)p.num_splits;
-    // either the full count or, once the last one has moved it on, the next generation
-    auto complete = [&](uint32_t now) { return now == full || (now & 0xffff0000u) != (before & 0xffff0000u); };
-    if (before + 1u == full) {
-        // last to arrive: full count -> next generation, no arrivals (nobody needs the result of this one)
-        __hip_atomic_fetch_add(unit_ctr, 0x10000u - (uint32_t)p.num_splits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const UnitWord word(unit_ctr, p.num_splits);
+    if (word.last()) {
+        word.next_generation();
         a.last = 1;
     } else if (share >= 0) {
         const unsigned long long t_begin = wall_clock64();
-        while (!complete(__hip_atomic_load(unit_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+        while (!word.complete(__hip_atomic_load(unit_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
             if (wall_clock64() - t_begin >= p.merge_wait_ticks) {
-                // The mark is in memory before this workgroup looks once more: if the others have all arrived by
-                // then, the last of them may have read the marks already, and this workgroup merges its share
-                // itself (twice the same values at worst); if not, the last one will find the mark.
-                // (acquire-release on the mark, acquire on the look that follows: the two stay in this order)
-                (void)__hip_atomic_fetch_or(mark, bit, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-                a.go = complete(__hip_atomic_load(unit_ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)) ? 1 : 0;
-                // everyone is there after all: this workgroup merges its share itself and takes its mark back, so that
-                // no mark outlives the launch (if the last arrival has collected it already, the share is merged twice
-                // with the same values)
-                if (a.go) (void)__hip_atomic_fetch_and(mark, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_fetch_add(&g_attn_report.abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                a.go = word.abandon(share) ? 1 : 0;
                 break;
             }
             __builtin_amdgcn_s_sleep(4);
@@ -217,8 +251,8 @@ __device__ inline void combine_block(const AttnParams& p, int g, int rb, int qua
     const int qcol = lane & 31, hf = lane >> 5;
     const int R = rb * kRowsPerWave + qcol;
     if (R >= p.group * p.T) return;
-    const int node = p.group_shift >= 0 ? R >> p.group_shift : R / p.group;
-    const int head = g * p.group + (p.group_shift >= 0 ? R & (p.group - 1) : R % p.group);
+    const Quotient row = divide(R, p.group, p.group_inv);
+    const int node = row.q, head = g * p.group + row.r;
     const int d0 = (quad >> 2) * 32 + (quad & 3) * 8 + hf * 4;
     const float2* ml = reinterpret_cast<const float2*>(p.ml_part) + (size_t)g * p.num_splits * p.rows_pad + R;
     const X4* op = reinterpret_cast<const X4*>(p.o_part) +
@@ -294,8 +328,9 @@ __device__ inline CombineWhere<E> combine_where(const AttnParams& p, int g, int 
     const int qcol = lane & 31, hf = lane >> 5;
     const int R = rb * kRowsPerWave + qcol;
     w.valid = R < p.group * p.T;
-    w.node = p.group_shift >= 0 ? R >> p.group_shift : R / p.group;
-    w.head = g * p.group + (p.group_shift >= 0 ? R & (p.group - 1) : R % p.group);
+    const Quotient row = divide(R, p.group, p.group_inv);
+    w.node = row.q;
+    w.head = g * p.group + row.r;
     w.d0 = (quad >> 2) * 32 + (quad & 3) * 8 + hf * 4;
     w.ml = reinterpret_cast<const float2*>(p.ml_part) + (size_t)g * p.num_splits * p.rows_pad + R;
     w.op = reinterpret_cast<const X4*>(p.o_part) + (((size_t)g * p.num_splits) * nrb + rb) * 16 * 64 + quad * 64 + lane;
@@ -494,8 +529,8 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     // All launch arguments are fetched in one go, up front: left alone, the compiler fetches them in three batches as
     // the code first needs them, and each batch is a memory round trip of its own in front of the first K/V request.
     asm volatile("" ::"s"(p.q), "s"(p.k_pool), "s"(p.v_pool), "s"(p.block_table), "s"(p.kv_len), "s"(p.k_new), "s"(p.v_new), "s"(p.rope),
-                 "s"(p.mask), "s"(p.mask_words), "s"(p.mask_k_range), "s"(p.T), "s"(p.Hq), "s"(p.Hkv), "s"(p.group), "s"(p.group_shift),
-                 "s"(p.hkv_shift), "s"(p.num_splits), "s"(p.num_mtiles), "s"(p.ntiles_max), "s"(p.table_pages), "s"(p.window_blocks),
+                 "s"(p.mask), "s"(p.mask_words), "s"(p.mask_k_range), "s"(p.T), "s"(p.Hq), "s"(p.Hkv), "s"(p.group), "s"(p.group_inv),
+                 "s"(p.hkv_inv), "s"(p.num_splits), "s"(p.num_mtiles), "s"(p.ntiles_max), "s"(p.table_pages), "s"(p.window_blocks),
                  "s"(p.max_kv_len));
     CPMCU_CLOCK_VAR(tl_start);
     CPMCU_CLOCK_VAR(tl_loop);
@@ -512,8 +547,8 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     const int sh = blockIdx.x;
     const int mt = blockIdx.y;
     if (sh >= p.num_splits * p.Hkv) return;
-    const int g = p.hkv_shift >= 0 ? sh & (p.Hkv - 1) : sh % p.Hkv;
-    const int split = p.hkv_shift >= 0 ? sh >> p.hkv_shift : sh / p.Hkv;
+    const Quotient sh_of = divide(sh, p.Hkv, p.hkv_inv);
+    const int g = sh_of.r, split = sh_of.q;
 
     // The value as it is known here: keeps what is worked out from it in paths that few tiles take from being worked out ahead of
     // the loop, where it would hold registers that the loop needs.
@@ -536,8 +571,8 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     // 60-node tree) has nothing to compute: it still requests its share of every tile and meets every barrier, but
     // skips the tile arithmetic -- 6 % of the launch's matrix and vector work at that tree size.
     const bool wave_has_rows = __builtin_amdgcn_readfirstlane(mt * kRowsPerWg + rw * kRowsPerWave) < p.group * p.T;
-    const int node = !row_ok ? 0 : p.group_shift >= 0 ? R >> p.group_shift : R / p.group;
-    const int head = g * p.group + (!row_ok ? 0 : p.group_shift >= 0 ? R & (p.group - 1) : R % p.group);
+    const Quotient row = divide(row_ok ? R : 0, p.group, p.group_inv);
+    const int node = row.q, head = g * p.group + row.r;
 
     // Loads that do not depend on the KV length go first.
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
@@ -562,8 +597,8 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
             const int inst = x * kWaves + wave_u;  // 1 KB of the staging area: rows 4 * inst .. + 3
             const int r = inst * 4 + (lane >> 4);
             const int Rr = min(mt * kRowsPerWg + r, last_row);  // rows past the end re-read the last one (zeroed below)
-            const int nr = p.group_shift >= 0 ? Rr >> p.group_shift : Rr / p.group;
-            const int hr = g * p.group + (p.group_shift >= 0 ? Rr & (p.group - 1) : Rr % p.group);
+            const Quotient row = divide(Rr, p.group, p.group_inv);
+            const int nr = row.q, hr = g * p.group + row.r;
             const int piece = (lane & 15) ^ (r & 15);  // the K tile's swizzle: the reads below are conflict-free
             load_to_lds16_v(p.q + ((size_t)nr * p.Hq + hr) * kHeadDim + piece * 8, qstage + inst * 1024);
         }
@@ -1363,6 +1398,7 @@ struct LaunchPlan {
 constexpr int kMergeUnits = 256;    // (KV head, M-tile) units a launch may have on this path
 constexpr int kMergeBlocks = 32;    // workspaces with a block per device
 __device__ __align__(256) uint32_t g_merge_ctr[kMergeBlocks][kMergeUnits * kMergeUnitWords];
+__device__ DirectSlots g_direct_slots[kMergeBlocks];  // of the same workspaces
 
 // The split workgroups can merge in the launch when they are all resident at once (one per CU: a workgroup that
 // waits for the others must not keep them from starting) and few enough per counter.
@@ -1381,11 +1417,13 @@ std::map<std::pair<int, const void*>, MergeState> g_merge_states;
 std::vector<int> g_merge_free_blocks[64];
 bool g_merge_blocks_listed[64] = {false};
 uint32_t* g_merge_ctr_base[64] = {nullptr};
+DirectSlots* g_direct_slots_base[64] = {nullptr};
 
 // The counter block of a workspace on the current device.  words null: the launch has to be merged by the combine launch.  may_wait
 // false: so does one whose workgroups would wait for each other; the direct shape's last arrival, which waits for nobody, still merges.
 struct MergeCounters {
     uint32_t* words = nullptr;
+    DirectSlots* slots = nullptr;
     bool may_wait = false;
 };
 MergeCounters merge_counters_for(const void* workspace, hipStream_t st) {
@@ -1401,11 +1439,12 @@ MergeCounters merge_counters_for(const void* workspace, hipStream_t st) {
                 (void)hipGetLastError();
                 return {};
             }
-            void* ptr = nullptr;
-            if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_merge_ctr)) != hipSuccess) {
+            void *ptr = nullptr, *slots = nullptr;
+            if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_merge_ctr)) != hipSuccess || hipGetSymbolAddress(&slots, HIP_SYMBOL(g_direct_slots)) != hipSuccess) {
                 (void)hipGetLastError();
                 return {};
             }
+            g_direct_slots_base[dev] = (DirectSlots*)slots;
             g_merge_ctr_base[dev] = (uint32_t*)ptr;
         }
         if (!g_merge_blocks_listed[dev]) {
@@ -1418,14 +1457,15 @@ MergeCounters merge_counters_for(const void* workspace, hipStream_t st) {
         g_merge_free_blocks[dev].pop_back();
         it = g_merge_states.emplace(std::make_pair(dev, workspace), ns).first;
     }
-    return {g_merge_ctr_base[dev] + (size_t)it->second.block * kMergeUnits * kMergeUnitWords, !it->second.no_waits};
+    return {g_merge_ctr_base[dev] + (size_t)it->second.block * kMergeUnits * kMergeUnitWords, g_direct_slots_base[dev] + it->second.block, !it->second.no_waits};
 }
 // The direct shape's merge.  Up to kDirectLastMerges splits the last arrival reads one round trip's worth of partials and nobody waits;
-// from there on sharing is the faster form (one query, last arrival / shares, us per layer: 7.07 / 7.86 on 8 splits, 7.25 / 7.47 on 12, 7.63 /
-// 7.45 on 16, 8.30 / 7.56 on 24, 9.06 / 7.90 on 33, 22.99 / 20.41 on 64, 25.42 / 19.01 on 128), if there is a CU for each
+// from there on sharing is the faster form (one query, last arrival / shares by counted arrivals, us per layer: 7.07 / 7.86 on 8 splits, 7.25 / 7.47 on 12, 7.63 /
+// 7.45 on 16, 8.30 / 7.56 on 24, 9.06 / 7.90 on 33, 22.99 / 20.41 on 64, 25.42 / 19.01 on 128; by words, last arrival / shares: 6.3 / 6.45 on 10, 10 row tiles on
+// 10 splits 6.6 / 7.3, 16 on 5 7.4 / 9.5: every wave polls), if there is a CU for each
 // workgroup: those with a share wait for all others, so all have to be resident (two to a CU are not, always).
 int direct_merge_shares(int num_splits, int workgroups, int cus) {
-    return num_splits > kDirectLastMerges && workgroups <= cus ? std::min(num_splits, kDirectItems) : 0;
+    return num_splits > kDirectLastMerges && workgroups <= std::min(cus, kDirectSlots) ? std::min(num_splits, kDirectItems) : 0;
 }
 
 // The direct shape or one of the split shapes, and the splits of the direct one: from estimates of both, in us, fitted to a sweep
@@ -1548,20 +1588,20 @@ int attention_report_enqueue(hipStream_t st) {
     CPMCU_CHECK_ARG(dev >= 0 && dev < 64, "device index %d outside [0, 64)", dev);
     if (g_report_host[dev] == nullptr) {
         CPMCU_HIP(hipHostMalloc((void**)&g_report_host[dev], sizeof(AttnReport), hipHostMallocDefault));
-        *g_report_host[dev] = AttnReport{0, 0u};
+        *g_report_host[dev] = AttnReport{0, 0u, 0u};
     }
     CPMCU_HIP(hipMemcpyFromSymbolAsync(g_report_host[dev], HIP_SYMBOL(g_attn_report), sizeof(AttnReport), 0, hipMemcpyDeviceToHost, st));
     return CPMCU_OK;
 }
-int attention_report_take(int* bad_length, unsigned int* abandoned) {
+int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int* lost) {
     int dev = 0;
     CPMCU_HIP(hipGetDevice(&dev));
     *bad_length = 0;
-    *abandoned = 0;
+    *abandoned = *lost = 0;
     if (dev < 0 || dev >= 64 || g_report_host[dev] == nullptr) return CPMCU_OK;
     const AttnReport r = *g_report_host[dev];
-    if (r.bad_length != 0 || r.abandoned != 0) {
-        const AttnReport zero{0, 0u};
+    if (r.bad_length != 0 || r.abandoned != 0 || r.lost != 0) {
+        const AttnReport zero{0, 0u, 0u};
         CPMCU_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_attn_report), &zero, sizeof(zero)));
         *g_report_host[dev] = zero;
         if (r.abandoned != 0) {
@@ -1572,6 +1612,7 @@ int attention_report_take(int* bad_length, unsigned int* abandoned) {
     }
     *bad_length = r.bad_length;
     *abandoned = r.abandoned;
+    *lost = r.lost;
     return CPMCU_OK;
 }
 // Lets the launches on the workspaces of the current device wait again (cpmcu_set_option attn_merge_in_launch = 1).
@@ -1658,13 +1699,8 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     p.Hq = Hq;
     p.Hkv = Hkv;
     p.group = group;
-    auto log2_or_minus1 = [](int v) {
-        int sft = 0;
-        while ((1 << sft) < v) ++sft;
-        return (1 << sft) == v ? sft : -1;
-    };
-    p.group_shift = log2_or_minus1(group);
-    p.hkv_shift = log2_or_minus1(Hkv);
+    p.group_inv = inverse_of(group);
+    p.hkv_inv = inverse_of(Hkv);
     p.window_blocks = block_window_size / 128;
     hipStream_t st = resolve_stream(stream);
     DirectMerge direct_merge = usual_direct_merge();
@@ -1676,6 +1712,7 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
         plan = plan_launch(T, group, Hkv, max_kv_len, block_window_size, num_splits_override, rope_cos_sin != nullptr, direct_merge);
     }
     p.merge_ctr = plan.direct || counters.may_wait ? counters.words : nullptr;
+    p.slots = counters.slots;
     const int span = plan.span;
     const int G = plan.kv_groups;
     p.num_mtiles = plan.num_mtiles;
@@ -1704,11 +1741,16 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     const dim3 grid(kXcds * ceil_div(nsh, kXcds), p.num_mtiles);
     const bool is_bf16 = options().dtype == 1;
     if (plan.direct) {
+        if (p.num_splits > kDirectLastMerges && counters.slots != nullptr && (int)(grid.x * grid.y) <= kDirectSlots) {
+            p.o_part = (float*)p.slots->o;  // (addresses in device memory)
+            p.ml_part = (float*)p.slots->ml;
+        }
         p.merge_shares = direct_merge == DirectMerge::kMayWait ? direct_merge_shares(p.num_splits, (int)(grid.x * grid.y), device_cu_count()) : 0;
         p.append_rows = k_new ? ceil_div(ceil_div(T, kAppendRows) * Hkv, (int)grid.x * (kThreads / kAppendThreads)) : 0;
         const dim3 dgrid(grid.x, p.num_mtiles + p.append_rows);
-        if (is_bf16) hipLaunchKernelGGL(tree_attn_direct_bf16_kernel, dgrid, dim3(kThreads), 0, st, p);
-        else hipLaunchKernelGGL(tree_attn_direct_kernel, dgrid, dim3(kThreads), 0, st, p);
+        const auto kernel = p.merge_shares > 0 ? (is_bf16 ? tree_attn_direct_shares_bf16_kernel : tree_attn_direct_shares_kernel)
+                                               : (is_bf16 ? tree_attn_direct_bf16_kernel : tree_attn_direct_kernel);
+        hipLaunchKernelGGL(kernel, dgrid, dim3(kThreads), 0, st, p);
         CPMCU_LAUNCH_CHECK();
         return CPMCU_OK;
     }

@@ -221,3 +221,44 @@ def test_direct_launches_after_an_abandoned_wait(gpu, option, hkv, T, splits, ze
         ops._workspaces.pop(key)
         if saved is not None:
             ops._workspaces[key] = saved
+
+
+def test_words_of_launches_of_changing_shapes(gpu, option):
+    """Launches that merge in shares pass their partials on in the same slots, other splits and units in them each time (the edges of
+    one to eight waves an item, shares of several turns, 256 workgroups): no launch takes an older one's words for its own.  Reference: the same
+    launch merged by its last arrival, two orders of the same fp32 sums, rounded to fp16 once."""
+    from cpm.cu_amd import ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch = gpu
+    option("attn_direct", 1)
+    option("attn_merge_in_launch", 1)
+    shapes = [(1, 2, 34), (4, 2, 17), (1, 8, 32), (2, 4, 16), (1, 1, 128), (7, 4, 18), (1, 2, 64), (1, 2, 65), (3, 2, 33), (1, 2, 16)]
+    S, g = 9000, torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).half()
+    kv_len, caches, calls = torch.tensor([S], dtype=torch.int32, device="cuda"), {}, []
+    for hkv in (1, 2, 4, 8):
+        caches[hkv] = PagedKVCache(1, hkv, (S + 255) // 256)
+        caches[hkv].write_logical(0, 0, rnd(S, hkv, D), rnd(S, hkv, D))
+    for turn in range(3):
+        for T, hkv, splits in shapes[turn:] + shapes[:turn]:
+            q = rnd(T, 32, D)
+            calls.append((lambda q=q, hkv=hkv, splits=splits: ops.tree_attention(q, caches[hkv], 0, kv_len, S, num_splits=splits), (T, hkv, splits)))
+            assert ops.attention_plan(T, 32, hkv, S, num_splits=splits)[0] == "tree_attn_direct_kernel"
+    outs = [call() for call, _ in calls]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        replayed = [call() for call, _ in calls]
+    for _ in range(3):
+        for r in replayed:
+            r.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        for r, o, (_, shape) in zip(replayed, outs, calls):
+            assert torch.equal(r.view(torch.int16), o.view(torch.int16)), shape
+    option("attn_merge_wait_us", 0)
+    try:
+        for o, (call, shape) in zip(outs, calls):
+            ref = call()
+            assert float((o.float() - ref.float()).abs().max()) <= 2.0 ** -10 * float(ref.float().abs().max()), shape
+    finally:
+        option("attn_merge_wait_us", 2000)
