@@ -35,7 +35,6 @@ constexpr int kDirectLastMerges = 15;          // up to here the last arrival me
 constexpr int kDirectSlots = 256;                           // workgroups of such a launch
 constexpr int kSlotQuads = kDirectRows * 32 + kDirectRows;  // of 16 bytes: four dims of a row, then a row's maximum and sum
 constexpr int kSlotBytes = kSlotQuads * 16;
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 struct DirectSlots {
     uint32_t generation[kDirectSlots];
     u32x4 words[kDirectSlots][kSlotQuads];
@@ -574,7 +573,7 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         const bool merged = split >= p.merge_shares || merge_share(split, p.merge_wait_ticks);
         if (tid == 0) s_before = before;
         __syncthreads();
-        const UnitWord word(ctr, p.num_splits, s_before);
+        const UnitWord<false> word(ctr, p.num_splits, s_before);
         if (word.last()) {
             // (every workgroup of the unit has read the generations)
             if (wave == 0) {
@@ -594,7 +593,7 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
             if (s_arrival.go) merge_what_comes(split);
         }
         if (word.last()) {
-            if (tid < kDirectItems / 32) s_abandoned[tid] = collect_abandoned(ctr, tid);
+            if (tid < kDirectItems / 32) s_abandoned[tid] = word.collect_abandoned(tid);
             __syncthreads();
             for (int v = 0; v < kDirectItems / 32; ++v)
                 for (uint32_t left = s_abandoned[v]; left != 0; left &= left - 1) merge_what_comes(v * 32 + __builtin_ctz(left));
@@ -610,7 +609,7 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         store_dev64(ml_part + (split * kDirectRows + c) * 8, (uint64_t)__float_as_uint(M) | ((uint64_t)__float_as_uint(L) << 32));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0) s_arrival = arrive_at_unit(p, ctr, -1);
+    if (tid == 0) s_arrival = arrive_at_unit<false>(p, ctr, p.num_splits, -1);
     __syncthreads();
     const auto o_rsrc = __builtin_amdgcn_make_buffer_rsrc(o_part, 0, p.num_splits * kPartBytes, 0x00027000);
     if (!s_arrival.last) return;

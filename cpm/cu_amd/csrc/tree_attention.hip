@@ -35,7 +35,8 @@
 //  * The Q rows and the tree mask reach the registers through LDS (whole rows,
 //    coalesced), not through per-lane fetches in the MFMA operand layout.
 //  * Workgroups are mapped so that all M-tiles that stream the same KV range
-//    land on the same XCD (workgroup id modulo 8) and share its L2.
+//    land on the same XCD (workgroup id modulo 8) and share its L2; at short
+//    contexts all splits of an M-tile instead, which merge through that L2.
 #include "common.h"
 #include "internal.h"
 #include "kv_append.h"
@@ -74,6 +75,7 @@ constexpr int kXcds = 8;
 constexpr float kLazyLog2 = 8.f;  // slack of the lazily updated softmax reference, in log2 units
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Set by a launch whose device-side length does not fit what the host promised (above max_kv_len, or shorter
 // than the query rows / the masked range): the launch then works on the length clamped into that range -- every
@@ -83,7 +85,8 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 struct AttnReport {
     int bad_length;
     unsigned int abandoned;
-    unsigned int lost;  // words of a partial that never came (direct shape; a second after the last arrival): nothing makes this happen
+    unsigned int lost;  // partials that never came: words of the direct shape, a second after the last arrival, or a unit merged through the L2 of
+                        // an XCD whose workgroups turned out to be on two
 };
 __device__ AttnReport g_attn_report;
 
@@ -128,6 +131,8 @@ struct AttnParams {
     int T, Hq, Hkv, group;
     uint32_t group_inv, hkv_inv;  // inverse_of(group), inverse_of(Hkv)
     int num_splits, num_mtiles, rows_pad;
+    int xcd_units;                       // all splits of a unit on one XCD: units per XCD
+    uint32_t xcd_units_inv, mtiles_inv;  // inverse_of(xcd_units), inverse_of(num_mtiles)
     int append_rows;  // direct shape: leading grid rows whose workgroups write the appended rows to the pool, two runs each
     int ntiles_max;  // tiles the split partition spans: ceil(max_kv_len / 64), fixed by the host-side bound
                      // (with a window: the most tiles a window can hold, counted from its first tile)
@@ -153,6 +158,8 @@ struct AttnParams {
     uint32_t merge_wait_ticks;  // longest wait for the other workgroups of a unit, in ticks of the 100 MHz wall clock
 };
 
+constexpr int kMergeUnits = 256;    // (KV head, M-tile) units a launch may have on this path
+constexpr int kUnitXccWord = 32;      // of a unit's words: see UnitWord::abandon (another line than the words that an L2 works on)
 constexpr int kMergeUnitWords = 64;  // a unit's word sits in a 256-byte line of its own: every poll and every arrival is
                                      // a memory transaction, and those on one line queue behind each other
 
@@ -180,19 +187,45 @@ __device__ inline To bits_as(const From& v) {
 struct Arrival {
     int go;    // the partials of all splits are there, and this workgroup merges its share
     int last;  // nobody arrives behind this one: it also merges what was abandoned
+    uint32_t before;  // (UnitWord)
 };
+// Atomics on a unit's words.  LOCAL: all workgroups of the unit are on one XCD, and its L2 performs them (0.3 us; the words are
+// back in memory behind the launch).  Assembly, because the compiler turns an addition of zero into a load, which the CU's own cache may answer.
+template <bool LOCAL>
+struct UnitAtomics {
+    __device__ static inline uint32_t add(uint32_t* w, uint32_t v) { return __hip_atomic_fetch_add(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ static inline uint32_t mark(uint32_t* w, uint32_t v) { return __hip_atomic_fetch_or(w, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ static inline uint32_t keep(uint32_t* w, uint32_t v) { return __hip_atomic_fetch_and(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ static inline uint32_t take(uint32_t* w) { return __hip_atomic_exchange(w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ static inline uint32_t look(uint32_t* w) { return __hip_atomic_load(w, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ static inline uint32_t poll(uint32_t* w) { return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+};
+#define CPMCU_L2_ATOMIC(op, w, v)                                                                                                             \
+    uint32_t before;                                                                                                                          \
+    asm volatile("global_atomic_" op " %0, %1, %2, off sc0\n\ts_waitcnt vmcnt(0)" : "=&v"(before) : "v"(w), "v"(v) : "memory"); \
+    return before
+template <>
+struct UnitAtomics<true> {
+    __device__ static inline uint32_t add(uint32_t* w, uint32_t v) { CPMCU_L2_ATOMIC("add", w, v); }
+    __device__ static inline uint32_t mark(uint32_t* w, uint32_t v) { CPMCU_L2_ATOMIC("or", w, v); }
+    __device__ static inline uint32_t keep(uint32_t* w, uint32_t v) { CPMCU_L2_ATOMIC("and", w, v); }
+    __device__ static inline uint32_t take(uint32_t* w) { CPMCU_L2_ATOMIC("swap", w, 0u); }
+    __device__ static inline uint32_t look(uint32_t* w) { return add(w, 0u); }
+    __device__ static inline uint32_t poll(uint32_t* w) { return add(w, 0u); }
+};
+#undef CPMCU_L2_ATOMIC
+
 // A unit's word as an arrival found it: the generation of this launch above, the arrivals before it below.
+template <bool LOCAL>
 struct UnitWord {
+    typedef UnitAtomics<LOCAL> Atomics;
     uint32_t* ctr;
     uint32_t before, full;
-    __device__ inline UnitWord(uint32_t* c, int num_splits)
-        : ctr(c), before(__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)), full((before & 0xffff0000u) + (uint32_t)num_splits) {}
     __device__ inline UnitWord(uint32_t* c, int num_splits, uint32_t b) : ctr(c), before(b), full((b & 0xffff0000u) + (uint32_t)num_splits) {}
+    __device__ inline UnitWord(uint32_t* c, int num_splits) : UnitWord(c, num_splits, Atomics::add(c, 1u)) {}
     __device__ inline bool last() const { return before + 1u == full; }
     // last to arrive: full count -> next generation, no arrivals (nobody needs the result of this one)
-    __device__ inline void next_generation() const {
-        __hip_atomic_fetch_add(ctr, 0x10000u - (full & 0xffffu), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    __device__ inline void next_generation() const { (void)Atomics::add(ctr, 0x10000u - (full & 0xffffu)); }
     // either the full count or, once the last one has moved it on, the next generation
     __device__ inline bool complete(uint32_t now) const { return now == full || (now & 0xffff0000u) != (before & 0xffff0000u); }
     // Marks a share as abandoned.  True: everyone has arrived after all, and the workgroup merges its share itself.
@@ -201,50 +234,78 @@ struct UnitWord {
         // by its maker).
         uint32_t* const mark = ctr + 1 + (share >> 5);
         const uint32_t bit = 1u << (share & 31);
-        // The mark is in memory before this workgroup looks once more: if the others have all arrived by
+        // The mark is made before this workgroup looks once more: if the others have all arrived by
         // then, the last of them may have read the marks already, and this workgroup merges its share
         // itself (twice the same values at worst); if not, the last one will find the mark.
         // (acquire-release on the mark, acquire on the look that follows: the two stay in this order)
-        (void)__hip_atomic_fetch_or(mark, bit, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        const bool go = complete(__hip_atomic_load(ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT));
-        // everyone is there after all: this workgroup merges its share itself and takes its mark back, so that
-        // no mark outlives the launch (if the last arrival has collected it already, the share is merged twice
+        (void)Atomics::mark(mark, bit);
+        uint32_t here = 0, seen = 0;
+        if constexpr (LOCAL) {
+            // A unit whose workgroups are not on one XCD never counts them all, and every wait in it runs out: those from two XCDs meet in
+            // this word, in memory, which is zero between the launches of a unit on one XCD.
+            uint32_t xcc;
+            asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+            here = 1u << (xcc & 31);
+            seen = UnitAtomics<false>::mark(ctr + kUnitXccWord, here) & ~here;
+        }
+        const bool go = complete(Atomics::look(ctr));
+        // everyone is there after all: this workgroup merges its share itself and takes its marks back, so that
+        // none outlives the launch (if the last arrival has collected it already, the share is merged twice
         // with the same values)
-        if (go) (void)__hip_atomic_fetch_and(mark, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (go) {
+            (void)Atomics::keep(mark, ~bit);
+            if (LOCAL) (void)UnitAtomics<false>::keep(ctr + kUnitXccWord, ~here);
+        } else if (seen != 0) {
+            __hip_atomic_fetch_add(&g_attn_report.lost, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         __hip_atomic_fetch_add(&g_attn_report.abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return go;
     }
+    // The last arrival: shares 32 w .. 32 w + 31 that were abandoned.
+    __device__ inline uint32_t collect_abandoned(int w) const {
+        const uint32_t marks = Atomics::take(ctr + 1 + w);
+        if (LOCAL && marks != 0) __hip_atomic_store(ctr + kUnitXccWord, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return marks;
+    }
 };
-__device__ inline Arrival arrive_at_unit(const AttnParams& p, uint32_t* unit_ctr, int share) {
-    Arrival a = {share >= 0 ? 1 : 0, 0};
-    const UnitWord word(unit_ctr, p.num_splits);
+// of: how many arrive at the word
+template <bool LOCAL>
+__device__ inline Arrival arrive_at_unit(const AttnParams& p, uint32_t* unit_ctr, int of, int share) {
+    Arrival a = {share >= 0 ? 1 : 0, 0, 0};
+    const UnitWord<LOCAL> word(unit_ctr, of);
+    a.before = word.before;
     if (word.last()) {
         word.next_generation();
         a.last = 1;
     } else if (share >= 0) {
         const unsigned long long t_begin = wall_clock64();
-        while (!word.complete(__hip_atomic_load(unit_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+        while (!word.complete(UnitAtomics<LOCAL>::poll(unit_ctr))) {
             if (wall_clock64() - t_begin >= p.merge_wait_ticks) {
                 a.go = word.abandon(share) ? 1 : 0;
                 break;
             }
-            __builtin_amdgcn_s_sleep(4);
+            __builtin_amdgcn_s_sleep(LOCAL ? 1 : 4);
         }
     }
     return a;
 }
-// The last arrival: shares 32 w .. 32 w + 31 that were abandoned.
-__device__ inline uint32_t collect_abandoned(uint32_t* unit_ctr, int w) {
-    return __hip_atomic_exchange(unit_ctr + 1 + w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+template <typename E>
+__device__ inline typename Elem<E>::x8 zero8() {
+    typename Elem<E>::x8 z;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) z[i] = (E)0.f;
+    return z;
 }
 
 // Merge of the split partials of one 32-row block and one quad of output dims (one wave; lane = accumulator lane):
 // M = max_s m_s, L = sum_s l_s 2^(m_s - M), O = sum_s l_s 2^(m_s - M) (O_s / l_s) / L -- the log-sum-exp merge of
 // src/flash_attn/src/flash_fwd_kernel.h:2392-2472 in base-2 form.  The statistics and the O partials of up to 16
 // splits are all requested before any is used, so a block pays one memory round trip, not one per split.
-// DEV: the partials were written by other workgroups of this launch (device-scope loads).
+// FROM: who wrote the partials -- an earlier launch, other workgroups of this one (device-scope loads), or workgroups of this one on the same
+// XCD (what its L2 has; the CU's own cache cannot have a line of them yet.  Scalar offsets: 16 pointers would take the registers of the loop).
 constexpr int kCombineBatch = 16;
-template <bool DEV, typename E>
+enum class Partials { kOfALaunch, kOfTheDevice, kOfTheXcd };
+template <Partials FROM, typename E>
 __device__ inline void combine_block(const AttnParams& p, int g, int rb, int quad, int lane) {
     typedef typename Elem<E>::x4 X4;
     const int nrb = p.rows_pad / kRowsPerWave;  // 32-row blocks per kv head
@@ -259,6 +320,11 @@ __device__ inline void combine_block(const AttnParams& p, int g, int rb, int qua
                       (((size_t)g * p.num_splits) * nrb + rb) * 16 * 64 + quad * 64 + lane;
     const size_t ml_stride = (size_t)p.rows_pad;
     const size_t o_stride = (size_t)nrb * 16 * 64;
+    // (of a launch that merges itself: at most 256 workgroups' partials)
+    const int ml_bytes = p.num_splits * p.rows_pad * (int)sizeof(float2), o_bytes = p.num_splits * nrb * 16 * 64 * (int)sizeof(X4);
+    const auto ml_rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(p.ml_part) + (size_t)g * ml_bytes, 0, ml_bytes, 0x00027000);
+    const auto o_rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(p.o_part) + (size_t)g * o_bytes, 0, o_bytes, 0x00027000);
+    const int o_at = ((rb * 16 + quad) * 64 + lane) * (int)sizeof(X4);
 
     float M = -INFINITY, L = 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -268,10 +334,13 @@ __device__ inline void combine_block(const AttnParams& p, int g, int rb, int qua
 #pragma unroll
         for (int u = 0; u < kCombineBatch; ++u) {
             const int s = min(s0 + u, p.num_splits - 1);  // clamp: repeats are ignored below
-            if (DEV) {
+            if constexpr (FROM == Partials::kOfTheDevice) {
                 const uint64_t mlw = load_dev64(&ml[s * ml_stride]);
                 v[u] = make_float2(__uint_as_float((uint32_t)mlw), __uint_as_float((uint32_t)(mlw >> 32)));
                 o[u] = bits_as<X4>(load_dev64(&op[s * o_stride]));
+            } else if constexpr (FROM == Partials::kOfTheXcd) {
+                v[u] = bits_as<float2>(__builtin_amdgcn_raw_buffer_load_b64(ml_rsrc, R * (int)sizeof(float2), s * p.rows_pad * (int)sizeof(float2), 0));
+                o[u] = bits_as<X4>(__builtin_amdgcn_raw_buffer_load_b64(o_rsrc, o_at, s * nrb * 16 * 64 * (int)sizeof(X4), 0));
             } else {
                 v[u] = ml[s * ml_stride];
                 o[u] = op[s * o_stride];
@@ -289,12 +358,17 @@ __device__ inline void combine_block(const AttnParams& p, int g, int rb, int qua
         M = Mb;
 #pragma unroll
         for (int u = 0; u < kCombineBatch; ++u) {
-            // an empty split (l == 0) has no meaningful O partial: select it away, never scale it
-            if (!(s0 + u < p.num_splits && v[u].y > 0.f)) continue;
-            const float w = __builtin_amdgcn_exp2f(v[u].x - M) * v[u].y;  // partials are stored normalised
-            L += w;
+            // an empty split (l == 0) has no meaningful O partial: select it away, never scale it (a branch for each of 16 splits
+            // would cost more than its arithmetic)
+            const bool in = s0 + u < p.num_splits && v[u].y > 0.f;
+            const float l = in ? v[u].y : 0.f;
+            const uint64_t bits = in ? bits_as<uint64_t>(o[u]) : 0;
+            const X4 x = bits_as<X4>(bits);
+            // partials are stored normalised (the fused products are written out: who merges must not change a bit)
+            const float f = __builtin_amdgcn_exp2f(in ? v[u].x - M : -INFINITY), w = f * l;
+            L = __builtin_fmaf(f, l, L);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] += w * (float)o[u][e];
+            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(w, (float)x[e], acc[e]);
         }
     }
     const float inv = (L == 0.f || L != L) ? 1.f : 1.f / L;
@@ -396,13 +470,6 @@ __device__ inline void combine_store(const AttnParams& p, const CombineWhere<E>&
     *reinterpret_cast<X4*>(p.out + ((size_t)w.node * p.Hq + w.head) * kHeadDim + w.d0) = o;
 }
 
-template <typename E>
-__device__ inline typename Elem<E>::x8 zero8() {
-    typename Elem<E>::x8 z;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) z[i] = (E)0.f;
-    return z;
-}
 
 // Swizzled LDS byte offsets inside one stage.  K: row = key (16 pieces of 16 B), piece index is
 // XORed with key % 16.  V^T: row = dim (8 pieces), XORed with (dim / 2) % 8 -- even and odd rows
@@ -510,7 +577,10 @@ __device__ inline void issue_tile_append(const AttnParams& p, int g, int tile, i
 // none of that code, so its registers and schedule are those of a kernel without the feature.
 // E: the element type.  The kernels proper are thin wrappers below (`tree_attn_split_kernel<G, ROPE>` for fp16 keeps the name
 // it has in every profile, `tree_attn_split_bf16_kernel<G, ROPE>` for bf16).
-template <int G, bool ROPE, typename E>
+// LOCAL: all splits of a unit are on one XCD, and the unit's partials change hands through its L2 (units_per_xcd).  That they are is what workgroup
+// numbers say (x % 8: the dispatcher deals workgroups to the XCDs in turn, whichever comes first); a unit counted in full proves it, since another XCD's
+// L2 counts for itself, and one that is not is reported (UnitWord::abandon).
+template <int G, bool ROPE, bool LOCAL, typename E>
 __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     typedef typename Elem<E>::x8 X8;
     typedef typename Elem<E>::x4 X4;
@@ -523,7 +593,7 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     __shared__ uint64_t s_mask[kMaxTree * 2];                                            // the tree mask as handed in
     __shared__ int s_append_page[3];  // pages of the (at most three: T <= 128) tiles that hold appended rows, as their requests found them
 
-    // XCD-aware work mapping: the grid is (splits x KV heads, padded to a multiple of the XCD count) x M-tiles.
+    // XCD-aware work mapping (but for LOCAL, below): the grid is (splits x KV heads, padded to a multiple of the XCD count) x M-tiles.
     // Workgroups are numbered x first and consecutive numbers go to consecutive XCDs, so x % 8 picks the XCD:
     // all M-tiles of one (split, kv head) pair share an XCD and the K/V pages they stream meet in its L2.
     // All launch arguments are fetched in one go, up front: left alone, the compiler fetches them in three batches as
@@ -544,11 +614,24 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     CPMCU_CLOCK_VAR(tl_fix0);
     CPMCU_CLOCK_VAR(tl_fix1);
     CPMCU_CLOCK(tl_start);
-    const int sh = blockIdx.x;
-    const int mt = blockIdx.y;
-    if (sh >= p.num_splits * p.Hkv) return;
-    const Quotient sh_of = divide(sh, p.Hkv, p.hkv_inv);
-    const int g = sh_of.r, split = sh_of.q;
+    int g, split, mt;
+    if constexpr (LOCAL) {
+        // XCD x % 8 has units (x % 8) * xcd_units, + 1, ..., neighbours in number for the same split: their K/V tiles meet in its L2
+        const Quotient place = divide(blockIdx.x / kXcds, p.xcd_units, p.xcd_units_inv);
+        const int unit = (blockIdx.x % kXcds) * p.xcd_units + place.r;
+        if (unit >= p.Hkv * p.num_mtiles) return;
+        const Quotient unit_of = divide(unit, p.num_mtiles, p.mtiles_inv);
+        g = unit_of.q;
+        mt = unit_of.r;
+        split = place.q;
+    } else {
+        const int sh = blockIdx.x;
+        if (sh >= p.num_splits * p.Hkv) return;
+        const Quotient sh_of = divide(sh, p.Hkv, p.hkv_inv);
+        g = sh_of.r;
+        split = sh_of.q;
+        mt = blockIdx.y;
+    }
 
     // The value as it is known here: keeps what is worked out from it in paths that few tiles take from being worked out ahead of
     // the loop, where it would hold registers that the loop needs.
@@ -559,7 +642,7 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
-    uint32_t* const unit_ctr = p.merge_ctr ? p.merge_ctr + kMergeUnitWords * (g * p.num_mtiles + mt) : nullptr;  // merge inside the launch
+    const bool merge_here = LOCAL || p.merge_ctr != nullptr;  // merge inside the launch
     const int grp = wave / kRowWaves;  // KV group: takes tiles grp, grp + G, ...
     const int rw = wave % kRowWaves;
     const int qcol = lane & 31;
@@ -625,7 +708,7 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     auto clamp_length = [&]() {
         const int lo = max(p.T, p.mask_k_range);
         if (S > p.max_kv_len || S < lo) {
-            if (sh == 0 && mt == 0 && tid == 0) g_attn_report.bad_length = S == 0 ? -1 : S;
+            if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) g_attn_report.bad_length = S == 0 ? -1 : S;
             S = min(max(S, lo), p.max_kv_len);
         }
     };
@@ -689,6 +772,11 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
             if (it * G + e < n) issue_tile_i(it * G + e);
     };
 
+    // Accumulator db holds dims 32 * dims_of(db) .. + 31.  With two KV groups a wave keeps half of the dims in the end, group 0 the lower and
+    // group 1 the upper one: it is accumulators 0 and 1 in either (as branches that differ in their registers the exchange and the stores
+    // exist twice, and made one by the compiler they put the accumulators into scratch memory).
+    const int dims_turn = G == 2 ? 2 * __builtin_amdgcn_readfirstlane(grp) : 0;
+    auto dims_of = [&](int db) { return db ^ dims_turn; };
     f32x16 oacc[4];
 #pragma unroll
     for (int db = 0; db < 4; ++db)
@@ -984,7 +1072,7 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
             for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int db = 0; db < 4; ++db)
-                    vf[j * 4 + db] = *reinterpret_cast<const X8*>(stage + v_lds_off(db * 32 + qcol, 2 * j + hf));
+                    vf[j * 4 + db] = *reinterpret_cast<const X8*>(stage + v_lds_off(dims_of(db) * 32 + qcol, 2 * j + hf));
             __builtin_amdgcn_sched_barrier(0);
             // sacc[kb][r] is the score of key  c0 + kb*32 + 8*(r/4) + 4*hf + r%4  for query qcol.
             if (c0 + kTileN > Pm) {  // tile touches masked columns or the end of the stream
@@ -1080,20 +1168,15 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         const int i_last = niter > 0 ? 2 * (niter - 1) : 0;
         f32x4* xch = reinterpret_cast<f32x4*>(ring + ((i_last + 2) % kStages) * kStageBytes);  // [wave][8 quads][64 lanes]
         float2* xml = reinterpret_cast<float2*>(vstage);                                        // [wave][64 lanes]
-        auto send = [&](auto db0_c) {
-            constexpr int DB0 = decltype(db0_c)::value;
 #pragma unroll
-            for (int db = 0; db < 2; ++db)
+        for (int db = 0; db < 2; ++db)
 #pragma unroll
-                for (int rq = 0; rq < 4; ++rq) {
-                    f32x4 o;
+            for (int rq = 0; rq < 4; ++rq) {
+                f32x4 o;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = oacc[DB0 + db][rq * 4 + e];
-                    xch[(wave * 8 + db * 4 + rq) * 64 + lane] = o;
-                }
-        };
-        if (grp == 0) send(std::integral_constant<int, 2>{});
-        else send(std::integral_constant<int, 0>{});
+                for (int e = 0; e < 4; ++e) o[e] = oacc[2 + db][rq * 4 + e];
+                xch[(wave * 8 + db * 4 + rq) * 64 + lane] = o;
+            }
         xml[wave * 64 + lane] = make_float2(m_ref, l_run);
         __syncthreads();
         const int other = wave ^ kRowWaves;  // same rows, other group
@@ -1102,41 +1185,30 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         const float m_scaled = (m_new == -INFINITY) ? 0.f : m_new;
         const float a0 = __builtin_amdgcn_exp2f(m_ref - m_scaled);
         const float a1 = __builtin_amdgcn_exp2f(ml1.x - m_scaled);
-        auto receive = [&](auto db0_c) {
-            constexpr int DB0 = decltype(db0_c)::value;
 #pragma unroll
-            for (int db = 0; db < 2; ++db)
+        for (int db = 0; db < 2; ++db)
 #pragma unroll
-                for (int rq = 0; rq < 4; ++rq) {
-                    const f32x4 o = xch[(other * 8 + db * 4 + rq) * 64 + lane];
+            for (int rq = 0; rq < 4; ++rq) {
+                const f32x4 o = xch[(other * 8 + db * 4 + rq) * 64 + lane];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) oacc[DB0 + db][rq * 4 + e] = oacc[DB0 + db][rq * 4 + e] * a0 + o[e] * a1;
-                }
-        };
-        if (grp == 0) receive(std::integral_constant<int, 0>{});
-        else receive(std::integral_constant<int, 2>{});
-        l_run = l_run * a0 + ml1.y * a1;
+                for (int e = 0; e < 4; ++e)  // (which product is rounded is not left to the compiler: every instance gives the same bits)
+                    oacc[db][rq * 4 + e] = __builtin_fmaf(oacc[db][rq * 4 + e], a0, o[e] * a1);
+            }
+        l_run = __builtin_fmaf(l_run, a0, ml1.y * a1);
         m_ref = m_new;
     }
 
     CPMCU_CLOCK(tl_groups);
-    // oacc[db][r] is O[query qcol][d = db*32 + 8*(r/4) + 4*hf + r%4], unnormalised; with two KV groups a wave now holds
-    // the d blocks [2 * grp, 2 * grp + 2) of its rows.
+    // oacc[db][r] is O[query qcol][d = dims_of(db)*32 + 8*(r/4) + 4*hf + r%4], unnormalised; with two KV groups a wave's are the first two now.
     const float l_tot = l_run + __shfl_xor(l_run, 32);
-    // stores db blocks [DB0, DB0 + NDB) of this wave's rows through `put(db, rq, values)`
+    // stores this wave's dims of its rows through `put(dims block, rq, values)`
     auto for_my_blocks = [&](auto&& put) {
-        auto run = [&](auto db0_c, auto ndb_c) {
-            constexpr int DB0 = decltype(db0_c)::value, NDB = decltype(ndb_c)::value;
 #pragma unroll
-            for (int db = DB0; db < DB0 + NDB; ++db)
+        for (int db = 0; db < (G == 1 ? 4 : 2); ++db)
 #pragma unroll
-                for (int rq = 0; rq < 4; ++rq) put(db, rq, oacc[db]);
-        };
-        if constexpr (G == 1) run(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
-        else if (grp == 0) run(std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{});
-        else run(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
+            for (int rq = 0; rq < 4; ++rq) put(dims_of(db), rq, oacc[db]);
     };
-    if (p.num_splits == 1) {
+    if (!LOCAL && p.num_splits == 1) {
         if (!row_ok) return;
         const float inv = (l_tot == 0.f || l_tot != l_tot) ? 1.f : 1.f / l_tot;
         f16* orow = p.out + ((size_t)node * p.Hq + head) * kHeadDim;
@@ -1158,11 +1230,11 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
             X4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = (E)(acc[rq * 4 + e] * inv);
-            if (unit_ctr != nullptr) store_dev64(&op[(db * 4 + rq) * 64], bits_as<uint64_t>(o));
+            if (!LOCAL && merge_here) store_dev64(&op[(db * 4 + rq) * 64], bits_as<uint64_t>(o));
             else __builtin_nontemporal_store(o, &op[(db * 4 + rq) * 64]);  // streamed: nothing left to flush at kernel end
         });
         if (grp == 0 && hf == 0 && row_ok) {
-            if (unit_ctr != nullptr) {
+            if (!LOCAL && merge_here) {
                 store_dev64(&p.ml_part[prow * 2], (uint64_t)__float_as_uint(m_ref) | ((uint64_t)__float_as_uint(l_tot) << 32));
             } else {
                 p.ml_part[prow * 2 + 0] = m_ref;
@@ -1181,7 +1253,7 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
             CPMCU_STAMP_VALUE(g_attn_timeline, wg, 4, tl_stored);
             CPMCU_STAMP_VALUE(g_attn_timeline, wg, 5, tl_acked);
             CPMCU_STAMP_VALUE(g_attn_timeline, wg, 6, tl_go);
-            if (unit_ctr != nullptr) CPMCU_STAMP(g_attn_timeline, wg, 7);
+            if (merge_here) CPMCU_STAMP(g_attn_timeline, wg, 7);
             else CPMCU_STAMP(g_attn_timeline, wg, 4);  // partials issued; the launch ends with them
             CPMCU_STAMP_VALUE(g_attn_timeline, wg, 8, niter);
             CPMCU_STAMP_VALUE(g_attn_timeline, wg, 9, n);
@@ -1192,21 +1264,23 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
             CPMCU_STAMP_VALUE(g_attn_timeline, wg, 14, tl_fix0);
             CPMCU_STAMP_VALUE(g_attn_timeline, wg, 15, tl_fix1);
         };
-        if (unit_ctr == nullptr) tl_record();
+        if (!merge_here) tl_record();
 #endif
-        if (unit_ctr == nullptr) return;
+        if (!merge_here) return;
         // ---- merge inside the launch ----
         // Every workgroup of the unit (same KV head and M-tile, one per split) announces its partials once they
-        // have reached memory; when all have, each merges its share of the unit's 32-row x 4-dim-quad blocks
+        // have reached memory (LOCAL: the L2); when all have, each merges its share of the unit's 32-row x 4-dim-quad blocks
         // (share s: the blocks b with b % splits == s).
         __shared__ int s_merge_go, s_merge_last;
         __shared__ uint32_t s_merge_abandoned;
+        constexpr int kBlocks = kRowWaves * 16;
         CPMCU_CLOCK(tl_stored);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         CPMCU_CLOCK(tl_acked);
+        uint32_t* const ctr = p.merge_ctr + kMergeUnitWords * (g * p.num_mtiles + mt);
         if (tid == 0) {
-            const Arrival a = arrive_at_unit(p, unit_ctr, split);
+            const Arrival a = arrive_at_unit<LOCAL>(p, ctr, p.num_splits, split);
             s_merge_go = a.go;
             s_merge_last = a.last;
         }
@@ -1216,11 +1290,10 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         const bool last = s_merge_last != 0;
         // the last one collects the abandoned shares while it merges its own
         uint32_t abandoned = 0;
-        if (last && tid == 0) abandoned = collect_abandoned(unit_ctr, 0);
-        const int nblocks = kRowWaves * 16;
+        if (last && tid == 0) abandoned = UnitWord<LOCAL>(ctr, 0, 0u).collect_abandoned(0);
         auto merge_share = [&](int share) {
-            for (int b = share + p.num_splits * wave; b < nblocks; b += p.num_splits * kWaves)
-                combine_block<true, E>(p, g, mt * kRowWaves + (b >> 4), b & 15, lane);
+            for (int b = share + p.num_splits * wave; b < kBlocks; b += p.num_splits * kWaves)
+                combine_block<LOCAL ? Partials::kOfTheXcd : Partials::kOfTheDevice, E>(p, g, mt * kRowWaves + (b >> 4), b & 15, lane);
         };
         merge_share(split);
         if (last) {
@@ -1235,13 +1308,13 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
 }
 
 // The merge as a launch of its own: one wave per (kv head, 32-row block, quad), in the partial layout's own order.
-template <int G, bool ROPE>
+template <int G, bool ROPE, bool LOCAL>
 __global__ __launch_bounds__(kThreads, 1) void tree_attn_split_kernel(AttnParams p) {
-    tree_attn_split_body<G, ROPE, f16>(p);
+    tree_attn_split_body<G, ROPE, LOCAL, f16>(p);
 }
-template <int G, bool ROPE>
+template <int G, bool ROPE, bool LOCAL>
 __global__ __launch_bounds__(kThreads, 1) void tree_attn_split_bf16_kernel(AttnParams p) {
-    tree_attn_split_body<G, ROPE, bf16>(p);
+    tree_attn_split_body<G, ROPE, LOCAL, bf16>(p);
 }
 
 template <typename E>
@@ -1252,7 +1325,7 @@ __device__ __forceinline__ void tree_attn_combine_body(const AttnParams& p) {
     const int nrb = p.rows_pad / kRowsPerWave;  // 32-row blocks per kv head (16 * 64 = 1024 threads each)
     const int grb = idx >> 10;
     if (grb >= p.Hkv * nrb) return;
-    combine_block<false, E>(p, grb / nrb, grb % nrb, quad, lane);
+    combine_block<Partials::kOfALaunch, E>(p, grb / nrb, grb % nrb, quad, lane);
 }
 __global__ __launch_bounds__(256) void tree_attn_combine_kernel(AttnParams p) { tree_attn_combine_body<f16>(p); }
 __global__ __launch_bounds__(256) void tree_attn_combine_bf16_kernel(AttnParams p) { tree_attn_combine_body<bf16>(p); }
@@ -1386,6 +1459,7 @@ struct LaunchPlan {
                      // (the window starts on a block boundary at or above P - block_window_size)
     int kv_groups, num_mtiles, num_splits;
     bool merge_in_launch;  // the split workgroups merge their own partials (no combine launch)
+    int xcd_units;         // split shapes: units per XCD where all splits of a unit are on one, and merged there (0: they are not)
     bool direct;           // the direct shape: num_mtiles counts its 16-row tiles
 };
 
@@ -1395,7 +1469,6 @@ struct LaunchPlan {
 // attention_release_workspace: a captured launch keeps its block's address, so a block is never passed on to another
 // workspace.  A launch that cannot have one -- more workspaces than blocks, a first launch under capture -- is merged by
 // the combine launch instead.
-constexpr int kMergeUnits = 256;    // (KV head, M-tile) units a launch may have on this path
 constexpr int kMergeBlocks = 32;    // workspaces with a block per device
 __device__ __align__(256) uint32_t g_merge_ctr[kMergeBlocks][kMergeUnits * kMergeUnitWords];
 __device__ DirectSlots g_direct_slots[kMergeBlocks];  // of the same workspaces
@@ -1406,6 +1479,21 @@ bool can_merge_in_launch(int Hkv, int num_mtiles, int num_splits) {
     if (!options().attn_merge_in_launch || num_splits < 2 || num_splits > kMergeMaxSplits) return false;
     if (Hkv * num_mtiles > kMergeUnits) return false;
     return kXcds * ceil_div(num_splits * Hkv, kXcds) * num_mtiles <= device_cu_count();
+}
+
+// Units per XCD of a launch that merges itself, where all splits of a unit are put on one XCD (one workgroup per CU) and their partials change
+// hands through its L2: acknowledged there in 0.4 us instead of 1-2, counted and read back without a trip to memory.  0: they are not.
+// With a multiple of 8 KV heads a unit's splits are on one XCD however they are numbered.  With fewer, M-tiles that would share K/V tiles in one L2
+// come to lie on several XCDs, each of which fetches its head's whole context (four times the traffic on 2 heads, twice on 4), and
+// with less than a multiple of 8 units XCDs are left idle.  us per layer in replayed graphs, merged through memory / an XCD: 60 nodes on 2 heads 12.4 / 11.4
+// at 1024 keys, 13.3 / 11.9 at 2048, 15.3 / 13.7 at 4096, 17.3 / 17.6 at 6000, 19.2 / 19.2 at 8192, 45.6 / 50.9 at 32768; 32 nodes 14.7 / 13.3 at 4096, 16.8 /
+// 17.4 at 8192; 128 nodes 17.1 / 16.4 at 2048, 21.6 / 21.6 at 4096, 29.5 / 30.1 at 8192; on 4 heads 60 nodes 14.3 / 13.4 at 4096, 19.5 / 20.4 at 8192; 24
+// nodes on 2 heads (6 units) 13.6 / 13.8 at 3000, 13.8 / 12.9 at 4096; on 8 heads 33 nodes of bfloat16 at 10007 22.2 / 21.0, 16 at 20000 28.9 / 25.8.
+constexpr int kXcdSpan = 4608;  // keys
+int units_per_xcd(int Hkv, int num_mtiles, int num_splits, int span) {
+    const int units = Hkv * num_mtiles, on_one = ceil_div(units, kXcds);
+    if (on_one * num_splits > device_cu_count() / kXcds) return 0;
+    return Hkv % kXcds == 0 || (units % kXcds == 0 && span <= kXcdSpan) ? on_one : 0;
 }
 
 struct MergeState {
@@ -1521,6 +1609,7 @@ LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_wind
     pl.span = max_kv_len;
     if (window_blocks > 0 && window_blocks * 128 + T < pl.span) pl.span = window_blocks * 128 + T;
     const int tiles = ceil_div(group * T, kDirectRows);
+    pl.xcd_units = 0;
     const DirectPlan direct = choose_direct(T, Hkv, tiles, pl.span, rope, merge == DirectMerge::kMayWait);
     // (a split count asked for is one of the split shapes', unless the direct shape is forced)
     pl.direct = merge != DirectMerge::kNone && direct.use && (num_splits_override == 0 || options().attn_direct == 1);
@@ -1536,6 +1625,7 @@ LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_wind
     pl.num_mtiles = ceil_div(group * T, rows_per_wg(pl.kv_groups));
     pl.num_splits = num_splits_override > 0 ? num_splits_override : choose_splits(T, group, Hkv, pl.span, pl.kv_groups);
     pl.merge_in_launch = can_merge_in_launch(Hkv, pl.num_mtiles, pl.num_splits);
+    if (pl.merge_in_launch) pl.xcd_units = units_per_xcd(Hkv, pl.num_mtiles, pl.num_splits, pl.span);
     return pl;
 }
 
@@ -1556,7 +1646,7 @@ extern "C" int cpmcu_tree_attention_plan(int T, int Hq, int Hkv, int max_kv_len,
                  pl.num_splits <= 1 || pl.merge_in_launch ? "" : pl.num_splits > kMergeMaxSplits ? "+tree_attn_combine_wide_kernel" : "+tree_attn_combine_kernel");
     if (num_splits) *num_splits = pl.num_splits;
     if (kv_groups) *kv_groups = pl.kv_groups;
-    if (num_workgroups) *num_workgroups = kXcds * ceil_div(pl.num_splits * Hkv, kXcds) * pl.num_mtiles;
+    if (num_workgroups) *num_workgroups = pl.xcd_units > 0 ? kXcds * pl.xcd_units * pl.num_splits : kXcds * ceil_div(pl.num_splits * Hkv, kXcds) * pl.num_mtiles;
     return CPMCU_OK;
 }
 
@@ -1604,6 +1694,8 @@ int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int
         const AttnReport zero{0, 0u, 0u};
         CPMCU_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_attn_report), &zero, sizeof(zero)));
         *g_report_host[dev] = zero;
+        // (the words of a unit that two L2s have counted are at rest no more)
+        if (r.lost != 0 && g_merge_ctr_base[dev] != nullptr) CPMCU_HIP(hipMemset(g_merge_ctr_base[dev], 0, sizeof(g_merge_ctr)));
         if (r.abandoned != 0) {
             std::lock_guard<std::mutex> lock(g_merge_mu);
             for (auto& kv : g_merge_states)
@@ -1754,21 +1846,17 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
         CPMCU_LAUNCH_CHECK();
         return CPMCU_OK;
     }
-    if (is_bf16) {
-        if (p.rope != nullptr) {
-            if (G == 1) hipLaunchKernelGGL((tree_attn_split_bf16_kernel<1, true>), grid, dim3(kThreads), 0, st, p);
-            else hipLaunchKernelGGL((tree_attn_split_bf16_kernel<2, true>), grid, dim3(kThreads), 0, st, p);
-        } else {
-            if (G == 1) hipLaunchKernelGGL((tree_attn_split_bf16_kernel<1, false>), grid, dim3(kThreads), 0, st, p);
-            else hipLaunchKernelGGL((tree_attn_split_bf16_kernel<2, false>), grid, dim3(kThreads), 0, st, p);
-        }
-    } else if (p.rope != nullptr) {
-        if (G == 1) hipLaunchKernelGGL((tree_attn_split_kernel<1, true>), grid, dim3(kThreads), 0, st, p);
-        else hipLaunchKernelGGL((tree_attn_split_kernel<2, true>), grid, dim3(kThreads), 0, st, p);
-    } else {
-        if (G == 1) hipLaunchKernelGGL((tree_attn_split_kernel<1, false>), grid, dim3(kThreads), 0, st, p);
-        else hipLaunchKernelGGL((tree_attn_split_kernel<2, false>), grid, dim3(kThreads), 0, st, p);
-    }
+    const bool local = p.merge_ctr != nullptr && plan.xcd_units > 0;
+    p.xcd_units = plan.xcd_units;
+    p.xcd_units_inv = local ? inverse_of(plan.xcd_units) : 0;
+    p.mtiles_inv = inverse_of(p.num_mtiles);
+    const dim3 sgrid = local ? dim3(kXcds * plan.xcd_units * p.num_splits) : grid;
+#define CPMCU_SPLIT(g, rope, local) (is_bf16 ? tree_attn_split_bf16_kernel<g, rope, local> : tree_attn_split_kernel<g, rope, local>)
+#define CPMCU_SPLIT_ROPE(g, local) (p.rope != nullptr ? CPMCU_SPLIT(g, true, local) : CPMCU_SPLIT(g, false, local))
+    const auto kernel = G == 1 ? (local ? CPMCU_SPLIT_ROPE(1, true) : CPMCU_SPLIT_ROPE(1, false)) : (local ? CPMCU_SPLIT_ROPE(2, true) : CPMCU_SPLIT_ROPE(2, false));
+#undef CPMCU_SPLIT_ROPE
+#undef CPMCU_SPLIT
+    hipLaunchKernelGGL(kernel, sgrid, dim3(kThreads), 0, st, p);
     CPMCU_LAUNCH_CHECK();
     if (p.num_splits > 1 && p.merge_ctr == nullptr) {
         const int waves_total = Hkv * (p.rows_pad / kRowsPerWave) * 16;  // one per (kv head, 32-row block, quad)
