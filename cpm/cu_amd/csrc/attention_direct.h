@@ -9,7 +9,7 @@
 //   * which pages a workgroup reads follows from its number alone: the page ids are requested beside the length instead of behind
 //     it, and a bound above the length costs no imbalance;
 //   * the appended rows are a block of their own, read from k_new / v_new (split 0 takes it first, while its pages are on their
-//     way), so no tile has to be patched; workgroups of their own (the first grid rows) write them to the pool meanwhile;
+//     way), so no tile has to be patched; workgroups of their own (the first of the grid) write them to the pool meanwhile;
 //   * the partials of few splits are merged by the last workgroup of a unit to arrive: nobody polls or waits, so the launch may be larger
 //     than the chip.  Those of many splits are merged in shares, by words that say themselves whether they are there: a kernel of its own
 //     (tree_attn_direct_shares_kernel), since code that a launch jumps over is fetched all the same, 0.1-0.2 us.
@@ -110,25 +110,24 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     __shared__ int s_late[2];  // the merge in shares: a wave's wait for partials ran out
     asm volatile("" ::"s"(p.q), "s"(p.k_pool), "s"(p.v_pool), "s"(p.block_table), "s"(p.kv_len), "s"(p.k_new), "s"(p.v_new), "s"(p.rope),
                  "s"(p.mask), "s"(p.mask_words), "s"(p.mask_k_range), "s"(p.T), "s"(p.Hq), "s"(p.Hkv), "s"(p.group), "s"(p.group_inv),
-                 "s"(p.hkv_inv), "s"(p.num_splits), "s"(p.num_mtiles), "s"(p.table_pages), "s"(p.window_blocks), "s"(p.max_kv_len));
+                 "s"(p.hkv_inv), "s"(p.tile_groups), "s"(p.tile_groups_inv), "s"(p.num_splits), "s"(p.num_mtiles), "s"(p.table_pages), "s"(p.window_blocks), "s"(p.max_kv_len));
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int append = p.k_new != nullptr ? 1 : 0;
-    const int sh = blockIdx.x;
-    const int mt = (int)blockIdx.y - p.append_rows;
+    const int wg = (int)blockIdx.x - p.append_groups;
 
     int S;
     auto clamp_length = [&]() {
         const int lo = max(p.T, p.mask_k_range);
         if (S > p.max_kv_len || S < lo) {
-            if (sh == 0 && blockIdx.y == 0 && tid == 0) g_attn_report.bad_length = S == 0 ? -1 : S;
+            if (blockIdx.x == 0 && tid == 0) g_attn_report.bad_length = S == 0 ? -1 : S;
             S = min(max(S, lo), p.max_kv_len);
         }
     };
-    if (mt < 0) {  // the rows on their way into the pool
+    if (wg < 0) {  // the rows on their way into the pool
         const int runs = (p.T + kAppendRows - 1) / kAppendRows;
         constexpr int kHalves = kThreads / kAppendThreads;
-        const int y = (blockIdx.y * gridDim.x + sh) * kHalves + tid / kAppendThreads;
+        const int y = blockIdx.x * kHalves + tid / kAppendThreads;
         if (y / kHalves * kHalves < runs * p.Hkv) {
             const Quotient y_of = divide(y, p.Hkv, p.hkv_inv);
             const int gg = y_of.r, run = y_of.q;
@@ -141,6 +140,8 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         }
         return;
     }
+    const Quotient wg_of = divide(wg, p.tile_groups, p.tile_groups_inv);
+    const int mt = wg_of.q, sh = wg_of.r;
     if (sh >= p.num_splits * p.Hkv) return;
     const Quotient sh_of = divide(sh, p.Hkv, p.hkv_inv);
     const int g = sh_of.r, split = sh_of.q;
