@@ -1585,16 +1585,23 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope, bool ma
     const int most = std::min(kMaxSplits, std::max(cus / units, std::max(1, std::min(4, 2 * cus / units))));
     DirectPlan d = {1, false};
     float best = 1e30f;
-    for (int it = ceil_div(blocks, most); it <= blocks; it = it < 64 ? it + 1 : it * 2) {
-        const int splits = ceil_div(blocks, it);
+    auto consider = [&](int splits, bool all_cus) {
         const int workgroups = kXcds * ceil_div(splits * Hkv, kXcds) * tiles;
+        const bool shares = may_wait && direct_merge_shares(splits, workgroups, cus) > 0;
+        if (all_cus && !shares) return;
         const float per_cu = (float)workgroups / (float)cus;
         const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.6f);
-        const float merge = splits == 1 ? 0.f : 2.3f + (may_wait && direct_merge_shares(splits, workgroups, cus) > 0 ? 0.025f : 0.06f) * splits;
+        const float merge = splits == 1 ? 0.f : 2.3f + (shares ? 0.025f : 0.06f) * splits;
+        const float it = all_cus ? (float)blocks / (float)splits + 0.25f : (float)ceil_div(blocks, splits);
         const float t = 3.4f + (units * splits * 2 > cus ? 1.2f : 1.05f) * it * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
                         0.6f * (new_steps - 1) + merge;
         if (t < best) best = t, d.splits = splits;
-    }
+    };
+    for (int it = ceil_div(blocks, most); it <= blocks; it = it < 64 ? it + 1 : it * 2) consider(ceil_div(blocks, it), false);
+    // Merged in shares, splits that do not divide the blocks evenly take little more than what they have on average: the last block of some
+    // is behind the others' merge loads.  us per layer, splits of whole iterations / one for each CU: 2 KV heads, one query at 32768
+    // keys 12.8 / 12.3, four at 4096 8.45 / 7.8, at 8192 9.55 / 9.1, at 16384 13.6 / 12.9; on 4 heads at 8192 11.4 / 10.7.
+    consider(std::min(most, blocks), true);
     const float split_shape = 10.2f + std::min(3.f, span / 2000.f) + stream + 0.02f * T + (split_units > 16 ? 3.f : 0.f) + (rope ? 1.5f : 0.f);
     d.use = options().attn_direct >= 0 ? options().attn_direct != 0 : options().attn_kv_groups == 0 && best < split_shape;
     return d;
