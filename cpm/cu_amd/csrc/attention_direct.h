@@ -9,7 +9,7 @@
 //   * which pages a workgroup reads follows from its number alone: the page ids are requested beside the length instead of behind
 //     it, and a bound above the length costs no imbalance;
 //   * the appended rows are a block of their own, read from k_new / v_new (split 0 takes it first, while its pages are on their
-//     way), so no tile has to be patched; workgroups of their own (the first of the grid) write them to the pool meanwhile;
+//     way), so no tile has to be patched; workgroups of their own write them to the pool meanwhile;
 //   * the partials of few splits are merged by the last workgroup of a unit to arrive: nobody polls or waits, so the launch may be larger
 //     than the chip.  Those of many splits are merged in shares, by words that say themselves whether they are there: a kernel of its own
 //     (tree_attn_direct_shares_kernel), since code that a launch jumps over is fetched all the same, 0.1-0.2 us.
@@ -114,7 +114,8 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int append = p.k_new != nullptr ? 1 : 0;
-    const int wg = (int)blockIdx.x - p.append_groups;
+    const int wg = SHARES ? (int)blockIdx.x - p.append_groups : (int)blockIdx.x;
+    const int append_wg = SHARES ? blockIdx.x : wg - p.tile_groups * p.num_mtiles;
 
     int S;
     auto clamp_length = [&]() {
@@ -124,10 +125,10 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
             S = min(max(S, lo), p.max_kv_len);
         }
     };
-    if (wg < 0) {  // the rows on their way into the pool
+    if (SHARES ? wg < 0 : append_wg >= 0) {  // the rows on their way into the pool
         const int runs = (p.T + kAppendRows - 1) / kAppendRows;
         constexpr int kHalves = kThreads / kAppendThreads;
-        const int y = blockIdx.x * kHalves + tid / kAppendThreads;
+        const int y = append_wg * kHalves + tid / kAppendThreads;
         if (y / kHalves * kHalves < runs * p.Hkv) {
             const Quotient y_of = divide(y, p.Hkv, p.hkv_inv);
             const int gg = y_of.r, run = y_of.q;

@@ -133,9 +133,9 @@ struct AttnParams {
     int num_splits, num_mtiles, rows_pad;
     int xcd_units;                       // all splits of a unit on one XCD: units per XCD
     uint32_t xcd_units_inv, mtiles_inv;  // inverse_of(xcd_units), inverse_of(num_mtiles)
-    int append_groups;          // direct shape: leading workgroups that write the appended rows to the pool, two runs each
-    int tile_groups;            // ... and the workgroups of each row tile behind them
-    uint32_t tile_groups_inv;   // inverse_of(tile_groups)
+    int append_groups;         // direct shape: workgroups that write the appended rows to the pool, two runs each
+    int tile_groups;           // ... and those of each row tile
+    uint32_t tile_groups_inv;  // inverse_of(tile_groups)
     int ntiles_max;  // tiles the split partition spans: ceil(max_kv_len / 64), fixed by the host-side bound
                      // (with a window: the most tiles a window can hold, counted from its first tile)
     int table_pages;    // entries of block_table the caller guarantees: ceil(max_kv_len / 256)
@@ -1847,13 +1847,16 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
             p.ml_part = (float*)p.slots->ml;
         }
         p.merge_shares = direct_merge == DirectMerge::kMayWait ? direct_merge_shares(p.num_splits, (int)(grid.x * grid.y), device_cu_count()) : 0;
-        // The appended rows' workgroups are as many as have work, rounded up so that the tiles keep their XCDs.  As whole grid rows, most of them
-        // empty, they held up the first tiles (us per layer, whole rows / this: one query on 2 KV heads 10.4 / 10.2 at 16384 keys, 17.9 / 16.8
-        // at 60001; 8 nodes 9.65 / 9.4 at 6000; 16 nodes 7.9 / 7.6 at 1024).
-        p.append_groups = k_new ? kXcds * ceil_div(ceil_div(T, kAppendRows) * Hkv, kXcds * (kThreads / kAppendThreads)) : 0;
+        // The appended rows' workgroups are as many as have work.  (As whole grid rows in front, most of them empty, they held up the first tiles.)
+        // Where the merge is shared out they come in front, and rounded up so that the tiles keep their XCDs: one of them that starts late ends last.  Else
+        // they come behind: in front they put two tiles on one CU where there is a CU for each.  us per layer, whole rows / in front / behind: one
+        // query on 2 KV heads 7.15 / 7.07 / 7.12 at 4096 keys, 10.5 / 10.3 / 10.4 at 16384, 18.3 / 16.9 / 16.8 at 60001; 16 nodes on 4 heads at 700
+        // 7.45 / 7.8 / 7.15, on 2 at 1024 8.0 / 7.55 / 7.5; 10 in a window of 1024 6.6 / 6.65 / 6.5; 56 at 1024 11.8 / 12.1 / 12.1.
+        p.append_groups = k_new ? ceil_div(ceil_div(T, kAppendRows) * Hkv, kThreads / kAppendThreads) : 0;
+        if (p.merge_shares > 0) p.append_groups = kXcds * ceil_div(p.append_groups, kXcds);
         p.tile_groups = grid.x;
         p.tile_groups_inv = inverse_of(grid.x);
-        const dim3 dgrid(p.append_groups + grid.x * grid.y);
+        const dim3 dgrid(grid.x * grid.y + p.append_groups);
         const auto kernel = p.merge_shares > 0 ? (is_bf16 ? tree_attn_direct_shares_bf16_kernel : tree_attn_direct_shares_kernel)
                                                : (is_bf16 ? tree_attn_direct_bf16_kernel : tree_attn_direct_kernel);
         hipLaunchKernelGGL(kernel, dgrid, dim3(kThreads), 0, st, p);
