@@ -1414,6 +1414,11 @@ int choose_splits(int T, int group, int Hkv, int max_kv_len, int G) {
     // better on more, shorter splits at short contexts (60-node tree at 512 tokens: 12.7 us on 10 splits, 16.2 on 4).
     const int tile_cap = merge && splits <= kMergeMaxSplits ? ntiles : ntiles / G;
     if (splits > tile_cap) splits = tile_cap > 0 ? tile_cap : 1;
+    // The launch's merge reads 16 partials at once, and with more of them in two goes: 17 to 32 splits have to make up for 1.5 us, which they do
+    // once 16 splits have nearly two tiles more each.  us per layer, 2 KV heads, 24 splits / 16 (33 nodes) 13.4 / 11.9 at 1536 keys, 14.2 / 13.4 at 3600,
+    // 15.9 / 16.4 at 6000, 22.9 / 25.9 at 16384; 20 / 16 (48 nodes) 14.2 / 12.2 at 1536, 15.8 / 14.3 at 3600, 18.5 / 18.0 at 8192, 26.3 / 26.8 at
+    // 16384; 32 / 16 (24 nodes) 13.3 / 12.2 at 2304, 13.4 / 13.0 at 3600, 13.5 / 14.8 at 4400.
+    if (merge && splits > 16 && splits <= kMergeMaxSplits && ntiles * (splits - 16) <= 30 * splits) splits = 16;
     // More than 64 splits (one M-tile: plain decode, trees of up to 8 nodes) pay for their partials and per-workgroup
     // latencies once every KV group still gets a run of about 3 tiles: one query, 128 against 64 splits, us per layer:
     // 18.6 / 19.0 at 32K, 21.3 / 23.2 at 48K, 23.6 / 27.1 at 64K, 36.4 / 47.5 at 128K (15.8 / 15.1 at 16K).
@@ -1491,11 +1496,20 @@ bool can_merge_in_launch(int Hkv, int num_mtiles, int num_splits) {
 // at 1024 keys, 13.3 / 11.9 at 2048, 15.3 / 13.7 at 4096, 17.3 / 17.6 at 6000, 19.2 / 19.2 at 8192, 45.6 / 50.9 at 32768; 32 nodes 14.7 / 13.3 at 4096, 16.8 /
 // 17.4 at 8192; 128 nodes 17.1 / 16.4 at 2048, 21.6 / 21.6 at 4096, 29.5 / 30.1 at 8192; on 4 heads 60 nodes 14.3 / 13.4 at 4096, 19.5 / 20.4 at 8192; 24
 // nodes on 2 heads (6 units) 13.6 / 13.8 at 3000, 13.8 / 12.9 at 4096; on 8 heads 33 nodes of bfloat16 at 10007 22.2 / 21.0, 16 at 20000 28.9 / 25.8.
+// Where XCDs are left idle (10 to 14 units, two on each of five to seven XCDs), units that share an XCD should share their head's tiles there: 48 nodes, 16
+// splits, 14.2 / 12.7 at 3000, 15.2 / 14.7 at 4400; an odd number of M-tiles (one XCD has units of both heads) pays up to 2560 keys on 2 heads: 33 nodes 12.4 / 11.7 at
+// 2304, 13.3 / 13.7 at 3000; 56 nodes 13.3 / 12.3 at 2304, 15.3 / 16.0 at 4400; level on 4 heads at 1536.  One unit on each of six, up to 4096: 20 nodes, 16
+// splits, 12.1 / 11.3 at 2304, 12.8 / 11.9 at 3600, 32 splits 15.3 / 15.7 at 4400.
 constexpr int kXcdSpan = 4608;  // keys
 int units_per_xcd(int Hkv, int num_mtiles, int num_splits, int span) {
     const int units = Hkv * num_mtiles, on_one = ceil_div(units, kXcds);
     if (on_one * num_splits > device_cu_count() / kXcds) return 0;
-    return Hkv % kXcds == 0 || (units % kXcds == 0 && span <= kXcdSpan) ? on_one : 0;
+    if (Hkv % kXcds == 0) return on_one;
+    if (span > kXcdSpan) return 0;
+    if (units % kXcds == 0) return on_one;
+    if (on_one > 2 || 2 * units <= kXcds * on_one) return 0;
+    if (on_one == 1) return span <= 4096 ? 1 : 0;
+    return num_mtiles % 2 == 0 || span * Hkv <= 2 * 2560 ? 2 : 0;
 }
 
 struct MergeState {

@@ -11,10 +11,11 @@ D = 128
 @pytest.mark.parametrize("P,T,hq,hkv,splits,groups", [
     (4548, 60, 32, 2, 16, 2), (4549, 60, 32, 2, 16, 2), (4000, 60, 32, 2, 15, 2), (2000, 60, 32, 2, 2, 2), (3000, 32, 32, 2, 32, 2), (3001, 128, 32, 2, 8, 2),
     (3000, 128, 32, 2, 16, 1), (1500, 60, 32, 2, 32, 1), (4500, 96, 32, 4, 10, 1), (2500, 33, 32, 8, 16, 2), (9001, 33, 32, 8, 31, 1), (6000, 128, 32, 8, 8, 1),
-    (700, 20, 48, 16, 16, 2), (5000, 17, 24, 8, 9, 2)])
+    (700, 20, 48, 16, 16, 2), (5000, 17, 24, 8, 9, 2),
+    (4076, 20, 32, 2, 16, 2), (1000, 24, 32, 2, 32, 2), (4560, 48, 32, 2, 16, 2), (2527, 33, 32, 2, 16, 2), (2504, 56, 32, 2, 13, 2), (1300, 40, 16, 1, 32, 2)])
 def test_merge_on_one_xcd_equals_separate_merge(gpu, P, T, hq, hkv, splits, groups):
-    """Launches whose units merge through the L2 of an XCD (one to three units on each, full and half empty XCDs, the longest context that is numbered
-    for it and the next one, any length on a multiple of 8 KV heads), in both types: the bits of the separate merge launch, also where every wait runs out at
+    """Launches whose units merge through the L2 of an XCD (one to three units on each, full, half empty and idle XCDs, XCDs with units of two heads, the longest context
+    that is numbered for it and the next one, any length on a multiple of 8 KV heads), in both types: the bits of the separate merge launch, also where every wait runs out at
     once, and in replays."""
     torch = gpu
     from cpm.cu_amd import lib, ops
