@@ -1568,8 +1568,12 @@ MergeCounters merge_counters_for(const void* workspace, hipStream_t st) {
 // 7.45 on 16, 8.30 / 7.56 on 24, 9.06 / 7.90 on 33, 22.99 / 20.41 on 64, 25.42 / 19.01 on 128; by words, last arrival / shares: 6.3 / 6.45 on 10, 10 row tiles on
 // 10 splits 6.6 / 7.3, 16 on 5 7.4 / 9.5: every wave polls), if there is a CU for each
 // workgroup: those with a share wait for all others, so all have to be resident (two to a CU are not, always).
-int direct_merge_shares(int num_splits, int workgroups, int cus) {
-    return num_splits > kDirectLastMerges && workgroups <= std::min(cus, kDirectSlots) ? std::min(num_splits, kDirectItems) : 0;
+// 16 splits are left to the last arrival too where more than half of the CUs pull K/V of four heads or more: the polls are in their way (words / last arrival, 8
+// nodes on 8 heads 10.1 / 9.8 at 3000 keys, 12.4 / 11.6 at 6000, 21.2 / 20.1 at 16384, on 4 13.4 / 12.85 at 8192; on 2 8.4 / 8.7 at 3000, 9.65 / 9.75 at
+// 6000; one query on 8 at 1900 7.35 / 7.85).
+int direct_merge_shares(int num_splits, int Hkv, int workgroups, int cus) {
+    const int by_the_last = kDirectLastMerges + (Hkv >= 4 && 2 * workgroups > cus ? 1 : 0);
+    return num_splits > by_the_last && workgroups <= std::min(cus, kDirectSlots) ? std::min(num_splits, kDirectItems) : 0;
 }
 
 // The direct shape or one of the split shapes, and the splits of the direct one: from estimates of both, in us, fitted to a sweep
@@ -1601,7 +1605,7 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope, bool ma
     float best = 1e30f;
     auto consider = [&](int splits, bool all_cus) {
         const int workgroups = kXcds * ceil_div(splits * Hkv, kXcds) * tiles;
-        const bool shares = may_wait && direct_merge_shares(splits, workgroups, cus) > 0;
+        const bool shares = may_wait && direct_merge_shares(splits, Hkv, workgroups, cus) > 0;
         if (all_cus && !shares) return;
         const float per_cu = (float)workgroups / (float)cus;
         const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.6f);
@@ -1860,7 +1864,7 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
             p.o_part = (float*)p.slots->o;  // (addresses in device memory)
             p.ml_part = (float*)p.slots->ml;
         }
-        p.merge_shares = direct_merge == DirectMerge::kMayWait ? direct_merge_shares(p.num_splits, (int)(grid.x * grid.y), device_cu_count()) : 0;
+        p.merge_shares = direct_merge == DirectMerge::kMayWait ? direct_merge_shares(p.num_splits, Hkv, (int)(grid.x * grid.y), device_cu_count()) : 0;
         // The appended rows' workgroups are as many as have work.  (As whole grid rows in front, most of them empty, they held up the first tiles.)
         // Where the merge is shared out they come in front, and rounded up so that the tiles keep their XCDs: one of them that starts late ends last.  Else
         // they come behind: in front they put two tiles on one CU where there is a CU for each.  us per layer, whole rows / in front / behind: one
