@@ -143,10 +143,15 @@ __global__ __launch_bounds__(kTopkThreads) void draft_extend_kernel(DraftState s
     }
 }
 
-// One thread per history entry up to 1024 entries (two beyond): the counting loop is a chain of LDS
-// reads, and sixteen waves hide its latency where four would wait for it.
+// One thread per history entry up to 1024 entries (two beyond).  A count over all entries is two vector instructions per entry and wave on
+// one CU, 4 us of 7.2 with 510 entries, so entries that cannot be among the T - 1 largest are left out first: the (T - 1)-th largest of the 64
+// maxima over every 64th entry has T - 1 entries at or above it.  us a launch in replayed graphs, all entries counted /
+// those kept, with their vocabulary ids looked up under the count: 7.4 / 5.0 with 510 entries and a tree of 60, 7.0 / 4.5 with 456 and 32, 15.3 / 6.6 with
+// 784 and 60, 21.4 / 8.7 with 1056 and 64, 3.9 / 4.0 with 136 and 30.  A draft of 6 rounds of 10 360.6 -> 357.8.
 constexpr int kFinishThreads = 1024;
+constexpr int kFinishCountsAll = 192;  // entries
 
+template <bool BOUND>
 __global__ __launch_bounds__(kFinishThreads) void draft_finish_kernel(DraftState s, int k, int num_iter, int T, const int32_t* cache_length,
                                                                       const int32_t* remap, bool set_root, int32_t root_id, int32_t* ids_out, int32_t* tree_pos,
                                                                       uint64_t* tree_mask, int32_t* tree_parent) {
@@ -156,6 +161,8 @@ __global__ __launch_bounds__(kFinishThreads) void draft_finish_kernel(DraftState
     __shared__ int32_t s_hpar[64];           // history parent of the entries chosen in rounds >= 1 (k * num_iter <= 64 of them)
     __shared__ int32_t s_sel[kMaxTree];      // history index of tree node i + 1
     __shared__ int32_t s_par[kMaxTree];
+    __shared__ __attribute__((aligned(16))) uint32_t s_kept[BOUND ? kMaxTried : 4];
+    __shared__ int s_kept_count;
     const int tid = threadIdx.x;
     const int kk = k * k;
     const int total = k + (num_iter - 1) * kk;
@@ -164,6 +171,7 @@ __global__ __launch_bounds__(kFinishThreads) void draft_finish_kernel(DraftState
     for (int x = tid; x < ((total + 3) & ~3); x += kFinishThreads) {
         const bool in = x < total;
         s_keys[x] = in ? key32(s.tried_val[x], x) : 0;
+        if constexpr (BOUND) s_kept[x] = 0;
         if (in) {
             s_pos[x] = s.tried_pos[x];
             s_reverse[x] = 0;  // a parent that was not selected maps to the root
@@ -171,14 +179,48 @@ __global__ __launch_bounds__(kFinishThreads) void draft_finish_kernel(DraftState
     }
     if (tid < k * (num_iter - 1)) s_hpar[tid] = s.tried_parent[tid];
     const int P = cache_length[0];
+    if (BOUND && tid == 0) s_kept_count = 0;
     __syncthreads();
-    for (int x = tid; x < total; x += kFinishThreads) {
-        const int place = keys_above(s_keys, total, s_keys[x]);
+    const uint32_t* keys = s_keys;
+    int count = total;
+    if constexpr (BOUND) {
+        const int lane = tid & 63;
+        if (tid - lane < total) {
+            uint32_t top = 0;
+            for (int x = lane; x < total; x += 64) top = max(top, s_keys[x]);
+            uint32_t bound = 0;  // of the values (a key's upper half)
+            for (int b = 15; b >= 0; --b) {
+                const uint32_t higher = bound | (1u << b);
+                if (__popcll(__ballot((top >> 16) >= higher)) >= T - 1) bound = higher;
+            }
+            for (int x = tid; x - lane < total; x += kFinishThreads) {
+                const uint32_t key = x < total ? s_keys[x] : 0;
+                const bool kept = x < total && (key >> 16) >= bound;
+                const uint64_t who = __ballot(kept);
+                int first = 0;
+                if (lane == 0) first = atomicAdd(&s_kept_count, __popcll(who));
+                first = __builtin_amdgcn_readfirstlane(first);
+                if (kept) s_kept[first + __popcll(who & ((1ull << lane) - 1))] = key;
+            }
+        }
+        __syncthreads();
+        keys = s_kept;
+        count = s_kept_count;
+    }
+    for (int j = tid; j < count; j += kFinishThreads) {
+        const uint32_t key = keys[j];
+        const int x = BOUND ? 0xFFFF - (int)(key & 0xFFFF) : j;
+        auto id_of = [&]() {
+            const int32_t fr = s_pos[x];
+            return remap ? remap[max(fr, 0)] : fr;
+        };
+        int32_t id = 0;
+        if constexpr (BOUND) id = id_of();
+        const int place = keys_above(keys, count, key);
         if (place < T - 1) {
             s_sel[place] = x;
             s_reverse[x] = place + 1;
-            const int32_t fr = s_pos[x];
-            ids_out[place + 1] = remap ? remap[max(fr, 0)] : fr;
+            ids_out[place + 1] = BOUND ? id : id_of();
         }
     }
     __syncthreads();
@@ -269,7 +311,8 @@ static int draft_tree_finish(void* state, int k, int num_iter, int tree_size, co
     const int total = k + (num_iter - 1) * k * k;
     CPMCU_CHECK_ARG(tree_size >= 2 && tree_size <= kMaxTree && tree_size - 1 <= total,
                     "draft_tree_finish: tree_size=%d outside [2, min(%d, history %d + 1)]", tree_size, kMaxTree, total);
-    hipLaunchKernelGGL(draft_finish_kernel, dim3(1), dim3(kFinishThreads), 0, resolve_stream(stream), draft_state(state, k, num_iter), k,
+    const auto kernel = total > kFinishCountsAll && tree_size - 1 <= 64 ? draft_finish_kernel<true> : draft_finish_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kFinishThreads), 0, resolve_stream(stream), draft_state(state, k, num_iter), k,
                        num_iter, tree_size, cache_length, token_id_remap, root_id != nullptr, root_id ? *root_id : 0, tree_draft_ids,
                        tree_position_ids, tree_attn_mask, tree_parent);
     CPMCU_LAUNCH_CHECK();

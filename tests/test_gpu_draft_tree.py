@@ -96,6 +96,24 @@ def test_positions_of_minus_one_stay_inside_the_table(gpu, orc, k, num_iter, T, 
     assert np.array_equal(parent, o_parent) and np.array_equal(mask.view(np.uint64), o_mask)
 
 
+@pytest.mark.parametrize("k,num_iter,T,equal", [(8, 3, 64, 0.), (9, 3, 60, 0.), (8, 4, 2, 0.), (8, 4, 64, 0.), (8, 4, 65, 0.), (8, 4, 66, 0.), (12, 2, 60, 0.), (14, 2, 60, .3), (10, 6, 60, 1.), (10, 6, 60, .9), (8, 8, 65, .99),
+                                                (32, 2, 64, .5), (32, 2, 2, 0.), (10, 6, 30, -1.)])
+def test_entries_below_the_bound_are_left_out(gpu, orc, k, num_iter, T, equal):
+    """Histories around the length from which the last step bounds its entries, one and several entries a thread, the smallest and the largest tree that it is done
+    for and the next one, with ties at the bound (`equal` of the log-probs the same; -1: all of them -inf but for one a row)."""
+    torch = gpu
+    vals, poss = make_rows(k, num_iter, 500, k + T)
+    rng = np.random.default_rng(T)
+    for v in vals:
+        v[rng.random(v.shape) < equal] = np.float16(-0.5)
+        if equal < 0:
+            v[:, 1:] = np.float16(-np.inf)
+    (o_ids, o_pos, o_mask, o_parent), _ = run_oracle(orc, k, num_iter, T, 99, vals, poss, None)
+    (g_ids, g_pos, g_mask, g_parent), _, _ = run_gpu(torch, k, num_iter, T, 99, vals, poss, None)
+    assert np.array_equal(g_ids[1:], o_ids[1:]) and np.array_equal(g_pos, o_pos)
+    assert np.array_equal(g_parent, o_parent) and np.array_equal(g_mask, o_mask)
+
+
 def test_heavy_ties(gpu, orc):
     """All log-probs equal: every choice is made by the index rule alone."""
     torch = gpu
