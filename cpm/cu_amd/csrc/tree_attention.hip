@@ -1584,13 +1584,12 @@ int direct_merge_shares(int num_splits, int Hkv, int workgroups, int cus) {
 //           for a merge and per partial 0.06 by the last arrival, 0.025 in shares
 //   split   10.2, 1 per 2000 keys up to 3 (more splits, then longer ones), the bytes, 0.02 per node, 3 beyond 16 units of 128 rows;
 //           1.5 with the rotary embedding
-// Measured, split / direct, us per layer, 2 KV heads (`python -m cpm.cu_amd.sweep attention --direct --graph`): one query 10.4 / 6.3 at
-// 1024 keys, 12.7 / 7.6 at 4096, 18.8 / 13.6 at 32768, 24.1 / 19.5 at 65536, 37.6 / 31.3 at 131072: direct at every
-// length.  The estimates change over at about 30000 keys with 4 nodes (16.1 / 12.8 at 16384, 19.0 / 17.8 at 32768), 12000 with 8 (15.3 / 12.3 at
-// 8192, 16.4 / 16.5 at 16384), 7000 with 16 (16.0 / 16.7 at 8192), 3000 with 24 (13.4 / 10.5 at 2048, 14.5 / 14.5 at 4096) and 900 with 33 and 60
-// (11.9 / 9.4 and 12.2 / 9.9 at 512, 13.5 / 13.1 and 13.2 / 13.6 at 1536), and leave 128 nodes to the split shapes (15.6 / 26.0 at
-// 512), whose larger tiles win beyond (60 nodes at 4096: 16.0 / 21.5).  The shape taken is within 9 % of the other one in
-// every cell of the sweep but 33 nodes at 1024 (12.9 / 11.2) and 8 nodes at 65536 on 8 KV heads (62.8 / 56.6).  The estimates cost up to 0.5 us of host time a call.
+// Measured, split / direct, us per layer, 2 KV heads: one query 10.1 / 6.3 at 1024 keys, 12.3 / 7.0 at 4096, 16.1 / 10.3 at 16384, 19.4 / 12.3 at 32768: direct at every
+// length.  The estimates change over beyond 32768 keys with 4 nodes (16.4 / 12.9 at 16384, 19.8 / 18.3 at 32768), beyond 16384 with 8 (16.0 / 11.7 at
+// 8192, 19.3 / 17.9 at 16384, 22.6 / 27.7 at 32768), at 7000 with 16 (16.5 / 15.2 at 8192, 20.8 / 26.4 at 16384), 3000 with 24 (12.8 / 10.6 at 2048, 13.9 / 13.4 at
+// 3000) and 900 to 1200 with 33 and 60 (12.7 / 11.9 and 11.4 / 11.9 at 1024, 12.7 / 13.4 and 12.2 / 13.4 at 1536), and leave most of 128 nodes to the split shapes (13.7 / 29.6
+// at 512), whose larger tiles win beyond (60 nodes at 4096: 15.2 / 22.1).  In a sweep of 458 launches of 4 to 128 nodes on 2, 4 and 8 heads the shape taken is within 3 %
+// of the other one or better but in 12, within 11 % but in 2: 72 nodes on 2 heads at 512 (14.4 / 19.5) and 128 on 4 at 512 (14.4 / 16.7).  The estimates cost up to 0.5 us of host time a call.
 struct DirectPlan {
     int splits;
     bool use;
