@@ -1434,7 +1434,10 @@ int choose_splits(int T, int group, int Hkv, int max_kv_len, int G) {
 //     nodes, where the two-group shape has 1.25-1.5 times the splits per tile): two groups.  us per layer, 256-row
 //     shape / two groups: 24 nodes 34.6 / 26.9 at 32K, 49.0 / 42.3 at 64K, 82 / 81 at 128K; 40 nodes 40.3 / 33.3 at
 //     32K, 67.6 / 56.6 at 64K, 124.5 / 105.7 at 128K; 48 nodes 68.2 / 64.6 at 64K, 127.7 / 122.3 at 128K; 16 nodes or
-//     one 74.8 / 62.4 and 73.2 / 55.0 at 128K;
+//     one 74.8 / 62.4 and 73.2 / 55.0 at 128K -- but where two groups have 32 splits and the 256-row shape 64 (17 to 32 nodes on 2 heads),
+//     the latter from about 65K on for 6 units of 128 rows and 87K for 8, when half the tiles a split pay for the merge launch: two groups / 256 rows
+//     77.8 / 71.4 (20 nodes), 79.9 / 75.5 (24) and 87.4 / 83.0 (32) at 128K, 61.2 / 56.3, 62.3 / 58.5 and 67.2 / 65 at 96K, 44.5 / 42.3, 45.0 / 43.9
+//     and 47.8 / 48.5 at 64K; on 4 heads 20 nodes 84.9 / 77 at 128K, 65 / 60 at 96K;
 //   * 2 s2 well below s1 (81 to 96 nodes: 8 splits against 20): the 256-row shape from 8K on (96 nodes: 28.7 / 30.8
 //     at 8K, 40.0 / 45.9 at 16K, 64.6 / 78.2 at 32K; 21.3 / 19.0 at 2K);
 //   * 2 s2 = s1 otherwise: the 256-row shape once every workgroup has a run of at least 16 tiles to amortise its larger
@@ -1444,6 +1447,7 @@ int choose_splits(int T, int group, int Hkv, int max_kv_len, int G) {
 // The option attn_kv_groups (cpmcu_set_option; CPMCU_ATTN_KV_GROUPS=1|2 in the environment at load) overrides the
 // choice: tests exercise both shapes.
 constexpr int kLongRunTiles = 16;
+constexpr int kLongSplitTiles = 170;
 int splits_that_fill(int T, int group, int Hkv, int G) {
     const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
     const int s = (cus / ceil_div(group * T, rows_per_wg(G)) / kXcds * kXcds) / Hkv;
@@ -1454,6 +1458,9 @@ int choose_groups(int T, int group, int Hkv, int max_kv_len) {
     const int units = ceil_div(group * T, rows_per_wg(1)) * Hkv;
     const int ntiles = ceil_div(max_kv_len, kTileN);
     const int s1 = splits_that_fill(T, group, Hkv, 1), s2 = splits_that_fill(T, group, Hkv, 2);
+    const int units2 = ceil_div(group * T, rows_per_wg(2)) * Hkv;
+    const bool s2_merges = s2 < 2 * kMergeMaxSplits;  // (up to 63 are cut to what a launch merges itself)
+    if (s2_merges && s1 >= 2 * std::min(s2, kMergeMaxSplits) && s1 > kMergeMaxSplits && ntiles >= kLongSplitTiles * units2) return 1;
     if (units < 4 || s1 > kMergeMaxSplits) return 2;
     if (40 * s2 >= 23 * s1) return 2;                       // 2 s2 / s1 >= 1.15
     if (40 * s2 <= 17 * s1) return ntiles >= 128 ? 1 : 2;   // 2 s2 / s1 <= 0.85
