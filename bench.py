@@ -40,11 +40,11 @@ MFMA_F16_PEAK_TFLOPS = 2500.0
 # names the library reports for the dispatch taken: a different instantiation finds no entry and reports null.
 MEASURED_TRAFFIC = {
     "source": "profiles/verify_step_hbm_traffic.md, profiles/tree_attention_long_context_traffic.md",
-    # the library the counters were read on (git rev-parse --short HEAD of that run, all figures)
-    "measured_at_commit": "5ad0aba",
+    # the library the counters were read on (git rev-parse --short HEAD of that run)
+    "measured_at_commit": "8a0f682 (32768 and 131072: 5ad0aba)",
     "kib_per_launch": {
-        "tree_attn_split_kernel<2,false>": 15185 + 9463,  # the merge of the split partials runs inside the launch
-        "head_gemm_stream_kernel<4,2,256>": 591978 + 128,
+        "tree_attn_split_kernel<2,false>": 25520 + 9008,  # each head's context through four XCDs; the split partials are merged in their L2s and written back behind the launch
+        "head_gemm_stream_kernel<4,2,256>": 591970 + 128,
     },
     # the attention launch at the longer contexts (32 splits of 256-row workgroups), by prefix length
     "attention_kib_per_launch_by_context": {"32768": 52487 + 17894, "131072": 150806 + 17894},
