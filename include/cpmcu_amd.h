@@ -98,7 +98,8 @@ const char* cpmcu_version(void);
  *                           the K-chunked kernel (CPMCU_HEAD_NO_STREAM set);
  *   "attn_merge_in_launch"  1 = the workgroups of a split tree-attention launch merge their own partials when the
  *                           launch fits the GPU's CUs and has at most 32 splits, those of the direct shape always (in
- *                           shares from 16 splits on if the launch fits, else by the last to arrive) (default), 0 = always
+ *                           shares from 16 splits on -- 17 where more than half of the CUs work on four KV heads and
+ *                           more -- if the launch fits, else by the last to arrive) (default), 0 = always
  *                           the separate merge launch, and the direct shape for launches of one split only
  *                           (CPMCU_ATTN_SEPARATE_MERGE set);
  *   "attn_merge_wait_us"    longest time a workgroup of such a launch waits for the others of its merge before it
@@ -338,7 +339,8 @@ size_t cpmcu_tree_attention_workspace_bytes(int T, int Hq, int Hkv, int max_kv_l
  *   scale: softmax scale (1/sqrt(128) in the reference, flash_api.hpp:360).
  *   workspace: device scratch of at least ..._workspace_bytes(), may be NULL
  *           when that is 0.  Calls that may overlap on one GPU must use different
- *           workspaces: the split partials live there, and the library keys the
+ *           workspaces: the split partials live there (but for the direct shape's
+ *           with 16 splits and more, which the library has memory for), and the library keys the
  *           arrival counters of the in-launch merge by this pointer (a launch with at
  *           most 32 splits, of the direct shape with 16 to 128, and at most one workgroup
  *           per CU merges its own partials; its workgroups wait for each other, which
