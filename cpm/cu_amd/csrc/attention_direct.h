@@ -575,7 +575,7 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         const bool merged = split >= p.merge_shares || merge_share(split, p.merge_wait_ticks);
         if (tid == 0) s_before = before;
         __syncthreads();
-        const UnitWord<false> word(ctr, p.num_splits, s_before);
+        const UnitWord word(ctr, p.num_splits, s_before);
         if (word.last()) {
             // (every workgroup of the unit has read the generations)
             if (wave == 0) {
@@ -611,7 +611,7 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
         store_dev64(ml_part + (split * kDirectRows + c) * 8, (uint64_t)__float_as_uint(M) | ((uint64_t)__float_as_uint(L) << 32));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0) s_arrival = arrive_at_unit<false>(p, ctr, p.num_splits, -1);
+    if (tid == 0) s_arrival = arrive_at_unit(p, ctr, p.num_splits, -1);
     __syncthreads();
     const auto o_rsrc = __builtin_amdgcn_make_buffer_rsrc(o_part, 0, p.num_splits * kPartBytes, 0x00027000);
     if (!s_arrival.last) return;

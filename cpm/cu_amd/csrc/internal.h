@@ -15,18 +15,20 @@ struct Options {
     int head_stream_kernel = 1;    // 0 keeps tiled weights on the K-chunked kernel (tests compare the two)
     int attn_merge_in_launch = 1;  // 0: the split partials of tree attention are always merged by a launch of their own
     int attn_merge_wait_us = 2000; // longest wait of a workgroup for the others of its merge before it abandons its share
+    int attn_spread_units = 0;     // 1: launches that merge through the L2 of an XCD have their workgroups numbered apart (tests)
     int frspec_fused = 0;          // 1: the FR-Spec head with its top-k as one launch where the shape allows (measured no faster: off)
     int frspec_wait_us = 50000;    // longest wait of a finisher of the fused FR-Spec launch for the other workgroups' words
     int topk_row_kernel = 1;       // 0: top-k by k rounds per chunk of 2048 elements and a merge launch (tests compare the two)
 };
 Options& options();
 
-// tree_attention.hip -- two things an attention launch can leave behind for the host: a device-side length outside
-// [max(T, mask_k_range), max_kv_len] (the launch worked on the clamped length), and merge waits that ran out.
-// attention_report_enqueue copies both words to pinned host memory in stream order (ahead of a synchronisation, never
+// tree_attention.hip -- what an attention launch can leave behind for the host: a device-side length outside
+// [max(T, mask_k_range), max_kv_len] (the launch worked on the clamped length), merge waits that ran out, partials of the
+// direct shape that did not arrive within a second, and units to be merged on one XCD that were on several.
+// attention_report_enqueue copies the words to pinned host memory in stream order (ahead of a synchronisation, never
 // under a capture); attention_report_take reads that copy afterwards and clears what it found.
 int attention_report_enqueue(hipStream_t st);
-int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int* lost);
+int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int* lost, unsigned int* spread);
 void attention_merge_reenable();
 // Assigns the counters of the in-launch merge to a workspace on the current device (otherwise done by the first
 // launch that uses it outside a stream capture); they stay with it until it is released.

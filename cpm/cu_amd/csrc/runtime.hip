@@ -167,7 +167,7 @@ struct PerfScope {
 // Synchronises the stream and looks at what attention launches left behind for the host (the report words travel to
 // pinned memory in front of the synchronisation: no round trip of their own): a length outside what the host had
 // promised is an error; merge waits that ran out are counted for the summary.
-long g_abandoned_waits = 0;
+long g_abandoned_waits = 0, g_spread_units = 0;
 // Fused FR-Spec launches: rows finished from the published candidates, rows redone from the logits, waits that ran out.
 long g_frspec_fused_rows = 0, g_frspec_slow_rows = 0, g_frspec_timeouts = 0;
 int synchronize_and_check(hipStream_t st) {
@@ -177,10 +177,11 @@ int synchronize_and_check(hipStream_t st) {
     if (rc) return rc;
     CPMCU_HIP(hipStreamSynchronize(st));
     int bad = 0;
-    unsigned int abandoned = 0, lost = 0;
-    rc = attention_report_take(&bad, &abandoned, &lost);
+    unsigned int abandoned = 0, lost = 0, spread = 0;
+    rc = attention_report_take(&bad, &abandoned, &lost, &spread);
     if (rc) return rc;
     g_abandoned_waits += abandoned;
+    g_spread_units += spread;
     unsigned int fr_timeouts = 0, fr_slow = 0, fr_fused = 0;
     rc = head_fuse_report_take(&fr_timeouts, &fr_slow, &fr_fused);
     if (rc) return rc;
@@ -247,6 +248,9 @@ extern "C" int cpmcu_set_option(const char* name, int value) {
         CPMCU_CHECK_ARG(value == 0 || value == 1, "set_option: attn_merge_in_launch=%d must be 0 or 1", value);
         options().attn_merge_in_launch = value;
         if (value) attention_merge_reenable();  // also for workspaces whose launches have not waited since an abandoned wait
+    } else if (nm == "attn_spread_units") {
+        CPMCU_CHECK_ARG(value == 0 || value == 1, "set_option: attn_spread_units=%d must be 0 or 1", value);
+        options().attn_spread_units = value;
     } else if (nm == "frspec_fused") {
         CPMCU_CHECK_ARG(value == 0 || value == 1, "set_option: frspec_fused=%d must be 0 or 1", value);
         options().frspec_fused = value;
@@ -808,7 +812,7 @@ uint64_t step_signature(const Model& m, const StepArgs& a) {
         mix(v);
     // the options decide which kernels a capture records: a graph captured under other settings is another graph
     const Options& o = options();
-    for (int v : {o.dtype, o.attn_kv_groups, o.attn_direct, o.head_share_last_pass, o.head_stream_kernel, o.attn_merge_in_launch, o.attn_merge_wait_us, o.frspec_fused, o.frspec_wait_us, o.topk_row_kernel}) mix((uint64_t)(uint32_t)v);
+    for (int v : {o.dtype, o.attn_kv_groups, o.attn_direct, o.head_share_last_pass, o.head_stream_kernel, o.attn_merge_in_launch, o.attn_merge_wait_us, o.attn_spread_units, o.frspec_fused, o.frspec_wait_us, o.topk_row_kernel}) mix((uint64_t)(uint32_t)v);
     return h;
 }
 
@@ -997,6 +1001,7 @@ extern "C" int cpmcu_print_perf_summary(void) {
     if (hipMemGetInfo(&free_b, &total_b) == hipSuccess)
         printf("GPU memory: %.1f MiB used of %.1f MiB\n", (total_b - free_b) / 1048576.0, total_b / 1048576.0);
     printf("attention merge waits that ran out (share left to the last workgroup of its unit): %ld\n", g_abandoned_waits);
+    printf("attention units to be merged on one XCD that were on several: %ld\n", g_spread_units);
     printf("one-launch FR-Spec heads: %ld rows from the published candidates, %ld redone from the logits, %ld not finished\n",
            g_frspec_fused_rows, g_frspec_slow_rows, g_frspec_timeouts);
     fflush(stdout);
@@ -1008,6 +1013,7 @@ extern "C" int cpmcu_print_perf_summary(void) {
 // others of its unit and left its share of the merge to the last of them: the output was complete, but late, and nobody
 // waits in later launches on the device's workspaces (cpmcu_set_option("attn_merge_in_launch", 1) undoes that).
 extern "C" long cpmcu_attention_abandoned_waits(void) { return g_abandoned_waits; }
+extern "C" long cpmcu_attention_spread_units(void) { return g_spread_units; }
 
 // Rows of one-launch FR-Spec heads seen by the library's synchronisations so far: finished from the published candidates,
 // redone from the logits in memory (tie-heavy rows), and not finished because a wait ran out (an error at that

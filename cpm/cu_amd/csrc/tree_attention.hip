@@ -42,6 +42,7 @@
 #include "kv_append.h"
 #include "timeline.h"
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -85,8 +86,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 struct AttnReport {
     int bad_length;
     unsigned int abandoned;
-    unsigned int lost;  // partials that never came: words of the direct shape, a second after the last arrival, or a unit merged through the L2 of
-                        // an XCD whose workgroups turned out to be on two
+    unsigned int lost;    // partials that never came: words of the direct shape, a second after the last arrival
+    unsigned int spread;  // units to be merged through the L2 of an XCD whose workgroups turned out to be on several
 };
 __device__ AttnReport g_attn_report;
 
@@ -132,6 +133,7 @@ struct AttnParams {
     uint32_t group_inv, hkv_inv;  // inverse_of(group), inverse_of(Hkv)
     int num_splits, num_mtiles, rows_pad;
     int xcd_units;                       // all splits of a unit on one XCD: units per XCD
+    int xcd_turn;                        // ... 1: split s of a unit s XCDs on instead (tests)
     uint32_t xcd_units_inv, mtiles_inv;  // inverse_of(xcd_units), inverse_of(num_mtiles)
     int append_groups;         // direct shape: workgroups that write the appended rows to the pool, two runs each
     int tile_groups;           // ... and those of each row tile
@@ -161,7 +163,7 @@ struct AttnParams {
 };
 
 constexpr int kMergeUnits = 256;    // (KV head, M-tile) units a launch may have on this path
-constexpr int kUnitXccWord = 32;      // of a unit's words: see UnitWord::abandon (another line than the words that an L2 works on)
+constexpr int kUnitXcdWords = 32;     // of a unit's words: those of XcdUnit
 constexpr int kMergeUnitWords = 64;  // a unit's word sits in a 256-byte line of its own: every poll and every arrival is
                                      // a memory transaction, and those on one line queue behind each other
 
@@ -189,45 +191,20 @@ __device__ inline To bits_as(const From& v) {
 struct Arrival {
     int go;    // the partials of all splits are there, and this workgroup merges its share
     int last;  // nobody arrives behind this one: it also merges what was abandoned
-    uint32_t before;  // (UnitWord)
+    int spread;  // (XcdUnit)
 };
-// Atomics on a unit's words.  LOCAL: all workgroups of the unit are on one XCD, and its L2 performs them (0.3 us; the words are
-// back in memory behind the launch).  Assembly, because the compiler turns an addition of zero into a load, which the CU's own cache may answer.
-template <bool LOCAL>
-struct UnitAtomics {
-    __device__ static inline uint32_t add(uint32_t* w, uint32_t v) { return __hip_atomic_fetch_add(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-    __device__ static inline uint32_t mark(uint32_t* w, uint32_t v) { return __hip_atomic_fetch_or(w, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT); }
-    __device__ static inline uint32_t keep(uint32_t* w, uint32_t v) { return __hip_atomic_fetch_and(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-    __device__ static inline uint32_t take(uint32_t* w) { return __hip_atomic_exchange(w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-    __device__ static inline uint32_t look(uint32_t* w) { return __hip_atomic_load(w, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT); }
-    __device__ static inline uint32_t poll(uint32_t* w) { return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-};
-#define CPMCU_L2_ATOMIC(op, w, v)                                                                                                             \
-    uint32_t before;                                                                                                                          \
-    asm volatile("global_atomic_" op " %0, %1, %2, off sc0\n\ts_waitcnt vmcnt(0)" : "=&v"(before) : "v"(w), "v"(v) : "memory"); \
-    return before
-template <>
-struct UnitAtomics<true> {
-    __device__ static inline uint32_t add(uint32_t* w, uint32_t v) { CPMCU_L2_ATOMIC("add", w, v); }
-    __device__ static inline uint32_t mark(uint32_t* w, uint32_t v) { CPMCU_L2_ATOMIC("or", w, v); }
-    __device__ static inline uint32_t keep(uint32_t* w, uint32_t v) { CPMCU_L2_ATOMIC("and", w, v); }
-    __device__ static inline uint32_t take(uint32_t* w) { CPMCU_L2_ATOMIC("swap", w, 0u); }
-    __device__ static inline uint32_t look(uint32_t* w) { return add(w, 0u); }
-    __device__ static inline uint32_t poll(uint32_t* w) { return add(w, 0u); }
-};
-#undef CPMCU_L2_ATOMIC
-
 // A unit's word as an arrival found it: the generation of this launch above, the arrivals before it below.
-template <bool LOCAL>
 struct UnitWord {
-    typedef UnitAtomics<LOCAL> Atomics;
     uint32_t* ctr;
     uint32_t before, full;
     __device__ inline UnitWord(uint32_t* c, int num_splits, uint32_t b) : ctr(c), before(b), full((b & 0xffff0000u) + (uint32_t)num_splits) {}
-    __device__ inline UnitWord(uint32_t* c, int num_splits) : UnitWord(c, num_splits, Atomics::add(c, 1u)) {}
+    __device__ inline UnitWord(uint32_t* c, int num_splits)
+        : UnitWord(c, num_splits, __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {}
     __device__ inline bool last() const { return before + 1u == full; }
     // last to arrive: full count -> next generation, no arrivals (nobody needs the result of this one)
-    __device__ inline void next_generation() const { (void)Atomics::add(ctr, 0x10000u - (full & 0xffffu)); }
+    __device__ inline void next_generation() const {
+        __hip_atomic_fetch_add(ctr, 0x10000u - (full & 0xffffu), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     // either the full count or, once the last one has moved it on, the next generation
     __device__ inline bool complete(uint32_t now) const { return now == full || (now & 0xffff0000u) != (before & 0xffff0000u); }
     // Marks a share as abandoned.  True: everyone has arrived after all, and the workgroup merges its share itself.
@@ -236,61 +213,122 @@ struct UnitWord {
         // by its maker).
         uint32_t* const mark = ctr + 1 + (share >> 5);
         const uint32_t bit = 1u << (share & 31);
-        // The mark is made before this workgroup looks once more: if the others have all arrived by
+        // The mark is in memory before this workgroup looks once more: if the others have all arrived by
         // then, the last of them may have read the marks already, and this workgroup merges its share
         // itself (twice the same values at worst); if not, the last one will find the mark.
         // (acquire-release on the mark, acquire on the look that follows: the two stay in this order)
-        (void)Atomics::mark(mark, bit);
-        uint32_t here = 0, seen = 0;
-        if constexpr (LOCAL) {
-            // A unit whose workgroups are not on one XCD never counts them all, and every wait in it runs out: those from two XCDs meet in
-            // this word, in memory, which is zero between the launches of a unit on one XCD.
-            uint32_t xcc;
-            asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-            here = 1u << (xcc & 31);
-            seen = UnitAtomics<false>::mark(ctr + kUnitXccWord, here) & ~here;
-        }
-        const bool go = complete(Atomics::look(ctr));
-        // everyone is there after all: this workgroup merges its share itself and takes its marks back, so that
-        // none outlives the launch (if the last arrival has collected it already, the share is merged twice
+        (void)__hip_atomic_fetch_or(mark, bit, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        const bool go = complete(__hip_atomic_load(ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT));
+        // everyone is there after all: this workgroup merges its share itself and takes its mark back, so that
+        // no mark outlives the launch (if the last arrival has collected it already, the share is merged twice
         // with the same values)
-        if (go) {
-            (void)Atomics::keep(mark, ~bit);
-            if (LOCAL) (void)UnitAtomics<false>::keep(ctr + kUnitXccWord, ~here);
-        } else if (seen != 0) {
-            __hip_atomic_fetch_add(&g_attn_report.lost, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        if (go) (void)__hip_atomic_fetch_and(mark, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_fetch_add(&g_attn_report.abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return go;
     }
     // The last arrival: shares 32 w .. 32 w + 31 that were abandoned.
     __device__ inline uint32_t collect_abandoned(int w) const {
-        const uint32_t marks = Atomics::take(ctr + 1 + w);
-        if (LOCAL && marks != 0) __hip_atomic_store(ctr + kUnitXccWord, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return marks;
+        return __hip_atomic_exchange(ctr + 1 + w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 };
 // of: how many arrive at the word
-template <bool LOCAL>
 __device__ inline Arrival arrive_at_unit(const AttnParams& p, uint32_t* unit_ctr, int of, int share) {
     Arrival a = {share >= 0 ? 1 : 0, 0, 0};
-    const UnitWord<LOCAL> word(unit_ctr, of);
-    a.before = word.before;
+    const UnitWord word(unit_ctr, of);
     if (word.last()) {
         word.next_generation();
         a.last = 1;
     } else if (share >= 0) {
         const unsigned long long t_begin = wall_clock64();
-        while (!word.complete(UnitAtomics<LOCAL>::poll(unit_ctr))) {
+        while (!word.complete(__hip_atomic_load(unit_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
             if (wall_clock64() - t_begin >= p.merge_wait_ticks) {
                 a.go = word.abandon(share) ? 1 : 0;
                 break;
             }
-            __builtin_amdgcn_s_sleep(LOCAL ? 1 : 4);
+            __builtin_amdgcn_s_sleep(4);
         }
     }
     return a;
 }
+
+// The same for a unit whose workgroups are all on one XCD, as far as their numbers say, and whose partials change hands through that XCD's L2.
+// Where a workgroup is placed is the dispatcher's business, so an arrival adds its XCD's number and that number's square to the unit's word: with n arrivals, n
+// times the sum of the squares is the square of the sum if they are all of one XCD, and more if not.  (Atomics on the word are the device's, whoever is on
+// which XCD; on one XCD they take 0.3 us.)  From one XCD, all partials are in its L2.  Else the unit is spread, and what its workgroups have
+// merged is not valid: each writes its L2 back to memory, and the one that completes the mask of those that have done so merges all shares anew;
+// nobody waits for that.
+struct XcdUnit {
+    // arrivals (6 bits), sums of the XCDs' numbers (8) and their squares (11), zero between launches; a generation (7)
+    static constexpr int kSumBit = 6, kSquaresBit = 14, kGenerationBit = 25;
+    static_assert(kMergeMaxSplits < 1 << kSumBit && kMergeMaxSplits * (kXcds - 1) < 1 << (kSquaresBit - kSumBit) &&
+                  kMergeMaxSplits * (kXcds - 1) * (kXcds - 1) < 1 << (kGenerationBit - kSquaresBit), "the fields of the word");
+    uint32_t* word;
+    uint32_t* mark;  // shares abandoned, one bit each (at most 32); zero between launches
+    uint32_t* back;  // a spread unit: splits whose partials are in memory; zero between launches
+    __device__ inline explicit XcdUnit(uint32_t* unit_ctr) : word(unit_ctr + kUnitXcdWords), mark(word + 1), back(word + 2) {}
+    __device__ static inline uint32_t here() {
+        uint32_t xcc;
+        asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+        return xcc % kXcds;
+    }
+    // (assembly, because the compiler turns an addition of zero into a load, which is slower to see the others' additions; one thread: the answer may be
+    // a scalar)
+    __device__ inline uint32_t add(uint32_t v) const {
+        uint32_t before;
+        asm volatile("global_atomic_add %0, %1, %2, off sc0\n\ts_waitcnt vmcnt(0)" : "=&v"(before) : "v"(word), "v"(v) : "memory");
+        return __builtin_amdgcn_readfirstlane(before);
+    }
+    __device__ inline uint32_t collect_abandoned() const { return __hip_atomic_exchange(mark, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    // xcd: here()
+    __device__ inline Arrival arrive(const AttnParams& p, int share, uint32_t xcd) const {
+        Arrival a = {1, 0, 0};
+        const uint32_t of = (uint32_t)p.num_splits, one = 1u + (xcd << kSumBit) + (xcd * xcd << kSquaresBit), before = add(one);
+        uint32_t now = before + one;
+        // the full count, or the generation that the last arrival moves it on to: the next one, or the next but one if the unit is spread
+        auto complete = [&]() { return (now & ((1u << kSumBit) - 1)) == of || (now ^ before) >> kGenerationBit != 0; };
+        auto is_spread = [&]() {
+            const uint32_t sum = now >> kSumBit & ((1u << (kSquaresBit - kSumBit)) - 1), squares = now >> kSquaresBit & ((1u << (kGenerationBit - kSquaresBit)) - 1);
+            const uint32_t moved = (now >> kGenerationBit) - (before >> kGenerationBit);
+            return (of * squares != sum * sum ? 1 : 0) | (moved >> 1 & 1);
+        };
+        if ((now & ((1u << kSumBit) - 1)) == of) {
+            a.last = 1;
+            a.spread = is_spread();
+            const uint32_t on = (((before >> kGenerationBit) + 1u + a.spread) << kGenerationBit) - now;
+            asm volatile("global_atomic_add %0, %1, off" ::"v"(word), "v"(on) : "memory");
+            return a;
+        }
+        const unsigned long long t_begin = wall_clock64();
+        for (;;) {
+            now = add(0);
+            if (complete()) break;
+            if (wall_clock64() - t_begin >= p.merge_wait_ticks) {
+                // The last arrival may be on another XCD: the mark has this one's L2 written back in front of it (acquire-release).  The look
+                // behind it as in UnitWord::abandon.
+                const uint32_t bit = 1u << share;
+                (void)__hip_atomic_fetch_or(mark, bit, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+                now = add(0);
+                __hip_atomic_fetch_add(&g_attn_report.abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                a.go = complete() ? 1 : 0;
+                // (everyone is there after all: the mark is taken back; if the last arrival has it already, the share is merged twice with the
+                // same values, but a spread unit's mask gets each bit once)
+                if (a.go && (__hip_atomic_fetch_and(mark, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit) == 0 && is_spread()) a.go = 0;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        a.spread = is_spread();
+        return a;
+    }
+    // A spread unit: the partials of these splits may be read from memory by now, or will once this is done.  The shares that this workgroup merges.
+    __device__ inline uint32_t written_back(uint32_t splits, int of) const {
+        const uint32_t all = 0xffffffffu >> (32 - of);
+        if ((__hip_atomic_fetch_or(back, splits, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) | splits) != all) return 0;
+        __hip_atomic_store(back, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(&g_attn_report.spread, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return all;
+    }
+};
 template <typename E>
 __device__ inline typename Elem<E>::x8 zero8() {
     typename Elem<E>::x8 z;
@@ -304,7 +342,8 @@ __device__ inline typename Elem<E>::x8 zero8() {
 // src/flash_attn/src/flash_fwd_kernel.h:2392-2472 in base-2 form.  The statistics and the O partials of up to 16
 // splits are all requested before any is used, so a block pays one memory round trip, not one per split.
 // FROM: who wrote the partials -- an earlier launch, other workgroups of this one (device-scope loads), or workgroups of this one on the same
-// XCD (what its L2 has; the CU's own cache cannot have a line of them yet.  Scalar offsets: 16 pointers would take the registers of the loop).
+// XCD (what its L2 has, or memory behind XcdUnit's mask of a spread unit; the CU's own cache cannot have a line of them yet.  Scalar offsets: 16 pointers
+// would take the registers of the loop).
 constexpr int kCombineBatch = 16;
 enum class Partials { kOfALaunch, kOfTheDevice, kOfTheXcd };
 template <Partials FROM, typename E>
@@ -580,8 +619,7 @@ __device__ inline void issue_tile_append(const AttnParams& p, int g, int tile, i
 // E: the element type.  The kernels proper are thin wrappers below (`tree_attn_split_kernel<G, ROPE>` for fp16 keeps the name
 // it has in every profile, `tree_attn_split_bf16_kernel<G, ROPE>` for bf16).
 // LOCAL: all splits of a unit are on one XCD, and the unit's partials change hands through its L2 (units_per_xcd).  That they are is what workgroup
-// numbers say (x % 8: the dispatcher deals workgroups to the XCDs in turn, whichever comes first); a unit counted in full proves it, since another XCD's
-// L2 counts for itself, and one that is not is reported (UnitWord::abandon).
+// numbers say (x % 8: the dispatcher deals workgroups to the XCDs in turn, whichever comes first); whether it is so they count (XcdUnit).
 template <int G, bool ROPE, bool LOCAL, typename E>
 __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     typedef typename Elem<E>::x8 X8;
@@ -620,7 +658,7 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
     if constexpr (LOCAL) {
         // XCD x % 8 has units (x % 8) * xcd_units, + 1, ..., neighbours in number for the same split: their K/V tiles meet in its L2
         const Quotient place = divide(blockIdx.x / kXcds, p.xcd_units, p.xcd_units_inv);
-        const int unit = (blockIdx.x % kXcds) * p.xcd_units + place.r;
+        const int unit = ((blockIdx.x + p.xcd_turn * place.q) % kXcds) * p.xcd_units + place.r;
         if (unit >= p.Hkv * p.num_mtiles) return;
         const Quotient unit_of = divide(unit, p.num_mtiles, p.mtiles_inv);
         g = unit_of.q;
@@ -1277,28 +1315,39 @@ __device__ __forceinline__ void tree_attn_split_body(const AttnParams& p) {
         __shared__ uint32_t s_merge_abandoned;
         constexpr int kBlocks = kRowWaves * 16;
         CPMCU_CLOCK(tl_stored);
+        const uint32_t xcd = LOCAL ? XcdUnit::here() : 0;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         CPMCU_CLOCK(tl_acked);
         uint32_t* const ctr = p.merge_ctr + kMergeUnitWords * (g * p.num_mtiles + mt);
         if (tid == 0) {
-            const Arrival a = arrive_at_unit<LOCAL>(p, ctr, p.num_splits, split);
+            Arrival a;
+            if constexpr (LOCAL) a = XcdUnit(ctr).arrive(p, split, xcd);
+            else a = arrive_at_unit(p, ctr, p.num_splits, split);
             s_merge_go = a.go;
-            s_merge_last = a.last;
+            s_merge_last = a.last + 2 * a.spread;
         }
         __syncthreads();
         CPMCU_CLOCK(tl_go);
         if (!s_merge_go) return;
-        const bool last = s_merge_last != 0;
+        const int last_spread = s_merge_last;
         // the last one collects the abandoned shares while it merges its own
         uint32_t abandoned = 0;
-        if (last && tid == 0) abandoned = UnitWord<LOCAL>(ctr, 0, 0u).collect_abandoned(0);
+        if ((last_spread & 1) && tid == 0) {
+            if constexpr (LOCAL) abandoned = XcdUnit(ctr).collect_abandoned();
+            else abandoned = UnitWord(ctr, 0, 0u).collect_abandoned(0);
+        }
         auto merge_share = [&](int share) {
             for (int b = share + p.num_splits * wave; b < kBlocks; b += p.num_splits * kWaves)
                 combine_block<LOCAL ? Partials::kOfTheXcd : Partials::kOfTheDevice, E>(p, g, mt * kRowWaves + (b >> 4), b & 15, lane);
         };
         merge_share(split);
-        if (last) {
+        if (last_spread != 0) {
+            if (LOCAL && last_spread >= 2) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+                if (tid == 0) abandoned = XcdUnit(ctr).written_back(1u << split | abandoned, p.num_splits);
+            }
             if (tid == 0) s_merge_abandoned = abandoned;
             __syncthreads();
             for (uint32_t m = s_merge_abandoned; m != 0; m &= m - 1) merge_share(__builtin_ctz(m));
@@ -1508,8 +1557,12 @@ bool can_merge_in_launch(int Hkv, int num_mtiles, int num_splits) {
 // 2304, 13.3 / 13.7 at 3000; 56 nodes 13.3 / 12.3 at 2304, 15.3 / 16.0 at 4400; level on 4 heads at 1536.  One unit on each of six, up to 4096: 20 nodes, 16
 // splits, 12.1 / 11.3 at 2304, 12.8 / 11.9 at 3600, 32 splits 15.3 / 15.7 at 4400.
 constexpr int kXcdSpan = 4608;  // keys
+// A device on which a synchronisation has found spread units (XcdUnit) is left alone: a spread unit is merged by one workgroup.
+std::atomic<bool> g_spread_seen[64];
 int units_per_xcd(int Hkv, int num_mtiles, int num_splits, int span) {
     const int units = Hkv * num_mtiles, on_one = ceil_div(units, kXcds);
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 || g_spread_seen[dev]) return 0;
     if (on_one * num_splits > device_cu_count() / kXcds) return 0;
     if (Hkv % kXcds == 0) return on_one;
     if (span > kXcdSpan) return 0;
@@ -1711,24 +1764,23 @@ int attention_report_enqueue(hipStream_t st) {
     CPMCU_CHECK_ARG(dev >= 0 && dev < 64, "device index %d outside [0, 64)", dev);
     if (g_report_host[dev] == nullptr) {
         CPMCU_HIP(hipHostMalloc((void**)&g_report_host[dev], sizeof(AttnReport), hipHostMallocDefault));
-        *g_report_host[dev] = AttnReport{0, 0u, 0u};
+        *g_report_host[dev] = AttnReport{};
     }
     CPMCU_HIP(hipMemcpyFromSymbolAsync(g_report_host[dev], HIP_SYMBOL(g_attn_report), sizeof(AttnReport), 0, hipMemcpyDeviceToHost, st));
     return CPMCU_OK;
 }
-int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int* lost) {
+int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int* lost, unsigned int* spread) {
     int dev = 0;
     CPMCU_HIP(hipGetDevice(&dev));
     *bad_length = 0;
-    *abandoned = *lost = 0;
+    *abandoned = *lost = *spread = 0;
     if (dev < 0 || dev >= 64 || g_report_host[dev] == nullptr) return CPMCU_OK;
     const AttnReport r = *g_report_host[dev];
-    if (r.bad_length != 0 || r.abandoned != 0 || r.lost != 0) {
-        const AttnReport zero{0, 0u, 0u};
+    if (r.bad_length != 0 || r.abandoned != 0 || r.lost != 0 || r.spread != 0) {
+        const AttnReport zero{};
         CPMCU_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_attn_report), &zero, sizeof(zero)));
         *g_report_host[dev] = zero;
-        // (the words of a unit that two L2s have counted are at rest no more)
-        if (r.lost != 0 && g_merge_ctr_base[dev] != nullptr) CPMCU_HIP(hipMemset(g_merge_ctr_base[dev], 0, sizeof(g_merge_ctr)));
+        if (r.spread != 0) g_spread_seen[dev] = true;
         if (r.abandoned != 0) {
             std::lock_guard<std::mutex> lock(g_merge_mu);
             for (auto& kv : g_merge_states)
@@ -1738,12 +1790,14 @@ int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int
     *bad_length = r.bad_length;
     *abandoned = r.abandoned;
     *lost = r.lost;
+    *spread = r.spread;
     return CPMCU_OK;
 }
-// Lets the launches on the workspaces of the current device wait again (cpmcu_set_option attn_merge_in_launch = 1).
+// Lets the launches on the workspaces of the current device wait, and merge through the L2 of an XCD, again (cpmcu_set_option attn_merge_in_launch = 1).
 void attention_merge_reenable() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return;
+    if (dev >= 0 && dev < 64) g_spread_seen[dev] = false;
     std::lock_guard<std::mutex> lock(g_merge_mu);
     for (auto& kv : g_merge_states)
         if (kv.first.first == dev) kv.second.no_waits = false;
@@ -1889,6 +1943,7 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     }
     const bool local = p.merge_ctr != nullptr && plan.xcd_units > 0;
     p.xcd_units = plan.xcd_units;
+    p.xcd_turn = options().attn_spread_units;
     p.xcd_units_inv = local ? inverse_of(plan.xcd_units) : 0;
     p.mtiles_inv = inverse_of(p.num_mtiles);
     const dim3 sgrid = local ? dim3(kXcds * plan.xcd_units * p.num_splits) : grid;

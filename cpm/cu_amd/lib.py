@@ -50,6 +50,7 @@ SIGNATURES = {
     "cpmcu_stream": (c_u64, []),
     "cpmcu_synchronize": (c_int, []),
     "cpmcu_attention_abandoned_waits": (ctypes.c_long, []),
+    "cpmcu_attention_spread_units": (ctypes.c_long, []),
     "cpmcu_shutdown": (c_int, []),
     "cpmcu_kv_append": (c_int, [_P, _P, _P, _P, _P, _P, c_int, c_int, _P]),
     "cpmcu_tree_attention_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),

@@ -105,6 +105,11 @@ const char* cpmcu_version(void);
  *   "attn_merge_wait_us"    longest time a workgroup of such a launch waits for the others of its merge before it
  *                           leaves its share to the last one to arrive (default 2000; 0 = never wait: split launches leave
  *                           their shares at once, those of the direct shape are merged whole by the last to arrive);
+ *   "attn_spread_units"     1 = launches whose units merge through the L2 of one XCD each have their workgroups numbered
+ *                           so that they are on several, as on a GPU that places workgroups otherwise: each unit is
+ *                           merged through memory by one workgroup, and launches behind the next synchronisation that
+ *                           checks (cpmcu_synchronize) no longer try, until attn_merge_in_launch is set to 1 (tests;
+ *                           default 0);
  *   "topk_row_kernel"       1 = top-k by the one-launch row kernel (rows of more than 32768 elements in slices and a
  *                           merge of the slices' k best) (default), 0 = k rounds of a maximum search per chunk of 2048
  *                           elements and a merge launch, for chunks x k up to 2048: the same results, bit for bit,
@@ -294,6 +299,11 @@ int cpmcu_synchronize(void);
  * that arrives last.  Launches that a graph holds already keep the form in which they were recorded.
  * cpmcu_set_option("attn_merge_in_launch", 1) lets later ones wait again. */
 long cpmcu_attention_abandoned_waits(void);
+/* No reference counterpart: (KV head, M-tile) units of tree-attention launches that were to be merged through the L2 of
+ * one XCD and had workgroups on several (a CU mask, another order of dispatch), as counted by the synchronising calls so
+ * far.  Such a unit is merged by one workgroup, through memory: its output is complete.  Launches behind the call that has
+ * seen one are numbered and merged without regard to XCDs; those that a graph holds already keep their form. */
+long cpmcu_attention_spread_units(void);
 /* Free everything the global model owns (the reference never frees). */
 int cpmcu_shutdown(void);
 

@@ -35,7 +35,7 @@ def gpu():
 def set_option():
     """Sets kernel-shape options of the library for one test and restores the defaults afterwards."""
     from cpm.cu_amd import lib
-    defaults = {"dtype": 0, "attn_kv_groups": 0, "head_share_last_pass": 1, "head_stream_kernel": 1, "attn_merge_in_launch": 1, "attn_merge_wait_us": 2000,
+    defaults = {"dtype": 0, "attn_kv_groups": 0, "attn_direct": -1, "head_share_last_pass": 1, "head_stream_kernel": 1, "attn_merge_in_launch": 1, "attn_merge_wait_us": 2000, "attn_spread_units": 0,
                 "frspec_fused": 0, "frspec_wait_us": 50000, "topk_row_kernel": 1}
     touched = []
 

@@ -63,3 +63,74 @@ def test_merge_on_one_xcd_equals_separate_merge(gpu, P, T, hq, hkv, splits, grou
         option("attn_merge_wait_us", 2000)
         L.synchronize()
         option("attn_merge_in_launch", 1)
+
+
+@pytest.mark.parametrize("P,T,hq,hkv,splits,groups", [
+    (4000, 60, 32, 2, 16, 2), (2000, 60, 32, 2, 2, 2), (3000, 32, 32, 2, 32, 2), (1500, 128, 32, 2, 8, 2), (9001, 33, 32, 8, 31, 1), (2527, 33, 32, 2, 16, 2), (4076, 20, 32, 2, 16, 2)])
+def test_units_on_several_xcds_are_merged_all_the_same(gpu, set_option, P, T, hq, hkv, splits, groups):
+    """Launches numbered for one XCD a unit whose workgroups are then on several (each split of a unit on the next one; with 2 splits two, else all
+    eight): the bits are those of the separate merge, in replays, with launches on one XCD between them, and where waits run out (60 launches each; a mark or a count
+    that outlived its launch would complete a unit that is not there yet).  All units of those launches are counted as spread, and none of the others."""
+    torch = gpu
+    from cpm.cu_amd import lib, ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    L = lib.get()
+    set_option("attn_kv_groups", groups)
+    set_option("attn_direct", 0)
+    S = P + T
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).half()
+    cache = PagedKVCache(1, hkv, (S + 255) // 256 + 1)
+    cache.write_logical(0, 0, rnd(S, hkv, D), rnd(S, hkv, D))
+    q, kv_len = rnd(T, hq, D), torch.tensor([S], dtype=torch.int32, device="cuda")
+    mask = to_dev(torch, synth.random_tree(T, S, max_children=4, max_depth=9).mask)
+
+    def launch(out):
+        out.fill_(float("nan"))
+        if ("attn", q.device) in ops._workspaces:
+            ops._workspaces["attn", q.device].fill_(255)  # (no partials of the launch before: NaN)
+        ops.tree_attention(q, cache, 0, kv_len, S, mask, num_splits=splits, out=out)
+
+    def same(out, *what):
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), what
+
+    L.synchronize()
+    set_option("attn_merge_in_launch", 0)
+    ref = torch.empty_like(q)
+    launch(ref)
+    set_option("attn_merge_in_launch", 1)
+    out, graphs, seen = torch.empty_like(q), {}, L.raw.cpmcu_attention_abandoned_waits()
+    launch(out)  # (the workspace gets its counters outside the captures)
+    for spread in (0, 1):
+        set_option("attn_spread_units", spread)
+        graphs[spread] = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graphs[spread]):
+            launch(out)
+    set_option("attn_spread_units", 0)
+    for spread in (0, 0):
+        graphs[spread].replay()
+        same(out, spread)
+    L.synchronize()
+    spread_units = L.raw.cpmcu_attention_spread_units()
+    for spread in (1, 0, 1, 1, 0, 0, 1):
+        graphs[spread].replay()
+        same(out, spread)
+    L.synchronize()
+    units = hkv * -(-hq // hkv * T // (128 if groups == 2 else 256))
+    assert L.raw.cpmcu_attention_spread_units() - spread_units == 4 * units
+    assert L.raw.cpmcu_attention_abandoned_waits() == seen
+    try:
+        set_option("attn_merge_in_launch", 1)
+        for wait_us in (0, 1):
+            set_option("attn_merge_wait_us", wait_us)
+            for turn in range(60):
+                set_option("attn_spread_units", turn & 1)
+                launch(out)
+                same(out, wait_us, turn)
+    finally:
+        set_option("attn_merge_wait_us", 2000)
+        set_option("attn_spread_units", 0)
+        L.synchronize()
+        set_option("attn_merge_in_launch", 1)
+    assert L.raw.cpmcu_attention_abandoned_waits() > seen
