@@ -25,6 +25,8 @@ constexpr int kDirectRows = 16;        // packed query rows per workgroup
 constexpr int kBlockKeys = kPage / 2;  // keys per iteration
 constexpr int kDirectItems = kDirectRows * 4;  // pieces of a unit's output that are merged by themselves: 32 dims of a row
 constexpr int kDirectLastMerges = 15;          // up to here the last arrival merges all splits
+constexpr float kSumScale = 1.f / kMaxSplits;
+static_assert((kMaxSplits & (kMaxSplits - 1)) == 0, "kSumScale");
 // A partial that is merged in shares changes hands through memory of the library: every 8-byte word carries two outputs (or half of a
 // row's statistics) and the generation of its slot, so that a reader that sees the generation has the payload, and nothing is acknowledged
 // or counted in front of the reads (acknowledgement, arrival, poll and read were four round trips, store and poll are two).  A slot's
@@ -504,10 +506,12 @@ __device__ __forceinline__ void tree_attn_direct_body(const AttnParams& p) {
                     asm volatile("" ::: "memory");  // (loads anew)
                 }
                 if (!__all(there)) s_late[parity] = 1;
-                // sums over the wave's splits, relative to their own maximum
+                // Sums over the wave's splits, relative to their own maximum and times kSumScale (exact): a weighted partial is at most its split's own
+                // sum, so that all of them together stay finite where each of those was (bfloat16 V of 1e34 and 60000 keys).  Dividing each sum by its
+                // weights' instead took 0.2 us a layer.
                 const float m = my_split < p.num_splits ? __uint_as_float(ml[0]) : -INFINITY;
                 const float top = over_splits<true>(m);
-                const float weight = __uint_as_float(ml[2]) * __builtin_amdgcn_exp2f(m - (top == -INFINITY ? 0.f : top));
+                const float weight = __uint_as_float(ml[2]) * kSumScale * __builtin_amdgcn_exp2f(m - (top == -INFINITY ? 0.f : top));
                 const X8 x = bits_as<X8>(u32x4{xa[0], xa[2], xb[0], xb[2]});
                 f32x4 lo, hi;
 #pragma unroll

@@ -262,3 +262,22 @@ def test_words_of_launches_of_changing_shapes(gpu, option):
             assert float((o.float() - ref.float()).abs().max()) <= 2.0 ** -10 * float(ref.float().abs().max()), shape
     finally:
         option("attn_merge_wait_us", 2000)
+
+
+@pytest.mark.parametrize("splits", [8, 16, 20, 40, 128])
+def test_merges_of_large_values_stay_finite(gpu, option, splits):
+    """bfloat16 V of 1e34, keys of equal weight: no split's sum (at most 60001 / 8 x 1e34) and no output leaves the range of an fp32, and no merge of them does, by
+    the last arrival or in shares on one to eight waves.  The mean of equal values is the value, but for fp32 roundings far below bfloat16's."""
+    from cpm.cu_amd import ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch, S = gpu, 60001
+    option("dtype", 1)
+    option("attn_direct", 1)
+    bits = lambda t: t.to(torch.bfloat16).view(torch.float16)
+    cache = PagedKVCache(1, 2, (S + 255) // 256)
+    v = torch.full((S, 2, D), 1e34, device="cuda")
+    v[:, 1] *= -1
+    cache.write_logical(0, 0, bits(torch.randn(S, 2, D, device="cuda")), bits(v))
+    kv_len = torch.tensor([S], dtype=torch.int32, device="cuda")
+    out = ops.tree_attention(bits(torch.zeros(1, 32, D, device="cuda")), cache, 0, kv_len, S, num_splits=splits).view(torch.bfloat16)
+    assert torch.equal(out, v[:1].to(torch.bfloat16).repeat_interleave(16, 1))
