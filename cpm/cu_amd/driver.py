@@ -21,7 +21,7 @@ the reference's ``(padded_length, T)`` graph key (src/entry.cu:475-492).
 """
 import torch
 
-from . import ops
+from . import lib, ops
 
 
 class VerifyStep:
@@ -148,7 +148,8 @@ class GraphedSteps:
         return (need + self.pad_to - 1) // self.pad_to * self.pad_to
 
     def run(self):
-        """Replay (capturing first, if this padded length is new) one step; returns (a, ids)."""
+        """Replay (capturing first, if this padded length is new) one step; returns (a, ids).  A step whose attention has left an
+        error behind (a length beyond its padded one, partials that never came) raises."""
         st = self.step
         padded = self._padded()
         assert padded <= st.cache.num_pages * 256, "the paged cache is too small for this padded length"
@@ -164,6 +165,7 @@ class GraphedSteps:
         with torch.cuda.stream(self.stream):
             self.graphs[padded].replay()
         self.stream.synchronize()
+        lib.get().synchronize()  # what the attention launches report reaches the host through the library alone
         a = int(st.packed[0])
         self.prefix_bound += a
         return a, st.packed[1:1 + a].numpy().copy()

@@ -103,6 +103,28 @@ def test_graph_replayed_steps_equal_host_driven_steps(gpu, orc):
         assert np.array_equal(to_np(va).view(np.uint16), to_np(vb).view(np.uint16))
 
 
+def test_replayed_steps_report_what_their_attention_reports(gpu):
+    """A length on the device beyond the padded one of the graph (the kernels work on it clamped): the replay raises instead of returning ids, and the step
+    behind it, on a length that fits, is whole again."""
+    from cpm.cu_amd.driver import GraphedSteps, VerifyStep
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch = gpu
+    tree = synth.random_tree(T, 1, max_children=3, max_depth=6)
+    mask, parent, pos = [torch.from_numpy(x).cuda() for x in (tree.mask.view(np.int64), tree.parent, tree.positions(P0))]
+    step = VerifyStep(PagedKVCache(1, HKV, 10), to_dev(torch, synth.normal_f16((VOCAB, H), 3, 2, std=0.02)), mask, parent, pos, P0, commit=True)
+    gs = GraphedSteps(step, 1, HQ, HKV, H)  # (padded to 1024, which the first step fills, then 2048)
+    a, _ = gs.run()
+    step.kv_len.fill_(2222)
+    torch.cuda.synchronize()
+    with pytest.raises(RuntimeError, match="KV length of 2222"):
+        gs.run()
+    step.kv_len.copy_(step.cache_length + T)
+    want = P0 + a + int(step.packed[0])
+    torch.cuda.synchronize()
+    a, ids = gs.run()
+    assert a == len(ids) >= 1 and int(step.cache_length[0]) == want + a
+
+
 @pytest.mark.parametrize("commit", [False, True])
 def test_step_is_ready_on_every_stream_when_built(gpu, commit):
     """Built on a stream that is busy, read and written on another one without a wait: the lengths are there, and no fill of the
