@@ -1662,23 +1662,29 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope, bool ma
     const int most = std::min(kMaxSplits, std::max(cus / units, std::max(1, std::min(4, 2 * cus / units))));
     DirectPlan d = {1, false};
     float best = 1e30f;
-    auto consider = [&](int splits, bool all_cus) {
-        const int workgroups = kXcds * ceil_div(splits * Hkv, kXcds) * tiles;
-        const bool shares = may_wait && direct_merge_shares(splits, Hkv, workgroups, cus) > 0;
-        if (all_cus && !shares) return;
-        const float per_cu = (float)workgroups / (float)cus;
+    const auto workgroups_of = [&](int splits) { return kXcds * ceil_div(splits * Hkv, kXcds) * tiles; };
+    const auto shares = [&](int splits) { return may_wait && direct_merge_shares(splits, Hkv, workgroups_of(splits), cus) > 0; };
+    const auto estimate = [&](int splits, float iterations) {
+        const float per_cu = (float)workgroups_of(splits) / (float)cus;
         const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.6f);
-        const float merge = splits == 1 ? 0.f : 2.3f + (shares ? 0.025f : 0.06f) * splits;
-        const float it = all_cus ? (float)blocks / (float)splits + 0.25f : (float)ceil_div(blocks, splits);
-        const float t = 3.4f + (units * splits * 2 > cus ? 1.2f : 1.05f) * it * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
-                        0.6f * (new_steps - 1) + merge;
-        if (t < best) best = t, d.splits = splits;
+        const float merge = splits == 1 ? 0.f : 2.3f + (shares(splits) ? 0.025f : 0.06f) * splits;
+        return 3.4f + (units * splits * 2 > cus ? 1.2f : 1.05f) * iterations * crowd + 0.4f * stream + 4.f * (std::ceil(std::max(per_cu, 2.f) / 2.f) - 1.f) +
+               0.6f * (new_steps - 1) + merge;
     };
-    for (int it = ceil_div(blocks, most); it <= blocks; it = it < 64 ? it + 1 : it * 2) consider(ceil_div(blocks, it), false);
-    // Merged in shares, splits that do not divide the blocks evenly take little more than what they have on average: the last block of some
-    // is behind the others' merge loads.  us per layer, splits of whole iterations / one for each CU: 2 KV heads, one query at 32768
-    // keys 12.8 / 12.3, four at 4096 8.45 / 7.8, at 8192 9.55 / 9.1, at 16384 13.6 / 12.9; on 4 heads at 8192 11.4 / 10.7.
-    consider(std::min(most, blocks), true);
+    // Splits that have the same number of iterations, but for the last ones.  More of them, one for each CU, are faster only where the pool's keys come out
+    // even, at whole multiples of 128 keys per split, which the bound on the length does not tell: us per layer, even splits / one for each CU, 2 KV heads, one query at
+    // 16418 keys 10.2 / 11.5 (at 16384 10.25 / 9.95), at 99003 22.5 / 23.8, two at 9682 9.7 / 10.2 (at 8192 9.55 / 8.75), four at 4216 8.2 / 8.75 (at
+    // 8192 10.75 / 10.1), eight at 2168 8.25 / 8.75; on 8 heads four at 4216 10.35 / 11.4.  Over 44 lengths of 1000 to 131072 keys 1 to 6 % in favour of the even ones.
+    for (int it = ceil_div(blocks, most); it <= blocks; it = it < 64 ? it + 1 : it * 2) {
+        const int splits = ceil_div(blocks, it);
+        const float t = estimate(splits, (float)it);
+        if (t < best) best = t, d.splits = splits;
+    }
+    // Merged in shares, the last block of some splits is behind the others' merge loads: compared with the split shapes, what one for each CU would take on
+    // average is nearer to what is measured (split / direct, 1 KV head, two queries at 59575 keys 21.2 / 17.4, four at 25113 18.8 / 15.5; on 2 heads four at 34498 19.5 /
+    // 18.8, eight at 12806 16.1 / 15.35: whole iterations would leave the direct shape there).
+    const int filling = std::min(most, blocks);
+    if (shares(filling)) best = std::min(best, estimate(filling, (float)blocks / (float)filling + 0.25f));
     const float split_shape = 10.2f + std::min(3.f, span / 2000.f) + stream + 0.02f * T + (split_units > 16 ? 3.f : 0.f) + (rope ? 1.5f : 0.f);
     d.use = options().attn_direct >= 0 ? options().attn_direct != 0 : options().attn_kv_groups == 0 && best < split_shape;
     return d;

@@ -243,3 +243,18 @@ def test_row_major_heads_of_many_rows_take_the_faster_kernel(n, V, H, sliced):
     name, wg = ctypes.create_string_buffer(96), ctypes.c_int(0)
     lib.get().head_plan(n, V, H, 0, name, 96, ctypes.byref(wg))
     assert ("slice_kernel" in name.value.decode()) == sliced, name.value
+
+
+@pytest.mark.parametrize("hkv,T", [(1, 1), (1, 4), (1, 8), (2, 1), (2, 2), (2, 4), (2, 5), (2, 8), (4, 1), (4, 4), (4, 6), (8, 1), (8, 2), (8, 4)])
+def test_direct_splits_have_the_same_number_of_blocks(hkv, T):
+    """No more splits than give each the same number of 128-key blocks, but for the last ones: more of them are slower but for lengths that are whole
+    multiples of 128 keys per split.  (The plan counts 256 CUs where there is no device.)"""
+    from cpm.cu_amd import ops
+    direct = 0
+    for S in [*range(1024, 20000, 128), 32896, 37376, 60032, 65664, 99072]:
+        kernel, splits, _, _ = ops.attention_plan(T, 32, hkv, S)
+        if "direct" in kernel:
+            blocks = -(-S // 128) + 1
+            direct += 1
+            assert splits == -(-blocks // -(-blocks // splits)), S
+    assert direct > 50
