@@ -40,9 +40,6 @@ constexpr int kSlotBytes = kSlotQuads * 16;
 struct DirectSlots {
     uint32_t generation[kDirectSlots];
     u32x4 words[kDirectSlots][kSlotQuads];
-    // the partials of such a launch where nobody is to wait: the last arrival reads them once it has counted all
-    f16 o[kDirectSlots][kDirectRows][kHeadDim];
-    float2 ml[kDirectSlots][kDirectRows];
 };
 static_assert(kThreads == kDirectRows * 32, "the merge: 32 threads per row");
 // The keys of a group of 32 make two operand blocks.  Row m of the K operand of block b of a group is its key direct_key_of_row(m) + 8 b;

@@ -1926,10 +1926,6 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     const dim3 grid(kXcds * ceil_div(nsh, kXcds), p.num_mtiles);
     const bool is_bf16 = options().dtype == 1;
     if (plan.direct) {
-        if (p.num_splits > kDirectLastMerges && counters.slots != nullptr && (int)(grid.x * grid.y) <= kDirectSlots) {
-            p.o_part = (float*)p.slots->o;  // (addresses in device memory)
-            p.ml_part = (float*)p.slots->ml;
-        }
         p.merge_shares = direct_merge == DirectMerge::kMayWait ? direct_merge_shares(p.num_splits, Hkv, (int)(grid.x * grid.y), device_cu_count()) : 0;
         // The appended rows' workgroups are as many as have work.  (As whole grid rows in front, most of them empty, they held up the first tiles.)
         // Where the merge is shared out they come in front, and rounded up so that the tiles keep their XCDs: one of them that starts late ends last.  Else

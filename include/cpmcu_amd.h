@@ -349,8 +349,8 @@ size_t cpmcu_tree_attention_workspace_bytes(int T, int Hq, int Hkv, int max_kv_l
  *   scale: softmax scale (1/sqrt(128) in the reference, flash_api.hpp:360).
  *   workspace: device scratch of at least ..._workspace_bytes(), may be NULL
  *           when that is 0.  Calls that may overlap on one GPU must use different
- *           workspaces: the split partials live there (but for the direct shape's
- *           with 16 splits and more, which the library has memory for), and the library keys the
+ *           workspaces: the split partials live there (those that the direct shape merges
+ *           in shares pass through memory of the library), and the library keys the
  *           arrival counters of the in-launch merge by this pointer (a launch with at
  *           most 32 splits, of the direct shape with 16 to 128, and at most one workgroup
  *           per CU merges its own partials; its workgroups wait for each other, which
