@@ -41,9 +41,10 @@ MFMA_F16_PEAK_TFLOPS = 2500.0
 MEASURED_TRAFFIC = {
     "source": "profiles/verify_step_hbm_traffic.md, profiles/tree_attention_long_context_traffic.md",
     # the library the counters were read on (git rev-parse --short HEAD of that run)
-    "measured_at_commit": "8a0f682 (32768 and 131072: 5ad0aba)",
+    "measured_at_commit": "8a0f682 (merged through memory, 32768 and 131072: 5ad0aba)",
     "kib_per_launch": {
-        "tree_attn_split_kernel<2,false>": 25520 + 9008,  # each head's context through four XCDs; the split partials are merged in their L2s and written back behind the launch
+        "tree_attn_split_kernel<2,false,false>": 15185 + 9463,  # the split partials written through to memory and read back
+        "tree_attn_split_kernel<2,false,true>": 25520 + 9008,  # each head's context through four XCDs; the split partials are merged in their L2s and written back behind the launch
         "head_gemm_stream_kernel<4,2,256>": 591970 + 128,
     },
     # the attention launch at the longer contexts (32 splits of 256-row workgroups), by prefix length
@@ -773,7 +774,7 @@ def main():
         ctx_attn[str(Pc)] = dict(us_per_layer=round(r["ms_attn"] * 1e3, 2), tflops=round(tf, 1), frac_mfma=round(tf / MFMA_F16_PEAK_TFLOPS, 4),
                                  kernel=r["attn_plan"][0], step_minus_attention_us=round((r["ms_step"] - L * r["ms_attn"]) * 1e3, 1))
         kib = MEASURED_TRAFFIC["attention_kib_per_launch_by_context"].get(str(Pc))
-        if kib is not None and r["attn_plan"][0] == "tree_attn_split_kernel<1,false>":
+        if kib is not None and r["attn_plan"][0] == "tree_attn_split_kernel<1,false,false>":
             ctx_attn[str(Pc)]["traffic"] = kib * 1024
             ctx_attn[str(Pc)]["algorithmic_bytes"] = int(bytes_attn(Pc))
         if parity is not None:  # acceptance on the device's arg-max + compacted rows, as for the headline context

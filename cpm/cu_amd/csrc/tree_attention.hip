@@ -1438,13 +1438,14 @@ int device_cu_count() {
     }
     return cus[dev];
 }
+int planned_cu_count() { return device_cu_count() > 0 ? device_cu_count() : 256; }  // (plans are made where there is no device, too)
 
 int choose_splits(int T, int group, int Hkv, int max_kv_len, int G) {
     const int num_mtiles = ceil_div(group * T, rows_per_wg(G));
     const int ntiles = ceil_div(max_kv_len, kTileN);
     // One workgroup per CU.  The grid is (splits x KV heads, padded to a multiple of the XCD count) x M-tiles, and the padding
     // counts: 42 splits of 2 heads on 3 M-tiles are 88 x 3 = 264 workgroups -- too many for the launch to merge itself.
-    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const int cus = planned_cu_count();
     int splits = (cus / num_mtiles / kXcds * kXcds) / Hkv;
     if (splits < 1) splits = 1;
     const bool merge = options().attn_merge_in_launch != 0;
@@ -1498,7 +1499,7 @@ int choose_splits(int T, int group, int Hkv, int max_kv_len, int G) {
 constexpr int kLongRunTiles = 16;
 constexpr int kLongSplitTiles = 170;
 int splits_that_fill(int T, int group, int Hkv, int G) {
-    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const int cus = planned_cu_count();
     const int s = (cus / ceil_div(group * T, rows_per_wg(G)) / kXcds * kXcds) / Hkv;
     return s < 1 ? 1 : s;
 }
@@ -1524,6 +1525,7 @@ struct LaunchPlan {
     bool merge_in_launch;  // the split workgroups merge their own partials (no combine launch)
     int xcd_units;         // split shapes: units per XCD where all splits of a unit are on one, and merged there (0: they are not)
     bool direct;           // the direct shape: num_mtiles counts its 16-row tiles
+    int merge_shares;      // ... direct_merge_shares
 };
 
 // Counters of the in-launch merge.  They live in the library (zero when it is loaded, and back at zero arrivals after
@@ -1541,7 +1543,7 @@ __device__ DirectSlots g_direct_slots[kMergeBlocks];  // of the same workspaces
 bool can_merge_in_launch(int Hkv, int num_mtiles, int num_splits) {
     if (!options().attn_merge_in_launch || num_splits < 2 || num_splits > kMergeMaxSplits) return false;
     if (Hkv * num_mtiles > kMergeUnits) return false;
-    return kXcds * ceil_div(num_splits * Hkv, kXcds) * num_mtiles <= device_cu_count();
+    return kXcds * ceil_div(num_splits * Hkv, kXcds) * num_mtiles <= planned_cu_count();
 }
 
 // Units per XCD of a launch that merges itself, where all splits of a unit are put on one XCD (one workgroup per CU) and their partials change
@@ -1562,8 +1564,8 @@ std::atomic<bool> g_spread_seen[64];
 int units_per_xcd(int Hkv, int num_mtiles, int num_splits, int span) {
     const int units = Hkv * num_mtiles, on_one = ceil_div(units, kXcds);
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 || g_spread_seen[dev]) return 0;
-    if (on_one * num_splits > device_cu_count() / kXcds) return 0;
+    if (hipGetDevice(&dev) == hipSuccess && (dev < 0 || dev >= 64 || g_spread_seen[dev])) return 0;
+    if (on_one * num_splits > planned_cu_count() / kXcds) return 0;
     if (Hkv % kXcds == 0) return on_one;
     if (span > kXcdSpan) return 0;
     if (units % kXcds == 0) return on_one;
@@ -1658,7 +1660,7 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope, bool ma
     const int units = Hkv * tiles, blocks = ceil_div(span, kBlockKeys) + 1;  // (one more for the appended rows)
     const int new_steps = ceil_div(T, 32), split_units = Hkv * ceil_div(tiles * kDirectRows, rows_per_wg(2));
     const float stream = (float)span * Hkv * (2 * kHeadDim * sizeof(f16)) / 5.5e6f;
-    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const int cus = planned_cu_count();
     const int most = std::min(kMaxSplits, std::max(cus / units, std::max(1, std::min(4, 2 * cus / units))));
     DirectPlan d = {1, false};
     float best = 1e30f;
@@ -1701,7 +1703,7 @@ LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_wind
     pl.span = max_kv_len;
     if (window_blocks > 0 && window_blocks * 128 + T < pl.span) pl.span = window_blocks * 128 + T;
     const int tiles = ceil_div(group * T, kDirectRows);
-    pl.xcd_units = 0;
+    pl.xcd_units = pl.merge_shares = 0;
     const DirectPlan direct = choose_direct(T, Hkv, tiles, pl.span, rope, merge == DirectMerge::kMayWait);
     // (a split count asked for is one of the split shapes', unless the direct shape is forced)
     pl.direct = merge != DirectMerge::kNone && direct.use && (num_splits_override == 0 || options().attn_direct == 1);
@@ -1710,8 +1712,12 @@ LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_wind
         pl.num_mtiles = tiles;
         pl.num_splits = num_splits_override > 0 ? num_splits_override : direct.splits;
         pl.merge_in_launch = pl.num_splits > 1;
+        if (merge == DirectMerge::kMayWait)
+            pl.merge_shares = direct_merge_shares(pl.num_splits, Hkv, kXcds * ceil_div(pl.num_splits * Hkv, kXcds) * tiles,
+                                                  planned_cu_count());
         if (pl.num_splits == 1 || (options().attn_merge_in_launch && Hkv * tiles <= kMergeUnits)) return pl;
         pl.direct = false;
+        pl.merge_shares = 0;
     }
     pl.kv_groups = choose_groups(T, group, Hkv, pl.span);
     pl.num_mtiles = ceil_div(group * T, rows_per_wg(pl.kv_groups));
@@ -1732,10 +1738,15 @@ extern "C" int cpmcu_tree_attention_plan(int T, int Hq, int Hkv, int max_kv_len,
                                          int* kv_groups, int* num_workgroups) {
     CPMCU_CHECK_ARG(T >= 1 && T <= kMaxTree && Hkv >= 1 && Hq >= Hkv && Hq % Hkv == 0 && max_kv_len >= T, "tree_attention_plan: bad shape");
     const LaunchPlan pl = plan_launch(T, Hq / Hkv, Hkv, max_kv_len, block_window_size, num_splits_override, with_rope != 0, usual_direct_merge());
-    if (kernel_names && kernel_names_bytes > 0)
-        pl.direct ? snprintf(kernel_names, kernel_names_bytes, "tree_attn_direct_kernel") :
-        snprintf(kernel_names, kernel_names_bytes, "tree_attn_split_kernel<%d,%s>%s", pl.kv_groups, with_rope ? "true" : "false",
-                 pl.num_splits <= 1 || pl.merge_in_launch ? "" : pl.num_splits > kMergeMaxSplits ? "+tree_attn_combine_wide_kernel" : "+tree_attn_combine_kernel");
+    const char* const bf16_name = options().dtype == 1 ? "_bf16" : "";
+    if (kernel_names && kernel_names_bytes > 0 && pl.direct)
+        snprintf(kernel_names, kernel_names_bytes, "tree_attn_direct%s%s_kernel", pl.merge_shares > 0 ? "_shares" : "", bf16_name);
+    else if (kernel_names && kernel_names_bytes > 0) {
+        const int n = snprintf(kernel_names, kernel_names_bytes, "tree_attn_split%s_kernel<%d,%s,%s>", bf16_name, pl.kv_groups, with_rope ? "true" : "false",
+                               pl.xcd_units > 0 ? "true" : "false");
+        if (pl.num_splits > 1 && !pl.merge_in_launch && n > 0 && (size_t)n < kernel_names_bytes)
+            snprintf(kernel_names + n, kernel_names_bytes - n, "+tree_attn_combine%s%s_kernel", pl.num_splits > kMergeMaxSplits ? "_wide" : "", bf16_name);
+    }
     if (num_splits) *num_splits = pl.num_splits;
     if (kv_groups) *kv_groups = pl.kv_groups;
     if (num_workgroups) *num_workgroups = pl.xcd_units > 0 ? kXcds * pl.xcd_units * pl.num_splits : kXcds * ceil_div(pl.num_splits * Hkv, kXcds) * pl.num_mtiles;
@@ -1926,7 +1937,7 @@ static int tree_attention_impl(const void* q, void* k_pool, void* v_pool,
     const dim3 grid(kXcds * ceil_div(nsh, kXcds), p.num_mtiles);
     const bool is_bf16 = options().dtype == 1;
     if (plan.direct) {
-        p.merge_shares = direct_merge == DirectMerge::kMayWait ? direct_merge_shares(p.num_splits, Hkv, (int)(grid.x * grid.y), device_cu_count()) : 0;
+        p.merge_shares = plan.merge_shares;
         // The appended rows' workgroups are as many as have work.  (As whole grid rows in front, most of them empty, they held up the first tiles.)
         // Where the merge is shared out they come in front, and rounded up so that the tiles keep their XCDs: one of them that starts late ends last.  Else
         // they come behind: in front they put two tiles on one CU where there is a CU for each.  us per layer, whole rows / in front / behind: one

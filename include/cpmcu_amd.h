@@ -376,9 +376,15 @@ int cpmcu_tree_attention_merge_mode(const void* workspace);
 int cpmcu_tree_attention_release_workspace(const void* workspace);
 
 /* No reference counterpart: which kernels a cpmcu_tree_attention* call of this shape launches, without
- * launching -- for reports that must name the instantiation actually taken.  kernel_names receives e.g.
- * "tree_attn_split_kernel<2,false>+tree_attn_combine_kernel" (beyond 32 splits: "+tree_attn_combine_wide_kernel") or
- * "tree_attn_direct_kernel" (kv_groups 0); the outputs may each be NULL. */
+ * launching -- for reports that must name the instantiation actually taken.  kernel_names receives, for the element type set,
+ *   "tree_attn_split_kernel<G,rope,xcd>": G KV groups a workgroup, the rotary embedding fused or not, splits merged
+ *       through the L2 of an XCD each or not; with a merge launch "+tree_attn_combine_kernel" behind it, beyond 32 splits
+ *       "+tree_attn_combine_wide_kernel";
+ *   "tree_attn_direct_kernel" (kv_groups 0): one split, or merged by the last workgroup to arrive; "tree_attn_direct_shares_kernel":
+ *       merged in shares;
+ * in bfloat16 "..._bf16_kernel".  num_workgroups leaves out those of the direct shape that write k_new and v_new to the pool.  A
+ * workspace that has no counters, or no longer waits (cpmcu_tree_attention_merge_mode), is launched in the other form.  The
+ * outputs may each be NULL. */
 int cpmcu_tree_attention_plan(int T, int Hq, int Hkv, int max_kv_len, int with_rope, int block_window_size,
                               int num_splits_override, char* kernel_names, size_t kernel_names_bytes, int* num_splits,
                               int* kv_groups, int* num_workgroups);

@@ -258,3 +258,19 @@ def test_direct_splits_have_the_same_number_of_blocks(hkv, T):
             direct += 1
             assert splits == -(-blocks // -(-blocks // splits)), S
     assert direct > 50
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("T,S,rope,splits,name", [
+    (1, 512, False, 0, "tree_attn_direct{}_kernel"), (1, 4224, True, 0, "tree_attn_direct_shares{}_kernel"), (60, 32896, False, 0, "tree_attn_split{}_kernel<1,false,false>"), (60, 4224, True, 0, "tree_attn_split{}_kernel<2,true,true>"),
+    (16, 32896, True, 0, "tree_attn_split{}_kernel<2,true,false>+tree_attn_combine_wide{}_kernel"),
+    (60, 4224, False, 5, "tree_attn_split{}_kernel<2,false,false>+tree_attn_combine{}_kernel"), (60, 4224, False, 1, "tree_attn_split{}_kernel<2,false,false>")])
+def test_plans_name_the_kernels_that_are_launched(set_option, dtype, T, S, rope, splits, name):
+    """Direct or split, merged in shares or by the last arrival, rotary embedding, element type and merge launch, through an XCD's L2 or memory.
+    (The plan counts 256 CUs where there is no device.)"""
+    from cpm.cu_amd import ops
+    set_option("dtype", dtype)
+    if "combine{}_k" in name:
+        set_option("attn_merge_in_launch", 0)
+    kernel, used, _, _ = ops.attention_plan(T, 32, 2, S, rope, num_splits=splits)
+    assert kernel == name.format(*["_bf16" * dtype] * 2) and (not splits or used == splits)

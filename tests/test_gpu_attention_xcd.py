@@ -15,16 +15,21 @@ D = 128
     (4076, 20, 32, 2, 16, 2), (1000, 24, 32, 2, 32, 2), (4560, 48, 32, 2, 16, 2), (2527, 33, 32, 2, 16, 2), (2504, 56, 32, 2, 13, 2), (1300, 40, 16, 1, 32, 2)])
 def test_merge_on_one_xcd_equals_separate_merge(gpu, P, T, hq, hkv, splits, groups):
     """Launches whose units merge through the L2 of an XCD (one to three units on each, full, half empty and idle XCDs, XCDs with units of two heads, the longest context
-    that is numbered for it and the next one, any length on a multiple of 8 KV heads), in both types: the bits of the separate merge launch, also where every wait runs out at
-    once, and in replays."""
+    that is numbered for it, any length on a multiple of 8 KV heads), in both types: the bits of the separate merge launch, also where waits run out at
+    once, and in replays.  The next longer context, and three M-tiles of 4 heads at 4596 keys, are merged through memory.  That the plan is the one meant, that the workspace has counters, and
+    that waits ran out, is asserted: without any of them the bits would be the same."""
     torch = gpu
+    import ctypes
     from cpm.cu_amd import lib, ops
     from cpm.cu_amd.kvcache import PagedKVCache
     L = lib.get()
     option = lambda name, value: L.set_option(name.encode(), int(value))
+    L.synchronize()
+    seen = L.raw.cpmcu_attention_abandoned_waits()
     option("attn_kv_groups", groups)
     option("attn_direct", 0)
     S = P + T
+    on_one_xcd = (P, T, hkv) not in ((4549, 60, 2), (4500, 96, 4))
     g = torch.Generator(device="cuda").manual_seed(S)
     mask = to_dev(torch, synth.random_tree(T, S, max_children=4, max_depth=9).mask)
     kv_len = torch.tensor([S], dtype=torch.int32, device="cuda")
@@ -37,12 +42,13 @@ def test_merge_on_one_xcd_equals_separate_merge(gpu, P, T, hq, hkv, splits, grou
             q = rnd(T, hq, D)
             call = lambda out: ops.tree_attention(q, cache, 0, kv_len, S, mask, num_splits=splits, out=out)
             names, used, _, _ = ops.attention_plan(T, hq, hkv, S, num_splits=splits)
-            assert "combine" not in names and used == splits
+            assert (names, used) == ("tree_attn_split%s_kernel<%d,false,%s>" % ("_bf16" if dtype else "", groups, str(on_one_xcd).lower()), splits)
             option("attn_merge_in_launch", 0)
             ref = call(torch.empty_like(q))
             option("attn_merge_in_launch", 1)
             out = torch.empty_like(q)
             call(out)
+            assert L.raw.cpmcu_tree_attention_merge_mode(ctypes.c_void_p(ops._workspaces["attn", q.device].data_ptr())) == 1
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 for _ in range(2):
@@ -63,6 +69,7 @@ def test_merge_on_one_xcd_equals_separate_merge(gpu, P, T, hq, hkv, splits, grou
         option("attn_merge_wait_us", 2000)
         L.synchronize()
         option("attn_merge_in_launch", 1)
+    assert L.raw.cpmcu_attention_abandoned_waits() > seen
 
 
 @pytest.mark.parametrize("P,T,hq,hkv,splits,groups", [
