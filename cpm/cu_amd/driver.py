@@ -162,6 +162,7 @@ class GraphedSteps:
                 with torch.cuda.graph(g, stream=self.stream):
                     st.enqueue(self.q, self.k_new, self.v_new, self.hidden, self.draft_ids, attn_out=self.attn_out)
             self.graphs[padded] = g
+        self.stream.wait_stream(torch.cuda.current_stream())  # the caller's refills
         with torch.cuda.stream(self.stream):
             self.graphs[padded].replay()
         self.stream.synchronize()

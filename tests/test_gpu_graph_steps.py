@@ -125,6 +125,31 @@ def test_replayed_steps_report_what_their_attention_reports(gpu):
     assert a == len(ids) >= 1 and int(step.cache_length[0]) == want + a
 
 
+def test_replayed_steps_wait_for_the_refills_of_their_buffers(gpu):
+    """Buffers refilled on the caller's stream, which is busy: the replay reads the new hidden rows, whose arg-max is known."""
+    from cpm.cu_amd.driver import GraphedSteps, VerifyStep
+    from cpm.cu_amd.kvcache import PagedKVCache
+    torch = gpu
+    tree = synth.random_tree(T, 1, max_children=3, max_depth=6)
+    mask, parent, pos = [torch.from_numpy(x).cuda() for x in (tree.mask.view(np.int64), tree.parent, tree.positions(P0))]
+    head = torch.zeros((VOCAB, H), dtype=torch.float16, device="cuda")
+    head[torch.arange(VOCAB), torch.arange(VOCAB) % H] = 1  # a hidden row with one entry picks the first row that has it
+    gs = GraphedSteps(VerifyStep(PagedKVCache(1, HKV, 10), head, mask, parent, pos, P0, commit=True), 1, HQ, HKV, H)
+    rows = torch.zeros((4, T, H), dtype=torch.float16, device="cuda")
+    for turn in range(4):
+        rows[turn, :, 100 + turn] = 1
+    gs.draft_ids.fill_(VOCAB - 1)  # (nothing but the root is accepted)
+    gs.run()
+    used = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for turn in range(4):
+        with torch.cuda.stream(used):
+            torch.cuda._sleep(10_000_000)
+            gs.hidden.copy_(rows[turn])
+            a, ids = gs.run()
+        assert (a, ids.tolist()) == (1, [100 + turn])
+
+
 @pytest.mark.parametrize("commit", [False, True])
 def test_step_is_ready_on_every_stream_when_built(gpu, commit):
     """Built on a stream that is busy, read and written on another one without a wait: the lengths are there, and no fill of the
