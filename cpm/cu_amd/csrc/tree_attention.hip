@@ -1770,7 +1770,7 @@ void attention_release_workspace(const void* workspace) {
 // The report words of the current device, read without a round trip of their own: `attention_report_enqueue` puts a copy
 // into pinned host memory in stream order (call it ahead of a synchronisation of that stream, outside any capture),
 // `attention_report_take` looks at that copy afterwards and clears the device words only when something is there.
-// After any abandoned wait nobody waits in the launches of the device's workspaces: the split shapes go back to the combine launch, the
+// After any abandoned wait, or partials that never came, nobody waits in the launches of the device's workspaces: the split shapes go back to the combine launch, the
 // direct one to the merge by the last arrival.
 namespace {
 AttnReport* g_report_host[64] = {nullptr};
@@ -1798,7 +1798,7 @@ int attention_report_take(int* bad_length, unsigned int* abandoned, unsigned int
         CPMCU_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_attn_report), &zero, sizeof(zero)));
         *g_report_host[dev] = zero;
         if (r.spread != 0) g_spread_seen[dev] = true;
-        if (r.abandoned != 0) {
+        if (r.abandoned != 0 || r.lost != 0) {
             std::lock_guard<std::mutex> lock(g_merge_mu);
             for (auto& kv : g_merge_states)
                 if (kv.first.first == dev) kv.second.no_waits = true;

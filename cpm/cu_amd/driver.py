@@ -166,7 +166,11 @@ class GraphedSteps:
         with torch.cuda.stream(self.stream):
             self.graphs[padded].replay()
         self.stream.synchronize()
-        lib.get().synchronize()  # what the attention launches report reaches the host through the library alone
+        try:
+            lib.get().synchronize()  # what the attention launches report reaches the host through the library alone
+        except RuntimeError:
+            self.graphs.clear()  # captured anew: later launches may take another form
+            raise
         a = int(st.packed[0])
         self.prefix_bound += a
         return a, st.packed[1:1 + a].numpy().copy()

@@ -104,8 +104,8 @@ def test_graph_replayed_steps_equal_host_driven_steps(gpu, orc):
 
 
 def test_replayed_steps_report_what_their_attention_reports(gpu):
-    """A length on the device beyond the padded one of the graph (the kernels work on it clamped): the replay raises instead of returning ids, and the step
-    behind it, on a length that fits, is whole again."""
+    """A length on the device beyond the padded one of the graph (the kernels work on it clamped): the replay raises instead of returning ids, its graphs
+    are given up, and the step behind it, on a length that fits, is whole again."""
     from cpm.cu_amd.driver import GraphedSteps, VerifyStep
     from cpm.cu_amd.kvcache import PagedKVCache
     torch = gpu
@@ -118,6 +118,7 @@ def test_replayed_steps_report_what_their_attention_reports(gpu):
     torch.cuda.synchronize()
     with pytest.raises(RuntimeError, match="KV length of 2222"):
         gs.run()
+    assert not gs.graphs
     step.kv_len.copy_(step.cache_length + T)
     want = P0 + a + int(step.packed[0])
     torch.cuda.synchronize()
