@@ -1548,7 +1548,9 @@ bool can_merge_in_launch(int Hkv, int num_mtiles, int num_splits) {
 
 // Units per XCD of a launch that merges itself, where all splits of a unit are put on one XCD (one workgroup per CU) and their partials change
 // hands through its L2: acknowledged there in 0.4 us instead of 1-2, counted and read back without a trip to memory.  0: they are not.
-// With a multiple of 8 KV heads a unit's splits are on one XCD however they are numbered.  With fewer, M-tiles that would share K/V tiles in one L2
+// With a multiple of 8 KV heads a unit's splits are on one XCD however they are numbered.  It pays at any length up to 256 rows a head, beyond them
+// only at short contexts, where the hand-off is what counts (8 heads, 72 nodes 19.5 / 19.1 at 4096 keys, 25.9 / 26.4 at 8192, 44.3 / 44.9 at 20011, 128 nodes 22.8 / 22.2,
+// 31.5 / 32.2 and 54.6 / 55.9; 64 nodes 16.4 / 15.2, 21.3 / 21.2 and 35.6 / 35.5, 33 nodes 20.0 / 19.7 at 8192 and 43.6 / 42.6 at 32768).  With fewer heads, M-tiles that would share K/V tiles in one L2
 // come to lie on several XCDs, each of which fetches its head's whole context (four times the traffic on 2 heads, twice on 4), and
 // with less than a multiple of 8 units XCDs are left idle.  us per layer in replayed graphs, merged through memory / an XCD: 60 nodes on 2 heads 12.4 / 11.4
 // at 1024 keys, 13.3 / 11.9 at 2048, 15.3 / 13.7 at 4096, 17.3 / 17.6 at 6000, 19.2 / 19.2 at 8192, 45.6 / 50.9 at 32768; 32 nodes 14.7 / 13.3 at 4096, 16.8 /
@@ -1559,15 +1561,17 @@ bool can_merge_in_launch(int Hkv, int num_mtiles, int num_splits) {
 // 2304, 13.3 / 13.7 at 3000; 56 nodes 13.3 / 12.3 at 2304, 15.3 / 16.0 at 4400; level on 4 heads at 1536.  One unit on each of six, up to 4096: 20 nodes, 16
 // splits, 12.1 / 11.3 at 2304, 12.8 / 11.9 at 3600, 32 splits 15.3 / 15.7 at 4400.
 constexpr int kXcdSpan = 4608;  // keys
+constexpr int kXcdRows = 256;   // packed rows of a KV head
 // A device on which a synchronisation has found spread units (XcdUnit) is left alone: a spread unit is merged by one workgroup.
 std::atomic<bool> g_spread_seen[64];
-int units_per_xcd(int Hkv, int num_mtiles, int num_splits, int span) {
+int units_per_xcd(int Hkv, int num_mtiles, int num_splits, int rows, int span) {
     const int units = Hkv * num_mtiles, on_one = ceil_div(units, kXcds);
     int dev = 0;
     if (hipGetDevice(&dev) == hipSuccess && (dev < 0 || dev >= 64 || g_spread_seen[dev])) return 0;
     if (on_one * num_splits > planned_cu_count() / kXcds) return 0;
-    if (Hkv % kXcds == 0) return on_one;
+    if (Hkv % kXcds == 0 && rows <= kXcdRows) return on_one;
     if (span > kXcdSpan) return 0;
+    if (Hkv % kXcds == 0) return on_one;
     if (units % kXcds == 0) return on_one;
     if (on_one > 2 || 2 * units <= kXcds * on_one) return 0;
     if (on_one == 1) return span <= 4096 ? 1 : 0;
@@ -1723,7 +1727,7 @@ LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_wind
     pl.num_mtiles = ceil_div(group * T, rows_per_wg(pl.kv_groups));
     pl.num_splits = num_splits_override > 0 ? num_splits_override : choose_splits(T, group, Hkv, pl.span, pl.kv_groups);
     pl.merge_in_launch = can_merge_in_launch(Hkv, pl.num_mtiles, pl.num_splits);
-    if (pl.merge_in_launch) pl.xcd_units = units_per_xcd(Hkv, pl.num_mtiles, pl.num_splits, pl.span);
+    if (pl.merge_in_launch) pl.xcd_units = units_per_xcd(Hkv, pl.num_mtiles, pl.num_splits, group * T, pl.span);
     return pl;
 }
 
