@@ -1637,9 +1637,18 @@ MergeCounters merge_counters_for(const void* workspace, hipStream_t st) {
 // 16 splits are left to the last arrival too where more than half of the CUs pull K/V of four heads or more: the polls are in their way (words / last arrival, 8
 // nodes on 8 heads 10.1 / 9.8 at 3000 keys, 12.4 / 11.6 at 6000, 21.2 / 20.1 at 16384, on 4 13.4 / 12.85 at 8192; on 2 8.4 / 8.7 at 3000, 9.65 / 9.75 at
 // 6000; one query on 8 at 1900 7.35 / 7.85).
-int direct_merge_shares(int num_splits, int Hkv, int workgroups, int cus) {
+bool direct_can_share(int num_splits, int Hkv, int workgroups, int cus) {
     const int by_the_last = kDirectLastMerges + (Hkv >= 4 && 2 * workgroups > cus ? 1 : 0);
-    return num_splits > by_the_last && workgroups <= std::min(cus, kDirectSlots) ? std::min(num_splits, kDirectItems) : 0;
+    return num_splits > by_the_last && workgroups <= std::min(cus, kDirectSlots);
+}
+// Up to 20 splits of more than one block each are left to it too where many rows are polled for: from 160 packed rows of all heads on, 128 on 8 heads (words / last arrival:
+// six nodes on 4 heads, 17 splits, 12.6 / 12.0 at 8192 keys, 19 splits 17.0 / 16.5 at 16384; on 2 12.1 / 11.7 at 8192; eight on 2, 16 splits, 12.8 / 12.3 at 8192; four on 8, 17 splits,
+// 10.4 / 10.2 at 4216, 19 10.7 / 10.4 at 4600; but two on 8, 17 splits, 9.7 / 10.1 at 4216, four on 2 8.2 / 8.3 at 4216, six on 1 1.4 % more by the last arrival); with one block each
+// they have nothing else to do (six on 4 at 2168 7.55 / 7.9).
+int direct_merge_shares(int num_splits, int blocks, int rows, int Hkv, int workgroups, int cus) {
+    if (!direct_can_share(num_splits, Hkv, workgroups, cus)) return 0;
+    if (num_splits <= 20 && blocks > num_splits && Hkv >= 2 && rows >= (Hkv >= kXcds ? 128 : 160)) return 0;
+    return std::min(num_splits, kDirectItems);
 }
 
 // The direct shape or one of the split shapes, and the splits of the direct one: from estimates of both, in us, fitted to a sweep
@@ -1660,8 +1669,9 @@ struct DirectPlan {
     int splits;
     bool use;
 };
+int direct_blocks(int span) { return ceil_div(span, kBlockKeys) + 1; }  // (one more for the appended rows)
 DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope, bool may_wait) {
-    const int units = Hkv * tiles, blocks = ceil_div(span, kBlockKeys) + 1;  // (one more for the appended rows)
+    const int units = Hkv * tiles, blocks = direct_blocks(span);
     const int new_steps = ceil_div(T, 32), split_units = Hkv * ceil_div(tiles * kDirectRows, rows_per_wg(2));
     const float stream = (float)span * Hkv * (2 * kHeadDim * sizeof(f16)) / 5.5e6f;
     const int cus = planned_cu_count();
@@ -1669,7 +1679,7 @@ DirectPlan choose_direct(int T, int Hkv, int tiles, int span, bool rope, bool ma
     DirectPlan d = {1, false};
     float best = 1e30f;
     const auto workgroups_of = [&](int splits) { return kXcds * ceil_div(splits * Hkv, kXcds) * tiles; };
-    const auto shares = [&](int splits) { return may_wait && direct_merge_shares(splits, Hkv, workgroups_of(splits), cus) > 0; };
+    const auto shares = [&](int splits) { return may_wait && direct_can_share(splits, Hkv, workgroups_of(splits), cus); };  // (or as fast by the last arrival)
     const auto estimate = [&](int splits, float iterations) {
         const float per_cu = (float)workgroups_of(splits) / (float)cus;
         const float crowd = per_cu <= 1.f ? 1.f : std::max(per_cu, 1.6f);
@@ -1717,7 +1727,7 @@ LaunchPlan plan_launch(int T, int group, int Hkv, int max_kv_len, int block_wind
         pl.num_splits = num_splits_override > 0 ? num_splits_override : direct.splits;
         pl.merge_in_launch = pl.num_splits > 1;
         if (merge == DirectMerge::kMayWait)
-            pl.merge_shares = direct_merge_shares(pl.num_splits, Hkv, kXcds * ceil_div(pl.num_splits * Hkv, kXcds) * tiles,
+            pl.merge_shares = direct_merge_shares(pl.num_splits, direct_blocks(pl.span), group * T * Hkv, Hkv, kXcds * ceil_div(pl.num_splits * Hkv, kXcds) * tiles,
                                                   planned_cu_count());
         if (pl.num_splits == 1 || (options().attn_merge_in_launch && Hkv * tiles <= kMergeUnits)) return pl;
         pl.direct = false;

@@ -98,8 +98,8 @@ const char* cpmcu_version(void);
  *                           the K-chunked kernel (CPMCU_HEAD_NO_STREAM set);
  *   "attn_merge_in_launch"  1 = the workgroups of a split tree-attention launch merge their own partials when the
  *                           launch fits the GPU's CUs and has at most 32 splits, those of the direct shape always (in
- *                           shares from 16 splits on -- 17 where more than half of the CUs work on four KV heads and
- *                           more -- if the launch fits, else by the last to arrive) (default), 0 = always
+ *                           shares from 16 splits on -- 17 to 21 where many workgroups or rows would poll -- if the
+ *                           launch fits, else by the last to arrive) (default), 0 = always
  *                           the separate merge launch, and the direct shape for launches of one split only
  *                           (CPMCU_ATTN_SEPARATE_MERGE set);
  *   "attn_merge_wait_us"    longest time a workgroup of such a launch waits for the others of its merge before it

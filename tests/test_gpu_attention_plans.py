@@ -45,3 +45,24 @@ def test_plans_beside_their_lines(gpu, S, T, hkv, splits, shape):
         option("attn_direct", -1)
         option("attn_merge_in_launch", 1)
     assert (out.float() - ref.float()).abs().max().item() <= 4.4e-3
+
+
+@pytest.mark.parametrize("S,T,hkv,splits,shares", [
+    (2200, 6, 4, 19, True), (8200, 6, 4, 17, False), (8200, 3, 4, 22, True), (16500, 5, 4, 19, False), (8200, 8, 2, 14, False), (6000, 8, 2, 16, False), (6050, 4, 2, 25, True),
+    (4300, 4, 2, 18, True), (4300, 4, 8, 18, False), (4300, 3, 8, 18, True), (6000, 8, 1, 16, True), (5400, 5, 2, 22, True), (8200, 6, 2, 17, False)])
+def test_merges_of_the_direct_shape_beside_their_lines(gpu, set_option, S, T, hkv, splits, shares):
+    """The splits and the merge are those that the lines say, and both merges have the same partials: two orders of their fp32 sums, rounded to fp16 once."""
+    torch = gpu
+    from cpm.cu_amd import ops
+    from cpm.cu_amd.kvcache import PagedKVCache
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).to(torch.float16)
+    cache = PagedKVCache(1, hkv, (S + 255) // 256)
+    cache.write_logical(0, 0, rnd(S, hkv, D), rnd(S, hkv, D))
+    q, kv_len = rnd(T, 32, D), torch.tensor([S], dtype=torch.int32, device="cuda")
+    assert ops.attention_plan(T, 32, hkv, S)[:2] == ("tree_attn_direct%s_kernel" % ("_shares" if shares else ""), splits)
+    out = ops.tree_attention(q, cache, 0, kv_len, S)
+    set_option("attn_direct", 1)
+    set_option("attn_merge_wait_us", 0)
+    ref = ops.tree_attention(q, cache, 0, kv_len, S, num_splits=splits)
+    assert float((out.float() - ref.float()).abs().max()) <= 2.0 ** -10 * float(ref.float().abs().max())
